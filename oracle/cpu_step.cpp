@@ -260,7 +260,7 @@ struct Problem {
     mcoef.assign(2 * (size_t)op.nmult, 0.0);
     mperm.assign(op.nmult, 0);
     for (int G = 0; G < m.NX * m.NY; ++G)
-      for (int t = 0; t < op.ndof_owner[G]; ++t) mperm[op.owner_base[G] + t] = FH->F.cell_base[G] + t;
+      for (int t = 0; t < op.ndof_owner[G]; ++t) mperm[op.owner_base[G] + t] = FH->F.at(G, t);
     std::vector<double> gx;
     gauss01(k, gx, gw);
     for (int K = 0; K < m.ncellP; ++K)
@@ -432,24 +432,24 @@ struct Problem {
         for (int i = 0; i < 2 * nb; ++i)
           for (int a = 0; a < nb; ++a) acc[a] += B[i * nb + a] * W[(size_t)M * 2 * nb + i];
       }
-      const int pb = F.F.cell_base[R.ci[X] + R.N * R.cj[X]];
-      for (int a = 0; a < nb; ++a) g[pb + a] = acc[a];
+      const size_t gx = R.ci[X] + (size_t)R.N * R.cj[X];
+      for (int a = 0; a < nb; ++a) g[F.F.at(gx, a)] = acc[a];
     }
     F.solve(g, u, z);
 #pragma omp parallel for schedule(static) if (nc >= 1024)
     for (int M = 0; M < nc; ++M) {
       const LdgCellOps& C = O.cell[M];
       std::vector<double> s(2 * nb, 0.0);
-      const int pm = F.F.cell_base[R.ci[M] + R.N * R.cj[M]];
+      const size_t gm = R.ci[M] + (size_t)R.N * R.cj[M];
       for (int i = 0; i < 2 * nb; ++i)
-        for (int a = 0; a < nb; ++a) s[i] += C.Bself[i * nb + a] * u[pm + a];
+        for (int a = 0; a < nb; ++a) s[i] += C.Bself[i * nb + a] * u[F.F.at(gm, a)];
       for (int f = 0; f < 4; ++f) {
         const int X = R.nbr[4 * (size_t)M + f];
         if (X < 0) continue;
-        const int px = F.F.cell_base[R.ci[X] + R.N * R.cj[X]];
+        const size_t gx = R.ci[X] + (size_t)R.N * R.cj[X];
         const double* B = C.Bf.data() + (size_t)f * 2 * nb * nb;
         for (int i = 0; i < 2 * nb; ++i)
-          for (int a = 0; a < nb; ++a) s[i] += B[i * nb + a] * u[px + a];
+          for (int a = 0; a < nb; ++a) s[i] += B[i * nb + a] * u[F.F.at(gx, a)];
       }
       for (int h = 0; h < 2; ++h)
         for (int a = 0; a < nb; ++a) {
@@ -457,7 +457,7 @@ struct Problem {
           for (int r = 0; r < nb; ++r) t += C.Minv[a * nb + r] * s[h * nb + r];
           x[(size_t)h * nc * nb + (size_t)M * nb + a] = W[(size_t)M * 2 * nb + h * nb + a] - mu * t;
         }
-      for (int a = 0; a < nb; ++a) x[2 * (size_t)nc * nb + (size_t)M * nb + a] = u[pm + a];
+      for (int a = 0; a < nb; ++a) x[2 * (size_t)nc * nb + (size_t)M * nb + a] = u[F.F.at(gm, a)];
     }
   }
 

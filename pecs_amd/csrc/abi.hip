@@ -48,7 +48,7 @@ struct FactorDev {
   double nnz = 0.0;
   double tri_bytes = 0.0;      // algorithmic bytes of a forward + backward sweep
   double device_seconds = 0.0, device_flops = 0.0;  // numeric factorisation on the device (0: on the host)
-  std::vector<int> cell_base;  // host copy: grid cell -> permuted base
+  std::vector<int> cell_dof0, perm;  // host copy: grid cell -> its first DoF; DoF -> permuted index
   FactorLevels lv() const {
     return FactorLevels{foff.data(), boff.data(), goff.data(),  xoff.data(),  fw.data(), bw.data(),
                         fm.data(),   bm.data(),   fks.data(),   bks.data(),   froff.data(), broff.data(),
@@ -490,6 +490,26 @@ void tune_factor(pecs_ctx* c, PackedFactor& P, DevFactor& d, int nrhs) {
   rebuild_tiles(P);
 }
 
+// What a level, a stored entry and a front row cost one solve (forward and
+// backward) with nrhs right-hand sides, for the merging of tree levels: three
+// dependent launches per level; 8 bytes per entry and direction at the 4 TB/s
+// a sweep level streams or, with many right-hand sides, 2 flops per entry,
+// right-hand side and direction at the 40 TFLOP/s of the MFMA sweeps; the row's
+// vector entries.  PECS_SOLVE_COST=level,entry,row (seconds) overrides it.
+// Separators of whole cells, levels unmerged -> separators of DoFs, merged:
+// refinement 4, k = 1, 298 -> 165 us per step; refinement 8, k = 2, 4.83 ->
+// 1.63 ms.
+SolveCost solve_cost(int nrhs) {
+  const double nrp = nrhs > 2 ? mfma_rhs_pad(nrhs) : nrhs;
+  SolveCost q;
+  q.level = 16e-6;
+  q.entry = std::max(2 * 8 / 4.0e12, 4 * nrp / 40e12);
+  q.row = nrp * 8 * 8 / 4.0e12;
+  if (const char* e = std::getenv("PECS_SOLVE_COST"); e && std::sscanf(e, "%lf,%lf,%lf", &q.level, &q.entry, &q.row) != 3)
+    throw std::runtime_error("PECS_SOLVE_COST: expected level,entry,row in seconds");
+  return q;
+}
+
 // Factor S and upload the sweep layout.  The numeric factorisation runs on
 // the device (factor_on_device) after a host symbolic phase;
 // PECS_HOST_FACTOR=1 runs it on the host instead (cholesky_factor +
@@ -512,13 +532,14 @@ FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
   auto secs = [](std::chrono::steady_clock::time_point a, std::chrono::steady_clock::time_point b) {
     return std::chrono::duration<double>(b - a).count();
   };
+  const SolveCost cost = solve_cost(nrhs);
   const auto t0 = tnow();
   if (on_host) {
-    SupernodalFactor F = cholesky_factor(S, leaf);
+    SupernodalFactor F = cholesky_factor(S, leaf, cost);
     P = pack_factor(F);
   } else {
     FrontPlan plan;
-    SupernodalFactor F = cholesky_symbolic(S, leaf, plan);
+    SupernodalFactor F = cholesky_symbolic(S, leaf, plan, cost);
     P = pack_layout(F);
     if (trace) std::fprintf(stderr, "[setup] n=%d: symbolic + layout %.3f s\n", P.n, secs(t0, tnow()));
     HIPCHECK(hipMalloc(&dfwd, std::max<int64_t>(P.nvals, 1) * sizeof(double)));
@@ -538,7 +559,8 @@ FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
   }
   D.n = P.n;
   D.nlevels = P.nlevels;
-  D.cell_base = P.cell_base;
+  D.cell_dof0 = P.cell_dof0;
+  D.perm = P.perm;
   D.goff = P.goff;
   D.xoff = P.xoff;
   D.nnz = (double)P.nvals;
@@ -685,9 +707,11 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
   d.table = upload(c, O.table);
   d.stride = O.type_stride;
   d.sigma_nb = upload(c, sigma);
-  std::vector<int> pb(R.ncell);
-  for (int i = 0; i < R.ncell; ++i) pb[i] = F.cell_base[R.ci[i] + (size_t)R.NXg * R.cj[i]];
-  d.perm_base = upload(c, pb);
+  const int nb = O.nb;
+  std::vector<int> pm((size_t)R.ncell * nb);
+  for (int i = 0; i < R.ncell; ++i)
+    std::copy_n(&F.perm[F.cell_dof0[R.ci[i] + (size_t)R.NXg * R.cj[i]]], nb, &pm[(size_t)i * nb]);
+  d.perm = upload(c, pm);
   if (!O.hang.empty()) {  // couplings across hanging faces, by target cell and by row cell
     std::vector<double> blk;
     std::vector<std::vector<std::pair<int, int>>> byx(R.ncell), bym(R.ncell);
@@ -1122,7 +1146,7 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     c->P = to_params(params);
     for (int i = 0; i < B; ++i) c->Pb.push_back(to_params(&params[i]));
     c->k = params->degree;
-    const int leaf = params->leaf_cells > 0 ? params->leaf_cells : 16;
+    const int leaf = params->leaf_cells > 0 ? params->leaf_cells : 4;
     c->mesh = make_solarcell_mesh(mesh->n_refine, to_geo(mesh));
     c->T = std::make_unique<RefTables>(c->k);
     const RefTables& T = *c->T;
@@ -1209,7 +1233,7 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     for (int G = 0; G < m.NX * m.NY; ++G)
       for (int t = 0; t < op.ndof_owner[G]; ++t) {
         owner_of[op.owner_base[G] + t] = G;
-        mperm[op.owner_base[G] + t] = c->FH.cell_base[G] + t;
+        mperm[op.owner_base[G] + t] = c->FH.perm[c->FH.cell_dof0[G] + t];
       }
     gauss01(c->k, gx, gw);
     for (int K = 0; K < m.ncellP; ++K)

@@ -14,80 +14,229 @@ namespace pecs {
 namespace {
 
 struct NDNode {
-  std::vector<int> cells;  // grid cell ids
+  std::vector<int> dofs;  // DoFs in grid order
   std::vector<int> children;
   int parent = -1;
 };
 
+// The couplings of S between single DoFs: neighbours of each DoF (grid-order
+// numbering), from the nonzero entries of S's blocks in either triangle.
+struct DofGraph {
+  std::vector<int> dof0;     // per cell, and the total
+  std::vector<int> cell;     // per DoF
+  std::vector<int64_t> ptr;  // per DoF
+  std::vector<int> adj;
+  int n = 0;
+
+  explicit DofGraph(const BlockSPD& S) {
+    const int NG = S.NXc * S.NYc, no = S.noff();
+    dof0.assign(NG + 1, 0);
+    for (int X = 0; X < NG; ++X) dof0[X + 1] = dof0[X] + S.ndof[X];
+    n = dof0[NG];
+    cell.resize(n);
+    for (int X = 0; X < NG; ++X)
+      for (int d = dof0[X]; d < dof0[X + 1]; ++d) cell[d] = X;
+    std::vector<int> opp(no, -1);  // the opposite offset
+    for (int o = 0; o < no; ++o)
+      for (int q = 0; q < no; ++q)
+        if (S.offi[q] == -S.offi[o] && S.offj[q] == -S.offj[o]) opp[o] = q;
+    ptr.assign((size_t)n + 1, 0);
+    for (int pass = 0; pass < 2; ++pass) {
+#pragma omp parallel for schedule(dynamic, 256)
+      for (int X = 0; X < NG; ++X) {
+        const int nx = S.ndof[X];
+        if (nx == 0) continue;
+        const int xi = X % S.NXc, xj = X / S.NXc;
+        for (int a = 0; a < nx; ++a) {
+          int64_t cnt = 0;
+          const int64_t at = ptr[dof0[X] + a];
+          for (int o = 0; o < no; ++o) {
+            const int yi = xi + S.offi[o], yj = xj + S.offj[o];
+            if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
+            const int Y = yi + S.NXc * yj, ny = S.ndof[Y];
+            const std::vector<double>& B = S.blk[(size_t)X * no + o];
+            static const std::vector<double> none;
+            const std::vector<double>& C = opp[o] >= 0 ? S.blk[(size_t)Y * no + opp[o]] : none;
+            if (ny == 0 || (B.empty() && C.empty())) continue;
+            for (int b = 0; b < ny; ++b) {
+              if (!((!B.empty() && B[(size_t)a * ny + b] != 0.0) || (!C.empty() && C[(size_t)b * nx + a] != 0.0)))
+                continue;
+              if (pass) adj[at + cnt] = dof0[Y] + b;
+              ++cnt;
+            }
+          }
+          if (!pass) ptr[dof0[X] + a + 1] = cnt;
+        }
+      }
+      if (!pass) {
+        for (int d = 0; d < n; ++d) ptr[d + 1] += ptr[d];
+        adj.resize(ptr[n]);
+      }
+    }
+  }
+};
+
 struct NDBuilder {
   const BlockSPD& S;
-  int leaf;
+  const DofGraph& G;
+  int leaf, reach = 0;
   std::vector<NDNode> nodes;  // postorder
-  NDBuilder(const BlockSPD& s, int l) : S(s), leaf(l) {}
+  std::vector<char> taken;    // per DoF: already in a separator
+  // scratch of cover(): per DoF its index on its side of the cut
+  std::vector<int> side;
 
-  // Width of a separator starting at column (row) `mid` of the rectangle
-  // that leaves no coupling between the part before it and the part after
-  // it: the farthest reach past mid of any coupling from a cell before mid.
-  int reach(int i0, int i1, int j0, int j1, int mid, bool vertical) const {
-    const int no = S.noff();
-    int maxo = 0;
-    for (int o = 0; o < no; ++o) maxo = std::max(maxo, std::abs(vertical ? S.offi[o] : S.offj[o]));
-    int w = 1;
-    const int lo = std::max(vertical ? i0 : j0, mid - maxo);
-    for (int t = lo; t < mid; ++t) {
-      const int u0 = vertical ? j0 : i0, u1 = vertical ? j1 : i1;
-      for (int u = u0; u < u1; ++u) {
-        const int xi = vertical ? t : u, xj = vertical ? u : t;
-        const int X = xi + S.NXc * xj;
-        if (S.ndof[X] == 0) continue;
-        for (int o = 0; o < no; ++o) {
-          const int yi = xi + S.offi[o], yj = xj + S.offj[o];
-          if (yi < i0 || yi >= i1 || yj < j0 || yj >= j1) continue;
-          if (S.blk[(size_t)X * no + o].empty() || S.ndof[yi + S.NXc * yj] == 0) continue;
-          const int p = vertical ? yi : yj;
-          if (p >= mid) w = std::max(w, p - mid + 1);
+  NDBuilder(const BlockSPD& s, const DofGraph& g, int l) : S(s), G(g), leaf(l), taken(g.n, 0), side(g.n, -1) {
+    for (int o = 0; o < S.noff(); ++o) reach = std::max({reach, std::abs(S.offi[o]), std::abs(S.offj[o])});
+  }
+
+  // Minimum vertex cover of the couplings between the free DoFs of the
+  // rectangle before and after the cut at column (row) mid: a maximum
+  // matching of the bipartite graph (augmenting paths, a greedy start) and
+  // Koenig's construction.
+  std::vector<int> cover(int i0, int i1, int j0, int j1, int mid, bool vertical) {
+    std::vector<int> L, R;                  // DoFs with a crossing coupling
+    std::vector<int> eptr{0}, e;            // edges of L
+    const int lo = std::max(vertical ? i0 : j0, mid - reach);
+    const int u0 = vertical ? j0 : i0, u1 = vertical ? j1 : i1;
+    for (int u = u0; u < u1; ++u)
+      for (int t = lo; t < mid; ++t) {
+        const int X = vertical ? t + S.NXc * u : u + S.NXc * t;
+        for (int d = G.dof0[X]; d < G.dof0[X + 1]; ++d) {
+          if (taken[d]) continue;
+          const size_t before = e.size();
+          for (int64_t q = G.ptr[d]; q < G.ptr[d + 1]; ++q) {
+            const int v = G.adj[q], Y = G.cell[v], yi = Y % S.NXc, yj = Y / S.NXc;
+            if (taken[v] || (vertical ? yi : yj) < mid || yi < i0 || yi >= i1 || yj < j0 || yj >= j1) continue;
+            if (side[v] < 0) {
+              side[v] = (int)R.size();
+              R.push_back(v);
+            }
+            e.push_back(side[v]);
+          }
+          if (e.size() > before) {
+            L.push_back(d);
+            eptr.push_back((int)e.size());
+          }
+        }
+      }
+    for (int v : R) side[v] = -1;
+    const int nl = (int)L.size(), nr = (int)R.size();
+    std::vector<int> ml(nl, -1), mr(nr, -1);
+    for (int l = 0; l < nl; ++l)
+      for (int q = eptr[l]; q < eptr[l + 1] && ml[l] < 0; ++q)
+        if (mr[e[q]] < 0) {
+          ml[l] = e[q];
+          mr[e[q]] = l;
+        }
+    std::vector<char> seen(nr);
+    std::vector<int> stack, cur(nl);
+    for (bool grew = true; grew;) {  // phases of disjoint augmenting paths
+      grew = false;
+      std::fill(seen.begin(), seen.end(), 0);
+      for (int l = 0; l < nl; ++l) cur[l] = eptr[l];
+      for (int l = 0; l < nl; ++l) {
+        if (ml[l] >= 0) continue;
+        stack.assign(1, l);
+        while (!stack.empty()) {
+          const int x = stack.back();
+          if (cur[x] == eptr[x + 1]) {
+            stack.pop_back();
+            continue;
+          }
+          const int r = e[cur[x]++];
+          if (seen[r]) continue;
+          seen[r] = 1;
+          if (mr[r] >= 0) {
+            stack.push_back(mr[r]);
+            continue;
+          }
+          // free: flip the path on the stack (each entry's edge is cur - 1)
+          for (size_t i = stack.size(); i-- > 0;) {
+            const int y = stack[i];
+            ml[y] = e[cur[y] - 1];
+            mr[ml[y]] = y;
+          }
+          grew = true;
+          break;
         }
       }
     }
-    return w;
+    // Koenig: reachable from the unmatched L by alternating paths
+    std::vector<char> zl(nl, 0), zr(nr, 0);
+    stack.clear();
+    for (int l = 0; l < nl; ++l)
+      if (ml[l] < 0) {
+        zl[l] = 1;
+        stack.push_back(l);
+      }
+    while (!stack.empty()) {
+      const int x = stack.back();
+      stack.pop_back();
+      for (int q = eptr[x]; q < eptr[x + 1]; ++q) {
+        if (zr[e[q]]) continue;
+        zr[e[q]] = 1;
+        const int y = mr[e[q]];
+        if (y >= 0 && !zl[y]) {
+          zl[y] = 1;
+          stack.push_back(y);
+        }
+      }
+    }
+    std::vector<int> c;
+    for (int l = 0; l < nl; ++l)
+      if (!zl[l]) c.push_back(L[l]);
+    for (int r = 0; r < nr; ++r)
+      if (zr[r]) c.push_back(R[r]);
+    // along the cut
+    auto key = [&](int d) {
+      const int X = G.cell[d], i = X % S.NXc, j = X / S.NXc;
+      return vertical ? j : i;
+    };
+    std::sort(c.begin(), c.end(), [&](int a, int b) { return std::make_pair(key(a), a) < std::make_pair(key(b), b); });
+    return c;
+  }
+
+  int push(NDNode&& node) {
+    const int id = (int)nodes.size();
+    for (int k : node.children) nodes[k].parent = id;
+    nodes.push_back(std::move(node));
+    return id;
   }
 
   int build(int i0, int i1, int j0, int j1) {
-    const int ni = i1 - i0, nj = j1 - j0, w0 = S.sep_width > 0 ? S.sep_width : 2;
+    const int ni = i1 - i0, nj = j1 - j0;
     if (ni <= 0 || nj <= 0) return -1;
-    if (ni * nj <= leaf || (ni <= w0 && nj <= w0)) {
-      NDNode n;
+    NDNode node;
+    if (ni * nj <= leaf || (ni == 1 && nj == 1)) {
       for (int j = j0; j < j1; ++j)
-        for (int i = i0; i < i1; ++i) n.cells.push_back(i + S.NXc * j);
-      nodes.push_back(n);
-      return (int)nodes.size() - 1;
+        for (int i = i0; i < i1; ++i)
+          for (int d = G.dof0[i + S.NXc * j]; d < G.dof0[i + S.NXc * j + 1]; ++d)
+            if (!taken[d]) node.dofs.push_back(d);
+      return node.dofs.empty() ? -1 : push(std::move(node));
     }
-    std::vector<int> kids;
-    NDNode sep;
-    if (ni >= nj && ni > w0) {
-      const int mid = i0 + (ni - w0) / 2;
-      const int w = S.sep_width > 0 ? w0 : reach(i0, i1, j0, j1, mid, true);
-      int a = build(i0, mid, j0, j1);
-      int b = build(std::min(mid + w, i1), i1, j0, j1);
-      if (a >= 0) kids.push_back(a);
-      if (b >= 0) kids.push_back(b);
-      for (int j = j0; j < j1; ++j)
-        for (int i = mid; i < std::min(mid + w, i1); ++i) sep.cells.push_back(i + S.NXc * j);
-    } else {
-      const int mid = j0 + (nj - w0) / 2;
-      const int w = S.sep_width > 0 ? w0 : reach(i0, i1, j0, j1, mid, false);
-      int a = build(i0, i1, j0, mid);
-      int b = build(i0, i1, std::min(mid + w, j1), j1);
-      if (a >= 0) kids.push_back(a);
-      if (b >= 0) kids.push_back(b);
-      for (int j = mid; j < std::min(mid + w, j1); ++j)
-        for (int i = i0; i < i1; ++i) sep.cells.push_back(i + S.NXc * j);
+    const bool vertical = ni >= nj;
+    const int mid = vertical ? i0 + ni / 2 : j0 + nj / 2;
+    node.dofs = cover(i0, i1, j0, j1, mid, vertical);
+    for (int d : node.dofs) taken[d] = 1;
+    const int a = vertical ? build(i0, mid, j0, j1) : build(i0, i1, j0, mid);
+    const int b = vertical ? build(mid, i1, j0, j1) : build(i0, i1, mid, j1);
+    if (a >= 0) node.children.push_back(a);
+    if (b >= 0) node.children.push_back(b);
+    if (node.dofs.empty()) {
+      if (node.children.size() < 2) return a >= 0 ? a : b;
+      // uncoupled halves: a node needs DoFs of its own, so it takes the last
+      // one of its second child's subtree root (any set containing a
+      // separator is one)
+      NDNode& r = nodes[b];
+      node.dofs.push_back(r.dofs.back());
+      r.dofs.pop_back();
+      if (r.dofs.empty()) {  // the root held one DoF: this node replaces it
+        for (int k : r.children) node.children.push_back(k);
+        node.children.erase(node.children.begin() + 1);
+        nodes.pop_back();  // b was the last node pushed
+      }
     }
-    sep.children = kids;
-    nodes.push_back(sep);
-    const int id = (int)nodes.size() - 1;
-    for (int k : kids) nodes[k].parent = id;
-    return id;
+    return push(std::move(node));
   }
 };
 
@@ -210,97 +359,160 @@ void lower_inverse(const double* L, int n, int ld, double* X) {
 
 namespace {
 
-// Ordering, supernodes, row structure and levels (no numeric values).
-struct Symbolic {
-  SupernodalFactor F;
-  std::vector<NDNode> nodes;
-  std::vector<int> pos, node_pos0, node_pos1;
-  std::vector<std::vector<int>> structc;
-};
+// Levels of a postordered tree: height above the lowest leaf below.
+std::vector<int> tree_levels(const std::vector<NDNode>& nodes, int& nlevels) {
+  std::vector<int> lv(nodes.size(), 0);
+  nlevels = 0;
+  for (size_t s = 0; s < nodes.size(); ++s) {
+    for (int c : nodes[s].children) lv[s] = std::max(lv[s], lv[c] + 1);
+    nlevels = std::max(nlevels, lv[s] + 1);
+  }
+  return lv;
+}
 
-Symbolic symbolic(const BlockSPD& S, int leaf_cells) {
-  const int NG = S.NXc * S.NYc;
-  const int no = S.noff();
-  NDBuilder nd(S, leaf_cells);
+// Positions of the DoFs in the postordered nodes, and every node's struct
+// rows: the DoFs after the node that it or its descendants couple to
+// (positions, ascending).  Nodes of one level are independent.
+void structure(const DofGraph& G, const std::vector<NDNode>& nodes, std::vector<int>& pos,
+               std::vector<int>& p1, std::vector<std::vector<int>>& st) {
+  const int nn = (int)nodes.size();
+  pos.assign(G.n, -1);
+  p1.assign(nn, 0);
+  int p = 0;
+  for (int s = 0; s < nn; ++s) {
+    for (int d : nodes[s].dofs) pos[d] = p++;
+    p1[s] = p;
+  }
+  int nl = 0;
+  const std::vector<int> lv = tree_levels(nodes, nl);
+  std::vector<std::vector<int>> by(nl);
+  for (int s = 0; s < nn; ++s) by[lv[s]].push_back(s);
+  st.assign(nn, {});
+#pragma omp parallel
+  {
+    std::vector<int> mark(G.n, -1);
+    for (int l = 0; l < nl; ++l) {
+#pragma omp for schedule(dynamic, 4)
+      for (size_t i = 0; i < by[l].size(); ++i) {
+        const int s = by[l][i];
+        std::vector<int>& r = st[s];
+        auto consider = [&](int q) {
+          if (q >= p1[s] && mark[q] != s) {
+            mark[q] = s;
+            r.push_back(q);
+          }
+        };
+        for (int d : nodes[s].dofs)
+          for (int64_t q = G.ptr[d]; q < G.ptr[d + 1]; ++q) consider(pos[G.adj[q]]);
+        for (int c : nodes[s].children)
+          for (int q : st[c]) consider(q);
+        std::sort(r.begin(), r.end());
+      }
+    }
+  }
+}
+
+// Merge runs of adjacent tree levels.  A run [a, b] becomes one level: every
+// node in it whose parent lies above b absorbs its descendants of levels a..b.
+// The runs minimise the sum over levels of cost.level + cost.entry * stored
+// entries + cost.row * front rows, by dynamic programming over the levels.
+std::vector<NDNode> merge_levels(const std::vector<NDNode>& nodes, const std::vector<std::vector<int>>& st,
+                                 const SolveCost& cost) {
+  const int nn = (int)nodes.size();
+  int nl = 0;
+  const std::vector<int> lv = tree_levels(nodes, nl);
+  std::vector<double> best(nl + 1, 0.0);
+  std::vector<int> from(nl + 1, 0);
+  std::vector<std::vector<double>> run(nl, std::vector<double>(nl, 0.0));  // [a][b]
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int a = 0; a < nl; ++a) {
+    std::vector<double> own(nn, 0.0);  // DoFs of levels >= a in the subtree
+    for (int s = 0; s < nn; ++s) {
+      if (lv[s] < a) continue;
+      own[s] += (double)nodes[s].dofs.size();
+      if (nodes[s].parent >= 0) own[nodes[s].parent] += own[s];
+      const int up = nodes[s].parent >= 0 ? lv[nodes[s].parent] : nl;  // s is a run's root for lv <= b < up
+      const double n = own[s], m = (double)st[s].size();
+      const double c = cost.entry * (0.5 * n * (n + 1.0) + m * n) + cost.row * (n + m);
+      for (int b = lv[s]; b < up; ++b) run[a][b] += c;
+    }
+  }
+  for (int b = 0; b < nl; ++b) {
+    best[b + 1] = -1.0;
+    for (int a = 0; a <= b; ++a) {
+      const double c = best[a] + cost.level + run[a][b];
+      if (best[b + 1] < 0 || c < best[b + 1]) {
+        best[b + 1] = c;
+        from[b + 1] = a;
+      }
+    }
+  }
+  std::vector<int> group(nl, 0);
+  for (int b = nl; b > 0; b = from[b])
+    for (int l = from[b]; l < b; ++l) group[l] = b;
+  // roots of the runs, in postorder, with their members' DoFs in postorder
+  std::vector<NDNode> out;
+  std::vector<int> root(nn), id(nn, -1);
+  for (int s = nn; s-- > 0;) {
+    const int pa = nodes[s].parent;
+    root[s] = (pa >= 0 && group[lv[pa]] == group[lv[s]]) ? root[pa] : s;
+  }
+  std::vector<std::vector<int>> members(nn);
+  for (int s = 0; s < nn; ++s) members[root[s]].push_back(s);
+  for (int s = 0; s < nn; ++s) {
+    if (root[s] != s) continue;
+    NDNode m;
+    for (int t : members[s]) {
+      m.dofs.insert(m.dofs.end(), nodes[t].dofs.begin(), nodes[t].dofs.end());
+      for (int c : nodes[t].children)
+        if (root[c] == c) m.children.push_back(id[c]);
+    }
+    id[s] = (int)out.size();
+    for (int c : m.children) out[c].parent = id[s];
+    out.push_back(std::move(m));
+  }
+  return out;
+}
+
+// Ordering, supernodes, row structure and levels (no numeric values).
+SupernodalFactor symbolic(const BlockSPD& S, const DofGraph& G, int leaf_cells, const SolveCost& cost) {
+  NDBuilder nd(S, G, leaf_cells);
   nd.build(0, S.NXc, 0, S.NYc);
-  const int nn = (int)nd.nodes.size();
-  Symbolic Y;
-  SupernodalFactor& F = Y.F;
-  // cell positions and DoF bases
-  std::vector<int> pos(NG, -1), node_of(NG, -1);
-  std::vector<int> node_pos0(nn), node_pos1(nn);
-  F.cell_base.assign(NG, 0);
-  int p = 0, d = 0;
-  F.nodes.resize(nn);
-  for (int s = 0; s < nn; ++s) {
-    node_pos0[s] = p;
-    F.nodes[s].p0 = d;
-    for (int c : nd.nodes[s].cells) {
-      pos[c] = p++;
-      node_of[c] = s;
-      F.cell_base[c] = d;
-      d += S.ndof[c];
-    }
-    node_pos1[s] = p;
-    F.nodes[s].ns = d - F.nodes[s].p0;
-    F.nodes[s].parent = nd.nodes[s].parent;
+  std::vector<NDNode> nodes = std::move(nd.nodes);
+  SupernodalFactor F;
+  std::vector<int> p1;
+  std::vector<std::vector<int>> st;
+  structure(G, nodes, F.perm, p1, st);
+  if (cost.level > 0) {
+    nodes = merge_levels(nodes, st, cost);
+    structure(G, nodes, F.perm, p1, st);
   }
-  F.n = d;
-  // symbolic: struct cells per node (sorted by position)
-  std::vector<std::vector<int>> structc(nn);
-  std::vector<int> mark(NG, -1);
-  for (int s = 0; s < nn; ++s) {
-    std::vector<int> st;
-    auto consider = [&](int c) {
-      if (pos[c] >= node_pos1[s] && mark[c] != s) {
-        mark[c] = s;
-        st.push_back(c);
-      }
-    };
-    for (int X : nd.nodes[s].cells) {
-      const int xi = X % S.NXc, xj = X / S.NXc;
-      for (int o = 0; o < no; ++o) {
-        const int yi = xi + S.offi[o], yj = xj + S.offj[o];
-        if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
-        const int Y = yi + S.NXc * yj;
-        if (S.blk[(size_t)X * no + o].empty() || S.ndof[Y] == 0) continue;
-        consider(Y);
-      }
-    }
-    for (int c : nd.nodes[s].children)
-      for (int Y : structc[c]) consider(Y);
-    std::sort(st.begin(), st.end(), [&](int a, int b) { return pos[a] < pos[b]; });
-    structc[s] = st;
-  }
-  // levels (height in the elimination tree)
-  for (int s = 0; s < nn; ++s) {
-    int lv = 0;
-    for (int c : nd.nodes[s].children) lv = std::max(lv, F.nodes[c].level + 1);
-    F.nodes[s].level = lv;
-    F.nlevels = std::max(F.nlevels, lv + 1);
-  }
+  const int nn = (int)nodes.size();
+  F.n = G.n;
+  F.cell_dof0.assign(G.dof0.begin(), G.dof0.end() - 1);
+  const std::vector<int> lv = tree_levels(nodes, F.nlevels);
   F.level_nodes.assign(F.nlevels, {});
-  for (int s = 0; s < nn; ++s) F.level_nodes[F.nodes[s].level].push_back(s);
-  // offsets
+  F.nodes.resize(nn);
+  F.children.resize(nn);
   int64_t linv = 0, l21 = 0, rows = 0;
   for (int s = 0; s < nn; ++s) {
     SNode& N = F.nodes[s];
-    int ms = 0;
-    for (int c : structc[s]) ms += S.ndof[c];
-    N.ms = ms;
+    N.ns = (int)nodes[s].dofs.size();
+    N.p0 = p1[s] - N.ns;
+    N.ms = (int)st[s].size();
+    N.parent = nodes[s].parent;
+    N.level = lv[s];
+    F.level_nodes[lv[s]].push_back(s);
+    F.children[s] = nodes[s].children;
     N.linv_off = linv;
     N.l21_off = l21;
     N.rows_off = rows;
     linv += (int64_t)N.ns * N.ns;
-    l21 += (int64_t)ms * N.ns;
-    rows += ms;
+    l21 += (int64_t)N.ms * N.ns;
+    rows += N.ms;
   }
-  F.rows.assign(rows, 0);
-  for (int s = 0; s < nn; ++s) {
-    int t = 0;
-    for (int c : structc[s])
-      for (int a = 0; a < S.ndof[c]; ++a) F.rows[F.nodes[s].rows_off + t++] = F.cell_base[c] + a;
-  }
+  F.rows.resize(rows);
+  for (int s = 0; s < nn; ++s) std::copy(st[s].begin(), st[s].end(), F.rows.begin() + F.nodes[s].rows_off);
   F.linv_size = linv;
   F.l21_size = l21;
   // forward contribution lists
@@ -319,39 +531,49 @@ Symbolic symbolic(const BlockSPD& S, int leaf_cells) {
       F.contrib_row[fill[pp]] = r;
       fill[pp]++;
     }
-  Y.nodes = nd.nodes;
-  Y.pos = pos;
-  Y.node_pos0 = node_pos0;
-  Y.node_pos1 = node_pos1;
-  Y.structc = structc;
-  return Y;
+  return F;
+}
+
+// Positions of child c's struct rows in its parent's front (own rows, then
+// struct rows; both lists ascend).
+std::vector<int> child_map(const SupernodalFactor& F, int c) {
+  const SNode& C = F.nodes[c];
+  const SNode& N = F.nodes[C.parent];
+  std::vector<int> m(C.ms);
+  int j = 0;
+  for (int r = 0; r < C.ms; ++r) {
+    const int q = F.rows[C.rows_off + r];
+    if (q < N.p0 + N.ns) {
+      m[r] = q - N.p0;
+    } else {
+      while (j < N.ms && F.rows[N.rows_off + j] < q) ++j;
+      if (j == N.ms || F.rows[N.rows_off + j] != q) throw std::runtime_error("child_map: a child row is not in the parent");
+      m[r] = N.ns + j;
+    }
+    if (m[r] < 0) throw std::runtime_error("child_map: a child row precedes the parent");
+  }
+  return m;
 }
 
 }  // namespace
 
-SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
-  const int NG = S.NXc * S.NYc;
+SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveCost& cost) {
   const int no = S.noff();
-  Symbolic Y = symbolic(S, leaf_cells);
-  SupernodalFactor& F = Y.F;
+  const DofGraph G(S);
+  SupernodalFactor F = symbolic(S, G, leaf_cells, cost);
   const int nn = (int)F.nodes.size();
-  const auto& pos = Y.pos;
-  const auto& node_pos0 = Y.node_pos0;
-  const auto& node_pos1 = Y.node_pos1;
-  const auto& structc = Y.structc;
-  struct {
-    const std::vector<NDNode>& nodes;
-  } nd{Y.nodes};
+  std::vector<int> dof_at(F.n);  // permuted index -> DoF
+  for (int d = 0; d < F.n; ++d) dof_at[F.perm[d]] = d;
   F.Linv.assign(F.linv_size, 0.0);
   F.L21.assign(F.l21_size, 0.0);
   // numeric multifrontal factorisation, level by level on the elimination tree:
   // nodes of one level are independent (their children are in lower levels).
   std::vector<std::vector<double>> upd(nn);
   const int nthreads = omp_get_max_threads();
-  std::vector<std::vector<int>> front_off_t(nthreads, std::vector<int>(NG, -1));
+  std::vector<std::vector<int>> loc_t(nthreads, std::vector<int>(F.n, -1));
   std::vector<double> flops_t(nthreads, 0.0), ta_t(nthreads, 0.0), tf_t(nthreads, 0.0), ti_t(nthreads, 0.0);
   auto process = [&](int s, int tid) {
-    std::vector<int>& front_off = front_off_t[tid];
+    std::vector<int>& loc = loc_t[tid];  // permuted index -> struct row of this front
     const SNode& N = F.nodes[s];
     const int ns = N.ns, ms = N.ms, nf = ns + ms;
     const bool big = nf > 1024;
@@ -359,47 +581,31 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
     std::vector<double> Fr((size_t)nf * nf);
 #pragma omp parallel for schedule(static) if (big)
     for (int r = 0; r < nf; ++r) std::fill(&Fr[(size_t)r * nf], &Fr[(size_t)r * nf] + r + 1, 0.0);
-    int off = 0;
-    for (int c : nd.nodes[s].cells) {
-      front_off[c] = off;
-      off += S.ndof[c];
-    }
-    for (int c : structc[s]) {
-      front_off[c] = off;
-      off += S.ndof[c];
-    }
-    // original entries: each symmetric block pair once, by the earlier cell's node
-    for (int X : nd.nodes[s].cells) {
-      const int nx = S.ndof[X];
-      if (nx == 0) continue;
+    for (int r = 0; r < ms; ++r) loc[F.rows[N.rows_off + r]] = ns + r;
+    // original entries (p, q), p own and p <= q, into column p
+    for (int c = 0; c < ns; ++c) {
+      const int d = dof_at[N.p0 + c], X = G.cell[d], a = d - G.dof0[X];
       const int xi = X % S.NXc, xj = X / S.NXc;
-      const int rx = front_off[X];
       for (int o = 0; o < no; ++o) {
         const int yi = xi + S.offi[o], yj = xj + S.offj[o];
         if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
-        const int Y = yi + S.NXc * yj;
+        const int Y = yi + S.NXc * yj, ny = S.ndof[Y];
         const auto& B = S.blk[(size_t)X * no + o];
-        if (B.empty() || S.ndof[Y] == 0) continue;
-        const int ny = S.ndof[Y];
-        if (pos[Y] < node_pos0[s]) continue;
-        const int ry = front_off[Y];
-        if (pos[Y] < node_pos1[s]) {
-          for (int a = 0; a < nx; ++a)
-            for (int b = 0; b < ny; ++b)
-              if (rx + a >= ry + b) Fr[(size_t)(rx + a) * nf + ry + b] += B[(size_t)a * ny + b];
-        } else {
-          for (int a = 0; a < nx; ++a)
-            for (int b = 0; b < ny; ++b) Fr[(size_t)(ry + b) * nf + rx + a] += B[(size_t)a * ny + b];
+        if (B.empty()) continue;
+        for (int b = 0; b < ny; ++b) {
+          const double v = B[(size_t)a * ny + b];
+          const int q = F.perm[G.dof0[Y] + b];
+          if (v == 0.0 || q < N.p0 + c) continue;
+          const int r = q < N.p0 + ns ? q - N.p0 : loc[q];
+          Fr[(size_t)r * nf + c] += v;
         }
       }
     }
+    for (int r = 0; r < ms; ++r) loc[F.rows[N.rows_off + r]] = -1;
     // extend-add children
-    for (int c : nd.nodes[s].children) {
+    for (int c : F.children[s]) {
       const int mc = F.nodes[c].ms;
-      std::vector<int> map(mc);
-      int t = 0;
-      for (int Y : structc[c])
-        for (int a = 0; a < S.ndof[Y]; ++a) map[t++] = front_off[Y] + a;
+      const std::vector<int> map = child_map(F, c);
       const std::vector<double>& U = upd[c];
 #pragma omp parallel for schedule(dynamic, 64) if (big)
       for (int r = 0; r < mc; ++r) {
@@ -409,8 +615,6 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
       }
       std::vector<double>().swap(upd[c]);
     }
-    for (int c : nd.nodes[s].cells) front_off[c] = -1;
-    for (int c : structc[s]) front_off[c] = -1;
     auto tB = std::chrono::steady_clock::now();
     if (ns > 0) partial_cholesky(Fr.data(), nf, ns, flops_t[tid]);
     flops_t[tid] += (double)ns * ns * ns / 3.0;
@@ -449,30 +653,38 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
   return F;
 }
 
-SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan) {
+SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost) {
   const int no = S.noff();
-  Symbolic Y = symbolic(S, leaf_cells);
-  SupernodalFactor& F = Y.F;
+  const DofGraph G(S);
+  SupernodalFactor F = symbolic(S, G, leaf_cells, cost);
   const int nn = (int)F.nodes.size();
   const int NG = S.NXc * S.NYc;
   plan = FrontPlan{};
   plan.nlevels = F.nlevels;
   // S blocks, concatenated
-  plan.sblk_off.assign((size_t)NG * no, -1);
+  std::vector<const std::vector<double>*> blocks;
   int64_t sv = 0;
   for (int X = 0; X < NG; ++X)
     for (int o = 0; o < no; ++o) {
       const auto& B = S.blk[(size_t)X * no + o];
       if (B.empty()) continue;
-      plan.sblk_off[(size_t)X * no + o] = sv;
+      const int Y = X + S.offi[o] + S.NXc * S.offj[o];
+      if (S.ndof[X] == 0 || S.ndof[Y] == 0) continue;
+      blocks.push_back(&B);
+      plan.sb_src.push_back(sv);
+      plan.sb_x.push_back(G.dof0[X]);
+      plan.sb_y.push_back(G.dof0[Y]);
+      plan.sb_nx.push_back(S.ndof[X]);
+      plan.sb_ny.push_back(S.ndof[Y]);
       sv += (int64_t)B.size();
     }
   plan.svals.resize(sv);
-  for (int X = 0; X < NG; ++X)
-    for (int o = 0; o < no; ++o) {
-      const int64_t off = plan.sblk_off[(size_t)X * no + o];
-      if (off >= 0) std::copy(S.blk[(size_t)X * no + o].begin(), S.blk[(size_t)X * no + o].end(), &plan.svals[off]);
-    }
+#pragma omp parallel for schedule(static)
+  for (size_t i = 0; i < blocks.size(); ++i)
+    std::copy(blocks[i]->begin(), blocks[i]->end(), &plan.svals[plan.sb_src[i]]);
+  plan.node_of.resize(F.n);
+  for (int s = 0; s < nn; ++s)
+    std::fill_n(plan.node_of.begin() + F.nodes[s].p0, F.nodes[s].ns, s);
   // fronts, level by level (each level's fronts contiguous)
   plan.front_off.assign(nn, 0);
   plan.level_front.assign(F.nlevels + 1, 0);
@@ -487,70 +699,27 @@ SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan&
   }
   plan.level_front[F.nlevels] = fo;
   plan.front_total = fo;
-  // local front position of each cell of a node's front (own cells, then struct)
-  std::vector<int> loc(NG, -1);
-  plan.sc_level.assign(F.nlevels + 1, 0);
-  plan.ea_level.assign(2 * F.nlevels + 1, 0);
+  // child row maps into the parent's front
   plan.ea_map_off.assign(nn + 1, 0);
-  // child row maps into the parent's front, per child (ms entries)
-  std::vector<std::vector<int>> cmap(nn);
-  for (int l = 0; l < F.nlevels; ++l) {
-    plan.sc_level[l] = (int)plan.sc_src.size();
-    for (int s : F.level_nodes[l]) {
-      const int nf = F.nodes[s].ns + F.nodes[s].ms;
-      int off = 0;
-      for (int c : Y.nodes[s].cells) {
-        loc[c] = off;
-        off += S.ndof[c];
-      }
-      for (int c : Y.structc[s]) {
-        loc[c] = off;
-        off += S.ndof[c];
-      }
-      for (int X : Y.nodes[s].cells) {
-        const int nx = S.ndof[X];
-        if (nx == 0) continue;
-        const int xi = X % S.NXc, xj = X / S.NXc;
-        for (int o = 0; o < no; ++o) {
-          const int yi = xi + S.offi[o], yj = xj + S.offj[o];
-          if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
-          const int Yc = yi + S.NXc * yj;
-          const int64_t so = plan.sblk_off[(size_t)X * no + o];
-          if (so < 0 || S.ndof[Yc] == 0) continue;
-          if (Y.pos[Yc] < Y.node_pos0[s]) continue;
-          const bool own = Y.pos[Yc] < Y.node_pos1[s];
-          const int rx = loc[X], ry = loc[Yc];
-          plan.sc_src.push_back(so);
-          plan.sc_dst.push_back(plan.front_off[s] + (own ? (int64_t)rx * nf + ry : (int64_t)ry * nf + rx));
-          plan.sc_nx.push_back(nx);
-          plan.sc_ny.push_back(S.ndof[Yc]);
-          plan.sc_nf.push_back(nf);
-          plan.sc_mode.push_back(own ? 0 : 1);
-          plan.sc_rx.push_back(rx);
-          plan.sc_ry.push_back(ry);
-        }
-      }
-      for (int c : Y.nodes[s].children) {
-        std::vector<int>& m = cmap[c];
-        m.clear();
-        for (int Yc : Y.structc[c])
-          for (int a = 0; a < S.ndof[Yc]; ++a) m.push_back(loc[Yc] + a);
-      }
-      for (int c : Y.nodes[s].cells) loc[c] = -1;
-      for (int c : Y.structc[s]) loc[c] = -1;
-    }
-  }
-  plan.sc_level[F.nlevels] = (int)plan.sc_src.size();
-  for (int s = 0; s < nn; ++s) plan.ea_map_off[s + 1] = plan.ea_map_off[s] + (int64_t)cmap[s].size();
+  for (int s = 0; s < nn; ++s)
+    plan.ea_map_off[s + 1] = plan.ea_map_off[s] + (F.nodes[s].parent >= 0 ? F.nodes[s].ms : 0);
   plan.ea_map.resize(plan.ea_map_off[nn]);
-  for (int s = 0; s < nn; ++s) std::copy(cmap[s].begin(), cmap[s].end(), &plan.ea_map[plan.ea_map_off[s]]);
-  // extend-add rows, per parent level and pass (child 0, then child 1 of every parent)
+  for (int s = 0; s < nn; ++s) {
+    if (F.nodes[s].parent < 0) continue;
+    const std::vector<int> m = child_map(F, s);
+    std::copy(m.begin(), m.end(), plan.ea_map.begin() + plan.ea_map_off[s]);
+  }
+  // extend-add rows, per parent level and pass (child i of every parent)
+  size_t kids = 0;
+  for (int s = 0; s < nn; ++s) kids = std::max(kids, F.children[s].size());
+  plan.npass = (int)kids;
+  plan.ea_level.assign((size_t)plan.npass * F.nlevels + 1, 0);
   for (int l = 0; l < F.nlevels; ++l)
-    for (int pass = 0; pass < 2; ++pass) {
-      plan.ea_level[2 * l + pass] = (int)plan.ea_child.size();
+    for (int pass = 0; pass < plan.npass; ++pass) {
+      plan.ea_level[(size_t)plan.npass * l + pass] = (int)plan.ea_child.size();
       for (int s : F.level_nodes[l]) {
-        if ((int)Y.nodes[s].children.size() <= pass) continue;
-        const int c = Y.nodes[s].children[pass];
+        if ((int)F.children[s].size() <= pass) continue;
+        const int c = F.children[s][pass];
         for (int r = 0; r < F.nodes[c].ms; ++r) {
           plan.ea_child.push_back(c);
           plan.ea_row.push_back(r);
@@ -558,9 +727,7 @@ SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan&
         }
       }
     }
-  plan.ea_level[2 * F.nlevels] = (int)plan.ea_child.size();
-  for (int s = 0; s < nn; ++s)
-    if (Y.nodes[s].children.size() > 2) throw std::runtime_error("cholesky_symbolic: more than two children");
+  plan.ea_level[(size_t)plan.npass * F.nlevels] = (int)plan.ea_child.size();
   return F;
 }
 
@@ -571,22 +738,27 @@ void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::ve
   Linv.assign(F.linv_size, 0.0);
   L21.assign(F.l21_size, 0.0);
   double flops = 0.0;
-  for (int l = 0; l < F.nlevels; ++l) {
-    for (int i = plan.sc_level[l]; i < plan.sc_level[l + 1]; ++i) {
-      const int nx = plan.sc_nx[i], ny = plan.sc_ny[i], nf = plan.sc_nf[i];
-      for (int a = 0; a < nx; ++a)
-        for (int b = 0; b < ny; ++b) {
-          const double v = plan.svals.at(plan.sc_src[i] + (int64_t)a * ny + b);
-          if (plan.sc_mode[i] == 0) {
-            if (plan.sc_rx[i] + a < plan.sc_ry[i] + b) continue;
-            fr.at(plan.sc_dst[i] + (int64_t)a * nf + b) += v;
-          } else {
-            fr.at(plan.sc_dst[i] + (int64_t)b * nf + a) += v;
-          }
+  for (size_t i = 0; i < plan.sb_src.size(); ++i)
+    for (int a = 0; a < plan.sb_nx[i]; ++a)
+      for (int b = 0; b < plan.sb_ny[i]; ++b) {
+        const double v = plan.svals.at(plan.sb_src[i] + (int64_t)a * plan.sb_ny[i] + b);
+        const int p = F.perm[plan.sb_x[i] + a], q = F.perm[plan.sb_y[i] + b];
+        if (v == 0.0 || q < p) continue;
+        const int s = plan.node_of[p];
+        const SNode& N = F.nodes[s];
+        int r = q - N.p0;
+        if (r >= N.ns) {
+          const auto it = std::lower_bound(F.rows.begin() + N.rows_off, F.rows.begin() + N.rows_off + N.ms, q);
+          if (it == F.rows.begin() + N.rows_off + N.ms || *it != q)
+            throw std::runtime_error("execute_plan_host: an entry outside its front");
+          r = N.ns + (int)(it - F.rows.begin() - N.rows_off);
         }
-    }
-    for (int pass = 0; pass < 2; ++pass)
-      for (int i = plan.ea_level[2 * l + pass]; i < plan.ea_level[2 * l + pass + 1]; ++i) {
+        fr.at(plan.front_off[s] + (int64_t)r * (N.ns + N.ms) + (p - N.p0)) += v;
+      }
+  for (int l = 0; l < F.nlevels; ++l) {
+    for (int pass = 0; pass < plan.npass; ++pass)
+      for (int i = plan.ea_level[(size_t)plan.npass * l + pass]; i < plan.ea_level[(size_t)plan.npass * l + pass + 1];
+           ++i) {
         const int c = plan.ea_child[i], r = plan.ea_row[i], s = plan.ea_parent[i];
         const int nsc = F.nodes[c].ns, nfc = nsc + F.nodes[c].ms, nfp = F.nodes[s].ns + F.nodes[s].ms;
         const int* m = &plan.ea_map[plan.ea_map_off[c]];
@@ -614,7 +786,8 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
   const int nn = (int)F.nodes.size();
   P.n = F.n;
   P.nlevels = F.nlevels;
-  P.cell_base = F.cell_base;
+  P.cell_dof0 = F.cell_dof0;
+  P.perm = F.perm;
   P.p0.resize(nn);
   P.ns.resize(nn);
   P.ms.resize(nn);

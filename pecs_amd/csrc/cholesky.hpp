@@ -5,11 +5,24 @@
 // once by SolarCellProblem::set_solvers (SolarCell.cpp:1733-1747).  Here the
 // factored matrices are the SPD density Schur complements and the SPD Poisson
 // multiplier matrix (ops.hpp), ordered by geometric nested dissection on the
-// logically Cartesian cell grid (separators of `sep_width` cell columns/rows),
-// factored by a multifrontal method.  The factor is stored per supernode as
-// the explicit inverse of its diagonal block plus its off-diagonal panel, so
-// every per-step triangular solve is a sequence of dense matrix-vector
-// products scheduled level by level on the elimination tree.
+// logically Cartesian cell grid, factored by a multifrontal method.  The
+// factor is stored per supernode as the explicit inverse of its diagonal block
+// plus its off-diagonal panel, so every per-step triangular solve is a
+// sequence of dense matrix-vector products scheduled level by level on the
+// elimination tree.
+//
+// Separators are sets of DoFs, not of cells.  A cut between two columns (rows)
+// of cells is closed by a minimum vertex cover of the couplings that cross it.
+// For the LDG Schur complement these are the face-trace DoFs on the two sides
+// of the cut, 2 (k + 1) per cell of its length where whole cells to the reach
+// of the couplings would be 2 (k + 1)^2; for the multipliers the cut's own
+// faces, k where an owner cell holds 2 k.  The dense blocks of the large
+// separators shrink with the square: refinement 8, k = 2 stores 135 M entries
+// per Schur factor with leaves of 16 cells instead of 645 M.
+//
+// Adjacent tree levels are then merged where a launch costs more than the
+// entries the merge adds (merge_levels): each node of the merged range absorbs
+// its descendants in it into one dense block.
 #pragma once
 #include <cstdint>
 #include <vector>
@@ -25,13 +38,15 @@ struct SNode {
 
 struct SupernodalFactor {
   int n = 0;
-  std::vector<int> cell_base;      // per grid cell: permuted index of its first DoF
+  std::vector<int> cell_dof0;      // per grid cell: its first DoF, cells in grid order
+  std::vector<int> perm;           // per DoF (grid order): its permuted index
   std::vector<SNode> nodes;        // postorder
-  std::vector<int> rows;           // per node: ms permuted row indices (struct)
+  std::vector<int> rows;           // per node: ms permuted row indices (struct), ascending
   std::vector<double> Linv;        // per node: ns x ns row-major, lower triangular
   std::vector<double> L21;         // per node: ms x ns row-major
   int nlevels = 0;
   std::vector<std::vector<int>> level_nodes;
+  std::vector<std::vector<int>> children;  // per node
   // forward contributions: for each permuted row p the (node, panel row) pairs
   std::vector<int64_t> contrib_ptr;
   std::vector<int> contrib_node, contrib_row;
@@ -39,31 +54,40 @@ struct SupernodalFactor {
   double flops = 0.0;
   double t_assemble = 0.0, t_factor = 0.0, t_inverse = 0.0;
   int64_t nnz_L() const { return (int64_t)Linv.size() + (int64_t)L21.size(); }
+  int at(size_t cell, int a) const { return perm[(size_t)cell_dof0[cell] + a]; }
 };
 
-SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells);
+// Cost of a triangular solve (forward + backward) as merge_levels weighs it:
+// seconds per tree level, per stored factor entry and per front row.  All
+// zero: levels are not merged.
+struct SolveCost {
+  double level = 0.0, entry = 0.0, row = 0.0;
+};
+
+SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveCost& cost = {});
 
 // Index plan of the multifrontal factorisation for execution on the device:
 // each node's dense nf x nf row-major front (nf = ns + ms; fronts of one level
-// contiguous), the S blocks scattered into the fronts (mode 0: own-own block,
-// lower triangle kept; mode 1: block of a panel row, stored transposed), and
-// the extend-add rows (child c's update row r into its parent's front through
-// the child's row map), in two passes per level (first, then second child).
+// contiguous), the S blocks (every entry (p, q), p <= q in permuted order, goes
+// to column p of the front of the node that owns p), and the extend-add rows
+// (child c's update row r into its parent's front through the child's row
+// map), in `npass` passes per level (pass i: every parent's i-th child).
 struct FrontPlan {
-  int nlevels = 0;
+  int nlevels = 0, npass = 0;
   std::vector<int64_t> front_off, level_front;  // per node; per level [begin, end)
   int64_t front_total = 0;
   std::vector<double> svals;                    // S blocks concatenated
-  std::vector<int64_t> sblk_off;                // per (cell, offset): block offset or -1
-  std::vector<int64_t> sc_src, sc_dst;          // scatter items
-  std::vector<int> sc_nx, sc_ny, sc_nf, sc_mode, sc_rx, sc_ry, sc_level;
+  // per nonempty block: values offset, first DoF and count of its rows / columns
+  std::vector<int64_t> sb_src;
+  std::vector<int> sb_x, sb_y, sb_nx, sb_ny;
+  std::vector<int> node_of;                     // per permuted index: its node
   std::vector<int> ea_child, ea_row, ea_parent, ea_level;  // extend-add rows; ea_level per (level, pass)
   std::vector<int> ea_map;                      // per child: its panel rows' positions in the parent front
   std::vector<int64_t> ea_map_off;
 };
 // The ordering, supernodes and row structure of cholesky_factor (no numeric
 // values: Linv / L21 stay empty) and the device plan of its numeric phase.
-SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan);
+SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost = {});
 // Host execution of a plan (for checking the plan's indexing against
 // cholesky_factor): fills Linv and L21 as cholesky_factor does.
 void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::vector<double>& Linv,
@@ -85,7 +109,7 @@ inline int sweep_tile_rows(int w) { return w <= 16 ? 64 : (w == 32 ? 32 : 16); }
 struct PackedFactor {
   int n = 0, nlevels = 0;
   int64_t zlen = 0;
-  std::vector<int> cell_base, p0, ns, ms, rows;
+  std::vector<int> cell_dof0, perm, p0, ns, ms, rows;
   std::vector<int64_t> fwd_off, bwd_off, rows_off, z_off, cptr, czidx;
   std::vector<double> fwd, bwd;
   std::vector<int> ftiles, btiles;    // flattened (node, row0, nrows, 0) grouped by level

@@ -43,9 +43,9 @@ namespace {
       throw std::runtime_error(std::string(#x) + ": " + rocblas_status_to_string(s_));             \
   } while (0)
 
-struct ScItem {
-  int64_t src, dst;
-  int nx, ny, nf, mode, rx, ry;
+struct SbItem {
+  int64_t src;
+  int x, y, nx, ny;
 };
 struct EaItem {
   int child, row, parent;
@@ -78,22 +78,37 @@ struct Pool {
   }
 };
 
-// S blocks into the fronts of one level: one wave per (cell, neighbour) block.
-// Mode 0 (both cells own): the lower-triangle part of the block at rows rx..,
-// columns ry..; mode 1 (neighbour in the struct rows): the block transposed.
-// Items write disjoint positions of zeroed fronts.
-__global__ __launch_bounds__(64) void k_front_scatter(const double* __restrict__ sv, const ScItem* __restrict__ items,
-                                                      int i0, double* __restrict__ fr) {
-  const ScItem I = items[i0 + blockIdx.x];
+// S blocks into the fronts: one wave per block.  Entry (p, q) in permuted
+// order, p <= q, goes to column p of the front of the node that owns p, at q's
+// row: own, or found in the node's ascending struct rows.  The entries write
+// disjoint positions of zeroed fronts.
+__global__ __launch_bounds__(64) void k_front_scatter(const double* __restrict__ sv, const SbItem* __restrict__ items,
+                                                      const int* __restrict__ perm, const int* __restrict__ node_of,
+                                                      const int* __restrict__ p0_, const int* __restrict__ ns_,
+                                                      const int* __restrict__ ms_, const int64_t* __restrict__ rows_off,
+                                                      const int* __restrict__ rows_, const int64_t* __restrict__ front_off,
+                                                      double* __restrict__ fr) {
+  const SbItem I = items[blockIdx.x];
   const int n = I.nx * I.ny;
   for (int e = threadIdx.x; e < n; e += 64) {
     const int a = e / I.ny, b = e - a * I.ny;
     const double v = sv[I.src + e];
-    if (I.mode == 0) {
-      if (I.rx + a >= I.ry + b) fr[I.dst + (int64_t)a * I.nf + b] = v;
-    } else {
-      fr[I.dst + (int64_t)b * I.nf + a] = v;
+    const int p = perm[I.x + a], q = perm[I.y + b];
+    if (v == 0.0 || q < p) continue;
+    const int s = node_of[p], ns = ns_[s], ms = ms_[s];
+    int r = q - p0_[s];
+    if (r >= ns) {
+      const int* rows = rows_ + rows_off[s];
+      int lo = 0, hi = ms;
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (rows[mid] < q) lo = mid + 1;
+        else hi = mid;
+      }
+      if (lo == ms || rows[lo] != q) continue;  // (the row structure holds every coupling)
+      r = ns + lo;
     }
+    fr[front_off[s] + (int64_t)r * (ns + ms) + (p - p0_[s])] = v;
   }
 }
 
@@ -241,17 +256,21 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
   }
   Pool pool(st);
   // plan arrays
-  std::vector<ScItem> sc(plan.sc_src.size());
-  for (size_t i = 0; i < sc.size(); ++i)
-    sc[i] = ScItem{plan.sc_src[i], plan.sc_dst[i], plan.sc_nx[i], plan.sc_ny[i],
-                   plan.sc_nf[i],  plan.sc_mode[i], plan.sc_rx[i], plan.sc_ry[i]};
+  std::vector<SbItem> sb(plan.sb_src.size());
+  for (size_t i = 0; i < sb.size(); ++i)
+    sb[i] = SbItem{plan.sb_src[i], plan.sb_x[i], plan.sb_y[i], plan.sb_nx[i], plan.sb_ny[i]};
   std::vector<EaItem> ea(plan.ea_child.size());
   for (size_t i = 0; i < ea.size(); ++i) ea[i] = EaItem{plan.ea_child[i], plan.ea_row[i], plan.ea_parent[i]};
   std::vector<PkItem> pk;
   for (int s = 0; s < nn; ++s)
     for (int j0 = 0; j0 < P.ns[s]; j0 += 16) pk.push_back(PkItem{s, j0});
   double* sv = pool.up(plan.svals, st);
-  ScItem* d_sc = pool.up(sc, st);
+  SbItem* d_sb = pool.up(sb, st);
+  int* d_perm = pool.up(F.perm, st);
+  int* d_node_of = pool.up(plan.node_of, st);
+  int* d_p0 = pool.up(P.p0, st);
+  int* d_rows = pool.up(P.rows, st);
+  int64_t* d_rows_off = pool.up(P.rows_off, st);
   EaItem* d_ea = pool.up(ea, st);
   PkItem* d_pk = pool.up(pk, st);
   int* d_ns = pool.up(P.ns, st);
@@ -303,11 +322,12 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
     const double one = 1.0, minus_one = -1.0;
     size_t gi = 0;
     if (trace) DFCHECK(hipEventRecord(ev[0], st));
+    if (!sb.empty())
+      k_front_scatter<<<(unsigned)sb.size(), 64, 0, st>>>(sv, d_sb, d_perm, d_node_of, d_p0, d_ns, d_ms, d_rows_off,
+                                                          d_rows, d_front_off, fr);
     for (int l = 0; l < F.nlevels; ++l) {
-      const int s0 = plan.sc_level[l], s1 = plan.sc_level[l + 1];
-      if (s1 > s0) k_front_scatter<<<s1 - s0, 64, 0, st>>>(sv, d_sc, s0, fr);
-      for (int pass = 0; pass < 2; ++pass) {
-        const int e0 = plan.ea_level[2 * l + pass], e1 = plan.ea_level[2 * l + pass + 1];
+      for (int pass = 0; pass < plan.npass; ++pass) {
+        const int e0 = plan.ea_level[(size_t)plan.npass * l + pass], e1 = plan.ea_level[(size_t)plan.npass * l + pass + 1];
         if (e1 > e0) k_extend_add<<<e1 - e0, 64, 0, st>>>(d_ea, e0, d_ns, d_ms, d_front_off, d_map, d_map_off, fr);
       }
       DFCHECK(hipGetLastError());

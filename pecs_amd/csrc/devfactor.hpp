@@ -3,9 +3,9 @@
 // The symbolic phase (ordering, supernodes, row structure, front plan) runs
 // once on the host (cholesky_symbolic); the numeric phase runs here, level by
 // level of the nested-dissection tree:
-//   1. scatter the S blocks owned by the level's supernodes into their fronts;
+//   1. scatter the S blocks into the fronts (once, before the levels);
 //   2. extend-add each child's updated Schur complement into its parent's
-//      front (two passes: first children, then second children);
+//      front (one pass per child: first children, second children, ...);
 //   3. per group of fronts with equal (ns, ms): batched dense Cholesky of the
 //      leading block, triangular solve of the panel, Schur update of the
 //      trailing block, inverse of the leading factor and W21 = L21 Linv

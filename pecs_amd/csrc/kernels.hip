@@ -345,9 +345,9 @@ __device__ __forceinline__ void schur_rhs_one(const DevRegion& R, const double* 
       for (int a = 0; a < NB; ++a) a1[a] += B[i * NB + a] * w1[i];
     }
   }
-  const int pb = R.perm_base[X];
+  const int* __restrict__ pm = R.perm + (size_t)X * NB;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) g[pb + a] = a1[a];
+  for (int a = 0; a < NB; ++a) g[pm[a]] = a1[a];
 }
 
 // g = f_v + B^T W of cell X: its own block and its 4 face neighbours' blocks,
@@ -396,11 +396,11 @@ __global__ __launch_bounds__(64) void k_schur_rhs(DevRegion R, const double* __r
       }
     }
   }
-  const int pb = R.perm_base[X];
+  const int* __restrict__ pm = R.perm + (size_t)X * NB;
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
-    g1[pb + a] = a1[a];
-    if (NRHS > 1) g2[pb + a] = a2[a];
+    g1[pm[a]] = a1[a];
+    if (NRHS > 1) g2[pm[a]] = a2[a];
   }
 }
 
@@ -416,9 +416,9 @@ __device__ __forceinline__ void schur_recover_one(const DevRegion& R, const doub
   const int ty = wave_type<true>(R, M);
   const double* tb = R.table + (size_t)ty * R.stride;
   double sv[2 * NB], u[NB];
-  const int pb = R.perm_base[M];
+  const int* __restrict__ pm = R.perm + (size_t)M * NB;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) u[a] = x[pb + a];
+  for (int a = 0; a < NB; ++a) u[a] = x[pm[a]];
   for (int i = 0; i < 2 * NB; ++i) {
     double t = 0.0;
 #pragma unroll
@@ -431,10 +431,10 @@ __device__ __forceinline__ void schur_recover_one(const DevRegion& R, const doub
   for (int f = 0; f < 4; ++f) {
     const int X = R.nbr[4 * (size_t)M + f];
     if (X < 0) continue;
-    const int px = R.perm_base[X];
+    const int* __restrict__ px = R.perm + (size_t)X * NB;
     double v[NB];
 #pragma unroll
-    for (int a = 0; a < NB; ++a) v[a] = x[px + a];
+    for (int a = 0; a < NB; ++a) v[a] = x[px[a]];
     const double* B = tb + NB * NB + 2 * NB * NB + f * 2 * NB * NB;
     for (int i = 0; i < 2 * NB; ++i) {
       double t = 0.0;
@@ -484,11 +484,11 @@ __global__ __launch_bounds__(64) void k_schur_recover(DevRegion R, const double*
   const int ty = wave_type<UNI>(R, M);
   const double* tb = R.table + (size_t)ty * R.stride;
   double s1[2 * NB], s2[2 * NB], u1[NB], u2[NB];
-  const int pb = R.perm_base[M];
+  const int* __restrict__ pm = R.perm + (size_t)M * NB;
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
-    u1[a] = x1[pb + a];
-    u2[a] = (NRHS > 1) ? x2[pb + a] : 0.0;
+    u1[a] = x1[pm[a]];
+    u2[a] = (NRHS > 1) ? x2[pm[a]] : 0.0;
   }
   for (int i = 0; i < 2 * NB; ++i) {
     double t1 = 0.0, t2 = 0.0;
@@ -503,12 +503,12 @@ __global__ __launch_bounds__(64) void k_schur_recover(DevRegion R, const double*
   for (int f = 0; f < 4; ++f) {
     const int X = R.nbr[4 * (size_t)M + f];
     if (X < 0) continue;
-    const int px = R.perm_base[X];
+    const int* __restrict__ px = R.perm + (size_t)X * NB;
     double v1[NB], v2[NB];
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
-      v1[a] = x1[px + a];
-      v2[a] = (NRHS > 1) ? x2[px + a] : 0.0;
+      v1[a] = x1[px[a]];
+      v2[a] = (NRHS > 1) ? x2[px[a]] : 0.0;
     }
     const double* B = tb + NB * NB + 2 * NB * NB + f * 2 * NB * NB;
     for (int i = 0; i < 2 * NB; ++i) {
@@ -593,9 +593,9 @@ __device__ __forceinline__ void schur_rhs_one_f32(const DevRegion& R, const doub
       for (int a = 0; a < NB; ++a) acc[a] += B[i * NB + a] * w[i];
     }
   }
-  const int pb = R.perm_base[X];
+  const int* __restrict__ pm = R.perm + (size_t)X * NB;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) g[pb + a] = b[2 * nc * NB + (size_t)X * NB + a] + (double)acc[a];
+  for (int a = 0; a < NB; ++a) g[pm[a]] = b[2 * nc * NB + (size_t)X * NB + a] + (double)acc[a];
 }
 
 template <int K, int NRHS>
@@ -618,10 +618,10 @@ __device__ __forceinline__ void schur_recover_one_f32(const DevRegion& R, const 
   const size_t nc = R.ncell;
   float s[2 * NB], u[NB];
   double ud[NB];
-  const int pb = R.perm_base[M];
+  const int* __restrict__ pm = R.perm + (size_t)M * NB;
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
-    ud[a] = x[pb + a];
+    ud[a] = x[pm[a]];
     u[a] = (float)ud[a];
   }
   for (int i = 0; i < 2 * NB; ++i) {
@@ -633,10 +633,10 @@ __device__ __forceinline__ void schur_recover_one_f32(const DevRegion& R, const 
   for (int f = 0; f < 4; ++f) {
     const int X = R.nbr[4 * (size_t)M + f];
     if (X < 0) continue;
-    const int px = R.perm_base[X];
+    const int* __restrict__ px = R.perm + (size_t)X * NB;
     float v[NB];
 #pragma unroll
-    for (int a = 0; a < NB; ++a) v[a] = (float)x[px + a];
+    for (int a = 0; a < NB; ++a) v[a] = (float)x[px[a]];
     const float* B = tb + NB * NB + 2 * NB * NB + f * 2 * NB * NB;
     for (int i = 0; i < 2 * NB; ++i) {
       float t = 0.0f;
@@ -1917,11 +1917,11 @@ __global__ __launch_bounds__(64) void k_schur_rhs_hang(DevRegion R, const double
       }
     }
   }
-  const int pb = R.perm_base[R.hx_cell[t]];
+  const int* __restrict__ pm = R.perm + (size_t)R.hx_cell[t] * NB;
 #pragma unroll
   for (int a = 0; a < NB; ++a) {
-    g1[pb + a] += a1[a];
-    if (NRHS > 1) g2[pb + a] += a2[a];
+    g1[pm[a]] += a1[a];
+    if (NRHS > 1) g2[pm[a]] += a2[a];
   }
 }
 
@@ -1947,12 +1947,12 @@ __global__ __launch_bounds__(64) void k_schur_recover_hang(DevRegion R, const do
   for (int i = 0; i < 2 * NB; ++i) s1[i] = s2[i] = 0.0;
   for (int e = R.hm_ptr[t]; e < R.hm_ptr[t + 1]; ++e) {
     const double* B = R.hblk + (size_t)R.hm_blk[e] * 2 * NB * NB;
-    const int px = R.perm_base[R.hm_dst[e]];
+    const int* __restrict__ px = R.perm + (size_t)R.hm_dst[e] * NB;
     double v1[NB], v2[NB];
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
-      v1[a] = x1[px + a];
-      v2[a] = (NRHS > 1) ? x2[px + a] : 0.0;
+      v1[a] = x1[px[a]];
+      v2[a] = (NRHS > 1) ? x2[px[a]] : 0.0;
     }
     for (int i = 0; i < 2 * NB; ++i) {
 #pragma unroll

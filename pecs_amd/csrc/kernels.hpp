@@ -22,7 +22,7 @@ struct DevRegion {
   const double* table;   // per type: Minv | Bself | Bf[4]
   int stride;
   const int* sigma_nb;   // interface partner cell in the other region, or -1
-  const int* perm_base;  // permuted index of the cell's first density DoF in the Schur system
+  const int* perm;       // per cell: permuted indices of its (k + 1)^2 density DoFs in the Schur system
   // Cells grouped so that each group of 64 (one wave) shares the operator
   // types the Schur kernels read, groups padded with -1 (null: cells in
   // order, per-lane types): by the cell's own type (recovery), and by the

@@ -14,11 +14,11 @@
 
 using namespace pecs;
 
-static void block_matvec(const BlockSPD& S, const std::vector<int>& base, const double* x, double* y) {
+static void block_matvec(const BlockSPD& S, const SupernodalFactor& F, const double* x, double* y) {
   const int no = S.noff();
   for (int X = 0; X < S.NXc * S.NYc; ++X) {
     const int nx = S.ndof[X];
-    for (int a = 0; a < nx; ++a) y[base[X] + a] = 0.0;
+    for (int a = 0; a < nx; ++a) y[F.at(X, a)] = 0.0;
     const int xi = X % S.NXc, xj = X / S.NXc;
     for (int o = 0; o < no; ++o) {
       const int yi = xi + S.offi[o], yj = xj + S.offj[o];
@@ -28,7 +28,7 @@ static void block_matvec(const BlockSPD& S, const std::vector<int>& base, const 
       if (B.empty()) continue;
       const int ny = S.ndof[Y];
       for (int a = 0; a < nx; ++a)
-        for (int b = 0; b < ny; ++b) y[base[X] + a] += B[(size_t)a * ny + b] * x[base[Y] + b];
+        for (int b = 0; b < ny; ++b) y[F.at(X, a)] += B[(size_t)a * ny + b] * x[F.at(Y, b)];
     }
   }
 }
@@ -325,25 +325,37 @@ static void device_factor_emulate(const FrontPlan& plan, const SupernodalFactor&
     DEV_CHECK(i >= 0 && i < P.nvals, "bwd");
     return bwd[i];
   };
-  for (int l = 0; l < F.nlevels; ++l) {
-    // k_front_scatter: 64 lanes per item
-    for (int it = plan.sc_level[l]; it < plan.sc_level[l + 1]; ++it) {
-      const int nx = plan.sc_nx[it], ny = plan.sc_ny[it], nf = plan.sc_nf[it];
-      for (int t = 0; t < 64; ++t)
-        for (int e = t; e < nx * ny; e += 64) {
-          const int a = e / ny, b = e - a * ny;
-          DEV_CHECK(plan.sc_src[it] + e < (int64_t)plan.svals.size(), "svals");
-          const double v = plan.svals[plan.sc_src[it] + e];
-          if (plan.sc_mode[it] == 0) {
-            if (plan.sc_rx[it] + a >= plan.sc_ry[it] + b) FR(plan.sc_dst[it] + (int64_t)a * nf + b) = v;
-          } else {
-            FR(plan.sc_dst[it] + (int64_t)b * nf + a) = v;
+  // k_front_scatter: 64 lanes per block
+  for (size_t it = 0; it < plan.sb_src.size(); ++it) {
+    const int nx = plan.sb_nx[it], ny = plan.sb_ny[it];
+    for (int t = 0; t < 64; ++t)
+      for (int e = t; e < nx * ny; e += 64) {
+        const int a = e / ny, b = e - a * ny;
+        DEV_CHECK(plan.sb_src[it] + e < (int64_t)plan.svals.size(), "svals");
+        const double v = plan.svals[plan.sb_src[it] + e];
+        DEV_CHECK(plan.sb_x[it] + a < F.n && plan.sb_y[it] + b < F.n, "perm");
+        const int p = F.perm[plan.sb_x[it] + a], q = F.perm[plan.sb_y[it] + b];
+        if (v == 0.0 || q < p) continue;
+        const int s = plan.node_of[p], ns = P.ns[s], ms = P.ms[s];
+        int r = q - P.p0[s];
+        if (r >= ns) {
+          const int* rows = P.rows.data() + P.rows_off[s];
+          int lo = 0, hi = ms;
+          while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (rows[mid] < q) lo = mid + 1;
+            else hi = mid;
           }
+          DEV_CHECK(lo < ms && rows[lo] == q, "struct row");
+          r = ns + lo;
         }
-    }
-    // k_extend_add, two passes
-    for (int pass = 0; pass < 2; ++pass)
-      for (int it = plan.ea_level[2 * l + pass]; it < plan.ea_level[2 * l + pass + 1]; ++it) {
+        FR(plan.front_off[s] + (int64_t)r * (ns + ms) + (p - P.p0[s])) = v;
+      }
+  }
+  for (int l = 0; l < F.nlevels; ++l) {
+    // k_extend_add, one pass per child
+    for (int pass = 0; pass < plan.npass; ++pass)
+      for (int it = plan.ea_level[plan.npass * l + pass]; it < plan.ea_level[plan.npass * l + pass + 1]; ++it) {
         const int c = plan.ea_child[it], r = plan.ea_row[it], s = plan.ea_parent[it];
         const int nsc = P.ns[c], nfc = nsc + P.ms[c], nfp = P.ns[s] + P.ms[s];
         DEV_CHECK(r < P.ms[c], "child row");
@@ -501,20 +513,20 @@ static void blocked_emulate(const PackedFactor& P, const std::vector<double>& fw
   }
 }
 
-static double check(const char* name, const BlockSPD& S, int leaf) {
+static double check(const char* name, const BlockSPD& S, int leaf, const SolveCost& cost) {
   auto t0 = std::chrono::steady_clock::now();
-  SupernodalFactor F = cholesky_factor(S, leaf);
+  SupernodalFactor F = cholesky_factor(S, leaf, cost);
   {  // the device plan, executed on the host, must reproduce the factor
     FrontPlan plan;
-    SupernodalFactor G = cholesky_symbolic(S, leaf, plan);
+    SupernodalFactor G = cholesky_symbolic(S, leaf, plan, cost);
     std::vector<double> Li, L2;
     execute_plan_host(plan, G, Li, L2);
     double d = 0;
     for (size_t i = 0; i < Li.size(); ++i) d = std::max(d, std::fabs(Li[i] - F.Linv[i]));
     for (size_t i = 0; i < L2.size(); ++i) d = std::max(d, std::fabs(L2[i] - F.L21[i]));
-    std::printf("   front plan on host: max |diff| to cholesky_factor %.3e (fronts %.1f MB, %zu scatter items, %zu "
+    std::printf("   front plan on host: max |diff| to cholesky_factor %.3e (fronts %.1f MB, %zu S blocks, %zu "
                 "extend-add rows)\n",
-                d, plan.front_total * 8e-6, plan.sc_src.size(), plan.ea_child.size());
+                d, plan.front_total * 8e-6, plan.sb_src.size(), plan.ea_child.size());
     if (d != 0.0 || Li.size() != F.Linv.size() || L2.size() != F.L21.size()) {
       std::printf("front plan mismatch\n");
       std::exit(2);
@@ -550,9 +562,9 @@ static double check(const char* name, const BlockSPD& S, int leaf) {
   std::uniform_real_distribution<double> U(-1, 1);
   std::vector<double> x(F.n), b(F.n), xs(F.n), r(F.n);
   for (auto& v : x) v = U(rng);
-  block_matvec(S, F.cell_base, x.data(), b.data());
+  block_matvec(S, F, x.data(), b.data());
   factor_solve_host(F, b.data(), xs.data());
-  block_matvec(S, F.cell_base, xs.data(), r.data());
+  block_matvec(S, F, xs.data(), r.data());
   double nr = 0, nb = 0, ne = 0, nx = 0;
   for (int i = 0; i < F.n; ++i) {
     nr += (r[i] - b[i]) * (r[i] - b[i]);
@@ -565,7 +577,7 @@ static double check(const char* name, const BlockSPD& S, int leaf) {
     PackedFactor P = pack_factor(F);
     std::vector<double> xp(F.n), rp(F.n);
     packed_solve_host(P, b.data(), xp.data());
-    block_matvec(S, F.cell_base, xp.data(), rp.data());
+    block_matvec(S, F, xp.data(), rp.data());
     double nr2 = 0;
     for (int i = 0; i < F.n; ++i) nr2 += (rp[i] - b[i]) * (rp[i] - b[i]);
     double rel2 = std::sqrt(nr2 / nb);
@@ -654,9 +666,14 @@ int main(int argc, char** argv) {
   BlockSPD H = multiplier_matrix(m, op, T);
   std::printf("assemble S/H %.2fs\n", std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
   double worst = 0;
-  worst = std::max(worst, check("S_semi", Ss, leaf));
-  worst = std::max(worst, check("S_elec", Se, leaf));
-  worst = std::max(worst, check("H_poisson", H, leaf));
+  // the nested-dissection levels as they are, then merged (a level as dear as
+  // 20000 entries, so that runs of several lengths appear)
+  const SolveCost costs[2] = {{}, {2e4, 1.0, 0.0}};
+  for (const SolveCost& cost : costs) {
+    worst = std::max(worst, check("S_semi", Ss, leaf, cost));
+    worst = std::max(worst, check("S_elec", Se, leaf, cost));
+    worst = std::max(worst, check("H_poisson", H, leaf, cost));
+  }
   std::printf("%s\n", worst < 1e-12 ? "SELFTEST OK" : "SELFTEST FAIL");
   return worst < 1e-12 ? 0 : 1;
 }
