@@ -695,6 +695,7 @@ std::vector<int> wave_groups(int n, int nkey, KeyFn key) {
 DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegionOps& O,
                           const std::vector<int>& sigma, const FactorDev& F) {
   DevRegion d{};
+  const int nb = O.nb;
   d.N = R.N;
   d.ncell = R.ncell;
   d.V = upload(c, R.V);
@@ -706,8 +707,31 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
   d.type = upload(c, O.type);
   d.table = upload(c, O.table);
   d.stride = O.type_stride;
+  {  // the FP64 Schur kernels' tables: the face blocks without their zero rows and columns
+    const int n1 = c->k + 1, full = 2 * nb * nb, face = 2 * n1 * n1, head = 3 * nb * nb;
+    auto node = [&](int f, int m) { return f == 0 ? n1 * m : f == 1 ? n1 - 1 + n1 * m : f == 2 ? m : n1 * (n1 - 1) + m; };
+    std::vector<double> ct((size_t)O.ntype * schur_ctab_size(c->k));
+    for (int ty = 0; ty < O.ntype; ++ty) {
+      const double* src = &O.table[(size_t)ty * O.type_stride];
+      double* dst = &ct[(size_t)ty * schur_ctab_size(c->k)];
+      std::copy_n(src, head, dst);
+      for (int f = 0; f < 4; ++f) {
+        const double* B = src + head + f * full;
+        double kept = 0.0, all = 0.0;
+        for (int h = 0; h < 2; ++h)
+          for (int m = 0; m < n1; ++m)
+            for (int j = 0; j < n1; ++j) {
+              const double v = B[(h * nb + node(f, m)) * nb + node(f ^ 1, j)];
+              dst[head + f * face + (h * n1 + m) * n1 + j] = v;
+              kept += v != 0.0;
+            }
+        for (int i = 0; i < full; ++i) all += B[i] != 0.0;
+        if (kept != all) throw std::runtime_error("a face coupling reaches beyond the trace DoFs");
+      }
+    }
+    d.ctab = upload(c, ct);
+  }
   d.sigma_nb = upload(c, sigma);
-  const int nb = O.nb;
   std::vector<int> pm((size_t)R.ncell * nb);
   for (int i = 0; i < R.ncell; ++i)
     std::copy_n(&F.perm[F.cell_dof0[R.ci[i] + (size_t)R.NXg * R.cj[i]]], nb, &pm[(size_t)i * nb]);
@@ -782,9 +806,14 @@ void solve_carrier(pecs_ctx* c, int which, const double* b, double* x) {
   const FactorDev& Fc = (car == 1 && !share) ? F[1] : F[0];
   const double mu = c->P.mu[which];
   hipStream_t s = c->stream;
-  HIPCHECK((hipError_t)launch_schur_rhs(c->k, R, b, b, mu, mu, c->g[reg], c->g[reg], 1, s));
+  // W goes to the current part of x, which the recovery overwrites cell by cell
+  SchurPair sp{};
+  sp.side[0] = schur_side_of(R, b, b, x, x, mu, mu, c->g[reg], c->g[reg], x, x, 0, 0, 0);
+  const DevRegion* rs[2] = {&R, nullptr};
+  if (!R.table_f) HIPCHECK((hipError_t)launch_carrier_w(c->k, sp, 1, s));
+  HIPCHECK((hipError_t)launch_schur_rhs(c->k, rs, sp, 1, s));
   HIPCHECK((hipError_t)launch_chol_solve(Fc.d, Fc.lv(), c->g[reg], c->t[reg], 1, s));
-  HIPCHECK((hipError_t)launch_schur_recover(c->k, R, b, b, c->g[reg], c->g[reg], mu, mu, x, x, 1, s));
+  HIPCHECK((hipError_t)launch_schur_recover(c->k, rs, sp, 1, s));
 }
 
 // Poisson solves of instances [i0, i0 + n) from their condensed cell data yP:
@@ -839,15 +868,24 @@ inline int64_t gslot(const pecs_ctx* c, int reg, int car, int i) {
   return ((int64_t)car * c->B + i) * n;
 }
 
-void region_schur(pecs_ctx* c, int reg, hipStream_t s) {
+// one region's part of the step's Schur kernels (W in place of f_p in b)
+SchurPair step_side(pecs_ctx* c, int reg) {
   const DevRegion& R = reg == 0 ? c->Rs : c->Re;
   const int64_t N = reg == 0 ? c->Ns : c->Ne;
   const int64_t n = reg == 0 ? c->Fs[0].n : c->Fe[0].n;
-  const int c0 = 2 * reg, c1 = 2 * reg + 1, B = c->B;
-  // the instance stride of the g slots is n (slot = carrier * B + instance)
-  HIPCHECK((hipError_t)launch_schur_rhs(c->k, R, c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1],
-                                        c->g[reg] + gslot(c, reg, 0, 0), c->g[reg] + gslot(c, reg, 1, 0), 2, s, B, N,
-                                        n));
+  const int c0 = 2 * reg, c1 = 2 * reg + 1;
+  SchurPair sp{};
+  sp.side[0] = schur_side_of(R, c->b[c0], c->b[c1], c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1],
+                             c->g[reg] + gslot(c, reg, 0, 0), c->g[reg] + gslot(c, reg, 1, 0), c->u[c0], c->u[c1], N, n,
+                             N);
+  return sp;
+}
+
+void region_schur(pecs_ctx* c, int reg, hipStream_t s) {
+  const DevRegion* R[2] = {reg == 0 ? &c->Rs : &c->Re, nullptr};
+  const SchurPair sp = step_side(c, reg);
+  if (!R[0]->table_f) HIPCHECK((hipError_t)launch_carrier_w(c->k, sp, 2, s, c->B));
+  HIPCHECK((hipError_t)launch_schur_rhs(c->k, R, sp, 2, s, c->B));
 }
 
 void region_chol(pecs_ctx* c, int reg, hipStream_t s) {
@@ -863,13 +901,8 @@ void region_chol(pecs_ctx* c, int reg, hipStream_t s) {
 }
 
 void region_recover(pecs_ctx* c, int reg, hipStream_t s) {
-  const DevRegion& R = reg == 0 ? c->Rs : c->Re;
-  const int64_t N = reg == 0 ? c->Ns : c->Ne;
-  const int64_t n = reg == 0 ? c->Fs[0].n : c->Fe[0].n;
-  const int c0 = 2 * reg, c1 = 2 * reg + 1;
-  HIPCHECK((hipError_t)launch_schur_recover(c->k, R, c->b[c0], c->b[c1], c->g[reg] + gslot(c, reg, 0, 0),
-                                            c->g[reg] + gslot(c, reg, 1, 0), c->P.mu[c0], c->P.mu[c1], c->u[c0],
-                                            c->u[c1], 2, s, c->B, N, n, N));
+  const DevRegion* R[2] = {reg == 0 ? &c->Rs : &c->Re, nullptr};
+  HIPCHECK((hipError_t)launch_schur_recover(c->k, R, step_side(c, reg), 2, s, c->B));
 }
 
 // The Poisson phases of a step on the context stream (cell condensation,
@@ -1629,9 +1662,13 @@ int pecs_solve_dev_noalloc(pecs_ctx* ctx, int which, const double* rhs, double* 
       double* g = base + n + zl;
       double* t = g + n;
       const double mu = ctx->P.mu[which];
-      HIPCHECK((hipError_t)launch_schur_rhs(ctx->k, R, rhs, rhs, mu, mu, g, g, 1, s));
+      SchurPair sp{};
+      sp.side[0] = schur_side_of(R, rhs, rhs, x, x, mu, mu, g, g, x, x, 0, 0, 0);
+      const DevRegion* rs[2] = {&R, nullptr};
+      if (!R.table_f) HIPCHECK((hipError_t)launch_carrier_w(ctx->k, sp, 1, s));
+      HIPCHECK((hipError_t)launch_schur_rhs(ctx->k, rs, sp, 1, s));
       HIPCHECK((hipError_t)launch_chol_solve(d, Fc.lv(), g, t, 1, s));
-      HIPCHECK((hipError_t)launch_schur_recover(ctx->k, R, rhs, rhs, g, g, mu, mu, x, x, 1, s));
+      HIPCHECK((hipError_t)launch_schur_recover(ctx->k, rs, sp, 1, s));
     } else if (which == PECS_POISSON) {
       // scratch: X (nH), Z (zlen) of the multiplier factor, the condensed
       // cell data y (ysz), the multiplier right-hand side r (nH) and the

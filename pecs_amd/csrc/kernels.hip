@@ -303,11 +303,10 @@ __device__ __forceinline__ void schur_w(const DevRegion& R, const double* __rest
   }
 }
 
-// Cell of thread t.  UNI: cells come from a list grouped so that every
+// Cell of thread t on a wave-uniform cell list: cells grouped so that every
 // wave's cells share the operator types the kernel reads (groups padded to
-// whole waves with -1), and the table offsets are made wave-uniform: the
-// table entries are then fetched once per wave through the scalar cache and
-// used as scalar operands, instead of one vector load per lane and entry.
+// whole waves with -1), so that the table offsets are wave-uniform and the
+// table entries are fetched once per wave through the scalar cache.
 template <bool UNI>
 __device__ __forceinline__ int schur_cell(const int* __restrict__ list, int n, int t) {
   if (UNI) return t < n ? list[t] : -1;
@@ -320,231 +319,234 @@ __device__ __forceinline__ int wave_type(const DevRegion& R, int M) {
   return UNI ? __builtin_amdgcn_readfirstlane(t) : t;
 }
 
-// One right-hand side of k_schur_rhs on a wave-uniform cell list (the table
-// reads are scalar, so a pass per right-hand side costs no extra vector
-// loads; it halves the live registers, 165 -> 97 VGPRs, which pays off when
-// a batch of instances fills the chip and not for a single instance).
+// The FP64 Schur kernels: one lane per (cell, density DoF a), NB = (K + 1)^2
+// lanes per cell, 256 / NB cells per workgroup, both regions in one launch.
+//
+// They read W = mu A^{-1} f_p (k_carrier_w) in the place of the current part
+// of the right-hand side, and compact operator tables (ctab): per type Minv,
+// Bself and, per face f, the face's 2 (K + 1) x (K + 1) block of B: the trace
+// DoFs of the cell's own currents against the neighbour's trace DoFs, all
+// that is not zero of the 2 NB x NB block.  Per cell and right-hand side that
+// is 2 NB^2 + 8 (K + 1)^2 products and 5 NB + 8 (K + 1) loads for the
+// transform where whole blocks with W recomputed for 5 cells took 20 NB^2.
+// A lane keeps its rows of the tables in registers and runs over `per`
+// instances of a batch; a cell's W, u and s pass between its lanes in LDS.
+// A lane's node lies on at most two faces: one of x = 0, 1 and one of y = 0, 1.
+// One thread per cell with whole blocks (its chain of 700 to 4000 dependent
+// products and, on conic meshes, 9.7 KB of table per cell set the time) ->
+// this, per step: refinement 4, k = 3, distinct mobilities 344 -> 236 us;
+// refinement 7 conic 822 -> 594 us; 16 bias points at refinement 6 conic
+// 940 -> 686 us; refinement 8 planar 1627 -> 1608 us.
 template <int K>
-__device__ __forceinline__ void schur_rhs_one(const DevRegion& R, const double* __restrict__ b, double mu,
-                                              double* __restrict__ g, int X) {
-  constexpr int NB = Sz<K>::NB;
-  const size_t nc = R.ncell;
-  double a1[NB];
-#pragma unroll
-  for (int a = 0; a < NB; ++a) a1[a] = b[2 * nc * NB + (size_t)X * NB + a];
-  for (int f = -1; f < 4; ++f) {
-    const int M = f < 0 ? X : R.nbr[4 * (size_t)X + f];
-    if (M < 0) continue;
-    const int ty = wave_type<true>(R, M);
-    const double* B = R.table + (size_t)ty * R.stride + NB * NB +
-                      (f < 0 ? 0 : 2 * NB * NB + (f ^ 1) * 2 * NB * NB);
-    double w1[2 * NB];
-    schur_w<K>(R, b, mu, M, ty, w1);
-    for (int i = 0; i < 2 * NB; ++i) {
-#pragma unroll
-      for (int a = 0; a < NB; ++a) a1[a] += B[i * NB + a] * w1[i];
-    }
+struct SchurLane {
+  static constexpr int NB = Sz<K>::NB, N1 = K + 1, CPB = 256 / NB;
+  static constexpr int TAB = 3 * NB * NB + 8 * N1 * N1;  // doubles per type in ctab
+  static constexpr int FACE = 3 * NB * NB;
+  __device__ static __forceinline__ int node(int f, int m) {
+    return f == 0 ? N1 * m : f == 1 ? K + N1 * m : f == 2 ? m : N1 * K + m;
   }
-  const int* __restrict__ pm = R.perm + (size_t)X * NB;
-#pragma unroll
-  for (int a = 0; a < NB; ++a) g[pm[a]] = a1[a];
-}
+};
 
-// g = f_v + B^T W of cell X: its own block and its 4 face neighbours' blocks,
-// each neighbour's W recomputed from its right-hand side (no W in memory)
-template <int K, int NRHS, bool UNI, bool SPLIT>
-__global__ __launch_bounds__(64) void k_schur_rhs(DevRegion R, const double* __restrict__ b1,
-                                                  const double* __restrict__ b2, double mu1, double mu2,
-                                                  double* __restrict__ g1, double* __restrict__ g2, int64_t sb,
-                                                  int64_t sg) {
-  constexpr int NB = Sz<K>::NB;
-  const int X = schur_cell<UNI>(R.ucell_nbh, UNI ? R.nu_nbh : R.ncell, blockIdx.x * blockDim.x + threadIdx.x);
-  if (X < 0) return;
-  {
-    const int64_t i = blockIdx.y;
-    b1 += i * sb;
-    b2 += i * sb;
-    g1 += i * sg;
-    g2 += i * sg;
-  }
-  if constexpr (UNI && SPLIT) {
-    schur_rhs_one<K>(R, b1, mu1, g1, X);
-    if (NRHS > 1) schur_rhs_one<K>(R, b2, mu2, g2, X);
-    return;
-  }
-  const size_t nc = R.ncell;
-  double a1[NB], a2[NB];
-#pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    a1[a] = b1[2 * nc * NB + (size_t)X * NB + a];
-    a2[a] = (NRHS > 1) ? b2[2 * nc * NB + (size_t)X * NB + a] : 0.0;
-  }
-  for (int f = -1; f < 4; ++f) {
-    const int M = f < 0 ? X : R.nbr[4 * (size_t)X + f];
-    if (M < 0) continue;
-    const int ty = wave_type<UNI>(R, M);
-    const double* B = R.table + (size_t)ty * R.stride + NB * NB +
-                      (f < 0 ? 0 : 2 * NB * NB + (f ^ 1) * 2 * NB * NB);
-    double w1[2 * NB], w2[2 * NB];
-    schur_w<K>(R, b1, mu1, M, ty, w1);
-    if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
-    for (int i = 0; i < 2 * NB; ++i) {
-#pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        a1[a] += B[i * NB + a] * w1[i];
-        if (NRHS > 1) a2[a] += B[i * NB + a] * w2[i];
-      }
-    }
-  }
-  const int* __restrict__ pm = R.perm + (size_t)X * NB;
-#pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    g1[pm[a]] = a1[a];
-    if (NRHS > 1) g2[pm[a]] = a2[a];
-  }
-}
-
-// One right-hand side of k_schur_recover on a wave-uniform cell list (the
-// same operations as the kernel's per carrier; half the live registers, for
-// batches that fill the chip).
+// the region of this workgroup and its first cell
 template <int K>
-__device__ __forceinline__ void schur_recover_one(const DevRegion& R, const double* __restrict__ b,
-                                                  const double* __restrict__ x, double mu, double* __restrict__ o,
-                                                  int M) {
-  constexpr int NB = Sz<K>::NB;
-  const size_t nc = R.ncell;
-  const int ty = wave_type<true>(R, M);
-  const double* tb = R.table + (size_t)ty * R.stride;
-  double sv[2 * NB], u[NB];
-  const int* __restrict__ pm = R.perm + (size_t)M * NB;
+__device__ __forceinline__ const SchurSide& schur_side(const SchurPair& P, int& c0) {
+  const bool first = (int)blockIdx.x < P.nblk0;
+  c0 = ((int)blockIdx.x - (first ? 0 : P.nblk0)) * SchurLane<K>::CPB;
+  return first ? P.side[0] : P.side[1];
+}
+
+// W = mu A^{-1} f_p of every cell (the current part of a carrier right-hand
+// side): the cell-local inverse mass block times the two current components.
+// In place when w == b.
+template <int K>
+__global__ __launch_bounds__(256) void k_carrier_w(SchurPair P, int nrhs, int ninst, int per) {
+  using S = SchurLane<K>;
+  constexpr int NB = S::NB, CPB = S::CPB;
+  __shared__ double sf[2][CPB * NB];
+  int c0;
+  const SchurSide& R = schur_side<K>(P, c0);
+  const int t = threadIdx.x, lc = t / NB, a = t % NB, c = c0 + lc;
+  const bool on = lc < CPB && c < R.ncell;
+  const size_t nb = (size_t)R.ncell * NB, at = (size_t)c * NB + a;
+  double m[NB];
+  if (on) {
+    const double* tb = R.tab + (size_t)R.type[c] * S::TAB + a * NB;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) u[a] = x[pm[a]];
-  for (int i = 0; i < 2 * NB; ++i) {
-    double t = 0.0;
-#pragma unroll
-    for (int a = 0; a < NB; ++a) t += tb[NB * NB + i * NB + a] * u[a];
-    sv[i] = t;
+    for (int q = 0; q < NB; ++q) m[q] = tb[q];
   }
-  // u is final: stored now, so that it is not live through the rest
+  const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
+  for (int i = blockIdx.y * per; i < i1; ++i)
+    for (int h = 0; h < nrhs; ++h) {
+      const double* b = R.b[h] + i * R.sb;
+      double* w = R.w[h] + i * R.sb;
+      if (on) {
+        sf[0][t] = b[at];
+        sf[1][t] = b[nb + at];
+      }
+      __syncthreads();
+      if (on) {
+        double x = 0.0, y = 0.0;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) o[2 * nc * NB + (size_t)M * NB + a] = u[a];
-  for (int f = 0; f < 4; ++f) {
-    const int X = R.nbr[4 * (size_t)M + f];
-    if (X < 0) continue;
-    const int* __restrict__ px = R.perm + (size_t)X * NB;
-    double v[NB];
-#pragma unroll
-    for (int a = 0; a < NB; ++a) v[a] = x[px[a]];
-    const double* B = tb + NB * NB + 2 * NB * NB + f * 2 * NB * NB;
-    for (int i = 0; i < 2 * NB; ++i) {
-      double t = 0.0;
-#pragma unroll
-      for (int a = 0; a < NB; ++a) t += B[i * NB + a] * v[a];
-      sv[i] += t;
-    }
-  }
-  double w[2 * NB];
-  schur_w<K>(R, b, mu, M, ty, w);
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      double t = 0.0;
-#pragma unroll
-      for (int q = 0; q < NB; ++q) t += tb[a * NB + q] * sv[h * NB + q];
-      o[(size_t)h * nc * NB + (size_t)M * NB + a] = w[h * NB + a] - mu * t;
+        for (int q = 0; q < NB; ++q) {
+          x += m[q] * sf[0][lc * NB + q];
+          y += m[q] * sf[1][lc * NB + q];
+        }
+        w[at] = R.mu[h] * x;
+        w[nb + at] = R.mu[h] * y;
+      }
+      __syncthreads();
     }
 }
 
-// q = W - A^{-1} B u; writes [Jx | Jy | u] (W recomputed from the RHS b)
-template <int K, int NRHS, bool UNI, bool SPLIT>
-__global__ __launch_bounds__(64) void k_schur_recover(DevRegion R, const double* __restrict__ b1,
-                                                      const double* __restrict__ b2, const double* __restrict__ x1,
-                                                      const double* __restrict__ x2, double mu1, double mu2,
-                                                      double* __restrict__ o1, double* __restrict__ o2, int64_t sb,
-                                                      int64_t sx, int64_t so) {
-  constexpr int NB = Sz<K>::NB;
-  const int M = schur_cell<UNI>(R.ucell_own, UNI ? R.nu_own : R.ncell, blockIdx.x * blockDim.x + threadIdx.x);
-  if (M < 0) return;
-  {
-    const int64_t i = blockIdx.y;
-    b1 += i * sb;
-    b2 += i * sb;
-    x1 += i * sx;
-    x2 += i * sx;
-    o1 += i * so;
-    o2 += i * so;
-  }
-  if constexpr (UNI && SPLIT) {
-    schur_recover_one<K>(R, b1, x1, mu1, o1, M);
-    if (NRHS > 1) schur_recover_one<K>(R, b2, x2, mu2, o2, M);
-    return;
-  }
-  const size_t nc = R.ncell;
-  const int ty = wave_type<UNI>(R, M);
-  const double* tb = R.table + (size_t)ty * R.stride;
-  double s1[2 * NB], s2[2 * NB], u1[NB], u2[NB];
-  const int* __restrict__ pm = R.perm + (size_t)M * NB;
+// g = f_v + B^T W: the cell's own block and its face neighbours' traces of W
+template <int K>
+__global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ninst, int per) {
+  using S = SchurLane<K>;
+  constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
+  __shared__ double sw[2][2][CPB * NB];  // two buffers: one barrier per right-hand side
+  int c0;
+  const SchurSide& R = schur_side<K>(P, c0);
+  const int t = threadIdx.x, lc = t / NB, a = t % NB, c = c0 + lc;
+  const bool on = lc < CPB && c < R.ncell;
+  const size_t nb = (size_t)R.ncell * NB, at = (size_t)c * NB + a;
+  const int ax = a % N1, ay = a / N1;
+  double bs[2 * NB], bf[2][2 * N1];
+  int M[2] = {-1, -1}, fc[2];
+  fc[0] = ax == 0 ? 0 : 1;
+  fc[1] = ay == 0 ? 2 : 3;
+  size_t pm = 0;
+  if (on) {
+    const double* tb = R.tab + (size_t)R.type[c] * S::TAB + NB * NB + a;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    u1[a] = x1[pm[a]];
-    u2[a] = (NRHS > 1) ? x2[pm[a]] : 0.0;
-  }
-  for (int i = 0; i < 2 * NB; ++i) {
-    double t1 = 0.0, t2 = 0.0;
+    for (int i = 0; i < 2 * NB; ++i) bs[i] = tb[i * NB];
+    if (ax == 0 || ax == K) M[0] = R.nbr[4 * (size_t)c + fc[0]];
+    if (ay == 0 || ay == K) M[1] = R.nbr[4 * (size_t)c + fc[1]];
 #pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      t1 += tb[NB * NB + i * NB + a] * u1[a];
-      if (NRHS > 1) t2 += tb[NB * NB + i * NB + a] * u2[a];
+    for (int e = 0; e < 2; ++e) {
+      if (M[e] < 0) continue;
+      // the neighbour's block on its side of the face, this node's column
+      const double* fb = R.tab + (size_t)R.type[M[e]] * S::TAB + S::FACE + (fc[e] ^ 1) * 2 * N1 * N1 + (e ? ax : ay);
+#pragma unroll
+      for (int i = 0; i < 2 * N1; ++i) bf[e][i] = fb[i * N1];
     }
-    s1[i] = t1;
-    s2[i] = t2;
+    pm = R.perm[at];
   }
-  for (int f = 0; f < 4; ++f) {
-    const int X = R.nbr[4 * (size_t)M + f];
-    if (X < 0) continue;
-    const int* __restrict__ px = R.perm + (size_t)X * NB;
-    double v1[NB], v2[NB];
+  int buf = 0;
+  const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
+  for (int i = blockIdx.y * per; i < i1; ++i)
+    for (int h = 0; h < nrhs; ++h, buf ^= 1) {
+      const double* w = R.w[h] + i * R.sb;
+      double acc = 0.0;
+      if (on) {
+        sw[buf][0][t] = w[at];
+        sw[buf][1][t] = w[nb + at];
+        acc = R.b[h][i * R.sb + 2 * nb + at];
 #pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      v1[a] = x1[px[a]];
-      v2[a] = (NRHS > 1) ? x2[px[a]] : 0.0;
-    }
-    const double* B = tb + NB * NB + 2 * NB * NB + f * 2 * NB * NB;
-    for (int i = 0; i < 2 * NB; ++i) {
-      double t1 = 0.0, t2 = 0.0;
+        for (int e = 0; e < 2; ++e) {
+          if (M[e] < 0) continue;
+          const double* wm = w + (size_t)M[e] * NB;
 #pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        t1 += B[i * NB + a] * v1[a];
-        if (NRHS > 1) t2 += B[i * NB + a] * v2[a];
+          for (int m = 0; m < N1; ++m) {
+            const int n = S::node(fc[e] ^ 1, m);
+            acc += bf[e][m] * wm[n] + bf[e][N1 + m] * wm[nb + n];
+          }
+        }
       }
-      s1[i] += t1;
-      s2[i] += t2;
-    }
-  }
-  double w1[2 * NB], w2[2 * NB];
-  schur_w<K>(R, b1, mu1, M, ty, w1);
-  if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
-  const double* Minv = tb;
+      __syncthreads();
+      if (on) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      double t1 = 0.0, t2 = 0.0;
-#pragma unroll
-      for (int t = 0; t < NB; ++t) {
-        t1 += Minv[a * NB + t] * s1[h * NB + t];
-        if (NRHS > 1) t2 += Minv[a * NB + t] * s2[h * NB + t];
+        for (int q = 0; q < NB; ++q) acc += bs[q] * sw[buf][0][lc * NB + q] + bs[NB + q] * sw[buf][1][lc * NB + q];
+        R.g[h][i * R.sg + pm] = acc;
       }
-      const size_t off = (size_t)h * nc * NB + (size_t)M * NB + a;
-      o1[off] = w1[h * NB + a] - mu1 * t1;
-      if (NRHS > 1) o2[off] = w2[h * NB + a] - mu2 * t2;
     }
+}
+
+// q = W - mu A^{-1} B u; writes [Jx | Jy | u]
+template <int K>
+__global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, int ninst, int per) {
+  using S = SchurLane<K>;
+  constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
+  __shared__ double su[CPB * NB], ss[2][CPB * NB];
+  int c0;
+  const SchurSide& R = schur_side<K>(P, c0);
+  const int t = threadIdx.x, lc = t / NB, a = t % NB, c = c0 + lc;
+  const bool on = lc < CPB && c < R.ncell;
+  const size_t nb = (size_t)R.ncell * NB, at = (size_t)c * NB + a;
+  const int ax = a % N1, ay = a / N1;
+  double mi[NB], bs[2][NB], bf[2][2][N1];
+  int M[2] = {-1, -1}, fc[2], pn[2][N1];
+  fc[0] = ax == 0 ? 0 : 1;
+  fc[1] = ay == 0 ? 2 : 3;
+  size_t pm = 0;
+  if (on) {
+    const double* tb = R.tab + (size_t)R.type[c] * S::TAB;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    o1[2 * nc * NB + (size_t)M * NB + a] = u1[a];
-    if (NRHS > 1) o2[2 * nc * NB + (size_t)M * NB + a] = u2[a];
+    for (int q = 0; q < NB; ++q) {
+      mi[q] = tb[a * NB + q];
+      bs[0][q] = tb[NB * NB + a * NB + q];
+      bs[1][q] = tb[NB * NB + (NB + a) * NB + q];
+    }
+    if (ax == 0 || ax == K) M[0] = R.nbr[4 * (size_t)c + fc[0]];
+    if (ay == 0 || ay == K) M[1] = R.nbr[4 * (size_t)c + fc[1]];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (M[e] < 0) continue;
+      const double* fb = tb + S::FACE + fc[e] * 2 * N1 * N1 + (e ? ax : ay) * N1;
+#pragma unroll
+      for (int j = 0; j < N1; ++j) {
+        bf[e][0][j] = fb[j];
+        bf[e][1][j] = fb[N1 * N1 + j];
+        pn[e][j] = R.perm[(size_t)M[e] * NB + S::node(fc[e] ^ 1, j)];
+      }
+    }
+    pm = R.perm[at];
   }
+  const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
+  for (int i = blockIdx.y * per; i < i1; ++i)
+    for (int h = 0; h < nrhs; ++h) {
+      const double* x = R.g[h] + i * R.sg;
+      double* o = R.o[h] + i * R.so;
+      double s0 = 0.0, s1 = 0.0, w0 = 0.0, w1 = 0.0;
+      if (on) {
+        const double u = x[pm];
+        su[t] = u;
+        o[2 * nb + at] = u;
+        w0 = R.w[h][i * R.sb + at];
+        w1 = R.w[h][i * R.sb + nb + at];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          if (M[e] < 0) continue;
+#pragma unroll
+          for (int j = 0; j < N1; ++j) {
+            const double v = x[pn[e][j]];
+            s0 += bf[e][0][j] * v;
+            s1 += bf[e][1][j] * v;
+          }
+        }
+      }
+      __syncthreads();
+      if (on) {
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          const double v = su[lc * NB + q];
+          s0 += bs[0][q] * v;
+          s1 += bs[1][q] * v;
+        }
+        ss[0][t] = s0;
+        ss[1][t] = s1;
+      }
+      __syncthreads();
+      if (on) {
+        double q0 = 0.0, q1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          q0 += mi[q] * ss[0][lc * NB + q];
+          q1 += mi[q] * ss[1][lc * NB + q];
+        }
+        o[at] = w0 - R.mu[h] * q0;
+        o[nb + at] = w1 - R.mu[h] * q1;
+      }
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -1884,7 +1886,8 @@ inline int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 // are absent from the neighbour lists); these kernels add them afterwards, in
 // FP64, one thread per cell that has such a coupling.  Both are linear in the
 // terms they add, so the sum equals the one over all couplings.
-template <int K, int NRHS>
+// W: the current part of b holds W (the FP64 path), else f_p.
+template <int K, int NRHS, bool W>
 __global__ __launch_bounds__(64) void k_schur_rhs_hang(DevRegion R, const double* __restrict__ b1,
                                                        const double* __restrict__ b2, double mu1, double mu2,
                                                        double* __restrict__ g1, double* __restrict__ g2, int64_t sb,
@@ -1907,8 +1910,21 @@ __global__ __launch_bounds__(64) void k_schur_rhs_hang(DevRegion R, const double
     const double* B = R.hblk + (size_t)R.hx_blk[e] * 2 * NB * NB;
     const int ty = R.type[M];
     double w1[2 * NB], w2[2 * NB];
-    schur_w<K>(R, b1, mu1, M, ty, w1);
-    if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
+    if (W) {
+      const size_t nc = R.ncell;
+#pragma unroll
+      for (int a = 0; a < NB; ++a) {
+        w1[a] = b1[(size_t)M * NB + a];
+        w1[NB + a] = b1[nc * NB + (size_t)M * NB + a];
+        if (NRHS > 1) {
+          w2[a] = b2[(size_t)M * NB + a];
+          w2[NB + a] = b2[nc * NB + (size_t)M * NB + a];
+        }
+      }
+    } else {
+      schur_w<K>(R, b1, mu1, M, ty, w1);
+      if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
+    }
     for (int i = 0; i < 2 * NB; ++i) {
 #pragma unroll
       for (int a = 0; a < NB; ++a) {
@@ -2037,6 +2053,8 @@ __global__ __launch_bounds__(64) void k_poisson_recover_hang(DevPoisson P, const
   }
 }
 
+static inline int nblk1(int64_t n, int b) { return (int)((n + b - 1) / b); }
+
 int launch_rhs_carrier(int k, bool semi, const DevRegion& R, const DevRegion& O, const DevPoisson& P,
                        const DevTabs& T, const DevPhys* phs, const double* u1, const double* u2, const double* ou1,
                        const double* ou2, const double* pvec, double* b1, double* b2, hipStream_t s, int nb,
@@ -2053,66 +2071,33 @@ int launch_rhs_carrier(int k, bool semi, const DevRegion& R, const DevRegion& O,
   return (int)hipGetLastError();
 }
 
-static int launch_schur_rhs_main(int k, const DevRegion& R, const double* b1, const double* b2, double mu1, double mu2,
-                     double* g1, double* g2, int nrhs, hipStream_t s, int nb, int64_t sb, int64_t sg) {
-#define PECS_SCHUR_RHS(UU, SS, NCELL)                                                                       \
-  {                                                                                                         \
-    const dim3 g(nblk(NCELL, 64), nb);                                                                      \
-    if (nrhs == 2) {                                                                                        \
-      PECS_DISPATCH_K(k, (k_schur_rhs<KK, 2, UU, SS><<<g, 64, 0, s>>>(R, b1, b2, mu1, mu2, g1, g2, sb, sg))); \
-    } else {                                                                                                \
-      PECS_DISPATCH_K(k, (k_schur_rhs<KK, 1, UU, SS><<<g, 64, 0, s>>>(R, b1, b1, mu1, mu1, g1, g1, sb, sg))); \
-    }                                                                                                       \
-    return (int)hipGetLastError();                                                                          \
-  }
-  if (R.table_f && R.ucell_nbh) {  // mixed precision
-    const dim3 g(nblk(R.nu_nbh, 64), nb);
-    if (nrhs == 2) {
-      PECS_DISPATCH_K(k, (k_schur_rhs_f32<KK, 2><<<g, 64, 0, s>>>(R, b1, b2, mu1, mu2, g1, g2, sb, sg)));
-    } else {
-      PECS_DISPATCH_K(k, (k_schur_rhs_f32<KK, 1><<<g, 64, 0, s>>>(R, b1, b1, mu1, mu1, g1, g1, sb, sg)));
-    }
-    return (int)hipGetLastError();
-  }
-  // a pass per right-hand side once a batch fills the chip (4 or more instances)
-  if (R.ucell_nbh && nb >= 4) PECS_SCHUR_RHS(true, true, R.nu_nbh)
-  if (R.ucell_nbh) PECS_SCHUR_RHS(true, false, R.nu_nbh)
-  PECS_SCHUR_RHS(false, false, R.ncell)
-#undef PECS_SCHUR_RHS
+// Instances of a batch per workgroup of the Schur kernels: enough that the
+// table rows a lane loads are used again, few enough that the launch still
+// has several thousand workgroups.
+static int schur_per(int nblk, int nb) {
+  int per = 1;
+  while (per < 16 && per < nb && (int64_t)nblk * nblk1(nb, 2 * per) >= 4096) per *= 2;
+  return per;
 }
 
-static int launch_schur_recover_main(int k, const DevRegion& R, const double* b1, const double* b2, const double* xs1,
-                         const double* xs2, double mu1, double mu2, double* out1, double* out2, int nrhs,
-                         hipStream_t s, int nb, int64_t sb, int64_t sx, int64_t so) {
-#define PECS_RECOVER(UU, SS, NCELL)                                                                             \
-  {                                                                                                             \
-    const dim3 g(nblk(NCELL, 64), nb);                                                                          \
-    if (nrhs == 2) {                                                                                            \
-      PECS_DISPATCH_K(k, (k_schur_recover<KK, 2, UU, SS><<<g, 64, 0, s>>>(R, b1, b2, xs1, xs2, mu1, mu2, out1,   \
-                                                                          out2, sb, sx, so)));                  \
-    } else {                                                                                                    \
-      PECS_DISPATCH_K(k, (k_schur_recover<KK, 1, UU, SS><<<g, 64, 0, s>>>(R, b1, b1, xs1, xs1, mu1, mu1, out1,   \
-                                                                          out1, sb, sx, so)));                  \
-    }                                                                                                           \
-    return (int)hipGetLastError();                                                                              \
-  }
-  if (R.table_f && R.ucell_own) {  // mixed precision
-    const dim3 g(nblk(R.nu_own, 64), nb);
-    if (nrhs == 2) {
-      PECS_DISPATCH_K(k, (k_schur_recover_f32<KK, 2><<<g, 64, 0, s>>>(R, b1, b2, xs1, xs2, mu1, mu2, out1, out2, sb,
-                                                                      sx, so)));
-    } else {
-      PECS_DISPATCH_K(k, (k_schur_recover_f32<KK, 1><<<g, 64, 0, s>>>(R, b1, b1, xs1, xs1, mu1, mu1, out1, out1, sb,
-                                                                      sx, so)));
-    }
-    return (int)hipGetLastError();
-  }
-  // a pass per right-hand side once a batch fills the chip (4 or more instances)
-  if (R.ucell_own && nb >= 4) PECS_RECOVER(true, true, R.nu_own)
-  if (R.ucell_own) PECS_RECOVER(true, false, R.nu_own)
-  PECS_RECOVER(false, false, R.ncell)
-#undef PECS_RECOVER
+int schur_ctab_size(int k) { return 3 * (k + 1) * (k + 1) * (k + 1) * (k + 1) + 8 * (k + 1) * (k + 1); }
+
+#define PECS_SCHUR_LAUNCH(KERNEL)                                                        \
+  P.nblk0 = nblk1(P.side[0].ncell, 256 / ((k + 1) * (k + 1)));                           \
+  const int n = P.nblk0 + nblk1(P.side[1].ncell, 256 / ((k + 1) * (k + 1)));             \
+  if (n == 0) return 0;                                                                  \
+  const int per = schur_per(n, nb);                                                      \
+  PECS_DISPATCH_K(k, (KERNEL<KK><<<dim3(n, nblk1(nb, per)), 256, 0, s>>>(P, nrhs, nb, per))); \
+  return (int)hipGetLastError()
+
+int launch_carrier_w(int k, SchurPair P, int nrhs, hipStream_t s, int nb) { PECS_SCHUR_LAUNCH(k_carrier_w); }
+
+static int launch_schur_rhs_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) { PECS_SCHUR_LAUNCH(k_schur_rhs); }
+
+static int launch_schur_recover_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
+  PECS_SCHUR_LAUNCH(k_schur_recover);
 }
+#undef PECS_SCHUR_LAUNCH
 
 template <int NRHS, bool FWD>
 static int sweep_dispatch(const DevFactor& F, const int4* tl, int nt, int w, int maxr, const double* v0,
@@ -2336,29 +2321,81 @@ static int launch_poisson_recover_main(int k, const DevPoisson& P, const double*
   return (int)hipGetLastError();
 }
 
-int launch_schur_rhs(int k, const DevRegion& R, const double* b1, const double* b2, double mu1, double mu2,
-                     double* g1, double* g2, int nrhs, hipStream_t s, int nb, int64_t sb, int64_t sg) {
-  const int rc = launch_schur_rhs_main(k, R, b1, b2, mu1, mu2, g1, g2, nrhs, s, nb, sb, sg);
-  if (rc || R.nhx == 0) return rc;
-  const dim3 g(nblk(R.nhx, 64), nb);
-  if (nrhs == 2) {
-    PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, 2><<<g, 64, 0, s>>>(R, b1, b2, mu1, mu2, g1, g2, sb, sg)));
-  } else {
-    PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, 1><<<g, 64, 0, s>>>(R, b1, b1, mu1, mu1, g1, g1, sb, sg)));
+SchurSide schur_side_of(const DevRegion& R, const double* b1, const double* b2, double* w1, double* w2, double mu1,
+                        double mu2, double* g1, double* g2, double* o1, double* o2, int64_t sb, int64_t sg, int64_t so) {
+  return SchurSide{R.ncell, R.nbr, R.type, R.perm, R.ctab, {b1, b2}, {w1, w2}, {g1, g2}, {o1, o2}, {mu1, mu2}, sb, sg,
+                   so};
+}
+
+int launch_schur_rhs(int k, const DevRegion* const* R, const SchurPair& P, int nrhs, hipStream_t s, int nb) {
+  bool f32 = false;
+  for (int r = 0; r < 2; ++r) f32 = f32 || (R[r] && R[r]->table_f);
+  if (!f32) {
+    const int rc = launch_schur_rhs_main(k, P, nrhs, s, nb);
+    if (rc) return rc;
+  }
+  for (int r = 0; r < 2; ++r) {
+    if (!R[r] || P.side[r].ncell == 0) continue;
+    const SchurSide& S = P.side[r];
+    if (f32) {  // mixed precision
+      const dim3 g(nblk(R[r]->nu_nbh, 64), nb);
+      if (nrhs == 2) {
+        PECS_DISPATCH_K(k, (k_schur_rhs_f32<KK, 2><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[1], S.mu[0], S.mu[1], S.g[0],
+                                                                    S.g[1], S.sb, S.sg)));
+      } else {
+        PECS_DISPATCH_K(k, (k_schur_rhs_f32<KK, 1><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[0], S.mu[0], S.mu[0], S.g[0],
+                                                                    S.g[0], S.sb, S.sg)));
+      }
+    }
+    if (R[r]->nhx == 0) continue;
+    const dim3 g(nblk(R[r]->nhx, 64), nb);
+#define PECS_HANG(NN, WW, B1, B2)                                                                              \
+  PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, NN, WW><<<g, 64, 0, s>>>(*R[r], B1, B2, S.mu[0], S.mu[NN - 1], S.g[0], \
+                                                                    S.g[NN - 1], S.sb, S.sg)))
+    if (f32 && nrhs == 2) {
+      PECS_HANG(2, false, S.b[0], S.b[1]);
+    } else if (f32) {
+      PECS_HANG(1, false, S.b[0], S.b[0]);
+    } else if (nrhs == 2) {
+      PECS_HANG(2, true, S.w[0], S.w[1]);
+    } else {
+      PECS_HANG(1, true, S.w[0], S.w[0]);
+    }
+#undef PECS_HANG
   }
   return (int)hipGetLastError();
 }
 
-int launch_schur_recover(int k, const DevRegion& R, const double* b1, const double* b2, const double* xs1,
-                         const double* xs2, double mu1, double mu2, double* out1, double* out2, int nrhs,
-                         hipStream_t s, int nb, int64_t sb, int64_t sx, int64_t so) {
-  const int rc = launch_schur_recover_main(k, R, b1, b2, xs1, xs2, mu1, mu2, out1, out2, nrhs, s, nb, sb, sx, so);
-  if (rc || R.nhm == 0) return rc;
-  const dim3 g(nblk(R.nhm, 64), nb);
-  if (nrhs == 2) {
-    PECS_DISPATCH_K(k, (k_schur_recover_hang<KK, 2><<<g, 64, 0, s>>>(R, xs1, xs2, mu1, mu2, out1, out2, sx, so)));
-  } else {
-    PECS_DISPATCH_K(k, (k_schur_recover_hang<KK, 1><<<g, 64, 0, s>>>(R, xs1, xs1, mu1, mu1, out1, out1, sx, so)));
+int launch_schur_recover(int k, const DevRegion* const* R, const SchurPair& P, int nrhs, hipStream_t s, int nb) {
+  bool f32 = false;
+  for (int r = 0; r < 2; ++r) f32 = f32 || (R[r] && R[r]->table_f);
+  if (!f32) {
+    const int rc = launch_schur_recover_main(k, P, nrhs, s, nb);
+    if (rc) return rc;
+  }
+  for (int r = 0; r < 2; ++r) {
+    if (!R[r] || P.side[r].ncell == 0) continue;
+    const SchurSide& S = P.side[r];
+    const int h = nrhs - 1;
+    if (f32) {  // mixed precision
+      const dim3 g(nblk(R[r]->nu_own, 64), nb);
+      if (nrhs == 2) {
+        PECS_DISPATCH_K(k, (k_schur_recover_f32<KK, 2><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[1], S.g[0], S.g[1], S.mu[0],
+                                                                        S.mu[1], S.o[0], S.o[1], S.sb, S.sg, S.so)));
+      } else {
+        PECS_DISPATCH_K(k, (k_schur_recover_f32<KK, 1><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[0], S.g[0], S.g[0], S.mu[0],
+                                                                        S.mu[0], S.o[0], S.o[0], S.sb, S.sg, S.so)));
+      }
+    }
+    if (R[r]->nhm == 0) continue;
+    const dim3 g(nblk(R[r]->nhm, 64), nb);
+    if (nrhs == 2) {
+      PECS_DISPATCH_K(k, (k_schur_recover_hang<KK, 2><<<g, 64, 0, s>>>(*R[r], S.g[0], S.g[1], S.mu[0], S.mu[1], S.o[0],
+                                                                       S.o[1], S.sg, S.so)));
+    } else {
+      PECS_DISPATCH_K(k, (k_schur_recover_hang<KK, 1><<<g, 64, 0, s>>>(*R[r], S.g[h], S.g[h], S.mu[h], S.mu[h],
+                                                                       S.o[h], S.o[h], S.sg, S.so)));
+    }
   }
   return (int)hipGetLastError();
 }

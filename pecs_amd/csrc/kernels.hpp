@@ -21,11 +21,12 @@ struct DevRegion {
   const int* type;       // LDG operator type per cell
   const double* table;   // per type: Minv | Bself | Bf[4]
   int stride;
+  const double* ctab;    // per type: Minv | Bself | the trace blocks of Bf[4] (schur_ctab_size(k) doubles)
   const int* sigma_nb;   // interface partner cell in the other region, or -1
   const int* perm;       // per cell: permuted indices of its (k + 1)^2 density DoFs in the Schur system
   // Cells grouped so that each group of 64 (one wave) shares the operator
-  // types the Schur kernels read, groups padded with -1 (null: cells in
-  // order, per-lane types): by the cell's own type (recovery), and by the
+  // types the mixed-precision Schur kernels read, groups padded with -1
+  // (null: too many types): by the cell's own type (recovery), and by the
   // types of the cell and its 4 face neighbours (right-hand side).
   const int* ucell_own;
   const int* ucell_nbh;
@@ -168,14 +169,37 @@ int launch_rhs_carrier(int k, bool semi, const DevRegion& R, const DevRegion& O,
                        const DevTabs& T, const DevPhys* phs, const double* u1, const double* u2, const double* ou1,
                        const double* ou2, const double* pvec, double* b1, double* b2, hipStream_t s, int nb = 1,
                        int64_t sR = 0, int64_t sO = 0, int64_t sP = 0);
-// Schur transform g = f_v + B^T (mu A^{-1} f_p) and recovery
-// q = mu A^{-1} f_p - mu A^{-1} B u of one region's carriers (b: the LDG RHS
-// [f_p | f_v] of each carrier; g / xs in the factor's permuted order).
-int launch_schur_rhs(int k, const DevRegion& R, const double* b1, const double* b2, double mu1, double mu2,
-                     double* g1, double* g2, int nrhs, hipStream_t s, int nb = 1, int64_t sb = 0, int64_t sg = 0);
-int launch_schur_recover(int k, const DevRegion& R, const double* b1, const double* b2, const double* xs1,
-                         const double* xs2, double mu1, double mu2, double* out1, double* out2, int nrhs,
-                         hipStream_t s, int nb = 1, int64_t sb = 0, int64_t sx = 0, int64_t so = 0);
+// One region's part in a launch of the Schur kernels.  Carriers h = 0, 1: the
+// right-hand side b ([f_p | f_v]), W = mu A^{-1} f_p in the place of f_p (w:
+// b itself or another vector of its layout), the Schur right-hand side or
+// solution g in the factor's permuted order, the solution o.  sb, sg, so: the
+// instance strides of b and w, g, o.
+struct SchurSide {
+  int ncell;
+  const int *nbr, *type, *perm;
+  const double* tab;
+  const double* b[2];
+  double* w[2];
+  double* g[2];
+  double* o[2];
+  double mu[2];
+  int64_t sb, sg, so;
+};
+// Both regions (side[1].ncell 0: one); nblk0 is set by the launchers.
+struct SchurPair {
+  SchurSide side[2];
+  int nblk0;
+};
+int schur_ctab_size(int k);
+SchurSide schur_side_of(const DevRegion& R, const double* b1, const double* b2, double* w1, double* w2, double mu1,
+                        double mu2, double* g1, double* g2, double* o1, double* o2, int64_t sb, int64_t sg, int64_t so);
+// W = mu A^{-1} f_p into w; Schur transform g = f_v + B^T W; recovery
+// q = W - mu A^{-1} B u.  nrhs: carriers per region.  R: the regions of
+// P.side (mixed precision, which reads f_p in b instead of W, and the hanging
+// faces).
+int launch_carrier_w(int k, SchurPair P, int nrhs, hipStream_t s, int nb = 1);
+int launch_schur_rhs(int k, const DevRegion* const* R, const SchurPair& P, int nrhs, hipStream_t s, int nb = 1);
+int launch_schur_recover(int k, const DevRegion* const* R, const SchurPair& P, int nrhs, hipStream_t s, int nb = 1);
 // One level's sweep over `nt` row tiles.  w > 0: W = w lanes per row and
 // `maxr` row passes per tile (W in {8,16,32,64} with maxr in {1,2,4}, or W in
 // {32,64} with maxr 8; every tile has at most (256 / W) * maxr rows), for 1 or
