@@ -63,7 +63,6 @@ struct pecs_ctx {
   hipStream_t stream = nullptr;
   hipStream_t side = nullptr;            // second stream for the concurrent region solves
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
-  hipEvent_t rhs_ev[2] = {};  // a region's right-hand side done (it has read the other region's old state)
   // one time step captured as a graph (pecs_step replays it); cap is the
   // stream it is captured on (capture needs a stream other than the null stream)
   hipStream_t cap = nullptr;
@@ -146,8 +145,6 @@ struct pecs_ctx {
     }
     if (fork_ev) (void)hipEventDestroy(fork_ev);
     if (join_ev) (void)hipEventDestroy(join_ev);
-    for (hipEvent_t e : rhs_ev)
-      if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : events) (void)hipEventDestroy(e);
     for (void* p : allocs) (void)hipFree(p);
     factor_handle_destroy(blas);
@@ -869,23 +866,43 @@ inline int64_t gslot(const pecs_ctx* c, int reg, int car, int i) {
 }
 
 // one region's part of the step's Schur kernels (W in place of f_p in b)
-SchurPair step_side(pecs_ctx* c, int reg) {
+SchurSide step_side(pecs_ctx* c, int reg) {
   const DevRegion& R = reg == 0 ? c->Rs : c->Re;
   const int64_t N = reg == 0 ? c->Ns : c->Ne;
   const int64_t n = reg == 0 ? c->Fs[0].n : c->Fe[0].n;
   const int c0 = 2 * reg, c1 = 2 * reg + 1;
-  SchurPair sp{};
-  sp.side[0] = schur_side_of(R, c->b[c0], c->b[c1], c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1],
-                             c->g[reg] + gslot(c, reg, 0, 0), c->g[reg] + gslot(c, reg, 1, 0), c->u[c0], c->u[c1], N, n,
-                             N);
-  return sp;
+  return schur_side_of(R, c->b[c0], c->b[c1], c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1],
+                       c->g[reg] + gslot(c, reg, 0, 0), c->g[reg] + gslot(c, reg, 1, 0), c->u[c0], c->u[c1], N, n, N);
 }
 
-void region_schur(pecs_ctx* c, int reg, hipStream_t s) {
-  const DevRegion* R[2] = {reg == 0 ? &c->Rs : &c->Re, nullptr};
-  const SchurPair sp = step_side(c, reg);
-  if (!R[0]->table_f) HIPCHECK((hipError_t)launch_carrier_w(c->k, sp, 2, s, c->B));
+// right-hand sides of one region (reg 0, 1) or both (2), W in place of f_p
+// except in mixed precision, whose kernels read f_p
+void step_rhs(pecs_ctx* c, int reg, hipStream_t s) {
+  RhsPair rp{};
+  rp.wmode = c->Rs.table_f ? 0 : 1;
+  int n = 0;
+  if (reg != 1)
+    rp.side[n++] = rhs_side_of(c->Rs, c->Re, true, c->u[0], c->u[1], c->u[2], c->u[3], c->b[0], c->b[1], c->P.mu[0],
+                               c->P.mu[1], c->Ns, c->Ne);
+  if (reg != 0)
+    rp.side[n++] = rhs_side_of(c->Re, c->Rs, false, c->u[2], c->u[3], c->u[0], c->u[1], c->b[2], c->b[3], c->P.mu[2],
+                               c->P.mu[3], c->Ne, c->Ns);
+  HIPCHECK((hipError_t)launch_rhs_carrier(c->k, rp, c->Pd, c->tabs, c->phs_d, c->pv, s, c->B, c->NP));
+}
+
+// Schur transforms and recoveries of both regions, one launch each
+void step_schur(pecs_ctx* c, hipStream_t s) {
+  const DevRegion* R[2] = {&c->Rs, &c->Re};
+  SchurPair sp{};
+  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r);
   HIPCHECK((hipError_t)launch_schur_rhs(c->k, R, sp, 2, s, c->B));
+}
+
+void step_recover(pecs_ctx* c, hipStream_t s) {
+  const DevRegion* R[2] = {&c->Rs, &c->Re};
+  SchurPair sp{};
+  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r);
+  HIPCHECK((hipError_t)launch_schur_recover(c->k, R, sp, 2, s, c->B));
 }
 
 void region_chol(pecs_ctx* c, int reg, hipStream_t s) {
@@ -898,11 +915,6 @@ void region_chol(pecs_ctx* c, int reg, hipStream_t s) {
     HIPCHECK((hipError_t)launch_chol_solve(F[0].d, F[0].lv(), c->g[reg], c->t[reg], c->B, s));
     HIPCHECK((hipError_t)launch_chol_solve(F[1].d, F[1].lv(), c->g[reg] + h1, c->t[reg], c->B, s));
   }
-}
-
-void region_recover(pecs_ctx* c, int reg, hipStream_t s) {
-  const DevRegion* R[2] = {reg == 0 ? &c->Rs : &c->Re, nullptr};
-  HIPCHECK((hipError_t)launch_schur_recover(c->k, R, step_side(c, reg), 2, s, c->B));
 }
 
 // The Poisson phases of a step on the context stream (cell condensation,
@@ -928,44 +940,15 @@ void step_once(pecs_ctx* c) {
     c->ev_used += NPHASE + 1;
     pm.mark();
   }
-  const int64_t Ns = c->Ns, Ne = c->Ne, NP = c->NP;
-  const int B = c->B;
-  if (!pm.ev) {
-    // Without per-phase timing each region's chain (right-hand side, Schur
-    // transform, solve, recovery) runs on its own stream, joined before the
-    // Poisson phase.  A region's recovery writes its new state, which the
-    // other region's right-hand side reads as the old one (the lagged
-    // interface traces): it waits for that right-hand side.
-    hipStream_t d = c->side;
-    HIPCHECK(hipEventRecord(c->fork_ev, s));
-    HIPCHECK(hipStreamWaitEvent(d, c->fork_ev, 0));
-    HIPCHECK((hipError_t)launch_rhs_carrier(c->k, true, c->Rs, c->Re, c->Pd, c->tabs, c->phs_d, c->u[0], c->u[1],
-                                            c->u[2], c->u[3], c->pv, c->b[0], c->b[1], s, B, Ns, Ne, NP));
-    HIPCHECK(hipEventRecord(c->rhs_ev[0], s));
-    HIPCHECK((hipError_t)launch_rhs_carrier(c->k, false, c->Re, c->Rs, c->Pd, c->tabs, c->phs_d, c->u[2], c->u[3],
-                                            c->u[0], c->u[1], c->pv, c->b[2], c->b[3], d, B, Ne, Ns, NP));
-    HIPCHECK(hipEventRecord(c->rhs_ev[1], d));
-    region_schur(c, 0, s);
-    region_schur(c, 1, d);
-    region_chol(c, 0, s);
-    region_chol(c, 1, d);
-    HIPCHECK(hipStreamWaitEvent(s, c->rhs_ev[1], 0));
-    region_recover(c, 0, s);
-    HIPCHECK(hipStreamWaitEvent(d, c->rhs_ev[0], 0));
-    region_recover(c, 1, d);
-    HIPCHECK(hipEventRecord(c->join_ev, d));
-    HIPCHECK(hipStreamWaitEvent(s, c->join_ev, 0));
-    poisson_step(c);
-    return;
+  if (pm.ev) {  // a launch per region, so that each has its own time
+    step_rhs(c, 0, s);
+    pm.mark();
+    step_rhs(c, 1, s);
+    pm.mark();
+  } else {
+    step_rhs(c, 2, s);
   }
-  HIPCHECK((hipError_t)launch_rhs_carrier(c->k, true, c->Rs, c->Re, c->Pd, c->tabs, c->phs_d, c->u[0], c->u[1],
-                                          c->u[2], c->u[3], c->pv, c->b[0], c->b[1], s, B, Ns, Ne, NP));
-  pm.mark();
-  HIPCHECK((hipError_t)launch_rhs_carrier(c->k, false, c->Re, c->Rs, c->Pd, c->tabs, c->phs_d, c->u[2], c->u[3],
-                                          c->u[0], c->u[1], c->pv, c->b[2], c->b[3], s, B, Ne, Ns, NP));
-  pm.mark();
-  region_schur(c, 0, s);
-  region_schur(c, 1, s);
+  step_schur(c, s);
   pm.mark();
   // the two regions' solves share no data: the electrolyte runs on the side
   // stream so its launches fill the GPU where the semiconductor's leave gaps
@@ -976,10 +959,9 @@ void step_once(pecs_ctx* c) {
   HIPCHECK(hipEventRecord(c->join_ev, c->side));
   HIPCHECK(hipStreamWaitEvent(s, c->join_ev, 0));
   pm.mark();
-  region_recover(c, 0, s);
-  region_recover(c, 1, s);
+  step_recover(c, s);
   pm.mark();
-  poisson_step(c, &pm);
+  poisson_step(c, pm.ev ? &pm : nullptr);
 }
 
 // The state before the last step of a pecs_step call (for the steady residual).
@@ -1175,7 +1157,6 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     HIPCHECK(hipStreamCreateWithFlags(&c->cap, hipStreamNonBlocking));
     HIPCHECK(hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming));
     HIPCHECK(hipEventCreateWithFlags(&c->join_ev, hipEventDisableTiming));
-    for (hipEvent_t& e : c->rhs_ev) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     c->P = to_params(params);
     for (int i = 0; i < B; ++i) c->Pb.push_back(to_params(&params[i]));
     c->k = params->degree;
@@ -1589,16 +1570,18 @@ static void d2h(pecs_ctx* c, double* h, const double* d, int64_t n) {
 int pecs_rhs_semiconductor_dev(pecs_ctx* ctx, const double* un, const double* up, const double* pv,
                                const double* ur, const double* uo, double* bn, double* bp) {
   PECS_TRY(ctx, {
-    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, true, ctx->Rs, ctx->Re, ctx->Pd, ctx->tabs, ctx->phs_d, un, up, ur,
-                                            uo, pv, bn, bp, ctx->stream));
+    RhsPair rp{};
+    rp.side[0] = rhs_side_of(ctx->Rs, ctx->Re, true, un, up, ur, uo, bn, bp);
+    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, rp, ctx->Pd, ctx->tabs, ctx->phs_d, pv, ctx->stream));
   })
 }
 
 int pecs_rhs_electrolyte_dev(pecs_ctx* ctx, const double* ur, const double* uo, const double* pv,
                              const double* un, const double* up, double* br, double* bo) {
   PECS_TRY(ctx, {
-    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, false, ctx->Re, ctx->Rs, ctx->Pd, ctx->tabs, ctx->phs_d, ur, uo,
-                                            un, up, pv, br, bo, ctx->stream));
+    RhsPair rp{};
+    rp.side[0] = rhs_side_of(ctx->Re, ctx->Rs, false, ur, uo, un, up, br, bo);
+    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, rp, ctx->Pd, ctx->tabs, ctx->phs_d, pv, ctx->stream));
   })
 }
 
@@ -1704,9 +1687,10 @@ int pecs_rhs_semiconductor(pecs_ctx* ctx, const double* un, const double* up, co
     h2d(ctx, ctx->io[2], ur, ctx->Ne);
     h2d(ctx, ctx->io[3], uo, ctx->Ne);
     h2d(ctx, ctx->old[4], poisson_in(ctx, pv, false), ctx->NP);
-    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, true, ctx->Rs, ctx->Re, ctx->Pd, ctx->tabs, ctx->phs_d, ctx->io[0],
-                                            ctx->io[1], ctx->io[2], ctx->io[3], ctx->old[4], ctx->b[0], ctx->b[1],
-                                            ctx->stream));
+    RhsPair rp{};
+    rp.side[0] = rhs_side_of(ctx->Rs, ctx->Re, true, ctx->io[0], ctx->io[1], ctx->io[2], ctx->io[3], ctx->b[0],
+                             ctx->b[1]);
+    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, rp, ctx->Pd, ctx->tabs, ctx->phs_d, ctx->old[4], ctx->stream));
     d2h(ctx, bn, ctx->b[0], ctx->Ns);
     d2h(ctx, bp, ctx->b[1], ctx->Ns);
   })
@@ -1720,9 +1704,10 @@ int pecs_rhs_electrolyte(pecs_ctx* ctx, const double* ur, const double* uo, cons
     h2d(ctx, ctx->io[2], ur, ctx->Ne);
     h2d(ctx, ctx->io[3], uo, ctx->Ne);
     h2d(ctx, ctx->old[4], poisson_in(ctx, pv, false), ctx->NP);
-    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, false, ctx->Re, ctx->Rs, ctx->Pd, ctx->tabs, ctx->phs_d, ctx->io[2],
-                                            ctx->io[3], ctx->io[0], ctx->io[1], ctx->old[4], ctx->b[2], ctx->b[3],
-                                            ctx->stream));
+    RhsPair rp{};
+    rp.side[0] = rhs_side_of(ctx->Re, ctx->Rs, false, ctx->io[2], ctx->io[3], ctx->io[0], ctx->io[1], ctx->b[2],
+                             ctx->b[3]);
+    HIPCHECK((hipError_t)launch_rhs_carrier(ctx->k, rp, ctx->Pd, ctx->tabs, ctx->phs_d, ctx->old[4], ctx->stream));
     d2h(ctx, br, ctx->b[2], ctx->Ne);
     d2h(ctx, bo, ctx->b[3], ctx->Ne);
   })

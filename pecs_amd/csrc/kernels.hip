@@ -75,6 +75,14 @@ struct Sz {
   static constexpr int NL = NRT + NPHI;
 };
 
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// doubles per type of the Schur kernels' operator tables (ctab)
+template <int K>
+constexpr int schur_tab() {
+  return 3 * Sz<K>::NB * Sz<K>::NB + 8 * (K + 1) * (K + 1);
+}
+
 // local RT index of face node m of face f (RT_{K-1} nodal basis)
 template <int K>
 __device__ __forceinline__ int rt_face(int f, int m) {
@@ -87,188 +95,227 @@ __device__ __forceinline__ int rt_face(int f, int m) {
 // ------------------------------------------------------------------------
 // Carrier right-hand sides (SolarCell.cpp:1073-1414 and 1451-1726)
 // ------------------------------------------------------------------------
-template <int K, bool SEMI>
-__global__ __launch_bounds__(64) void k_rhs_carrier(DevRegion R, DevRegion O, DevPoisson P, DevTabs T,
-                                                    const DevPhys* __restrict__ phs, const double* __restrict__ u1,
-                                                    const double* __restrict__ u2, const double* __restrict__ ou1,
-                                                    const double* __restrict__ ou2, const double* __restrict__ pvec,
-                                                    double* __restrict__ b1, double* __restrict__ b2, int64_t sR,
-                                                    int64_t sO, int64_t sP) {
+// Both regions in one launch; a wave takes 16 cells of one region, lane
+// l = 16 kq + col cell col, and the element contractions run on FP64 MFMA
+// (16x16x4): values at the quadrature points from the DoFs, and the DoF rows
+// from the pointwise integrands.  The result layout (lane l, register r: row
+// kq + 4 r, cell col) of the first is the operand layout (k = kq of step r) of
+// the second, so a lane computes the integrands of its own points
+// q = 16 qb + 4 r + kq in registers and nothing moves between lanes.  The
+// faces on the boundary and the interface take the same two steps over the
+// face points, skipped where no cell of the wave has one.
+// W (wmode): the current part is multiplied by mu A^{-1} before it is stored
+// (what the Schur kernels read), one (cell, DoF) per thread from LDS.
+// One thread per cell with the whole quadrature loop (255 VGPRs, about 4000
+// dependent FP64 operations) took 36 + 36 us at refinement 8, k = 2, and
+// 58 + 74 us at refinement 4, k = 3, the regions one after the other.
+template <int K>
+__global__ __launch_bounds__(256) void k_rhs_carrier(RhsPair A, DevPoisson P, DevTabs T,
+                                                     const DevPhys* __restrict__ phs, const double* __restrict__ pvec,
+                                                     int64_t sP) {
   using S = Sz<K>;
-  constexpr int NB = S::NB, NQ = S::NQ, NF = S::NF, NRT = S::NRT;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= R.ncell) return;
-  // instance blockIdx.y of a batch: its physics and vectors
-  const DevPhys ph = phs[blockIdx.y];
-  {
-    const int64_t i = blockIdx.y;
-    u1 += i * sR;
-    u2 += i * sR;
-    b1 += i * sR;
-    b2 += i * sR;
-    ou1 += i * sO;
-    ou2 += i * sO;
-    pvec += i * sP;
-  }
-  const int nc = R.ncell;
+  constexpr int NB = S::NB, NQ = S::NQ, NF = S::NF, NX = S::NRTX;
+  constexpr int SA = (NB + 3) / 4, SX = (NX + 3) / 4, QB = (NQ + 15) / 16, SF = (NF + 3) / 4;
+  __shared__ double sf[4][64 * NB];  // [carrier, component][cell][DoF] (wmode)
+  const bool first = (int)blockIdx.x < A.nblk0;
+  const RhsSide& R = first ? A.side[0] : A.side[1];
+  const bool semi = R.semi != 0;
+  const int c0 = ((int)blockIdx.x - (first ? 0 : A.nblk0)) * 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, kq = lane >> 4;
+  const int cw = c0 + 16 * wave + col, nc = R.ncell;
+  const bool on = cw < nc;
+  const int c = on ? cw : nc - 1;  // (lanes past the last cell repeat it and store nothing)
+  const int64_t inst = blockIdx.y;
+  const DevPhys ph = phs[inst];
+  const double* __restrict__ u1 = R.u[0] + inst * R.s;
+  const double* __restrict__ u2 = R.u[1] + inst * R.s;
+  pvec += inst * sP;
+  const size_t nn = (size_t)nc * NB, uo = 2 * nn + (size_t)c * NB;
   double v[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) v[t] = R.V[8 * (size_t)c + t];
-  double d1[NB], d2[NB];
-  const size_t ub = 2 * (size_t)nc * NB + (size_t)c * NB;
+  double d1[SA], d2[SA];
 #pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    d1[a] = u1[ub + a];
-    d2[a] = u2[ub + a];
+  for (int t = 0; t < SA; ++t) {
+    const int a = 4 * t + kq;
+    d1[t] = a < NB ? u1[uo + a] : 0.0;
+    d2[t] = a < NB ? u2[uo + a] : 0.0;
   }
-  const int pc = SEMI ? c : P.ncell_semi + c;
-  double dp[NRT];
+  const int* __restrict__ id = P.idx + (size_t)(semi ? c : P.ncell_semi + c) * P.nloc;
+  double ex[SX], ey[SX];
 #pragma unroll
-  for (int i = 0; i < NRT; ++i) dp[i] = pvec[P.idx[(size_t)pc * P.nloc + i]];
-  double a1p[2 * NB], a1v[NB], a2p[2 * NB], a2v[NB];
-#pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    a1p[a] = a1p[NB + a] = a1v[a] = 0.0;
-    a2p[a] = a2p[NB + a] = a2v[a] = 0.0;
+  for (int t = 0; t < SX; ++t) {
+    const int i = 4 * t + kq;
+    ex[t] = i < NX ? pvec[id[i]] : 0.0;
+    ey[t] = i < NX ? pvec[id[NX + i]] : 0.0;
   }
-  const double inv_perm = 1.0 / (SEMI ? ph.eps_s : ph.eps_e);
-  const double idt = 1.0 / ph.dt;
-  for (int q = 0; q < NQ; ++q) {
-    const GeoD g = bilin(v, T.qx[q], T.qy[q]);
-    const double jxw = T.qw[q] * g.det;
-    double n1 = 0.0, n2 = 0.0;
+  const v4d zero = {0.0, 0.0, 0.0, 0.0};
+  v4d ax1 = zero, ay1 = zero, av1 = zero, ax2 = zero, ay2 = zero, av2 = zero;
+  const double inv_perm = 1.0 / (semi ? ph.eps_s : ph.eps_e), idt = 1.0 / ph.dt;
 #pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      const double ph_a = T.phi[a * NQ + q];
-      n1 += d1[a] * ph_a;
-      n2 += d2[a] * ph_a;
-    }
-    double hx = 0.0, hy = 0.0;
+  for (int qb = 0; qb < QB; ++qb) {
+    v4d n1 = zero, n2 = zero, hx = zero, hy = zero;
+    const int qr = 16 * qb + col;  // this lane's row of the first operand
 #pragma unroll
-    for (int i = 0; i < NRT; ++i) {
-      hx += dp[i] * T.psix[i * NQ + q];
-      hy += dp[i] * T.psiy[i * NQ + q];
+    for (int t = 0; t < SA; ++t) {
+      const int a = 4 * t + kq;
+      const double f = (qr < NQ && a < NB) ? T.phi[a * NQ + qr] : 0.0;
+      n1 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, d1[t], n1, 0, 0, 0);
+      n2 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, d2[t], n2, 0, 0, 0);
     }
-    const double Ex = (g.J00 * hx + g.J01 * hy) / g.det;
-    const double Ey = (g.J10 * hx + g.J11 * hy) / g.det;
-    double src = 0.0;
-    if (SEMI) {
-      if (ph.gen_mode == 0) src = ph.alpha * ph.G0 * exp(ph.alpha * (g.y - ph.H));
-      else if (ph.gen_mode == 1) src = ph.G0 * exp(-ph.alpha * g.x);
-      if (ph.srh)
-        src += (ph.ni * ph.ni - n1 * n2) / (ph.tau_n * (n1 + ph.ni) + ph.tau_p * (n2 + ph.ni));
-    }
-    if (R.msrc) src += R.msrc[(size_t)c * NQ + q];
-    const double sv1 = jxw * (n1 * idt + src), sv2 = jxw * (n2 * idt + src);
-    const double cp1 = -1.0 * inv_perm * n1 * jxw, cp2 = 1.0 * inv_perm * n2 * jxw;
 #pragma unroll
-    for (int a = 0; a < NB; ++a) {
-      const double ph_a = T.phi[a * NQ + q];
-      a1v[a] += sv1 * ph_a;
-      a2v[a] += sv2 * ph_a;
-      a1p[a] += cp1 * Ex * ph_a;
-      a1p[NB + a] += cp1 * Ey * ph_a;
-      a2p[a] += cp2 * Ex * ph_a;
-      a2p[NB + a] += cp2 * Ey * ph_a;
+    for (int t = 0; t < SX; ++t) {
+      const int i = 4 * t + kq;
+      const bool in = qr < NQ && i < NX;
+      const double fx = in ? T.psix[i * NQ + qr] : 0.0, fy = in ? T.psiy[(NX + i) * NQ + qr] : 0.0;
+      hx = __builtin_amdgcn_mfma_f64_16x16x4f64(fx, ex[t], hx, 0, 0, 0);
+      hy = __builtin_amdgcn_mfma_f64_16x16x4f64(fy, ey[t], hy, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (16 * qb + 4 * r >= NQ) continue;
+      const int q = 16 * qb + 4 * r + kq;
+      const bool in = q < NQ;
+      const int qc = in ? q : NQ - 1;
+      const GeoD g = bilin(v, T.qx[qc], T.qy[qc]);
+      const double jxw = T.qw[qc] * g.det;
+      const double Ex = (g.J00 * hx[r] + g.J01 * hy[r]) / g.det;
+      const double Ey = (g.J10 * hx[r] + g.J11 * hy[r]) / g.det;
+      double src = 0.0;
+      if (semi) {
+        if (ph.gen_mode == 0) src = ph.alpha * ph.G0 * exp(ph.alpha * (g.y - ph.H));
+        else if (ph.gen_mode == 1) src = ph.G0 * exp(-ph.alpha * g.x);
+        if (ph.srh)
+          src += (ph.ni * ph.ni - n1[r] * n2[r]) / (ph.tau_n * (n1[r] + ph.ni) + ph.tau_p * (n2[r] + ph.ni));
+      }
+      if (R.msrc) src += R.msrc[(size_t)c * NQ + qc];
+      // (selected, not multiplied by zero: rows past the last point may hold no number)
+      const double sv1 = in ? jxw * (n1[r] * idt + src) : 0.0, sv2 = in ? jxw * (n2[r] * idt + src) : 0.0;
+      const double cp1 = -inv_perm * n1[r] * jxw, cp2 = inv_perm * n2[r] * jxw;
+      const double x1 = in ? cp1 * Ex : 0.0, y1 = in ? cp1 * Ey : 0.0;
+      const double x2 = in ? cp2 * Ex : 0.0, y2 = in ? cp2 * Ey : 0.0;
+      const double f = (in && col < NB) ? T.phi[col * NQ + q] : 0.0;
+      av1 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, sv1, av1, 0, 0, 0);
+      av2 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, sv2, av2, 0, 0, 0);
+      ax1 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, x1, ax1, 0, 0, 0);
+      ay1 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, y1, ay1, 0, 0, 0);
+      ax2 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, x2, ax2, 0, 0, 0);
+      ay2 = __builtin_amdgcn_mfma_f64_16x16x4f64(f, y2, ay2, 0, 0, 0);
     }
   }
   const double hc = R.h[c];
   for (int f = 0; f < 4; ++f) {
     const int bid = R.bid[4 * (size_t)c + f];
-    if (bid < 0) continue;
+    const int e = bid == 0 ? R.sigma_nb[c] : -1;
+    const bool flux = R.mflux && (bid == 0 || bid == 2);  // manufactured data: prescribed normal flux, -<v, h>
+    const bool dir = bid == 1, iface = bid == 0 && e >= 0, sch = semi && bid == 3;
+    if (!__any(flux || dir || iface || sch)) continue;  // wave-uniform
+    const double* fph = T.fphi + (size_t)f * NB * NF;
+    const double* foph = T.fphi + (size_t)(f ^ 1) * NB * NF;
+    v4d t1 = zero, t2 = zero, o1 = zero, o2 = zero;  // own and other side's traces
+    if (__any(iface || sch)) {
+      const size_t ob = 2 * (size_t)R.ncell_o * NB + (size_t)(e < 0 ? 0 : e) * NB;
+      const double* __restrict__ ou1 = R.ou[0] + inst * R.so;
+      const double* __restrict__ ou2 = R.ou[1] + inst * R.so;
+#pragma unroll
+      for (int t = 0; t < SA; ++t) {
+        const int a = 4 * t + kq;
+        const bool in = col < NF && a < NB;
+        const double fo = in ? fph[a * NF + col] : 0.0, fe = in ? foph[a * NF + col] : 0.0;
+        t1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fo, d1[t], t1, 0, 0, 0);
+        t2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fo, d2[t], t2, 0, 0, 0);
+        const bool ld = iface && a < NB;
+        o1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fe, ld ? ou1[ob + a] : 0.0, o1, 0, 0, 0);
+        o2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fe, ld ? ou2[ob + a] : 0.0, o2, 0, 0, 0);
+      }
+    }
     double nx, ny, len;
     face_nrm(v, f, nx, ny, len);
-    const double* fph = T.fphi + (size_t)f * NB * NF;
-    if (R.mflux && (bid == 0 || bid == 2)) {  // manufactured data: prescribed normal flux, -<v, h>
-      for (int q = 0; q < NF; ++q) {
-        const double w = -R.mflux[(4 * (size_t)c + f) * NF + q] * T.fw[q] * len;
 #pragma unroll
-        for (int a = 0; a < NB; ++a) {
-          a1v[a] += fph[a * NF + q] * w;
-          a2v[a] += fph[a * NF + q] * w;
-        }
-      }
-    }
-    if (bid == 2) continue;  // Neumann: nothing (SolarCell.cpp:1403-1406)
-    if (!SEMI && bid == 3) continue;
-    if (bid == 1) {  // Dirichlet
-      const double c1 = SEMI ? ph.ne : ph.rinf, c2 = SEMI ? ph.pe : ph.oinf;
-      const double pen = ph.penalty / hc;
-      for (int q = 0; q < NF; ++q) {
-        const double jw = T.fw[q] * len;
-        const double e1 = R.mdir ? R.mdir[(4 * (size_t)c + f) * NF + q] : c1;
-        const double e2 = R.mdir ? e1 : c2;
-#pragma unroll
-        for (int a = 0; a < NB; ++a) {
-          const double fa = fph[a * NF + q];
-          a1p[a] -= fa * nx * jw * e1;
-          a1p[NB + a] -= fa * ny * jw * e1;
-          a1v[a] += pen * fa * jw * e1;
-          a2p[a] -= fa * nx * jw * e2;
-          a2p[NB + a] -= fa * ny * jw * e2;
-          a2v[a] += pen * fa * jw * e2;
-        }
-      }
-      continue;
-    }
-    // interface (0) and Schottky (3) use the own traces
-    double o1[NB], o2[NB];
-    const double* foph = T.fphi + (size_t)(f ^ 1) * NB * NF;
-    if (bid == 0) {
-      const int e = R.sigma_nb[c];
-      if (e < 0) continue;
-      const size_t ob = 2 * (size_t)O.ncell * NB + (size_t)e * NB;
-#pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        o1[a] = ou1[ob + a];
-        o2[a] = ou2[ob + a];
-      }
-    }
-    for (int q = 0; q < NF; ++q) {
-      const double jw = T.fw[q] * len;
-      double t1 = 0.0, t2 = 0.0;
-#pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        t1 += d1[a] * fph[a * NF + q];
-        t2 += d2[a] * fph[a * NF + q];
-      }
-      double w1, w2;
-      if (bid == 0) {
-        double r1 = 0.0, r2 = 0.0;
-#pragma unroll
-        for (int a = 0; a < NB; ++a) {
-          r1 += o1[a] * foph[a * NF + q];
-          r2 += o2[a] * foph[a * NF + q];
-        }
-        if (SEMI) {
-          w1 = -ph.k_et * (t1 - ph.ne) * r2 * jw;  // -v k_et (n - n^e) o
-          w2 = ph.k_ht * (t2 - ph.pe) * r1 * jw;   // +v k_ht (p - p^e) r
+    for (int r = 0; r < SF; ++r) {
+      const int q = 4 * r + kq;
+      const bool in = q < NF;
+      const int qc = in ? q : NF - 1;
+      const double jw = T.fw[qc] * len;
+      double w1 = 0.0, w2 = 0.0, x1 = 0.0, y1 = 0.0, x2 = 0.0, y2 = 0.0;
+      if (flux) w1 = w2 = -R.mflux[(4 * (size_t)c + f) * NF + qc] * jw;
+      if (dir) {  // Dirichlet
+        const double pen = ph.penalty / hc;
+        const double md = R.mdir ? R.mdir[(4 * (size_t)c + f) * NF + qc] : 0.0;
+        const double e1 = jw * (R.mdir ? md : semi ? ph.ne : ph.rinf), e2 = jw * (R.mdir ? md : semi ? ph.pe : ph.oinf);
+        x1 = -nx * e1;
+        y1 = -ny * e1;
+        w1 = pen * e1;
+        x2 = -nx * e2;
+        y2 = -ny * e2;
+        w2 = pen * e2;
+      } else if (iface) {
+        if (semi) {
+          w1 += -ph.k_et * (t1[r] - ph.ne) * o2[r] * jw;  // -v k_et (n - n^e) o
+          w2 += ph.k_ht * (t2[r] - ph.pe) * o1[r] * jw;   // +v k_ht (p - p^e) r
         } else {
-          const double cur = (-ph.k_et * (r1 - ph.ne) * t2 + ph.k_ht * (r2 - ph.pe) * t1) * jw;
-          w1 = cur;
-          w2 = -cur;
+          const double cur = (-ph.k_et * (o1[r] - ph.ne) * t2[r] + ph.k_ht * (o2[r] - ph.pe) * t1[r]) * jw;
+          w1 += cur;
+          w2 -= cur;
         }
-      } else {  // Schottky (SolarCell.cpp:1348-1402)
-        w1 = -ph.v_rec_n * (t1 - ph.ne) * jw;
-        w2 = ph.v_rec_p * (t2 - ph.pe) * jw;
-      }
-#pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        const double fa = fph[a * NF + q];
-        a1v[a] += fa * w1;
-        a2v[a] += fa * w2;
+      } else if (sch) {  // Schottky (SolarCell.cpp:1348-1402)
+        w1 += -ph.v_rec_n * (t1[r] - ph.ne) * jw;
+        w2 += ph.v_rec_p * (t2[r] - ph.pe) * jw;
+      }  // Neumann: nothing (SolarCell.cpp:1403-1406)
+      if (!in) w1 = w2 = x1 = y1 = x2 = y2 = 0.0;
+      const double fa = (in && col < NB) ? fph[col * NF + q] : 0.0;
+      av1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, w1, av1, 0, 0, 0);
+      av2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, w2, av2, 0, 0, 0);
+      if (__any(dir)) {
+        ax1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, x1, ax1, 0, 0, 0);
+        ay1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, y1, ay1, 0, 0, 0);
+        ax2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, x2, ax2, 0, 0, 0);
+        ay2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, y2, ay2, 0, 0, 0);
       }
     }
   }
-  const size_t jxo = (size_t)c * NB, jyo = (size_t)nc * NB + (size_t)c * NB, uo = 2 * (size_t)nc * NB + (size_t)c * NB;
+  double* __restrict__ b1 = R.b[0] + inst * R.s;
+  double* __restrict__ b2 = R.b[1] + inst * R.s;
+  const bool wm = A.wmode != 0;
 #pragma unroll
-  for (int a = 0; a < NB; ++a) {
-    b1[jxo + a] = a1p[a];
-    b1[jyo + a] = a1p[NB + a];
-    b1[uo + a] = a1v[a];
-    b2[jxo + a] = a2p[a];
-    b2[jyo + a] = a2p[NB + a];
-    b2[uo + a] = a2v[a];
+  for (int r = 0; r < (NB + 3) / 4; ++r) {
+    const int a = 4 * r + kq;
+    if (a >= NB || !on) continue;
+    const size_t at = (size_t)c * NB + a;
+    b1[2 * nn + at] = av1[r];
+    b2[2 * nn + at] = av2[r];
+    if (wm) {
+      const int l = (16 * wave + col) * NB + a;
+      sf[0][l] = ax1[r];
+      sf[1][l] = ay1[r];
+      sf[2][l] = ax2[r];
+      sf[3][l] = ay2[r];
+    } else {
+      b1[at] = ax1[r];
+      b1[nn + at] = ay1[r];
+      b2[at] = ax2[r];
+      b2[nn + at] = ay2[r];
+    }
+  }
+  if (!wm) return;
+  __syncthreads();
+  const int last = min(64, nc - c0) * NB;
+  for (int l = threadIdx.x; l < last; l += 256) {
+    const int lc = l / NB, a = l % NB;
+    const double* tb = R.tab + (size_t)R.type[c0 + lc] * schur_tab<K>() + a * NB;
+    double w[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const double m = tb[q];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) w[h] += m * sf[h][lc * NB + q];
+    }
+    const size_t at = (size_t)c0 * NB + l;
+    b1[at] = R.mu[0] * w[0];
+    b1[nn + at] = R.mu[0] * w[1];
+    b2[at] = R.mu[1] * w[2];
+    b2[nn + at] = R.mu[1] * w[3];
   }
 }
 
@@ -340,7 +387,7 @@ __device__ __forceinline__ int wave_type(const DevRegion& R, int M) {
 template <int K>
 struct SchurLane {
   static constexpr int NB = Sz<K>::NB, N1 = K + 1, CPB = 256 / NB;
-  static constexpr int TAB = 3 * NB * NB + 8 * N1 * N1;  // doubles per type in ctab
+  static constexpr int TAB = schur_tab<K>();
   static constexpr int FACE = 3 * NB * NB;
   __device__ static __forceinline__ int node(int f, int m) {
     return f == 0 ? N1 * m : f == 1 ? K + N1 * m : f == 2 ? m : N1 * K + m;
@@ -927,8 +974,6 @@ __global__ __launch_bounds__(256) void k_sweep(DevFactor F, const int4* __restri
 // whose B operand holds the vector at the same columns (lane l: column
 // 4(l/16)+e, right-hand side l%16), so the k order of A and B agree.
 // Accumulator lane l, register r holds row l/16 + 4r, right-hand side l%16.
-typedef double v4d __attribute__((ext_vector_type(4)));
-
 // The interleaved vectors from and to one vector per right-hand side (entry
 // p of right-hand side h at [h * n + p]): a tile of IL_TP rows passes through
 // LDS, so that the per-right-hand-side side moves IL_TP consecutive rows
@@ -2055,19 +2100,19 @@ __global__ __launch_bounds__(64) void k_poisson_recover_hang(DevPoisson P, const
 
 static inline int nblk1(int64_t n, int b) { return (int)((n + b - 1) / b); }
 
-int launch_rhs_carrier(int k, bool semi, const DevRegion& R, const DevRegion& O, const DevPoisson& P,
-                       const DevTabs& T, const DevPhys* phs, const double* u1, const double* u2, const double* ou1,
-                       const double* ou2, const double* pvec, double* b1, double* b2, hipStream_t s, int nb,
-                       int64_t sR, int64_t sO, int64_t sP) {
-  if (R.ncell == 0) return 0;
-  const dim3 g(nblk(R.ncell, 64), nb);
-  if (semi) {
-    PECS_DISPATCH_K(k, (k_rhs_carrier<KK, true><<<g, 64, 0, s>>>(R, O, P, T, phs, u1, u2, ou1, ou2, pvec, b1, b2, sR,
-                                                                 sO, sP)));
-  } else {
-    PECS_DISPATCH_K(k, (k_rhs_carrier<KK, false><<<g, 64, 0, s>>>(R, O, P, T, phs, u1, u2, ou1, ou2, pvec, b1, b2, sR,
-                                                                  sO, sP)));
-  }
+RhsSide rhs_side_of(const DevRegion& R, const DevRegion& O, bool semi, const double* u1, const double* u2,
+                    const double* ou1, const double* ou2, double* b1, double* b2, double mu1, double mu2, int64_t s,
+                    int64_t so) {
+  return RhsSide{R.ncell, O.ncell, semi ? 1 : 0, R.V,   R.h,          R.bid,        R.type, R.sigma_nb, R.ctab,
+                 R.msrc,  R.mdir,  R.mflux,      {u1, u2}, {ou1, ou2}, {b1, b2},    {mu1, mu2}, s,      so};
+}
+
+int launch_rhs_carrier(int k, RhsPair A, const DevPoisson& P, const DevTabs& T, const DevPhys* phs, const double* pvec,
+                       hipStream_t s, int nb, int64_t sP) {
+  A.nblk0 = nblk1(A.side[0].ncell, 64);
+  const int n = A.nblk0 + nblk1(A.side[1].ncell, 64);
+  if (n == 0) return 0;
+  PECS_DISPATCH_K(k, (k_rhs_carrier<KK><<<dim3(n, nb), 256, 0, s>>>(A, P, T, phs, pvec, sP)));
   return (int)hipGetLastError();
 }
 

@@ -165,10 +165,33 @@ struct FactorLevels {
 // launchers (return hipError_t as int).  The cell-local launchers run nb
 // instances of a batch at once (grid dimension y); each vector argument of
 // instance i is at its pointer + i * (its stride), physics at phs[i].
-int launch_rhs_carrier(int k, bool semi, const DevRegion& R, const DevRegion& O, const DevPoisson& P,
-                       const DevTabs& T, const DevPhys* phs, const double* u1, const double* u2, const double* ou1,
-                       const double* ou2, const double* pvec, double* b1, double* b2, hipStream_t s, int nb = 1,
-                       int64_t sR = 0, int64_t sO = 0, int64_t sP = 0);
+//
+// One region's part in a launch of the carrier right-hand sides: its own
+// carriers' states u, the other region's ou (interface traces), the results b
+// ([f_p | f_v]); s, so: the instance strides of u and b, of ou.
+struct RhsSide {
+  int ncell, ncell_o, semi;
+  const double *V, *h;
+  const int *bid, *type, *sigma_nb;
+  const double* tab;
+  const double *msrc, *mdir, *mflux;
+  const double* u[2];
+  const double* ou[2];
+  double* b[2];
+  double mu[2];
+  int64_t s, so;
+};
+// Both regions (side[1].ncell 0: one).  wmode: W = mu A^{-1} f_p is stored in
+// the place of f_p; nblk0 is set by the launcher.
+struct RhsPair {
+  RhsSide side[2];
+  int nblk0, wmode;
+};
+RhsSide rhs_side_of(const DevRegion& R, const DevRegion& O, bool semi, const double* u1, const double* u2,
+                    const double* ou1, const double* ou2, double* b1, double* b2, double mu1 = 1.0, double mu2 = 1.0,
+                    int64_t s = 0, int64_t so = 0);
+int launch_rhs_carrier(int k, RhsPair A, const DevPoisson& P, const DevTabs& T, const DevPhys* phs, const double* pvec,
+                       hipStream_t s, int nb = 1, int64_t sP = 0);
 // One region's part in a launch of the Schur kernels.  Carriers h = 0, 1: the
 // right-hand side b ([f_p | f_v]), W = mu A^{-1} f_p in the place of f_p (w:
 // b itself or another vector of its layout), the Schur right-hand side or
