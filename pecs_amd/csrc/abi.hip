@@ -45,14 +45,21 @@ struct FactorDev {
   std::vector<int> foff, boff, goff, xoff, fw, bw, fm, bm, frows, brows, fks, bks, froff, broff, fpf,
       bpf;  // per level
   int nlevels = 0, n = 0;
-  double nnz = 0.0;
-  double tri_bytes = 0.0;      // algorithmic bytes of a forward + backward sweep
+  int nsys = 0;
+  std::vector<double> nnz;        // per system: stored entries
+  std::vector<double> tri_bytes;  // per system: algorithmic bytes of a forward + backward sweep
+  int rows(int k) const { return sys_p0[k + 1] - sys_p0[k]; }
   double device_seconds = 0.0, device_flops = 0.0;  // numeric factorisation on the device (0: on the host)
-  std::vector<int> cell_dof0, perm;  // host copy: grid cell -> its first DoF; DoF -> permuted index
+  // host copies: per system grid cell -> its first DoF; DoF -> permuted index;
+  // per system its first row and first update slot (and the ends)
+  std::vector<std::vector<int>> cell_dof0;
+  std::vector<int> perm, sys_p0;
+  std::vector<int64_t> sys_z0;
   FactorLevels lv() const {
     return FactorLevels{foff.data(), boff.data(), goff.data(),  xoff.data(),  fw.data(), bw.data(),
                         fm.data(),   bm.data(),   fks.data(),   bks.data(),   froff.data(), broff.data(),
-                        nlevels,     fpf.empty() ? nullptr : fpf.data(), bpf.empty() ? nullptr : bpf.data()};
+                        nlevels,     nsys,        sys_p0.data(), fpf.empty() ? nullptr : fpf.data(),
+                        bpf.empty() ? nullptr : bpf.data()};
   }
 };
 
@@ -87,16 +94,25 @@ struct pecs_ctx {
   std::vector<float> tabf_host[3];
   float* tabf_dev[3] = {};
   DevPhys ph{};  // instance 0
-  FactorDev Fs[2], Fe[2], FH;
-  bool share_s = false, share_e = false;
+  // The carriers' Schur factors.  The carriers of a region share one system
+  // when their mobilities agree (share).  Regions that agree in that are one
+  // factor (a forest), whose levels both regions' solves run through together;
+  // otherwise there are two.  Carrier car of region r is system sys[r][car] of
+  // Fc[fr[r]]; its Schur vectors begin gcar[r] entries after those of carrier 0
+  // of the region when both are solved together.
+  FactorDev Fc[2], FH;
+  int nf = 0, fr[2] = {}, sys[2][2] = {}, nrhs_f[2] = {};
+  int64_t gcar[2] = {};
+  bool share[2] = {};
   int64_t Ns = 0, Ne = 0, NP = 0;
   // device vectors, instance-major (instance i at offset i * per-instance size)
   double* u[4] = {};
   double* pv = nullptr;
   double* b[4] = {};
 
-  // per region: the Schur right-hand sides / solutions of all carriers and
-  // instances, h-major with h = carrier * B + instance (region factor order)
+  // per factor: the Schur right-hand sides / solutions of all its systems and
+  // instances, h-major (factor order), h = carrier * B + instance where the
+  // carriers share a system, else h = instance
   double* g[2] = {};
   double* t[2] = {};
   double* yP = nullptr;
@@ -321,7 +337,7 @@ void tune_factor(pecs_ctx* c, PackedFactor& P, DevFactor& d, int nrhs) {
   size_t tcap = 0;
   for (int l = 0; l < P.nlevels; ++l) {
     size_t rows = 0;
-    for (int q = P.lnoff[l]; q < P.lnoff[l + 1]; ++q) rows += P.ns[P.lnodes[q]] + P.ms[P.lnodes[q]];
+    for (int q = P.lnoff[l * P.nsys]; q < P.lnoff[(l + 1) * P.nsys]; ++q) rows += P.ns[P.lnodes[q]] + P.ms[P.lnodes[q]];
     tcap = std::max(tcap, rows);  // at most one tile per row
   }
   auto release = [&]() {
@@ -383,7 +399,7 @@ void tune_factor(pecs_ctx* c, PackedFactor& P, DevFactor& d, int nrhs) {
         } else {
           // the prefetching variant is a candidate on levels with few nodes,
           // where each lane's chain of load latencies sets the time
-          const bool few = P.lnoff[l + 1] - P.lnoff[l] <= 64;
+          const bool few = P.lnoff[(l + 1) * P.nsys] - P.lnoff[l * P.nsys] <= 64;
           for (int pf = 0; pf < (few ? 2 : 1); ++pf)
             for (int w : {8, 16, 32, 64})
               for (int m : {1, 2, 4, 8}) {
@@ -445,7 +461,7 @@ void tune_factor(pecs_ctx* c, PackedFactor& P, DevFactor& d, int nrhs) {
           // the level's factor bytes (MFMA-blocked copy when batched) and nodes
           double bytes = 0.0;
           int maxns = 0;
-          for (int q = P.lnoff[l]; q < P.lnoff[l + 1]; ++q) {
+          for (int q = P.lnoff[l * P.nsys]; q < P.lnoff[(l + 1) * P.nsys]; ++q) {
             const int sn = P.lnodes[q];
             maxns = std::max(maxns, P.ns[sn]);
             if (nrhs > 2) {
@@ -461,7 +477,7 @@ void tune_factor(pecs_ctx* c, PackedFactor& P, DevFactor& d, int nrhs) {
                        "[setup] tune n=%d level %d %s: W %d MAXR %d rows %d segment %d%s (%.3f ms) nodes %d max ns %d"
                        " factor %.1f MB (%.2f TB/s)\n",
                        P.n, l, fwd ? "fwd" : "bwd", bw, bm, br, bk, bpf ? " prefetch" : "", best,
-                       P.lnoff[l + 1] - P.lnoff[l], maxns, bytes / 1e6, bytes / (best * 1e-3) / 1e12);
+                       P.lnoff[(l + 1) * P.nsys] - P.lnoff[l * P.nsys], maxns, bytes / 1e6, bytes / (best * 1e-3) / 1e12);
         }
         if (fwd) {
           P.fw[l] = bw;
@@ -511,7 +527,7 @@ SolveCost solve_cost(int nrhs) {
 // the device (factor_on_device) after a host symbolic phase;
 // PECS_HOST_FACTOR=1 runs it on the host instead (cholesky_factor +
 // pack_factor), for comparison.
-FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
+FactorDev make_factor(pecs_ctx* c, const Systems& S, int leaf, int nrhs, const std::vector<int>& twin = {}) {
   const char* hf = std::getenv("PECS_HOST_FACTOR");
   const bool on_host = hf && std::string(hf) == "1";
   PackedFactor P;
@@ -532,11 +548,11 @@ FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
   const SolveCost cost = solve_cost(nrhs);
   const auto t0 = tnow();
   if (on_host) {
-    SupernodalFactor F = cholesky_factor(S, leaf, cost);
+    SupernodalFactor F = cholesky_factor(S, leaf, cost, twin);
     P = pack_factor(F);
   } else {
     FrontPlan plan;
-    SupernodalFactor F = cholesky_symbolic(S, leaf, plan, cost);
+    SupernodalFactor F = cholesky_symbolic(S, leaf, plan, cost, twin);
     P = pack_layout(F);
     if (trace) std::fprintf(stderr, "[setup] n=%d: symbolic + layout %.3f s\n", P.n, secs(t0, tnow()));
     HIPCHECK(hipMalloc(&dfwd, std::max<int64_t>(P.nvals, 1) * sizeof(double)));
@@ -560,7 +576,13 @@ FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
   D.perm = P.perm;
   D.goff = P.goff;
   D.xoff = P.xoff;
-  D.nnz = (double)P.nvals;
+  D.nsys = P.nsys;
+  D.sys_p0 = P.sys_p0;
+  for (int k = 0; k <= P.nsys; ++k) {
+    const int s = P.sys_node0[k], e = (int)P.p0.size();
+    D.sys_z0.push_back(s < e ? P.z_off[s] : P.zlen);
+    if (k > 0) D.nnz.push_back((double)((s < e ? P.fwd_off[s] : P.nvals) - P.fwd_off[P.sys_node0[k - 1]]));
+  }
   D.tri_bytes = P.tri_bytes;
   const int nn = (int)P.p0.size();
   DevFactor& d = D.d;
@@ -645,8 +667,8 @@ FactorDev make_factor(pecs_ctx* c, const BlockSPD& S, int leaf, int nrhs) {
   size_t part = 0;
   const int nrs = nrhs > 2 ? mfma_rhs_pad(nrhs) : nrhs;
   for (int l = 0; l < P.nlevels; ++l) {
-    if (P.fks[l] > 0) part = std::max(part, (size_t)(P.foff[l + 1] - P.foff[l]) * 64 * P.fm[l] * nrs);
-    if (P.bks[l] > 0) part = std::max(part, (size_t)(P.boff[l + 1] - P.boff[l]) * 64 * P.bm[l] * nrs);
+    if (P.fks[l] > 0) part = std::max(part, (size_t)(P.foff[(l + 1) * P.nsys] - P.foff[l * P.nsys]) * 64 * P.fm[l] * nrs);
+    if (P.bks[l] > 0) part = std::max(part, (size_t)(P.boff[(l + 1) * P.nsys] - P.boff[l * P.nsys]) * 64 * P.bm[l] * nrs);
   }
   d.Part = part > 0 ? dalloc<double>(c, part) : nullptr;
   D.foff = P.foff;
@@ -690,7 +712,7 @@ std::vector<int> wave_groups(int n, int nkey, KeyFn key) {
 }
 
 DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegionOps& O,
-                          const std::vector<int>& sigma, const FactorDev& F) {
+                          const std::vector<int>& sigma, const FactorDev& F, int sys) {
   DevRegion d{};
   const int nb = O.nb;
   d.N = R.N;
@@ -731,7 +753,7 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
   d.sigma_nb = upload(c, sigma);
   std::vector<int> pm((size_t)R.ncell * nb);
   for (int i = 0; i < R.ncell; ++i)
-    std::copy_n(&F.perm[F.cell_dof0[R.ci[i] + (size_t)R.NXg * R.cj[i]]], nb, &pm[(size_t)i * nb]);
+    std::copy_n(&F.perm[F.cell_dof0[sys][R.ci[i] + (size_t)R.NXg * R.cj[i]]], nb, &pm[(size_t)i * nb]);
   d.perm = upload(c, pm);
   if (!O.hang.empty()) {  // couplings across hanging faces, by target cell and by row cell
     std::vector<double> blk;
@@ -794,22 +816,25 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
   return d;
 }
 
-// single-carrier solve with its own factor (instance 0's scratch)
+// single-carrier solve with its own system (instance 0's scratch)
 void solve_carrier(pecs_ctx* c, int which, const double* b, double* x) {
-  const int reg = which / 2, car = which % 2;
+  const int reg = which / 2, car = which % 2, f = c->fr[reg];
   const DevRegion& R = reg == 0 ? c->Rs : c->Re;
-  FactorDev* F = reg == 0 ? c->Fs : c->Fe;
-  const bool share = reg == 0 ? c->share_s : c->share_e;
-  const FactorDev& Fc = (car == 1 && !share) ? F[1] : F[0];
+  const FactorDev& F = c->Fc[f];
   const double mu = c->P.mu[which];
   hipStream_t s = c->stream;
+  // (the region's row permutation is that of its first system)
+  const int64_t off = c->share[reg] || car == 0 ? 0 : c->gcar[reg];
+  double* g = c->g[f] + off;
+  double* sol = chol_solution(F.d, F.lv(), c->g[f]) + off;
   // W goes to the current part of x, which the recovery overwrites cell by cell
   SchurPair sp{};
-  sp.side[0] = schur_side_of(R, b, b, x, x, mu, mu, c->g[reg], c->g[reg], x, x, 0, 0, 0);
+  sp.side[0] = schur_side_of(R, b, b, x, x, mu, mu, g, g, x, x, 0, 0, 0);
   const DevRegion* rs[2] = {&R, nullptr};
   if (!R.table_f) HIPCHECK((hipError_t)launch_carrier_w(c->k, sp, 1, s));
   HIPCHECK((hipError_t)launch_schur_rhs(c->k, rs, sp, 1, s));
-  HIPCHECK((hipError_t)launch_chol_solve(Fc.d, Fc.lv(), c->g[reg], c->t[reg], 1, s));
+  HIPCHECK((hipError_t)launch_chol_solve(F.d, F.lv(), c->g[f], c->t[f], 1, s, c->sys[reg][car]));
+  sp.side[0].g[0] = sp.side[0].g[1] = sol;
   HIPCHECK((hipError_t)launch_schur_recover(c->k, rs, sp, 1, s));
 }
 
@@ -821,7 +846,8 @@ void poisson_solve_from_y(pecs_ctx* c, int i0, int n, double* out) {
   const int64_t nH = c->FH.n;
   HIPCHECK((hipError_t)launch_poisson_face(c->Pd, c->yP + i0 * c->ysz, c->rH, s, n, c->ysz, nH));
   HIPCHECK((hipError_t)launch_chol_solve(c->FH.d, c->FH.lv(), c->rH, c->tH, n, s));
-  HIPCHECK((hipError_t)launch_poisson_recover(c->k, c->Pd, c->rH, c->yP + i0 * c->ysz, out, s, n, nH, c->ysz, c->NP));
+  HIPCHECK((hipError_t)launch_poisson_recover(c->k, c->Pd, chol_solution(c->FH.d, c->FH.lv(), c->rH),
+                                              c->yP + i0 * c->ysz, out, s, n, nH, c->ysz, c->NP));
 }
 
 // Poisson condensation of instance i from its densities
@@ -844,9 +870,7 @@ void poisson_all_from_densities(pecs_ctx* c) {
 
 // Phases of one step (timing mode records an event on the context stream
 // after each): 0 rhs semiconductor, 1 rhs electrolyte, 2 Schur transforms of
-// both regions, 3 the carrier Cholesky solves of both regions (run
-// concurrently on the context stream and a second stream, joined before the
-// mark), 4 recoveries of both regions, 5 Poisson condensation, 6 Poisson
+// both regions, 3 the carrier Cholesky solves of both regions, 4 recoveries of both regions, 5 Poisson condensation, 6 Poisson
 // multiplier Cholesky, 7 Poisson recovery.  Every phase covers all instances.
 constexpr int NPHASE = 8;
 
@@ -859,20 +883,17 @@ struct PhaseMarks {
   }
 };
 
-// right-hand side slot of carrier car (0, 1) of instance i in a region's g / t
-inline int64_t gslot(const pecs_ctx* c, int reg, int car, int i) {
-  const int64_t n = reg == 0 ? c->Fs[0].n : c->Fe[0].n;
-  return ((int64_t)car * c->B + i) * n;
-}
-
-// one region's part of the step's Schur kernels (W in place of f_p in b)
-SchurSide step_side(pecs_ctx* c, int reg) {
+// one region's part of the step's Schur kernels (W in place of f_p in b; g:
+// the Schur right-hand sides, or the solutions)
+SchurSide step_side(pecs_ctx* c, int reg, bool solution) {
   const DevRegion& R = reg == 0 ? c->Rs : c->Re;
   const int64_t N = reg == 0 ? c->Ns : c->Ne;
-  const int64_t n = reg == 0 ? c->Fs[0].n : c->Fe[0].n;
+  const FactorDev& F = c->Fc[c->fr[reg]];
   const int c0 = 2 * reg, c1 = 2 * reg + 1;
-  return schur_side_of(R, c->b[c0], c->b[c1], c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1],
-                       c->g[reg] + gslot(c, reg, 0, 0), c->g[reg] + gslot(c, reg, 1, 0), c->u[c0], c->u[c1], N, n, N);
+  double* g = c->g[c->fr[reg]];
+  if (solution) g = chol_solution(F.d, F.lv(), g);
+  return schur_side_of(R, c->b[c0], c->b[c1], c->b[c0], c->b[c1], c->P.mu[c0], c->P.mu[c1], g, g + c->gcar[reg], c->u[c0],
+                       c->u[c1], N, F.n, N);
 }
 
 // right-hand sides of one region (reg 0, 1) or both (2), W in place of f_p
@@ -894,26 +915,30 @@ void step_rhs(pecs_ctx* c, int reg, hipStream_t s) {
 void step_schur(pecs_ctx* c, hipStream_t s) {
   const DevRegion* R[2] = {&c->Rs, &c->Re};
   SchurPair sp{};
-  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r);
+  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r, false);
   HIPCHECK((hipError_t)launch_schur_rhs(c->k, R, sp, 2, s, c->B));
 }
 
 void step_recover(pecs_ctx* c, hipStream_t s) {
   const DevRegion* R[2] = {&c->Rs, &c->Re};
   SchurPair sp{};
-  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r);
+  for (int r = 0; r < 2; ++r) sp.side[r] = step_side(c, r, true);
   HIPCHECK((hipError_t)launch_schur_recover(c->k, R, sp, 2, s, c->B));
 }
 
-void region_chol(pecs_ctx* c, int reg, hipStream_t s) {
-  FactorDev* F = reg == 0 ? c->Fs : c->Fe;
-  const bool share = reg == 0 ? c->share_s : c->share_e;
-  if (share) {  // both carriers of all instances against one factor read
-    HIPCHECK((hipError_t)launch_chol_solve(F[0].d, F[0].lv(), c->g[reg], c->t[reg], 2 * c->B, s));
-  } else {  // one factor per carrier, one after the other on the same stream (t is reused)
-    const int64_t h1 = gslot(c, reg, 1, 0);
-    HIPCHECK((hipError_t)launch_chol_solve(F[0].d, F[0].lv(), c->g[reg], c->t[reg], c->B, s));
-    HIPCHECK((hipError_t)launch_chol_solve(F[1].d, F[1].lv(), c->g[reg] + h1, c->t[reg], c->B, s));
+// The carrier solves.  Two factors share no data: the second one runs on the
+// side stream, so that its launches fill the GPU where the first one's leave
+// gaps.
+void step_chol(pecs_ctx* c, hipStream_t s) {
+  if (c->nf == 2) {
+    HIPCHECK(hipEventRecord(c->fork_ev, s));
+    HIPCHECK(hipStreamWaitEvent(c->side, c->fork_ev, 0));
+  }
+  for (int f = 0; f < c->nf; ++f)
+    HIPCHECK((hipError_t)launch_chol_solve(c->Fc[f].d, c->Fc[f].lv(), c->g[f], c->t[f], c->nrhs_f[f], f ? c->side : s));
+  if (c->nf == 2) {
+    HIPCHECK(hipEventRecord(c->join_ev, c->side));
+    HIPCHECK(hipStreamWaitEvent(s, c->join_ev, 0));
   }
 }
 
@@ -928,7 +953,8 @@ void poisson_step(pecs_ctx* c, PhaseMarks* pm = nullptr) {
   HIPCHECK((hipError_t)launch_poisson_face(c->Pd, c->yP, c->rH, s, B, c->ysz, nH));
   HIPCHECK((hipError_t)launch_chol_solve(c->FH.d, c->FH.lv(), c->rH, c->tH, B, s));
   if (pm) pm->mark();
-  HIPCHECK((hipError_t)launch_poisson_recover(c->k, c->Pd, c->rH, c->yP, c->pv, s, B, nH, c->ysz, c->NP));
+  HIPCHECK((hipError_t)launch_poisson_recover(c->k, c->Pd, chol_solution(c->FH.d, c->FH.lv(), c->rH), c->yP, c->pv, s, B,
+                                              nH, c->ysz, c->NP));
   if (pm) pm->mark();
 }
 
@@ -950,14 +976,7 @@ void step_once(pecs_ctx* c) {
   }
   step_schur(c, s);
   pm.mark();
-  // the two regions' solves share no data: the electrolyte runs on the side
-  // stream so its launches fill the GPU where the semiconductor's leave gaps
-  HIPCHECK(hipEventRecord(c->fork_ev, s));
-  HIPCHECK(hipStreamWaitEvent(c->side, c->fork_ev, 0));
-  region_chol(c, 0, s);
-  region_chol(c, 1, c->side);
-  HIPCHECK(hipEventRecord(c->join_ev, c->side));
-  HIPCHECK(hipStreamWaitEvent(s, c->join_ev, 0));
+  step_chol(c, s);
   pm.mark();
   step_recover(c, s);
   pm.mark();
@@ -1177,8 +1196,6 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     if (tr && std::string(tr) == "1")
       std::fprintf(stderr, "[setup] mesh + local operators %.3f s\n",
                    std::chrono::duration<double>(tf - t0).count());
-    c->share_s = c->P.mu[0] == c->P.mu[1];
-    c->share_e = c->P.mu[2] == c->P.mu[3];
     auto timed = [&](const char* what, auto&& build) {
       const auto ta = std::chrono::steady_clock::now();
       BlockSPD S = build();
@@ -1190,11 +1207,37 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     auto schur = [&](const Region& R, const LdgRegionOps& o, double mu) {
       return timed("Schur", [&] { return schur_matrix(R, o, mu); });
     };
-    c->Fs[0] = make_factor(c.get(), schur(c->mesh.semi, os, c->P.mu[0]), leaf, c->share_s ? 2 * B : B);
-    if (!c->share_s) c->Fs[1] = make_factor(c.get(), schur(c->mesh.semi, os, c->P.mu[1]), leaf, B);
-    c->Fe[0] = make_factor(c.get(), schur(c->mesh.elec, oe, c->P.mu[2]), leaf, c->share_e ? 2 * B : B);
-    if (!c->share_e) c->Fe[1] = make_factor(c.get(), schur(c->mesh.elec, oe, c->P.mu[3]), leaf, B);
-    c->FH = make_factor(c.get(), timed("multiplier", [&] { return multiplier_matrix(c->mesh, op, T); }), leaf, B);
+    for (int r = 0; r < 2; ++r) {
+      c->share[r] = c->P.mu[2 * r] == c->P.mu[2 * r + 1];
+      c->fr[r] = r == 0 || c->share[1] == c->share[0] ? 0 : 1;
+      c->nf = c->fr[r] + 1;
+    }
+    for (int f = 0; f < c->nf; ++f) {
+      std::vector<BlockSPD> mats;
+      std::vector<int> twin;
+      mats.reserve(4);
+      for (int r = 0; r < 2; ++r) {
+        if (c->fr[r] != f) continue;
+        c->nrhs_f[f] = c->share[r] ? 2 * B : B;
+        for (int car = 0; car < 2; ++car) {
+          if (car == 0 || !c->share[r]) {
+            mats.push_back(r == 0 ? schur(c->mesh.semi, os, c->P.mu[car]) : schur(c->mesh.elec, oe, c->P.mu[2 + car]));
+            twin.push_back(r);
+          }
+          c->sys[r][car] = (int)mats.size() - 1;
+        }
+      }
+      Systems S;
+      for (const BlockSPD& m : mats) S.push_back(&m);
+      c->Fc[f] = make_factor(c.get(), S, leaf, c->nrhs_f[f], twin);
+      for (int r = 0; r < 2; ++r)
+        if (c->fr[r] == f)
+          c->gcar[r] = c->share[r] ? (int64_t)B * c->Fc[f].n : c->Fc[f].sys_p0[c->sys[r][1]] - c->Fc[f].sys_p0[c->sys[r][0]];
+    }
+    {
+      const BlockSPD H = timed("multiplier", [&] { return multiplier_matrix(c->mesh, op, T); });
+      c->FH = make_factor(c.get(), {&H}, leaf, B);
+    }
     c->factor_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - tf).count();
     // reference tables
     DevTabs& tb = c->tabs;
@@ -1211,8 +1254,8 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     tb.fpsix = upload(c.get(), T.fpsix);
     tb.fpsiy = upload(c.get(), T.fpsiy);
     // regions
-    c->Rs = make_region_dev(c.get(), 0, c->mesh.semi, os, c->mesh.semi_sigma_nb, c->Fs[0]);
-    c->Re = make_region_dev(c.get(), 1, c->mesh.elec, oe, c->mesh.elec_sigma_nb, c->Fe[0]);
+    c->Rs = make_region_dev(c.get(), 0, c->mesh.semi, os, c->mesh.semi_sigma_nb, c->Fc[c->fr[0]], c->sys[0][0]);
+    c->Re = make_region_dev(c.get(), 1, c->mesh.elec, oe, c->mesh.elec_sigma_nb, c->Fc[c->fr[1]], c->sys[1][0]);
     // Poisson
     DevPoisson& P = c->Pd;
     const SolarCellMesh& m = c->mesh;
@@ -1247,7 +1290,7 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     for (int G = 0; G < m.NX * m.NY; ++G)
       for (int t = 0; t < op.ndof_owner[G]; ++t) {
         owner_of[op.owner_base[G] + t] = G;
-        mperm[op.owner_base[G] + t] = c->FH.perm[c->FH.cell_dof0[G] + t];
+        mperm[op.owner_base[G] + t] = c->FH.perm[c->FH.cell_dof0[0][G] + t];
       }
     gauss01(c->k, gx, gw);
     for (int K = 0; K < m.ncellP; ++K)
@@ -1314,11 +1357,12 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     // scratch right-hand sides of a solve: 2B (or B) h-major, or the padded
     // interleaved block of the MFMA sweep
     auto scratch_rhs = [](int nrhs) { return nrhs > 2 ? mfma_rhs_pad(nrhs) : nrhs; };
-    for (int r = 0; r < 2; ++r) {
-      const int64_t n = r == 0 ? c->Fs[0].n : c->Fe[0].n;
-      c->g[r] = dalloc<double>(c.get(), 2 * B * n);
-      c->t[r] = dalloc<double>(c.get(), std::max(2 * B, scratch_rhs(2 * B)) * n);
-      HIPCHECK(hipMemset(c->t[r], 0, std::max(2 * B, scratch_rhs(2 * B)) * n * sizeof(double)));
+    for (int f = 0; f < c->nf; ++f) {
+      const int64_t n = c->Fc[f].n, nr = c->nrhs_f[f];
+      c->g[f] = dalloc<double>(c.get(), nr * n);
+      c->t[f] = dalloc<double>(c.get(), std::max<int64_t>(nr, scratch_rhs((int)nr)) * n);
+      HIPCHECK(hipMemset(c->g[f], 0, nr * n * sizeof(double)));
+      HIPCHECK(hipMemset(c->t[f], 0, std::max<int64_t>(nr, scratch_rhs((int)nr)) * n * sizeof(double)));
     }
     c->ysz = (int64_t)m.ncellP * op.nloc;
     c->yP = dalloc<double>(c.get(), B * c->ysz);
@@ -1453,15 +1497,16 @@ int pecs_sizes(pecs_ctx* ctx, int64_t* ns, int64_t* ne, int64_t* np) {
 
 int pecs_stats(pecs_ctx* ctx, double* o, int n) {
   if (!ctx || !o) return -1;
-  const FactorDev* fs[5] = {&ctx->Fs[0], &ctx->Fs[1], &ctx->Fe[0], &ctx->Fe[1], &ctx->FH};
-  double dev_s = 0.0, dev_flops = 0.0;
-  for (const FactorDev* f : fs) {
-    dev_s += f->device_seconds;
-    dev_flops += f->device_flops;
+  double dev_s = ctx->FH.device_seconds, dev_flops = ctx->FH.device_flops, nnz[2] = {};
+  for (int f = 0; f < ctx->nf; ++f) {
+    dev_s += ctx->Fc[f].device_seconds;
+    dev_flops += ctx->Fc[f].device_flops;
   }
-  const double v[12] = {ctx->Fs[0].nnz + ctx->Fs[1].nnz, ctx->Fe[0].nnz + ctx->Fe[1].nnz, ctx->FH.nnz,
-                        ctx->setup_seconds, ctx->factor_seconds, (double)ctx->Fs[0].nlevels,
-                        (double)ctx->Fe[0].nlevels, (double)ctx->FH.nlevels, (double)ctx->Fs[0].n,
+  for (int r = 0; r < 2; ++r)
+    for (int car = 0; car < (ctx->share[r] ? 1 : 2); ++car) nnz[r] += ctx->Fc[ctx->fr[r]].nnz[ctx->sys[r][car]];
+  const FactorDev &F0 = ctx->Fc[ctx->fr[0]], &F1 = ctx->Fc[ctx->fr[1]];
+  const double v[12] = {nnz[0], nnz[1], ctx->FH.nnz[0], ctx->setup_seconds, ctx->factor_seconds, (double)F0.nlevels,
+                        (double)F1.nlevels, (double)ctx->FH.nlevels, (double)F0.rows(ctx->sys[0][0]),
                         (double)ctx->FH.n, dev_s, dev_flops};
   for (int i = 0; i < n && i < 12; ++i) o[i] = v[i];
   return 0;
@@ -1628,29 +1673,33 @@ int pecs_solve_dev_noalloc(pecs_ctx* ctx, int which, const double* rhs, double* 
     if (which >= PECS_ELECTRONS && which <= PECS_OXIDANTS) {
       // scratch: X (n), Z (zlen) of the factor, then the Schur right-hand side
       // g (n) and the forward output t (n); every entry is written before it is read
-      const int reg = which / 2, car = which % 2;
+      const int reg = which / 2, car = which % 2, k = ctx->sys[reg][car];
       const DevRegion& R = reg == 0 ? ctx->Rs : ctx->Re;
-      FactorDev* F = reg == 0 ? ctx->Fs : ctx->Fe;
-      const bool share = reg == 0 ? ctx->share_s : ctx->share_e;
-      const FactorDev& Fc = (car == 1 && !share) ? F[1] : F[0];
-      const size_t n = (size_t)Fc.n, zl = (size_t)std::max<int64_t>(Fc.d.zlen, 1);
+      const FactorDev& F = ctx->Fc[ctx->fr[reg]];
+      const int64_t p0 = F.sys_p0[k], z0 = F.sys_z0[k];
+      const size_t n = (size_t)F.rows(k), zl = (size_t)std::max<int64_t>(F.sys_z0[k + 1] - z0, 1);
       const size_t need = 3 * n + zl;
       if (need > cap)
         throw std::runtime_error("pecs_solve_dev_noalloc: carrier solve needs " + std::to_string(need * 8) +
                                  " bytes of scratch, above the limit of " + std::to_string(cap * 8));
-      DevFactor d = Fc.d;
-      d.X = base;
-      d.Z = base + n;
+      // the solve touches only the system's own rows and update slots: the
+      // factor's scratch vectors begin so far before the array that these fall
+      // on it (the region's row permutation is that of its first system)
+      DevFactor d = F.d;
+      d.X = base - p0;
+      d.Z = base + n - z0;
       d.Part = nullptr;
-      double* g = base + n + zl;
+      double* g = base + n + zl - p0;
       double* t = g + n;
+      const int64_t off = ctx->share[reg] || car == 0 ? 0 : ctx->gcar[reg];
       const double mu = ctx->P.mu[which];
       SchurPair sp{};
-      sp.side[0] = schur_side_of(R, rhs, rhs, x, x, mu, mu, g, g, x, x, 0, 0, 0);
+      sp.side[0] = schur_side_of(R, rhs, rhs, x, x, mu, mu, g + off, g + off, x, x, 0, 0, 0);
       const DevRegion* rs[2] = {&R, nullptr};
       if (!R.table_f) HIPCHECK((hipError_t)launch_carrier_w(ctx->k, sp, 1, s));
       HIPCHECK((hipError_t)launch_schur_rhs(ctx->k, rs, sp, 1, s));
-      HIPCHECK((hipError_t)launch_chol_solve(d, Fc.lv(), g, t, 1, s));
+      HIPCHECK((hipError_t)launch_chol_solve(d, F.lv(), g, t, 1, s, k));
+      sp.side[0].g[0] = sp.side[0].g[1] = chol_solution(d, F.lv(), g) + off;
       HIPCHECK((hipError_t)launch_schur_recover(ctx->k, rs, sp, 1, s));
     } else if (which == PECS_POISSON) {
       // scratch: X (nH), Z (zlen) of the multiplier factor, the condensed
@@ -1672,7 +1721,8 @@ int pecs_solve_dev_noalloc(pecs_ctx* ctx, int which, const double* rhs, double* 
       HIPCHECK((hipError_t)launch_poisson_cell_from_b(ctx->Pd, rhs, y, s));
       HIPCHECK((hipError_t)launch_poisson_face(ctx->Pd, y, r, s, 1, ctx->ysz, (int64_t)nH));
       HIPCHECK((hipError_t)launch_chol_solve(d, FH.lv(), r, t, 1, s));
-      HIPCHECK((hipError_t)launch_poisson_recover(ctx->k, ctx->Pd, r, y, x, s, 1, (int64_t)nH, ctx->ysz, ctx->NP));
+      HIPCHECK((hipError_t)launch_poisson_recover(ctx->k, ctx->Pd, chol_solution(d, FH.lv(), r), y, x, s, 1, (int64_t)nH,
+                                                  ctx->ysz, ctx->NP));
     } else {
       throw std::runtime_error("unknown system id");
     }
@@ -2125,7 +2175,7 @@ int pecs_uniform_lists(pecs_ctx* ctx, int* flags) {
 
 int pecs_sweep_config(pecs_ctx* ctx, int which, int* out, int n, int* nlevels) {
   PECS_TRY(ctx, {
-    const FactorDev* F = which == 0 ? &ctx->Fs[0] : which == 1 ? &ctx->Fe[0] : which == 2 ? &ctx->FH : nullptr;
+    const FactorDev* F = which == 0 || which == 1 ? &ctx->Fc[ctx->fr[which]] : which == 2 ? &ctx->FH : nullptr;
     if (!F) throw std::runtime_error("which must be 0 (semiconductor), 1 (electrolyte) or 2 (Poisson multipliers)");
     if (nlevels) *nlevels = F->nlevels;
     for (int l = 0; l < F->nlevels && 6 * l + 5 < n; ++l) {
@@ -2165,8 +2215,7 @@ int pecs_factor_bytes(pecs_ctx* ctx, int which, double* bytes) {
   // 2: Poisson multipliers): the lower triangles of the inverse diagonal
   // blocks and the off-diagonal panels, read once per sweep, 8 B per value.
   if (!ctx || !bytes) return -1;
-  const FactorDev* F = which == 0 ? &ctx->Fs[0] : (which == 1 ? &ctx->Fe[0] : &ctx->FH);
-  *bytes = F->tri_bytes;
+  *bytes = which == 0 || which == 1 ? ctx->Fc[ctx->fr[which]].tri_bytes[ctx->sys[which][0]] : ctx->FH.tri_bytes[0];
   return 0;
 }
 

@@ -19,53 +19,76 @@ struct NDNode {
   int parent = -1;
 };
 
-// The couplings of S between single DoFs: neighbours of each DoF (grid-order
-// numbering), from the nonzero entries of S's blocks in either triangle.
+// The couplings between single DoFs of the systems: neighbours of each DoF
+// (grid-order numbering, one system after the other), from the nonzero entries
+// of the blocks in either triangle, of the system or of one of its twins.
 struct DofGraph {
-  std::vector<int> dof0;     // per cell, and the total
-  std::vector<int> cell;     // per DoF
-  std::vector<int64_t> ptr;  // per DoF
+  std::vector<std::vector<int>> dof0;  // per system: per cell, and its end
+  std::vector<int> cell;               // per DoF
+  std::vector<int> sys;                // per DoF
+  std::vector<int64_t> ptr;            // per DoF
   std::vector<int> adj;
   int n = 0;
 
-  explicit DofGraph(const BlockSPD& S) {
-    const int NG = S.NXc * S.NYc, no = S.noff();
-    dof0.assign(NG + 1, 0);
-    for (int X = 0; X < NG; ++X) dof0[X + 1] = dof0[X] + S.ndof[X];
-    n = dof0[NG];
+  DofGraph(const Systems& Ss, const std::vector<int>& twin) {
+    for (const BlockSPD* S : Ss) {
+      const int NG = S->NXc * S->NYc;
+      std::vector<int> d(NG + 1, n);
+      for (int X = 0; X < NG; ++X) d[X + 1] = d[X] + S->ndof[X];
+      n = d[NG];
+      dof0.push_back(std::move(d));
+    }
     cell.resize(n);
-    for (int X = 0; X < NG; ++X)
-      for (int d = dof0[X]; d < dof0[X + 1]; ++d) cell[d] = X;
-    std::vector<int> opp(no, -1);  // the opposite offset
-    for (int o = 0; o < no; ++o)
-      for (int q = 0; q < no; ++q)
-        if (S.offi[q] == -S.offi[o] && S.offj[q] == -S.offj[o]) opp[o] = q;
+    sys.resize(n);
+    for (size_t k = 0; k < Ss.size(); ++k)
+      for (int X = 0; X + 1 < (int)dof0[k].size(); ++X)
+        for (int d = dof0[k][X]; d < dof0[k][X + 1]; ++d) {
+          cell[d] = X;
+          sys[d] = (int)k;
+        }
     ptr.assign((size_t)n + 1, 0);
     for (int pass = 0; pass < 2; ++pass) {
+      for (size_t k = 0; k < Ss.size(); ++k) {
+        const BlockSPD& S = *Ss[k];
+        const int NG = S.NXc * S.NYc, no = S.noff();
+        std::vector<const BlockSPD*> like;  // the system and its twins
+        for (size_t j = 0; j < Ss.size(); ++j)
+          if (j == k || (!twin.empty() && twin[j] == twin[k])) like.push_back(Ss[j]);
+        for (const BlockSPD* T : like)
+          if (T->ndof != S.ndof || T->offi != S.offi || T->offj != S.offj)
+            throw std::runtime_error("twin systems on different grids");
+        std::vector<int> opp(no, -1);  // the opposite offset
+        for (int o = 0; o < no; ++o)
+          for (int q = 0; q < no; ++q)
+            if (S.offi[q] == -S.offi[o] && S.offj[q] == -S.offj[o]) opp[o] = q;
 #pragma omp parallel for schedule(dynamic, 256)
-      for (int X = 0; X < NG; ++X) {
-        const int nx = S.ndof[X];
-        if (nx == 0) continue;
-        const int xi = X % S.NXc, xj = X / S.NXc;
-        for (int a = 0; a < nx; ++a) {
-          int64_t cnt = 0;
-          const int64_t at = ptr[dof0[X] + a];
-          for (int o = 0; o < no; ++o) {
-            const int yi = xi + S.offi[o], yj = xj + S.offj[o];
-            if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
-            const int Y = yi + S.NXc * yj, ny = S.ndof[Y];
-            const std::vector<double>& B = S.blk[(size_t)X * no + o];
-            static const std::vector<double> none;
-            const std::vector<double>& C = opp[o] >= 0 ? S.blk[(size_t)Y * no + opp[o]] : none;
-            if (ny == 0 || (B.empty() && C.empty())) continue;
-            for (int b = 0; b < ny; ++b) {
-              if (!((!B.empty() && B[(size_t)a * ny + b] != 0.0) || (!C.empty() && C[(size_t)b * nx + a] != 0.0)))
-                continue;
-              if (pass) adj[at + cnt] = dof0[Y] + b;
-              ++cnt;
+        for (int X = 0; X < NG; ++X) {
+          const int nx = S.ndof[X];
+          if (nx == 0) continue;
+          const int xi = X % S.NXc, xj = X / S.NXc;
+          for (int a = 0; a < nx; ++a) {
+            int64_t cnt = 0;
+            const int64_t at = ptr[dof0[k][X] + a];
+            for (int o = 0; o < no; ++o) {
+              const int yi = xi + S.offi[o], yj = xj + S.offj[o];
+              if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
+              const int Y = yi + S.NXc * yj, ny = S.ndof[Y];
+              for (int b = 0; b < ny; ++b) {
+                bool nz = false;
+                for (const BlockSPD* T : like) {
+                  const std::vector<double>& B = T->blk[(size_t)X * no + o];
+                  nz = nz || (!B.empty() && B[(size_t)a * ny + b] != 0.0);
+                  if (nz || opp[o] < 0) continue;
+                  const std::vector<double>& C = T->blk[(size_t)Y * no + opp[o]];
+                  nz = !C.empty() && C[(size_t)b * nx + a] != 0.0;
+                }
+                if (!nz) continue;
+                if (pass) adj[at + cnt] = dof0[k][Y] + b;
+                ++cnt;
+              }
             }
+            if (!pass) ptr[dof0[k][X] + a + 1] = cnt;
           }
-          if (!pass) ptr[dof0[X] + a + 1] = cnt;
         }
       }
       if (!pass) {
@@ -79,13 +102,15 @@ struct DofGraph {
 struct NDBuilder {
   const BlockSPD& S;
   const DofGraph& G;
+  const std::vector<int>& dof0;  // of this system
   int leaf, reach = 0;
-  std::vector<NDNode> nodes;  // postorder
+  std::vector<NDNode>& nodes;  // postorder
   std::vector<char> taken;    // per DoF: already in a separator
   // scratch of cover(): per DoF its index on its side of the cut
   std::vector<int> side;
 
-  NDBuilder(const BlockSPD& s, const DofGraph& g, int l) : S(s), G(g), leaf(l), taken(g.n, 0), side(g.n, -1) {
+  NDBuilder(const BlockSPD& s, const DofGraph& g, int k, int l, std::vector<NDNode>& out)
+      : S(s), G(g), dof0(g.dof0[k]), leaf(l), nodes(out), taken(g.n, 0), side(g.n, -1) {
     for (int o = 0; o < S.noff(); ++o) reach = std::max({reach, std::abs(S.offi[o]), std::abs(S.offj[o])});
   }
 
@@ -101,7 +126,7 @@ struct NDBuilder {
     for (int u = u0; u < u1; ++u)
       for (int t = lo; t < mid; ++t) {
         const int X = vertical ? t + S.NXc * u : u + S.NXc * t;
-        for (int d = G.dof0[X]; d < G.dof0[X + 1]; ++d) {
+        for (int d = dof0[X]; d < dof0[X + 1]; ++d) {
           if (taken[d]) continue;
           const size_t before = e.size();
           for (int64_t q = G.ptr[d]; q < G.ptr[d + 1]; ++q) {
@@ -210,7 +235,7 @@ struct NDBuilder {
     if (ni * nj <= leaf || (ni == 1 && nj == 1)) {
       for (int j = j0; j < j1; ++j)
         for (int i = i0; i < i1; ++i)
-          for (int d = G.dof0[i + S.NXc * j]; d < G.dof0[i + S.NXc * j + 1]; ++d)
+          for (int d = dof0[i + S.NXc * j]; d < dof0[i + S.NXc * j + 1]; ++d)
             if (!taken[d]) node.dofs.push_back(d);
       return node.dofs.empty() ? -1 : push(std::move(node));
     }
@@ -475,10 +500,10 @@ std::vector<NDNode> merge_levels(const std::vector<NDNode>& nodes, const std::ve
 }
 
 // Ordering, supernodes, row structure and levels (no numeric values).
-SupernodalFactor symbolic(const BlockSPD& S, const DofGraph& G, int leaf_cells, const SolveCost& cost) {
-  NDBuilder nd(S, G, leaf_cells);
-  nd.build(0, S.NXc, 0, S.NYc);
-  std::vector<NDNode> nodes = std::move(nd.nodes);
+SupernodalFactor symbolic(const Systems& S, const DofGraph& G, int leaf_cells, const SolveCost& cost) {
+  std::vector<NDNode> nodes;
+  for (size_t k = 0; k < S.size(); ++k)
+    NDBuilder(*S[k], G, (int)k, leaf_cells, nodes).build(0, S[k]->NXc, 0, S[k]->NYc);
   SupernodalFactor F;
   std::vector<int> p1;
   std::vector<std::vector<int>> st;
@@ -489,7 +514,15 @@ SupernodalFactor symbolic(const BlockSPD& S, const DofGraph& G, int leaf_cells, 
   }
   const int nn = (int)nodes.size();
   F.n = G.n;
-  F.cell_dof0.assign(G.dof0.begin(), G.dof0.end() - 1);
+  for (const std::vector<int>& d : G.dof0) {
+    F.sys_p0.push_back(d.front());
+    F.cell_dof0.emplace_back(d.begin(), d.end() - 1);
+  }
+  F.sys_p0.push_back(G.n);
+  F.sys_node0.assign(S.size() + 1, nn);
+  for (int s = nn; s-- > 0;)
+    if (!nodes[s].dofs.empty()) F.sys_node0[G.sys[nodes[s].dofs[0]]] = s;
+  for (size_t k = S.size(); k-- > 0;) F.sys_node0[k] = std::min(F.sys_node0[k], F.sys_node0[k + 1]);
   const std::vector<int> lv = tree_levels(nodes, F.nlevels);
   F.level_nodes.assign(F.nlevels, {});
   F.nodes.resize(nn);
@@ -557,10 +590,10 @@ std::vector<int> child_map(const SupernodalFactor& F, int c) {
 
 }  // namespace
 
-SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveCost& cost) {
-  const int no = S.noff();
-  const DofGraph G(S);
-  SupernodalFactor F = symbolic(S, G, leaf_cells, cost);
+SupernodalFactor cholesky_factor(const Systems& Ss, int leaf_cells, const SolveCost& cost,
+                                 const std::vector<int>& twin) {
+  const DofGraph G(Ss, twin);
+  SupernodalFactor F = symbolic(Ss, G, leaf_cells, cost);
   const int nn = (int)F.nodes.size();
   std::vector<int> dof_at(F.n);  // permuted index -> DoF
   for (int d = 0; d < F.n; ++d) dof_at[F.perm[d]] = d;
@@ -584,7 +617,10 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveC
     for (int r = 0; r < ms; ++r) loc[F.rows[N.rows_off + r]] = ns + r;
     // original entries (p, q), p own and p <= q, into column p
     for (int c = 0; c < ns; ++c) {
-      const int d = dof_at[N.p0 + c], X = G.cell[d], a = d - G.dof0[X];
+      const int d = dof_at[N.p0 + c], X = G.cell[d];
+      const BlockSPD& S = *Ss[G.sys[d]];
+      const std::vector<int>& dof0 = G.dof0[G.sys[d]];
+      const int a = d - dof0[X], no = S.noff();
       const int xi = X % S.NXc, xj = X / S.NXc;
       for (int o = 0; o < no; ++o) {
         const int yi = xi + S.offi[o], yj = xj + S.offj[o];
@@ -594,7 +630,7 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveC
         if (B.empty()) continue;
         for (int b = 0; b < ny; ++b) {
           const double v = B[(size_t)a * ny + b];
-          const int q = F.perm[G.dof0[Y] + b];
+          const int q = F.perm[dof0[Y] + b];
           if (v == 0.0 || q < N.p0 + c) continue;
           const int r = q < N.p0 + ns ? q - N.p0 : loc[q];
           Fr[(size_t)r * nf + c] += v;
@@ -653,31 +689,34 @@ SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveC
   return F;
 }
 
-SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost) {
-  const int no = S.noff();
-  const DofGraph G(S);
-  SupernodalFactor F = symbolic(S, G, leaf_cells, cost);
+SupernodalFactor cholesky_symbolic(const Systems& Ss, int leaf_cells, FrontPlan& plan, const SolveCost& cost,
+                                   const std::vector<int>& twin) {
+  const DofGraph G(Ss, twin);
+  SupernodalFactor F = symbolic(Ss, G, leaf_cells, cost);
   const int nn = (int)F.nodes.size();
-  const int NG = S.NXc * S.NYc;
   plan = FrontPlan{};
   plan.nlevels = F.nlevels;
   // S blocks, concatenated
   std::vector<const std::vector<double>*> blocks;
   int64_t sv = 0;
-  for (int X = 0; X < NG; ++X)
-    for (int o = 0; o < no; ++o) {
-      const auto& B = S.blk[(size_t)X * no + o];
-      if (B.empty()) continue;
-      const int Y = X + S.offi[o] + S.NXc * S.offj[o];
-      if (S.ndof[X] == 0 || S.ndof[Y] == 0) continue;
-      blocks.push_back(&B);
-      plan.sb_src.push_back(sv);
-      plan.sb_x.push_back(G.dof0[X]);
-      plan.sb_y.push_back(G.dof0[Y]);
-      plan.sb_nx.push_back(S.ndof[X]);
-      plan.sb_ny.push_back(S.ndof[Y]);
-      sv += (int64_t)B.size();
-    }
+  for (size_t k = 0; k < Ss.size(); ++k) {
+    const BlockSPD& S = *Ss[k];
+    const int NG = S.NXc * S.NYc, no = S.noff();
+    for (int X = 0; X < NG; ++X)
+      for (int o = 0; o < no; ++o) {
+        const auto& B = S.blk[(size_t)X * no + o];
+        if (B.empty()) continue;
+        const int Y = X + S.offi[o] + S.NXc * S.offj[o];
+        if (S.ndof[X] == 0 || S.ndof[Y] == 0) continue;
+        blocks.push_back(&B);
+        plan.sb_src.push_back(sv);
+        plan.sb_x.push_back(G.dof0[k][X]);
+        plan.sb_y.push_back(G.dof0[k][Y]);
+        plan.sb_nx.push_back(S.ndof[X]);
+        plan.sb_ny.push_back(S.ndof[Y]);
+        sv += (int64_t)B.size();
+      }
+  }
   plan.svals.resize(sv);
 #pragma omp parallel for schedule(static)
   for (size_t i = 0; i < blocks.size(); ++i)
@@ -786,8 +825,14 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
   const int nn = (int)F.nodes.size();
   P.n = F.n;
   P.nlevels = F.nlevels;
+  P.nsys = F.nsys();
+  P.sys_p0 = F.sys_p0;
+  P.sys_node0 = F.sys_node0;
   P.cell_dof0 = F.cell_dof0;
   P.perm = F.perm;
+  P.tri_bytes.assign(P.nsys, 0.0);
+  const int K = P.nsys;
+  int sys = 0;
   P.p0.resize(nn);
   P.ns.resize(nn);
   P.ms.resize(nn);
@@ -807,7 +852,8 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
     P.z_off[s] = zl;
     nf += n_ * (n_ + 1) / 2 + m_ * n_;
     zl += m_;
-    P.tri_bytes += 2.0 * 8.0 * (0.5 * n_ * (n_ + 1.0) + (double)m_ * n_);
+    while (s >= F.sys_node0[sys + 1]) ++sys;
+    P.tri_bytes[sys] += 2.0 * 8.0 * (0.5 * n_ * (n_ + 1.0) + (double)m_ * n_);
   }
   P.zlen = zl;
   P.nvals = nf;
@@ -817,8 +863,8 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
     while (w < 64 && w * 8 < mean) w *= 2;
     return w;
   };
-  P.goff.assign(F.nlevels + 1, 0);
-  P.xoff.assign(F.nlevels + 1, 0);
+  P.goff.assign(F.nlevels * K + 1, 0);
+  P.xoff.assign(F.nlevels * K + 1, 0);
   P.fw.assign(F.nlevels, 64);
   P.bw.assign(F.nlevels, 64);
   P.fm.assign(F.nlevels, 1);
@@ -827,7 +873,7 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
   P.bpf.assign(F.nlevels, 0);
   P.frows.assign(F.nlevels, 4);
   P.brows.assign(F.nlevels, 4);
-  P.lnoff.assign(F.nlevels + 1, 0);
+  P.lnoff.assign(F.nlevels * K + 1, 0);
   for (int l = 0; l < F.nlevels; ++l) {
     double fl = 0, fr = 0, bl = 0, br = 0;
     for (int s : F.level_nodes[l]) {
@@ -851,23 +897,27 @@ PackedFactor pack_layout(const SupernodalFactor& F) {
     P.brows[l] = height(P.bw[l], br);
     P.fm[l] = std::max(1, P.frows[l] / (256 / P.fw[l]));
     P.bm[l] = std::max(1, P.brows[l] / (256 / P.bw[l]));
-    P.goff[l] = (int)P.lrows.size();
-    P.xoff[l] = (int)P.xidx.size();
-    P.lnoff[l] = (int)P.lnodes.size();
-    for (int s : F.level_nodes[l]) {
-      P.lnodes.push_back(s);
-      for (int r = 0; r < P.ns[s]; ++r) P.lrows.push_back(P.p0[s] + r);
-      for (int i = 0; i < P.ms[s]; ++i) P.xidx.push_back(P.rows_off[s] + i);
+    size_t i = 0;  // (a level's nodes ascend, so its systems follow each other)
+    for (int k = 0; k < K; ++k) {
+      P.goff[l * K + k] = (int)P.lrows.size();
+      P.xoff[l * K + k] = (int)P.xidx.size();
+      P.lnoff[l * K + k] = (int)P.lnodes.size();
+      for (; i < F.level_nodes[l].size() && F.level_nodes[l][i] < F.sys_node0[k + 1]; ++i) {
+        const int s = F.level_nodes[l][i];
+        P.lnodes.push_back(s);
+        for (int r = 0; r < P.ns[s]; ++r) P.lrows.push_back(P.p0[s] + r);
+        for (int j = 0; j < P.ms[s]; ++j) P.xidx.push_back(P.rows_off[s] + j);
+      }
     }
   }
-  P.goff[F.nlevels] = (int)P.lrows.size();
-  P.xoff[F.nlevels] = (int)P.xidx.size();
-  P.lnoff[F.nlevels] = (int)P.lnodes.size();
+  P.goff[F.nlevels * K] = (int)P.lrows.size();
+  P.xoff[F.nlevels * K] = (int)P.xidx.size();
+  P.lnoff[F.nlevels * K] = (int)P.lnodes.size();
   rebuild_tiles(P);
   P.rows = F.rows;
   P.cptr = F.contrib_ptr;
   // the solves read the leaf level's right-hand side without a gather
-  for (int q = P.goff[0]; q < P.goff[1]; ++q)
+  for (int q = P.goff[0]; q < P.goff[K]; ++q)
     if (P.cptr[P.lrows[q] + 1] != P.cptr[P.lrows[q]])
       throw std::runtime_error("pack_layout: a leaf-level row is owed contributions");
   P.czidx.resize(F.contrib_node.size());
@@ -992,29 +1042,22 @@ void pack_blocked(PackedFactor& P) {
   std::vector<double>().swap(P.bwd);
 }
 
-void level_tiles(const PackedFactor& P, int l, bool fwd, int rows, std::vector<int>& out) {
-  if (rows < 1) throw std::runtime_error("level_tiles: rows must be >= 1");
-  for (int q = P.lnoff[l]; q < P.lnoff[l + 1]; ++q) {
-    const int s = P.lnodes[q];
-    const int nr = fwd ? P.ns[s] + P.ms[s] : P.ns[s];
-    for (int r0 = 0; r0 < nr; r0 += rows) out.insert(out.end(), {s, r0, std::min(rows, nr - r0), -1});
-  }
-}
-
 bool level_tiles_split(const PackedFactor& P, int l, bool fwd, int rows, int ks, std::vector<int>& tiles,
-                       std::vector<int>& rtiles) {
-  if (ks <= 0) {
-    level_tiles(P, l, fwd, rows, tiles);
-    return true;
-  }
-  if (ks % 16 != 0) throw std::runtime_error("level_tiles_split: segment length must be a multiple of 16");
-  const int t_base = (int)(tiles.size() / 4);
-  for (int q = P.lnoff[l]; q < P.lnoff[l + 1]; ++q) {
+                       std::vector<int>& rtiles, int sys, int t_base) {
+  if (rows < 1) throw std::runtime_error("level_tiles: rows must be >= 1");
+  if (ks > 0 && ks % 16 != 0) throw std::runtime_error("level_tiles_split: segment length must be a multiple of 16");
+  if (t_base < 0) t_base = (int)(tiles.size() / 4);
+  const int q0 = P.lnoff[l * P.nsys + std::max(sys, 0)], q1 = P.lnoff[sys < 0 ? (l + 1) * P.nsys : l * P.nsys + sys + 1];
+  for (int q = q0; q < q1; ++q) {
     const int s = P.lnodes[q];
     const int ns = P.ns[s], ms = P.ms[s];
     const int nr = fwd ? ns + ms : ns;
     for (int r0 = 0; r0 < nr; r0 += rows) {
       const int n = std::min(rows, nr - r0);
+      if (ks <= 0) {
+        tiles.insert(tiles.end(), {s, r0, n, -1});
+        continue;
+      }
       const int last = r0 + n - 1;
       // columns the row tile touches: forward [0, longest row), backward [r0, ns + ms)
       const int cbeg = fwd ? 0 : r0;
@@ -1034,10 +1077,11 @@ void rebuild_tiles(PackedFactor& P) {
   P.btiles.clear();
   P.frtiles.clear();
   P.brtiles.clear();
-  P.foff.assign(P.nlevels + 1, 0);
-  P.boff.assign(P.nlevels + 1, 0);
-  P.froff.assign(P.nlevels + 1, 0);
-  P.broff.assign(P.nlevels + 1, 0);
+  const int K = P.nsys;
+  P.foff.assign(P.nlevels * K + 1, 0);
+  P.boff.assign(P.nlevels * K + 1, 0);
+  P.froff.assign(P.nlevels * K + 1, 0);
+  P.broff.assign(P.nlevels * K + 1, 0);
   if ((int)P.fks.size() != P.nlevels) P.fks.assign(P.nlevels, 0);
   if ((int)P.bks.size() != P.nlevels) P.bks.assign(P.nlevels, 0);
   for (int l = 0; l < P.nlevels; ++l) {
@@ -1049,18 +1093,21 @@ void rebuild_tiles(PackedFactor& P) {
       throw std::runtime_error("rebuild_tiles: tile height exceeds the rows one workgroup covers");
     if ((P.fks[l] && P.fw[l] > 0) || (P.bks[l] && P.bw[l] > 0))
       throw std::runtime_error("rebuild_tiles: only the MFMA sweep splits columns");
-    P.foff[l] = (int)(P.ftiles.size() / 4);
-    P.boff[l] = (int)(P.btiles.size() / 4);
-    P.froff[l] = (int)(P.frtiles.size() / 4);
-    P.broff[l] = (int)(P.brtiles.size() / 4);
-    if (!level_tiles_split(P, l, true, P.frows[l], P.fks[l], P.ftiles, P.frtiles) ||
-        !level_tiles_split(P, l, false, P.brows[l], P.bks[l], P.btiles, P.brtiles))
-      throw std::runtime_error("rebuild_tiles: too many column segments");
+    const int ft = (int)(P.ftiles.size() / 4), bt = (int)(P.btiles.size() / 4);
+    for (int k = 0; k < K; ++k) {
+      P.foff[l * K + k] = (int)(P.ftiles.size() / 4);
+      P.boff[l * K + k] = (int)(P.btiles.size() / 4);
+      P.froff[l * K + k] = (int)(P.frtiles.size() / 4);
+      P.broff[l * K + k] = (int)(P.brtiles.size() / 4);
+      if (!level_tiles_split(P, l, true, P.frows[l], P.fks[l], P.ftiles, P.frtiles, k, ft) ||
+          !level_tiles_split(P, l, false, P.brows[l], P.bks[l], P.btiles, P.brtiles, k, bt))
+        throw std::runtime_error("rebuild_tiles: too many column segments");
+    }
   }
-  P.foff[P.nlevels] = (int)(P.ftiles.size() / 4);
-  P.boff[P.nlevels] = (int)(P.btiles.size() / 4);
-  P.froff[P.nlevels] = (int)(P.frtiles.size() / 4);
-  P.broff[P.nlevels] = (int)(P.brtiles.size() / 4);
+  P.foff[P.nlevels * K] = (int)(P.ftiles.size() / 4);
+  P.boff[P.nlevels * K] = (int)(P.btiles.size() / 4);
+  P.froff[P.nlevels * K] = (int)(P.frtiles.size() / 4);
+  P.broff[P.nlevels * K] = (int)(P.brtiles.size() / 4);
 }
 
 }  // namespace pecs

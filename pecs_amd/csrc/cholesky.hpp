@@ -38,7 +38,11 @@ struct SNode {
 
 struct SupernodalFactor {
   int n = 0;
-  std::vector<int> cell_dof0;      // per grid cell: its first DoF, cells in grid order
+  // A factor may hold several systems without couplings between them (a
+  // forest, one tree each), solved level by level together: DoFs, permuted
+  // rows and nodes of system k are contiguous, from sys_p0[k] and sys_node0[k].
+  std::vector<int> sys_p0, sys_node0;          // per system, and the totals
+  std::vector<std::vector<int>> cell_dof0;     // per system and grid cell: its first DoF, cells in grid order
   std::vector<int> perm;           // per DoF (grid order): its permuted index
   std::vector<SNode> nodes;        // postorder
   std::vector<int> rows;           // per node: ms permuted row indices (struct), ascending
@@ -54,7 +58,8 @@ struct SupernodalFactor {
   double flops = 0.0;
   double t_assemble = 0.0, t_factor = 0.0, t_inverse = 0.0;
   int64_t nnz_L() const { return (int64_t)Linv.size() + (int64_t)L21.size(); }
-  int at(size_t cell, int a) const { return perm[(size_t)cell_dof0[cell] + a]; }
+  int nsys() const { return (int)cell_dof0.size(); }
+  int at(size_t cell, int a, int sys = 0) const { return perm[(size_t)cell_dof0[sys][cell] + a]; }
 };
 
 // Cost of a triangular solve (forward + backward) as merge_levels weighs it:
@@ -64,7 +69,15 @@ struct SolveCost {
   double level = 0.0, entry = 0.0, row = 0.0;
 };
 
-SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells, const SolveCost& cost = {});
+// Systems on the same grid with the same twin number (their own index when
+// `twin` is empty) are ordered alike, by the union of their patterns: their
+// permutations differ by a constant.
+using Systems = std::vector<const BlockSPD*>;
+SupernodalFactor cholesky_factor(const Systems& S, int leaf_cells, const SolveCost& cost = {},
+                                 const std::vector<int>& twin = {});
+inline SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
+  return cholesky_factor(Systems{&S}, leaf_cells);
+}
 
 // Index plan of the multifrontal factorisation for execution on the device:
 // each node's dense nf x nf row-major front (nf = ns + ms; fronts of one level
@@ -87,7 +100,8 @@ struct FrontPlan {
 };
 // The ordering, supernodes and row structure of cholesky_factor (no numeric
 // values: Linv / L21 stay empty) and the device plan of its numeric phase.
-SupernodalFactor cholesky_symbolic(const BlockSPD& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost = {});
+SupernodalFactor cholesky_symbolic(const Systems& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost = {},
+                                   const std::vector<int>& twin = {});
 // Host execution of a plan (for checking the plan's indexing against
 // cholesky_factor): fills Linv and L21 as cholesky_factor does.
 void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::vector<double>& Linv,
@@ -109,24 +123,28 @@ inline int sweep_tile_rows(int w) { return w <= 16 ? 64 : (w == 32 ? 32 : 16); }
 struct PackedFactor {
   int n = 0, nlevels = 0;
   int64_t zlen = 0;
-  std::vector<int> cell_dof0, perm, p0, ns, ms, rows;
+  int nsys = 1;
+  std::vector<int> sys_p0, sys_node0;
+  std::vector<std::vector<int>> cell_dof0;
+  std::vector<int> perm, p0, ns, ms, rows;
   std::vector<int64_t> fwd_off, bwd_off, rows_off, z_off, cptr, czidx;
   std::vector<double> fwd, bwd;
   std::vector<int> ftiles, btiles;    // flattened (node, row0, nrows, 0) grouped by level
-  std::vector<int> foff, boff;        // per level offsets (tiles)
+  // offsets are per level and system, system k of level l at l * nsys + k
+  std::vector<int> foff, boff;        // offsets (tiles)
   std::vector<int> lrows, goff;       // own rows of each level's nodes + offsets
   std::vector<int64_t> xidx;          // panel-row positions of each level's nodes
-  std::vector<int> xoff;              // per level offsets into xidx
+  std::vector<int> xoff;              // offsets into xidx
   std::vector<int> fw, bw;            // lanes per row of the sweeps per level
   std::vector<int> fm, bm;            // row passes per tile per level
   std::vector<int> frows, brows;      // tile height per level (<= (256 / W) * MAXR)
   std::vector<int> fks, bks;          // per level column-segment length of split tiles (0: no split)
   std::vector<int> fpf, bpf;          // per level: the scalar sweep's prefetching variant (0 / 1)
   std::vector<int> frtiles, brtiles;  // split levels: row tiles (node, row0, nrows, 64 * first tile + nseg)
-  std::vector<int> froff, broff;      // per level offsets into frtiles / brtiles
+  std::vector<int> froff, broff;      // offsets into frtiles / brtiles
   std::vector<int> lnodes, lnoff;     // nodes of each level + offsets
   int64_t nvals = 0;                  // entries of fwd (= of bwd)
-  double tri_bytes = 0.0;             // bytes read by one forward + backward sweep
+  std::vector<double> tri_bytes;      // per system: bytes read by one forward + backward sweep
   // MFMA-blocked copies (see pack_blocked): per node, blocks of 16 rows; a
   // block holds its columns [clo, clo + 16 nsteps) in 16-column steps of four
   // 64-entry groups in MFMA A-operand lane order
@@ -160,14 +178,15 @@ inline int blk_chi(bool fwd, int b, int ns, int ms) {
 
 // Row tiles of level l (forward: all ns + ms rows of each node; backward: the
 // ns own rows) with `rows` rows per tile, appended as (node, row0, nrows, -1).
-void level_tiles(const PackedFactor& P, int l, bool fwd, int rows, std::vector<int>& out);
-// Split tiles: each row tile is cut into column segments of ks columns
+// With ks > 0 the row tiles are cut into column segments of ks columns
 // (multiple of 16), one tile (node, row0, nrows, segment) per non-empty
-// segment, and one row tile (node, row0, nrows, 64 * first tile + nseg) per
-// row tile for the deterministic reduction of the segments' partial sums.
-// Returns false if a row tile would need more than 63 segments.
+// segment, and rtiles gets one row tile (node, row0, nrows, 64 * first tile +
+// nseg) per row tile for the deterministic reduction of the segments' partial
+// sums, first tile counted from t_base (-1: the end of `tiles`).  Returns
+// false if a row tile would need more than 63 segments.  sys: the nodes of one
+// system (-1: all).
 bool level_tiles_split(const PackedFactor& P, int l, bool fwd, int rows, int ks, std::vector<int>& tiles,
-                       std::vector<int>& rtiles);
+                       std::vector<int>& rtiles, int sys = -1, int t_base = -1);
 // Rebuild ftiles/btiles and their level offsets from fw/fm/frows, bw/bm/brows.
 void rebuild_tiles(PackedFactor& P);
 

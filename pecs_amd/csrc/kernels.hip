@@ -982,29 +982,29 @@ __global__ __launch_bounds__(256) void k_sweep(DevFactor F, const int4* __restri
 constexpr int IL_TP = 32;
 
 template <int NRP>
-__global__ __launch_bounds__(256) void k_pack_il(DevFactor F, const double* __restrict__ v, int nrhs) {
+__global__ __launch_bounds__(256) void k_pack_il(DevFactor F, const double* __restrict__ v, int nrhs, int pb, int pe) {
   __shared__ double s[NRP * (IL_TP + 1)];
-  const int64_t n = F.n, p0 = (int64_t)blockIdx.x * IL_TP;
+  const int64_t n = F.n, p0 = pb + (int64_t)blockIdx.x * IL_TP;
   for (int e = threadIdx.x; e < NRP * IL_TP; e += 256) {
     const int h = e / IL_TP, pp = e % IL_TP;
-    s[h * (IL_TP + 1) + pp] = (h < nrhs && p0 + pp < n) ? v[(int64_t)h * n + p0 + pp] : 0.0;
+    s[h * (IL_TP + 1) + pp] = (h < nrhs && p0 + pp < pe) ? v[(int64_t)h * n + p0 + pp] : 0.0;
   }
   __syncthreads();
   for (int e = threadIdx.x; e < IL_TP * NRP / 2; e += 256) {
     const int pp = e / (NRP / 2), h = 2 * (e % (NRP / 2));
-    if (p0 + pp < n)
+    if (p0 + pp < pe)
       *reinterpret_cast<double2*>(F.X + (p0 + pp) * NRP + h) =
           double2{s[h * (IL_TP + 1) + pp], s[(h + 1) * (IL_TP + 1) + pp]};
   }
 }
 
 template <int NRP>
-__global__ __launch_bounds__(256) void k_unpack_il(DevFactor F, double* __restrict__ v, int nrhs) {
+__global__ __launch_bounds__(256) void k_unpack_il(DevFactor F, double* __restrict__ v, int nrhs, int pb, int pe) {
   __shared__ double s[NRP * (IL_TP + 1)];
-  const int64_t n = F.n, p0 = (int64_t)blockIdx.x * IL_TP;
+  const int64_t n = F.n, p0 = pb + (int64_t)blockIdx.x * IL_TP;
   for (int e = threadIdx.x; e < IL_TP * NRP / 2; e += 256) {
     const int pp = e / (NRP / 2), h = 2 * (e % (NRP / 2));
-    if (p0 + pp < n) {
+    if (p0 + pp < pe) {
       const double2 x = *reinterpret_cast<const double2*>(F.X + (p0 + pp) * NRP + h);
       s[h * (IL_TP + 1) + pp] = x.x;
       s[(h + 1) * (IL_TP + 1) + pp] = x.y;
@@ -1013,7 +1013,7 @@ __global__ __launch_bounds__(256) void k_unpack_il(DevFactor F, double* __restri
   __syncthreads();
   for (int e = threadIdx.x; e < nrhs * IL_TP; e += 256) {
     const int h = e / IL_TP, pp = e % IL_TP;
-    if (p0 + pp < n) v[(int64_t)h * n + p0 + pp] = s[h * (IL_TP + 1) + pp];
+    if (p0 + pp < pe) v[(int64_t)h * n + p0 + pp] = s[h * (IL_TP + 1) + pp];
   }
 }
 
@@ -1065,7 +1065,7 @@ __global__ __launch_bounds__(256) void k_bwd_gather_il(DevFactor F, const int64_
 }
 
 // ks > 0: the tile is column segment tl.w (columns [tl.w ks, (tl.w + 1) ks))
-// of its row tile and writes its partial sums to Part (slot blockIdx.x, rows
+// of its row tile and writes its partial sums to Part (slot tbase + tile, rows
 // relative to row0, 64 MB rows per slot); k_sweep_reduce adds the segments.
 // Single-block tiles (MB = 1) with up to 32 right-hand sides ask for 4 waves
 // per SIMD: the forward sweep then fits its accumulators in the VGPRs (111,
@@ -1093,7 +1093,7 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 
 template <int NRP, int MB, bool FWD, int HPW = NRP / 16>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(NRP, MB, HPW)))) void k_sweep_mfma(
-    DevFactor F, const int4* __restrict__ tiles, double* __restrict__ Y, int ks, double* __restrict__ Part) {
+    DevFactor F, const int4* __restrict__ tiles, double* __restrict__ Y, int ks, double* __restrict__ Part, int tbase) {
   constexpr int NH = HPW;                  // right-hand-side groups of this wave
   constexpr int WPR = NRP / 16 / HPW;      // waves per row block
   static_assert(WPR >= 1 && 4 % WPR == 0, "a row block's waves must divide the workgroup");
@@ -1220,7 +1220,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mfma_waves_
         if (lr >= row0 + nr) continue;
         const double v = acc[mb][hg][r];
         if (ks > 0) {
-          Part[((int64_t)ti * (64 * MB) + (lr - row0)) * NRP + h] = v;
+          Part[((int64_t)(tbase + ti) * (64 * MB) + (lr - row0)) * NRP + h] = v;
         } else if (FWD) {
           if (lr < ns) Y[(int64_t)(p0 + lr) * NRP + h] = v;
           else F.Z[(F.z_off[s] + (lr - ns)) * NRP + h] = v;
@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mfma_waves_
 template <int NRP, bool FWD, int MBL>
 __global__ __launch_bounds__(256) void k_sweep_mfma_lds(DevFactor F, const int4* __restrict__ tiles,
                                                         double* __restrict__ Y, int ks,
-                                                        double* __restrict__ Part) {
+                                                        double* __restrict__ Part, int tbase) {
   constexpr int NH = NRP / 16;
   constexpr int S = NRP + 4;   // LDS row stride (doubles): the 4 column groups of a read fall in 2 bank halves
   constexpr int K = NRP / 16;  // staged entries per thread per step
@@ -1394,7 +1394,7 @@ __global__ __launch_bounds__(256) void k_sweep_mfma_lds(DevFactor F, const int4*
         if (lr >= row0 + nr) continue;
         const double v = acc[j][hg][r];
         if (ks > 0) {
-          Part[((int64_t)ti * (64 * MBL) + (lr - row0)) * NRP + h] = v;
+          Part[((int64_t)(tbase + ti) * (64 * MBL) + (lr - row0)) * NRP + h] = v;
         } else if (FWD) {
           if (lr < ns) Y[(int64_t)(p0 + lr) * NRP + h] = v;
           else F.Z[(F.z_off[s] + (lr - ns)) * NRP + h] = v;
@@ -2164,17 +2164,17 @@ static int sweep_dispatch(const DevFactor& F, const int4* tl, int nt, int w, int
 
 template <bool FWD>
 static int sweep_mfma_dispatch(const DevFactor& F, const int4* tl, int nt, int mb, int nrp, bool split, double* Y,
-                               int ks, const int4* rtl, int nrt, hipStream_t s) {
+                               int ks, const int4* rtl, int nrt, hipStream_t s, int tbase) {
   if (ks > 0 && (!rtl || !F.Part)) return (int)hipErrorInvalidValue;
 #define PECS_MFMA_CASE(NN, MM)                                                              \
   if (!split && nrp == NN && mb == MM) {                                                    \
-    k_sweep_mfma<NN, MM, FWD><<<nt, 256, 0, s>>>(F, tl, Y, ks, F.Part);                     \
+    k_sweep_mfma<NN, MM, FWD><<<nt, 256, 0, s>>>(F, tl, Y, ks, F.Part, tbase);                   \
     if (ks > 0 && nrt > 0) k_sweep_reduce<NN, FWD><<<dim3(nrt, REDUCE_SPLIT), 256, 0, s>>>(F, rtl, 64 * MM, F.Part, Y); \
     return 0;                                                                               \
   }
 #define PECS_MFMA_SPLIT(NN, MM, HH)                                                         \
   if (split && nrp == NN && mb == MM) {                                                     \
-    k_sweep_mfma<NN, MM, FWD, HH><<<nt, 256, 0, s>>>(F, tl, Y, ks, F.Part);                 \
+    k_sweep_mfma<NN, MM, FWD, HH><<<nt, 256, 0, s>>>(F, tl, Y, ks, F.Part, tbase);               \
     if (ks > 0 && nrt > 0) k_sweep_reduce<NN, FWD><<<dim3(nrt, REDUCE_SPLIT), 256, 0, s>>>(F, rtl, 64 * MM, F.Part, Y); \
     return 0;                                                                               \
   }
@@ -2204,7 +2204,8 @@ int mfma_tile_rows(int nrp, int mb, bool split) {
 }
 
 int launch_sweep(const DevFactor& F, const int4* tiles, int nt, int w, int maxr, bool fwd, int nrhs,
-                 double* t, hipStream_t s, int ks, const int4* rtiles, int nrt, const double* src, bool pf) {
+                 double* t, hipStream_t s, int ks, const int4* rtiles, int nrt, const double* src, bool pf,
+                 int tbase) {
   if (nt <= 0) return 0;
   if (w <= 0) {  // 0: MFMA sweep, -1: its right-hand-side groups split over waves, -2: LDS-staged vector
     if (nrhs > MAX_MFMA_RHS) return (int)hipErrorInvalidValue;
@@ -2219,10 +2220,10 @@ int launch_sweep(const DevFactor& F, const int4* tiles, int nt, int w, int maxr,
 #define PECS_MFMA_LDS(NN, MM)                                                                    \
   if (nrp == NN && maxr == MM) {                                                                 \
     if (fwd) {                                                                                   \
-      k_sweep_mfma_lds<NN, true, MM><<<nt, 256, 0, s>>>(F, tiles, t, ks, F.Part);                \
+      k_sweep_mfma_lds<NN, true, MM><<<nt, 256, 0, s>>>(F, tiles, t, ks, F.Part, tbase);                \
       if (ks > 0 && nrt > 0) k_sweep_reduce<NN, true><<<dim3(nrt, REDUCE_SPLIT), 256, 0, s>>>(F, rtiles, 64 * MM, F.Part, t); \
     } else {                                                                                     \
-      k_sweep_mfma_lds<NN, false, MM><<<nt, 256, 0, s>>>(F, tiles, t, ks, F.Part);               \
+      k_sweep_mfma_lds<NN, false, MM><<<nt, 256, 0, s>>>(F, tiles, t, ks, F.Part, tbase);               \
       if (ks > 0 && nrt > 0) k_sweep_reduce<NN, false><<<dim3(nrt, REDUCE_SPLIT), 256, 0, s>>>(F, rtiles, 64 * MM, F.Part, t); \
     }                                                                                            \
     return (int)hipGetLastError();                                                               \
@@ -2233,8 +2234,8 @@ int launch_sweep(const DevFactor& F, const int4* tiles, int nt, int w, int maxr,
       return (int)hipErrorInvalidValue;
     }
     const bool split = w < 0 && nrp > 16;
-    return fwd ? sweep_mfma_dispatch<true>(F, tiles, nt, maxr, nrp, split, t, ks, rtiles, nrt, s)
-               : sweep_mfma_dispatch<false>(F, tiles, nt, maxr, nrp, split, t, ks, rtiles, nrt, s);
+    return fwd ? sweep_mfma_dispatch<true>(F, tiles, nt, maxr, nrp, split, t, ks, rtiles, nrt, s, tbase)
+               : sweep_mfma_dispatch<false>(F, tiles, nt, maxr, nrp, split, t, ks, rtiles, nrt, s, tbase);
   }
   if (nrhs > 2 || ks > 0) return (int)hipErrorInvalidValue;
   const double* v0 = fwd ? src : nullptr;
@@ -2247,75 +2248,82 @@ int launch_sweep(const DevFactor& F, const int4* tiles, int nt, int w, int maxr,
                    : sweep_dispatch<1, false>(F, tiles, nt, w, maxr, v0, v0, t, t1, s, pf);
 }
 
+// The tiles (rows, row tiles) of level l: of one system, or of all (sys -1).
+struct LevelRange {
+  int at, n, base;
+  LevelRange(const int* off, const FactorLevels& L, int l, int sys) {
+    base = off[l * L.nsys];
+    at = sys < 0 ? base : off[l * L.nsys + sys];
+    n = off[sys < 0 ? (l + 1) * L.nsys : l * L.nsys + sys + 1] - at;
+  }
+};
+
 template <int NRP>
-static int chol_solve_il(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s) {
-  k_pack_il<NRP><<<nblk(F.n, IL_TP), 256, 0, s>>>(F, v, nrhs);
+static int chol_solve_il(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s,
+                         int sys) {
+  const int pb = sys < 0 ? 0 : L.sys_p0[sys], pe = sys < 0 ? F.n : L.sys_p0[sys + 1];
+  k_pack_il<NRP><<<nblk(pe - pb, IL_TP), 256, 0, s>>>(F, v, nrhs, pb, pe);
   // the leaf level's rows are owed nothing (pack_layout checks it)
   for (int l = 0; l < L.nlevels; ++l) {
-    const int ng = L.goff[l + 1] - L.goff[l];
-    if (l > 0 && ng > 0)
-      k_fwd_gather_il<NRP><<<nblk((int64_t)ng * NRP / 2, 256), 256, 0, s>>>(F, F.lrows + L.goff[l], ng, nrhs);
-    const int nt = L.foff[l + 1] - L.foff[l];
+    const LevelRange g(L.goff, L, l, sys), f(L.foff, L, l, sys), r(L.froff, L, l, sys);
+    if (l > 0 && g.n > 0)
+      k_fwd_gather_il<NRP><<<nblk((int64_t)g.n * NRP / 2, 256), 256, 0, s>>>(F, F.lrows + g.at, g.n, nrhs);
     if (L.fw[l] > 0) return (int)hipErrorInvalidValue;
-    const int e = launch_sweep(F, F.ftiles + L.foff[l], nt, L.fw[l], L.fm[l], true, nrhs, t, s, L.fks[l],
-                               F.frtiles + L.froff[l], L.froff[l + 1] - L.froff[l]);
+    const int e = launch_sweep(F, F.ftiles + f.at, f.n, L.fw[l], L.fm[l], true, nrhs, t, s, L.fks[l], F.frtiles + r.at,
+                               r.n, nullptr, false, f.at - f.base);
     if (e) return e;
   }
   for (int l = L.nlevels - 1; l >= 0; --l) {
-    const int nx = L.xoff[l + 1] - L.xoff[l];
+    const LevelRange x(L.xoff, L, l, sys), b(L.boff, L, l, sys), r(L.broff, L, l, sys);
     // (the LDS-staged sweep, 32 or more right-hand sides, reads the panel
     // columns through the row index)
-    if (nx > 0 && !(L.bw[l] == -2 && NRP >= 32))
-      k_bwd_gather_il<NRP><<<nblk((int64_t)nx * NRP / 2, 256), 256, 0, s>>>(F, F.xidx + L.xoff[l], nx);
-    const int nt = L.boff[l + 1] - L.boff[l];
+    if (x.n > 0 && !(L.bw[l] == -2 && NRP >= 32))
+      k_bwd_gather_il<NRP><<<nblk((int64_t)x.n * NRP / 2, 256), 256, 0, s>>>(F, F.xidx + x.at, x.n);
     if (L.bw[l] > 0) return (int)hipErrorInvalidValue;
-    const int e = launch_sweep(F, F.btiles + L.boff[l], nt, L.bw[l], L.bm[l], false, nrhs, t, s, L.bks[l],
-                               F.brtiles + L.broff[l], L.broff[l + 1] - L.broff[l]);
+    const int e = launch_sweep(F, F.btiles + b.at, b.n, L.bw[l], L.bm[l], false, nrhs, t, s, L.bks[l], F.brtiles + r.at,
+                               r.n, nullptr, false, b.at - b.base);
     if (e) return e;
   }
-  k_unpack_il<NRP><<<nblk(F.n, IL_TP), 256, 0, s>>>(F, v, nrhs);
+  k_unpack_il<NRP><<<nblk(pe - pb, IL_TP), 256, 0, s>>>(F, v, nrhs, pb, pe);
   return (int)hipGetLastError();
 }
 
-int launch_chol_solve(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s) {
+int launch_chol_solve(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s,
+                      int sys) {
   if (L.nlevels > 0 && L.fw[0] <= 0) {  // MFMA-shaped factor: interleaved vectors
     if (nrhs > MAX_MFMA_RHS) return (int)hipErrorInvalidValue;
     switch (mfma_rhs_pad(nrhs)) {
-      case 16: return chol_solve_il<16>(F, L, v, t, nrhs, s);
-      case 32: return chol_solve_il<32>(F, L, v, t, nrhs, s);
-      case 64: return chol_solve_il<64>(F, L, v, t, nrhs, s);
-      default: return chol_solve_il<128>(F, L, v, t, nrhs, s);
+      case 16: return chol_solve_il<16>(F, L, v, t, nrhs, s, sys);
+      case 32: return chol_solve_il<32>(F, L, v, t, nrhs, s, sys);
+      case 64: return chol_solve_il<64>(F, L, v, t, nrhs, s, sys);
+      default: return chol_solve_il<128>(F, L, v, t, nrhs, s, sys);
     }
   }
   if (nrhs > 2) return (int)hipErrorInvalidValue;
   for (int l = 0; l < L.nlevels; ++l) {
     // level 0 (leaves) owes nothing to its rows: its sweep reads the right-hand side itself
-    const int ng = L.goff[l + 1] - L.goff[l];
-    if (l > 0 && ng > 0) {
-      const int* lr = F.lrows + L.goff[l];
-      if (ng >= 16384) {
-        if (nrhs == 2) k_fwd_gather<1, 2><<<nblk(ng, 256), 256, 0, s>>>(F, lr, ng, v);
-        else k_fwd_gather<1, 1><<<nblk(ng, 256), 256, 0, s>>>(F, lr, ng, v);
+    const LevelRange g(L.goff, L, l, sys), f(L.foff, L, l, sys);
+    if (l > 0 && g.n > 0) {
+      const int* lr = F.lrows + g.at;
+      if (g.n >= 16384) {
+        if (nrhs == 2) k_fwd_gather<1, 2><<<nblk(g.n, 256), 256, 0, s>>>(F, lr, g.n, v);
+        else k_fwd_gather<1, 1><<<nblk(g.n, 256), 256, 0, s>>>(F, lr, g.n, v);
       } else {
-        if (nrhs == 2) k_fwd_gather<8, 2><<<nblk(8 * (int64_t)ng, 256), 256, 0, s>>>(F, lr, ng, v);
-        else k_fwd_gather<8, 1><<<nblk(8 * (int64_t)ng, 256), 256, 0, s>>>(F, lr, ng, v);
+        if (nrhs == 2) k_fwd_gather<8, 2><<<nblk(8 * (int64_t)g.n, 256), 256, 0, s>>>(F, lr, g.n, v);
+        else k_fwd_gather<8, 1><<<nblk(8 * (int64_t)g.n, 256), 256, 0, s>>>(F, lr, g.n, v);
       }
     }
-    const int nt = L.foff[l + 1] - L.foff[l];
-    const int e = launch_sweep(F, F.ftiles + L.foff[l], nt, L.fw[l], L.fm[l], true, nrhs, t, s, 0, nullptr, 0,
+    const int e = launch_sweep(F, F.ftiles + f.at, f.n, L.fw[l], L.fm[l], true, nrhs, t, s, 0, nullptr, 0,
                                l == 0 ? v : nullptr, L.fpf && L.fpf[l]);
     if (e) return e;
   }
   for (int l = L.nlevels - 1; l >= 0; --l) {
     // the backward sweep reads the panel rows' x straight from X (no gather)
-    const int nt = L.boff[l + 1] - L.boff[l];
-    const int e = launch_sweep(F, F.btiles + L.boff[l], nt, L.bw[l], L.bm[l], false, nrhs, t, s, 0, nullptr, 0,
-                               nullptr, L.bpf && L.bpf[l]);
+    const LevelRange b(L.boff, L, l, sys);
+    const int e = launch_sweep(F, F.btiles + b.at, b.n, L.bw[l], L.bm[l], false, nrhs, t, s, 0, nullptr, 0, nullptr,
+                               L.bpf && L.bpf[l]);
     if (e) return e;
   }
-  // a kernel, not a memcpy node, so that the solve can be captured in a graph
-  const int64_t nx = (int64_t)nrhs * F.n;
-  k_copy<<<(unsigned)std::min<int64_t>(nblk(nx, 256), 4096), 256, 0, s>>>(F.X, v, nx);
   return (int)hipGetLastError();
 }
 

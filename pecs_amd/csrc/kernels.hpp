@@ -144,20 +144,23 @@ struct DevFactor {
   double* X;                // 2 * n scratch: forward t, then backward output
 };
 
+// (offsets per level and system: system k of level l at l * nsys + k)
 struct FactorLevels {
-  const int* foff;  // host: per level offsets into ftiles (nlevels+1)
-  const int* boff;  // host: per level offsets into btiles
-  const int* goff;  // host: per level offsets into lrows
-  const int* xoff;  // host: per level offsets into xidx
+  const int* foff;  // host: offsets into ftiles
+  const int* boff;  // host: offsets into btiles
+  const int* goff;  // host: offsets into lrows
+  const int* xoff;  // host: offsets into xidx
   const int* fw;    // host: lanes per row of the forward sweep per level
   const int* bw;    // host: lanes per row of the backward sweep per level
   const int* fm;    // host: row passes per tile (tile rows <= (256 / fw) * fm) per level
   const int* bm;    // host: the same for the backward sweep
   const int* fks;   // host: column-segment length of split forward tiles per level (0: no split)
   const int* bks;   // host: the same for the backward sweep
-  const int* froff; // host: per level offsets into frtiles (nlevels+1)
-  const int* broff; // host: per level offsets into brtiles
+  const int* froff; // host: offsets into frtiles
+  const int* broff; // host: offsets into brtiles
   int nlevels;
+  int nsys;
+  const int* sys_p0;  // host: first row of each system, and the end
   const int* fpf;   // host: scalar sweep, prefetching variant per forward level (null: none)
   const int* bpf;   // host: the same for the backward sweep
 };
@@ -232,10 +235,11 @@ int launch_schur_recover(int k, const DevRegion* const* R, const SchurPair& P, i
 // columns whose partial sums (F.Part) are added by a reduction over rtiles.
 // Vectors are h-major: right-hand side h at t[h * n].
 // src (scalar forward sweeps only): read t from src instead of X (the leaf
-// level, whose rows are owed no contributions).
+// level, whose rows are owed no contributions).  tbase: index of the first
+// tile in its level (the partial sums' slots are counted over the level).
 int launch_sweep(const DevFactor& F, const int4* tiles, int nt, int w, int maxr, bool fwd, int nrhs,
                  double* t, hipStream_t s, int ks = 0, const int4* rtiles = nullptr, int nrt = 0,
-                 const double* src = nullptr, bool pf = false);
+                 const double* src = nullptr, bool pf = false, int tbase = 0);
 // Padded right-hand-side count of the MFMA sweep (16 or 32).
 // Right-hand sides of the MFMA sweeps: padded to 16, 32, 64 or 128
 // interleaved columns; at most MAX_MFMA_RHS.  mfma_shape_ok: whether the
@@ -247,10 +251,16 @@ bool mfma_shape_ok(int nrp, int mb, bool split = false);
 // sides split over waves (sweep width -1) 64 mb / (waves per row block)
 int mfma_tile_rows(int nrp, int mb, bool split);
 // x = S^{-1} v for nrhs h-major right-hand sides in the factor's permuted
-// order (v is overwritten with x).  t is scratch: nrhs * n doubles for a
-// factor shaped for 1-2 right-hand sides, mfma_rhs_pad(nrhs) * n for an
-// MFMA-shaped one (whose scratch X, Z and t hold RHS-interleaved vectors).
-int launch_chol_solve(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s);
+// order, at chol_solution(F, L, v): F.X for a factor shaped for 1-2 right-hand
+// sides (h-major, stride F.n; v is kept), v itself for an MFMA-shaped one.  t
+// is scratch: nrhs * n doubles or mfma_rhs_pad(nrhs) * n (an MFMA-shaped
+// factor's scratch X, Z and t hold RHS-interleaved vectors).  sys: one system
+// of the factor (-1: all); the rows of the others are neither read nor written.
+int launch_chol_solve(const DevFactor& F, const FactorLevels& L, double* v, double* t, int nrhs, hipStream_t s,
+                      int sys = -1);
+inline double* chol_solution(const DevFactor& F, const FactorLevels& L, double* v) {
+  return L.nlevels > 0 && L.fw[0] <= 0 ? v : F.X;
+}
 int launch_poisson_cell(int k, const DevPoisson& P, const DevTabs& T, const DevPhys* phs, const double* un,
                         const double* up, const double* ur, const double* uo, int ncs, int nce, double* y,
                         hipStream_t s, int nb = 1, int64_t ss = 0, int64_t se = 0, int64_t sy = 0);

@@ -14,21 +14,24 @@
 
 using namespace pecs;
 
-static void block_matvec(const BlockSPD& S, const SupernodalFactor& F, const double* x, double* y) {
-  const int no = S.noff();
-  for (int X = 0; X < S.NXc * S.NYc; ++X) {
-    const int nx = S.ndof[X];
-    for (int a = 0; a < nx; ++a) y[F.at(X, a)] = 0.0;
-    const int xi = X % S.NXc, xj = X / S.NXc;
-    for (int o = 0; o < no; ++o) {
-      const int yi = xi + S.offi[o], yj = xj + S.offj[o];
-      if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
-      const int Y = yi + S.NXc * yj;
-      const auto& B = S.blk[(size_t)X * no + o];
-      if (B.empty()) continue;
-      const int ny = S.ndof[Y];
-      for (int a = 0; a < nx; ++a)
-        for (int b = 0; b < ny; ++b) y[F.at(X, a)] += B[(size_t)a * ny + b] * x[F.at(Y, b)];
+static void block_matvec(const Systems& Ss, const SupernodalFactor& F, const double* x, double* y) {
+  for (int k = 0; k < (int)Ss.size(); ++k) {
+    const BlockSPD& S = *Ss[k];
+    const int no = S.noff();
+    for (int X = 0; X < S.NXc * S.NYc; ++X) {
+      const int nx = S.ndof[X];
+      for (int a = 0; a < nx; ++a) y[F.at(X, a, k)] = 0.0;
+      const int xi = X % S.NXc, xj = X / S.NXc;
+      for (int o = 0; o < no; ++o) {
+        const int yi = xi + S.offi[o], yj = xj + S.offj[o];
+        if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
+        const int Y = yi + S.NXc * yj;
+        const auto& B = S.blk[(size_t)X * no + o];
+        if (B.empty()) continue;
+        const int ny = S.ndof[Y];
+        for (int a = 0; a < nx; ++a)
+          for (int b = 0; b < ny; ++b) y[F.at(X, a, k)] += B[(size_t)a * ny + b] * x[F.at(Y, b, k)];
+      }
     }
   }
 }
@@ -72,7 +75,7 @@ static void factor_solve_host(const SupernodalFactor& F, const double* b, double
 static void packed_solve_host(const PackedFactor& P, const double* b, double* x) {
   std::vector<double> Y(P.n), z(P.zlen), X(P.n), vec;
   for (int l = 0; l < P.nlevels; ++l)
-    for (int q = P.foff[l]; q < P.foff[l + 1]; ++q) {
+    for (int q = P.foff[l * P.nsys]; q < P.foff[(l + 1) * P.nsys]; ++q) {
       const int s = P.ftiles[4 * q], r0 = P.ftiles[4 * q + 1], nr = P.ftiles[4 * q + 2];
       const int ns = P.ns[s], p0 = P.p0[s];
       vec.assign(ns, 0.0);
@@ -98,7 +101,7 @@ static void packed_solve_host(const PackedFactor& P, const double* b, double* x)
       }
     }
   for (int l = P.nlevels - 1; l >= 0; --l)
-    for (int q = P.boff[l]; q < P.boff[l + 1]; ++q) {
+    for (int q = P.boff[l * P.nsys]; q < P.boff[(l + 1) * P.nsys]; ++q) {
       const int s = P.btiles[4 * q], r0 = P.btiles[4 * q + 1], nr = P.btiles[4 * q + 2];
       const int ns = P.ns[s], ms = P.ms[s], p0 = P.p0[s];
       vec.assign(ns + ms, 0.0);
@@ -143,7 +146,7 @@ static void mfma_solve_emulate(const PackedFactor& P, int nrhs, int MB, int KS, 
         if (l == 0)  // k_pack_il: the right-hand sides interleaved, padding zero
           for (int64_t p = 0; p < n; ++p)
             for (int h = 0; h < NRP; ++h) X[p * NRP + h] = h < nrhs ? b[h * n + p] : 0.0;
-        for (int i = P.goff[l]; i < P.goff[l + 1]; ++i)
+        for (int i = P.goff[l * P.nsys]; i < P.goff[(l + 1) * P.nsys]; ++i)
           for (int h = 0; h < nrhs && l > 0; ++h) {
             const int p = P.lrows[i];
             for (int64_t c = P.cptr[p]; c < P.cptr[p + 1]; ++c) {
@@ -152,7 +155,7 @@ static void mfma_solve_emulate(const PackedFactor& P, int nrhs, int MB, int KS, 
             }
           }
       } else {
-        for (int i = P.xoff[l]; i < P.xoff[l + 1]; ++i)
+        for (int i = P.xoff[l * P.nsys]; i < P.xoff[(l + 1) * P.nsys]; ++i)
           for (int h = 0; h < NRP; ++h) {
             const int64_t q = P.xidx[i];
             EMU_CHECK(q >= 0 && q < zl, "backward gather");
@@ -513,12 +516,13 @@ static void blocked_emulate(const PackedFactor& P, const std::vector<double>& fw
   }
 }
 
-static double check(const char* name, const BlockSPD& S, int leaf, const SolveCost& cost) {
+static double check(const char* name, const Systems& S, int leaf, const SolveCost& cost,
+                    const std::vector<int>& twin = {}) {
   auto t0 = std::chrono::steady_clock::now();
-  SupernodalFactor F = cholesky_factor(S, leaf, cost);
+  SupernodalFactor F = cholesky_factor(S, leaf, cost, twin);
   {  // the device plan, executed on the host, must reproduce the factor
     FrontPlan plan;
-    SupernodalFactor G = cholesky_symbolic(S, leaf, plan, cost);
+    SupernodalFactor G = cholesky_symbolic(S, leaf, plan, cost, twin);
     std::vector<double> Li, L2;
     execute_plan_host(plan, G, Li, L2);
     double d = 0;
@@ -608,13 +612,13 @@ static double check(const char* name, const BlockSPD& S, int leaf, const SolveCo
       for (int l = 0; l < P.nlevels; ++l) {
         double fb = 0, bb = 0;
         int nodes = 0, rowsf = 0, rowsb = 0, maxns = 0, maxms = 0;
-        for (int q = P.foff[l]; q < P.foff[l + 1]; ++q) {
+        for (int q = P.foff[l * P.nsys]; q < P.foff[(l + 1) * P.nsys]; ++q) {
           const int s = P.ftiles[4 * q], r0 = P.ftiles[4 * q + 1], nr = P.ftiles[4 * q + 2];
           for (int r = r0; r < r0 + nr; ++r) fb += 8.0 * (r < P.ns[s] ? r + 1 : P.ns[s]);
           if (r0 == 0) { nodes++; maxns = std::max(maxns, P.ns[s]); maxms = std::max(maxms, P.ms[s]); }
           rowsf += nr;
         }
-        for (int q = P.boff[l]; q < P.boff[l + 1]; ++q) {
+        for (int q = P.boff[l * P.nsys]; q < P.boff[(l + 1) * P.nsys]; ++q) {
           const int s = P.btiles[4 * q], r0 = P.btiles[4 * q + 1], nr = P.btiles[4 * q + 2];
           for (int j = r0; j < r0 + nr; ++j) bb += 8.0 * (P.ns[s] - j + P.ms[s]);
           rowsb += nr;
@@ -670,9 +674,20 @@ int main(int argc, char** argv) {
   // 20000 entries, so that runs of several lengths appear)
   const SolveCost costs[2] = {{}, {2e4, 1.0, 0.0}};
   for (const SolveCost& cost : costs) {
-    worst = std::max(worst, check("S_semi", Ss, leaf, cost));
-    worst = std::max(worst, check("S_elec", Se, leaf, cost));
-    worst = std::max(worst, check("H_poisson", H, leaf, cost));
+    worst = std::max(worst, check("S_semi + S_elec", {&Ss, &Se}, leaf, cost));
+    worst = std::max(worst, check("H_poisson", {&H}, leaf, cost));
+  }
+  {  // one factor per carrier of a region, ordered alike
+    BlockSPD S2 = schur_matrix(m.semi, os, 0.7);
+    worst = std::max(worst, check("S_semi, two carriers", {&Ss, &S2}, leaf, costs[1], {0, 0}));
+    FrontPlan plan;
+    const SupernodalFactor F = cholesky_symbolic({&Ss, &S2}, leaf, plan, costs[1], {0, 0});
+    const int n1 = F.sys_p0[1];
+    for (int d = 0; d < n1; ++d)
+      if (F.perm[n1 + d] != n1 + F.perm[d]) {
+        std::printf("twin systems ordered differently\n");
+        return 2;
+      }
   }
   std::printf("%s\n", worst < 1e-12 ? "SELFTEST OK" : "SELFTEST FAIL");
   return worst < 1e-12 ? 0 : 1;
