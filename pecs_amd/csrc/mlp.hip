@@ -9,13 +9,18 @@
 // file; the C-ABI (include/pecs_abi.h, pecs_mlp_*) moves host arrays in and
 // out.
 //
-// Every matrix product -- the dense layers, their gradients, and the
-// convolutions with their weight and input gradients as implicit GEMMs
-// (im2col gathered while staging the LDS tiles) -- is one kernel, k_mm, on
-// the matrix cores: v_mfma_f32_16x16x4f32 for FP32, v_mfma_f32_16x16x16bf16_1k
-// for BF16.  MFMA operand layout (both): lane l holds A[l%16][k], B[k][l%16]
-// with k = l/16 (FP32) or 4(l/16)..4(l/16)+3 (BF16); accumulator lane l,
-// register r holds C[4(l/16)+r][l%16].
+// Every matrix product runs on the matrix cores: v_mfma_f32_16x16x4f32 for
+// FP32, v_mfma_f32_16x16x16bf16_1k for BF16.  MFMA operand layout (both): lane
+// l holds A[l%16][k], B[k][l%16] with k = l/16 (FP32) or 4(l/16)..4(l/16)+3
+// (BF16); accumulator lane l, register r holds C[4(l/16)+r][l%16].
+//   k_dense    the dense layers and their gradients, one 16 x 16 tile per wave
+//   k_conv     the convolutions and their input gradients as implicit GEMMs on
+//              input strips staged in LDS
+//   k_conv_dw  their weight and bias gradients on the same strips
+//   k_mm       any of the convolution products, im2col gathered element by
+//              element: maps that do not divide into strips of whole rows
+// Every product adds its k terms in ascending order in groups of 4 (FP32) or
+// 16 (BF16), whichever kernel runs it: the forward pass is the same bit by bit.
 //
 // Parameters are one FP32 array: per dense layer W (n_in x n_out, row-major)
 // then b (n_out); per convolution W (cout x cin x 3 x 3) then b (cout).
@@ -76,7 +81,6 @@ __device__ __forceinline__ float ldv<uint16_t>(const uint16_t* p, int64_t i) {
 // An operand matrix of k_mm, read element by element while staging tiles.
 enum OpKind {
   OP_ROW = 0,     // (r, c) = p[r ld + c]
-  OP_TRANS = 1,   // (r, c) = p[c ld + r]
   OP_IM2COL = 2,  // (ci 9 + t, b R^2 + px): input pixel under tap t of output pixel px (conv forward B)
   OP_IM2COL_T = 3,  // its transpose (weight gradient B)
   OP_CHAN = 4,    // (ch, b R^2 + px) of a C x R x R map per sample (weight gradient A)
@@ -87,7 +91,7 @@ enum OpKind {
 struct Opnd {
   const void* p;
   int kind;
-  int ld;  // OP_ROW / OP_TRANS
+  int ld;  // OP_ROW
   int C;   // channels of the map read (OP_WT: cin)
   int R;   // side of the convolution's output (and upsampled input)
   int up;  // OP_IM2COL*: the input map is R/2 x R/2, upsampled by 2 (nearest)
@@ -99,8 +103,6 @@ __device__ __forceinline__ float opnd(const Opnd& o, int r, int c) {
   switch (o.kind) {
     case OP_ROW:
       return ldv(p, (int64_t)r * o.ld + c);
-    case OP_TRANS:
-      return ldv(p, (int64_t)c * o.ld + r);
     case OP_IM2COL:
     case OP_IM2COL_T: {
       const int k = o.kind == OP_IM2COL ? r : c, n = o.kind == OP_IM2COL ? c : r;
@@ -142,6 +144,7 @@ struct Dst {
   int bias_row;
   int relu;
   int bf16;  // store BF16 (hidden activations of BF16 inference)
+  const float* mask;  // ReLU backward: zero where mask (the layer's output, indexed as p) is not positive
 };
 
 constexpr int TM = 64, TN = 64, TK = 16;  // tile: 64 x 64 outputs, 16-deep k steps, 4 waves of 32 x 32
@@ -158,6 +161,7 @@ __device__ __forceinline__ void mm_store(const Dst& D, int m, int n, float v) {
   } else {
     o = (int64_t)m * D.ld + n;
   }
+  if (D.mask && D.mask[o] <= 0.f) v = 0.f;
   if (D.bf16) static_cast<uint16_t*>(D.p)[o] = f32_to_bf16(v);
   else static_cast<float*>(D.p)[o] = v;
 }
@@ -253,12 +257,293 @@ __global__ __launch_bounds__(256) void k_mm_reduce(const float* __restrict__ par
   mm_store(D, (int)(e / N), (int)(e % N), v);
 }
 
-// db[c] = sum over rows of dZ[r][c] (fixed order)
+// ---- dense products ---------------------------------------------------------
+// C[m][n] = sum_k a[m am + k ak] b[k bk + n bn], one 16 x 16 tile per wave, the
+// operands straight from L2 into registers (no LDS, no barriers), two groups of
+// DU steps in turn so that one's loads run under the other's MFMAs.  With the
+// few rows of a minibatch the 64 x 64 tiles of k_mm left 4 to 64 workgroups
+// with a barrier and a load latency per 16 k (42 us at 32 x 256 x 256, 449 us
+// at 32 x 256 x 4096).  blockIdx.z: k slice of kchunk (a multiple of 16), raw
+// sums to part.
+template <class T>
+__global__ __launch_bounds__(256) void k_dense(const T* __restrict__ a, int am, int ak, const T* __restrict__ b, int bk,
+                                               int bn, Dst D, int M, int N, int K, int kchunk,
+                                               float* __restrict__ part) {
+  constexpr bool BF = sizeof(T) == 2;
+  constexpr int KS = BF ? 16 : 4, E = BF ? 4 : 1, DU = BF ? 4 : 8;  // k per MFMA, entries per lane, steps per group
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n0 = (blockIdx.x * 4 + wave) * 16, m0 = blockIdx.y * 16;
+  if (n0 >= N) return;
+  const int li = lane & 15, lq = lane >> 4;
+  const int m = min(m0 + li, M - 1), n = min(n0 + li, N - 1);  // (rows and columns past the end are not stored)
+  const T* __restrict__ pa = a + (int64_t)m * am;
+  const T* __restrict__ pb = b + (int64_t)n * bn;
+  const int kbeg = blockIdx.z * kchunk, kend = min(K, kbeg + kchunk);
+  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  T A[2][DU][E], B[2][DU][E];
+  auto load = [&](int k0, T (&x)[DU][E], T (&y)[DU][E]) {
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int k = k0 + u * KS + lq * E + e, kc = min(k, kend - 1);
+        const T va = pa[(int64_t)kc * ak], vb = pb[(int64_t)kc * bk];
+        x[u][e] = k < kend ? va : T(0);
+        y[u][e] = k < kend ? vb : T(0);
+      }
+  };
+  auto mma = [&](const T (&x)[DU][E], const T (&y)[DU][E]) {
+#pragma unroll
+    for (int u = 0; u < DU; ++u) {
+      if constexpr (BF) {
+        v4s xa, yb;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          xa[e] = (short)x[u][e];
+          yb[e] = (short)y[u][e];
+        }
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xa, yb, acc, 0, 0, 0);
+      } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u][0], y[u][0], acc, 0, 0, 0);
+      }
+    }
+  };
+  load(kbeg, A[0], B[0]);
+  for (int k0 = kbeg; k0 < kend; k0 += 2 * DU * KS) {
+    if (k0 + DU * KS < kend) load(k0 + DU * KS, A[1], B[1]);
+    mma(A[0], B[0]);
+    if (k0 + DU * KS >= kend) break;
+    if (k0 + 2 * DU * KS < kend) load(k0 + 2 * DU * KS, A[0], B[0]);
+    mma(A[1], B[1]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int mm = m0 + 4 * lq + r, nn = n0 + li;
+    if (mm >= M || nn >= N) continue;
+    if (part) part[((int64_t)blockIdx.z * M + mm) * N + nn] = acc[r];
+    else mm_store(D, mm, nn, acc[r]);
+  }
+}
+
+// ---- convolutions on staged strips ------------------------------------------
+// A strip is P consecutive output pixels of one sample, whole rows; its input
+// (all channels, a border of one pixel, zeros outside the map, upsampled if the
+// stage upsamples) is staged in LDS once, so that the operand of tap (ci, t) at
+// a pixel is at (pixel offset) + (tap offset): two table look-ups per MFMA
+// instead of k_mm's divisions, bounds checks and loads per element.
+struct Conv {
+  int C;     // channels of the staged map
+  int R;     // side of the output (and of the upsampled input)
+  int up;    // the map read is R/2 x R/2
+  int P;     // output pixels per strip
+  int M, K;  // output channels, C * 9
+  int rows() const { return P / R; }
+  int ch() const { return (P / R + 2) * (R + 2); }  // staged entries per channel
+};
+
+// One wave stages one row at a time (two where a row is at most 32 entries).
+template <class T>
+__device__ __forceinline__ void conv_stage(const Conv& c, const T* __restrict__ in, int smp, int y0, T* sIn) {
+  const int W = c.R + 2, rows = c.P / c.R + 2, Ri = c.R >> c.up;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int par = W <= 32 ? 2 : 1, sub = W <= 32 ? lane >> 5 : 0, x0 = W <= 32 ? lane & 31 : lane, xs = 64 / par;
+  for (int q = wave * par + sub; q < c.C * rows; q += 4 * par) {
+    const int ci = q / rows, yy = q - ci * rows, y = y0 + yy - 1;
+    const bool yin = y >= 0 && y < c.R;
+    const T* src = in + (((int64_t)smp * c.C + ci) * Ri + (yin ? y >> c.up : 0)) * Ri;
+    for (int xx = x0; xx < W; xx += xs) {
+      const int x = xx - 1;
+      sIn[q * W + xx] = yin && x >= 0 && x < c.R ? src[x >> c.up] : T(0);
+    }
+  }
+}
+
+// Forward (FLIP 0): out[m][px] = sum over (ci, t) of w[m][ci][t] in[ci][px + off(t)];
+// input gradient (FLIP 1): the staged map is the output gradient (C = the
+// stage's output channels), out[m][px] = sum over (co, t) of w[co][m][t]
+// in[co][px - off(t)].  MW waves of 16 output channels, 4 / MW groups of NC
+// 16-pixel blocks.
+template <class T, int FLIP, int MW, int NC>
+__global__ __launch_bounds__(256) void k_conv(Conv c, const T* __restrict__ in, const T* __restrict__ w, Dst D) {
+  constexpr bool BF = sizeof(T) == 2;
+  constexpr int KS = BF ? 16 : 4, E = BF ? 4 : 1, DU = BF ? 2 : 8;
+  extern __shared__ __align__(16) char smem[];
+  int2* sK = reinterpret_cast<int2*>(smem);        // per k: tap offset in the strip, weight offset
+  T* sIn = reinterpret_cast<T*>(smem + (size_t)c.K * sizeof(int2));
+  const int W = c.R + 2, R2 = c.R * c.R, CH = (c.P / c.R + 2) * W;
+  const int64_t n0 = (int64_t)blockIdx.x * c.P;
+  const int smp = (int)(n0 / R2), px0 = (int)(n0 - (int64_t)smp * R2);
+  for (int k = threadIdx.x; k < c.K; k += 256) {
+    const int ci = k / 9, t = k - 9 * ci, ty = t / 3, tx = t - 3 * ty;
+    sK[k] = FLIP ? make_int2(ci * CH + (2 - ty) * W + 2 - tx, ci * c.M * 9 + t) : make_int2(ci * CH + ty * W + tx, k);
+  }
+  conv_stage(c, in, smp, px0 / c.R, sIn);
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int m0 = (blockIdx.y * MW + wave % MW) * 16;
+  if (m0 >= c.M) return;
+  const T* __restrict__ wm = w + (int64_t)min(m0 + li, c.M - 1) * (FLIP ? 9 : c.K);
+  int px[NC], po[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    px[j] = ((wave / MW) * NC + j) * 16 + li;
+    const int y = px[j] / c.R;
+    po[j] = y * W + px[j] - y * c.R;
+  }
+  v4f acc[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+  T A[2][DU][E];
+  int O[2][DU][E];
+  auto load = [&](int k0, T (&x)[DU][E], int (&o)[DU][E]) {
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int k = k0 + u * KS + lq * E + e;
+        const int2 ko = sK[min(k, c.K - 1)];
+        const T v = wm[ko.y];
+        x[u][e] = k < c.K ? v : T(0);
+        o[u][e] = k < c.K ? ko.x : -1;
+      }
+  };
+  auto mma = [&](const T (&x)[DU][E], const int (&o)[DU][E]) {
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        T b[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const T v = sIn[max(o[u][e], 0) + po[j]];
+          b[e] = o[u][e] >= 0 ? v : T(0);
+        }
+        if constexpr (BF) {
+          v4s xa, yb;
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            xa[e] = (short)x[u][e];
+            yb[e] = (short)b[e];
+          }
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xa, yb, acc[j], 0, 0, 0);
+        } else {
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u][0], b[0], acc[j], 0, 0, 0);
+        }
+      }
+  };
+  load(0, A[0], O[0]);
+  for (int k0 = 0; k0 < c.K; k0 += 2 * DU * KS) {
+    if (k0 + DU * KS < c.K) load(k0 + DU * KS, A[1], O[1]);
+    mma(A[0], O[0]);
+    if (k0 + DU * KS >= c.K) break;
+    if (k0 + 2 * DU * KS < c.K) load(k0 + 2 * DU * KS, A[0], O[0]);
+    mma(A[1], O[1]);
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 4 * lq + r;
+      if (m < c.M) mm_store(D, m, (int)(n0 + px[j]), acc[j][r]);
+    }
+}
+
+// dW[co][ci t] = sum over pixels of dOut[co][px] in[ci][px + off(t)], and the
+// bias gradient sum of dOut[co] as one more column block against ones.  A
+// workgroup takes every gridDim.x-th strip, keeps all of dW in registers (the
+// column blocks dealt to its 4 waves, NT per wave, MB row blocks each) and
+// writes raw sums to part; k_conv_dw_reduce adds the workgroups in order.
+// Split products over K = batch x pixels with k_mm read each element of both
+// operands through the im2col switch (187 to 247 us per stage at batch 32) and
+// summed the bias gradient over one workgroup per channel (up to 170 us).
+template <int MB, int NT>
+__global__ __launch_bounds__(256) void k_conv_dw(Conv c, const float* __restrict__ in, const float* __restrict__ dout,
+                                                 int strips, float* __restrict__ part) {
+  extern __shared__ __align__(16) char smem[];
+  float* sIn = reinterpret_cast<float*>(smem);
+  const int W = c.R + 2, R2 = c.R * c.R, CH = (c.P / c.R + 2) * W, lda = c.P + 4;
+  float* sA = sIn + c.C * CH;  // output gradient of the strip: [co][pixel]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lq = lane >> 4;
+  const int ncol = c.K + 1, nblk = (ncol + 15) / 16;  // column K: ones
+  int off[NT];  // tap offset of this lane's column; -1: ones, -2: none
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = (wave + 4 * j) * 16 + li;
+    const int ci = n / 9, t = n - 9 * ci, ty = t / 3;
+    off[j] = n < c.K ? ci * CH + ty * W + t - 3 * ty : n == c.K ? -1 : -2;
+  }
+  v4f acc[MB][NT];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int st = blockIdx.x; st < strips; st += gridDim.x) {
+    const int64_t n0 = (int64_t)st * c.P;
+    const int smp = (int)(n0 / R2), px0 = (int)(n0 - (int64_t)smp * R2);
+    __syncthreads();  // the previous strip has been read
+    conv_stage(c, in, smp, px0 / c.R, sIn);
+    for (int m = wave; m < 16 * MB; m += 4)
+      for (int x = lane; x < c.P; x += 64)
+        sA[m * lda + x] = m < c.M ? dout[((int64_t)smp * c.M + m) * R2 + px0 + x] : 0.f;
+    __syncthreads();
+    for (int y = 0; y < c.P / c.R; ++y)
+      for (int x = 0; x < c.R; x += 4) {
+        float a[MB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) a[i] = sA[(16 * i + li) * lda + y * c.R + x + lq];
+        const int po = y * W + x + lq;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          if (wave + 4 * j >= nblk) continue;  // wave-uniform
+          const float v = sIn[max(off[j], 0) + po];
+          const float b = off[j] >= 0 ? v : off[j] == -1 ? 1.f : 0.f;
+#pragma unroll
+          for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b, acc[i][j], 0, 0, 0);
+        }
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = 16 * i + 4 * lq + r, n = (wave + 4 * j) * 16 + li;
+        if (m < c.M && n < ncol) part[((int64_t)blockIdx.x * c.M + m) * ncol + n] = acc[i][j][r];
+      }
+}
+
+__global__ __launch_bounds__(256) void k_conv_dw_reduce(const float* __restrict__ part, int slices, int M, int K,
+                                                        float* __restrict__ dw, float* __restrict__ db) {
+  const int e = blockIdx.x * 256 + threadIdx.x, ncol = K + 1, n = M * ncol;
+  if (e >= n) return;
+  float v = 0.f;
+  for (int z0 = 0; z0 < slices; z0 += 8) {  // 8 loads in flight, added in order
+    float q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) q[u] = z0 + u < slices ? part[(int64_t)(z0 + u) * n + e] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v += q[u];
+  }
+  const int m = e / ncol, c = e - m * ncol;
+  if (c < K) dw[m * K + c] = v;
+  else db[m] = v;
+}
+
+// db[c] = sum over rows of dZ[r][c] (in order, 8 loads in flight)
 __global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ dZ, float* __restrict__ db, int m, int n) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= n) return;
   float s = 0.f;
-  for (int r = 0; r < m; ++r) s += dZ[(int64_t)r * n + c];
+  for (int r0 = 0; r0 < m; r0 += 8) {
+    float q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) q[u] = r0 + u < m ? dZ[(int64_t)(r0 + u) * n + c] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += q[u];
+  }
   db[c] = s;
 }
 
@@ -283,22 +568,18 @@ __global__ __launch_bounds__(256) void k_chansum(const float* __restrict__ dZ, f
   if (threadIdx.x == 0) db[ch] = s[0];
 }
 
-// gradient of a nearest x2 upsampling: each input pixel sums its 2 x 2 block
-__global__ __launch_bounds__(256) void k_down2_sum(const float* __restrict__ dUp, float* __restrict__ dIn,
-                                                   int64_t maps, int Ri) {
+// gradient of a nearest x2 upsampling, then of the ReLU before it: each input
+// pixel sums its 2 x 2 block, zero where A (that layer's output) is not positive
+__global__ __launch_bounds__(256) void k_down2_relu(const float* __restrict__ dUp, const float* __restrict__ A,
+                                                    float* __restrict__ dIn, int64_t maps, int Ri) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= maps * Ri * Ri) return;
   const int64_t mp = e / ((int64_t)Ri * Ri);
   const int px = (int)(e - mp * Ri * Ri), Y = px / Ri, X = px % Ri;
   const int R = 2 * Ri;
   const float* u = dUp + mp * R * R + (int64_t)(2 * Y) * R + 2 * X;
-  dIn[e] = (u[0] + u[1]) + (u[R] + u[R + 1]);
-}
-
-// dZ = dA where A > 0 (ReLU backward; A is the layer's output)
-__global__ __launch_bounds__(256) void k_relu_back(float* __restrict__ dA, const float* __restrict__ A, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n && A[i] <= 0.f) dA[i] = 0.f;
+  const float v = (u[0] + u[1]) + (u[R] + u[R + 1]);
+  dIn[e] = A[e] <= 0.f ? 0.f : v;
 }
 
 // dY = 2 (Y - T) / count; per-block partial sums of (Y - T)^2 into part
@@ -368,13 +649,89 @@ void mm(const Opnd& A, const Opnd& B, const Dst& D, int M, int N, int K, hipStre
   }
 }
 
+// Dense product.  k slices (where a scratch array is given) until about 512
+// waves are at work, each slice at least 128 deep.
+template <class T>
+void dense(const T* a, int am, int ak, const T* b, int bk, int bn, const Dst& D, int M, int N, int K, hipStream_t s,
+           float* part = nullptr, int64_t part_cap = 0) {
+  const int64_t waves = (int64_t)nblk(N, 16) * nblk(M, 16);
+  int splits = part ? (int)std::max<int64_t>(1, std::min<int64_t>(512 / waves, K / 128)) : 1;
+  if ((int64_t)splits * M * N > part_cap) splits = 1;
+  const int kchunk = splits > 1 ? ((K + splits - 1) / splits + 15) / 16 * 16 : K;
+  if (splits > 1) splits = (K + kchunk - 1) / kchunk;
+  k_dense<T><<<dim3(nblk(N, 64), nblk(M, 16), splits), 256, 0, s>>>(a, am, ak, b, bk, bn, D, M, N, K, kchunk,
+                                                                    splits > 1 ? part : nullptr);
+  MCHECK(hipGetLastError());
+  if (splits > 1) {
+    k_mm_reduce<<<nblk((int64_t)M * N, 256), 256, 0, s>>>(part, splits, D, M, N);
+    MCHECK(hipGetLastError());
+  }
+}
+
+// A stage's strips: P = 16 NC 4 / MW pixels, whole rows of one sample, the
+// largest NC of 4, 2, 1 that divides the map so and fits in 64 KB of LDS.
+constexpr size_t CONV_LDS = 64 << 10;
+inline int conv_mw(int M) { return M > 32 ? 4 : M > 16 ? 2 : 1; }
+inline bool conv_strip(Conv& c, int px, size_t per_entry, size_t extra) {
+  c.P = px;
+  return px % c.R == 0 && c.R * c.R % px == 0 && (size_t)c.C * c.ch() * per_entry + extra <= CONV_LDS;
+}
+
+// The convolution product on staged strips; false if the map does not divide.
+template <class T, int FLIP>
+bool conv(const T* in, int C, int R, int up, const T* w, int M, int batch, const Dst& D, hipStream_t s) {
+  const int mw = conv_mw(M);
+  Conv c{C, R, up, 0, M, C * 9};
+  int nc = 4;
+  while (nc && !conv_strip(c, 16 * nc * (4 / mw), sizeof(T), (size_t)c.K * sizeof(int2))) nc /= 2;
+  if (!nc) return false;
+  const size_t lds = (size_t)c.K * sizeof(int2) + (size_t)C * c.ch() * sizeof(T);
+  const dim3 g((unsigned)((int64_t)batch * R * R / c.P), nblk(M, 16 * mw));
+#define MLP_CONV(WW, NN)                                       \
+  if (mw == WW && nc == NN) {                                  \
+    k_conv<T, FLIP, WW, NN><<<g, 256, lds, s>>>(c, in, w, D);  \
+    MCHECK(hipGetLastError());                                 \
+    return true;                                               \
+  }
+  MLP_CONV(4, 4) MLP_CONV(4, 2) MLP_CONV(4, 1) MLP_CONV(2, 4) MLP_CONV(2, 2) MLP_CONV(2, 1)
+  MLP_CONV(1, 4) MLP_CONV(1, 2) MLP_CONV(1, 1)
+#undef MLP_CONV
+  return false;
+}
+
+// Weight and bias gradients of a convolution on staged strips; false if the
+// map does not divide, or dW does not fit in registers or its slices in part.
+inline bool conv_dw(const float* in, int C, int R, int up, const float* dout, int M, int batch, float* dw, float* db,
+                    float* part, int64_t part_cap, hipStream_t s) {
+  Conv c{C, R, up, 0, M, C * 9};
+  const int mb = nblk(M, 16), nt = nblk(nblk(c.K + 1, 16), 4);
+  if (R % 4 || mb > 4 || nt > 10 || mb == 3) return false;
+  bool fits = false;
+  for (int px = 256; px >= 16 && !fits; px /= 2) fits = conv_strip(c, px, 4, (size_t)16 * mb * (px + 4) * 4);
+  if (!fits) return false;
+  const size_t lds = ((size_t)C * c.ch() + (size_t)16 * mb * (c.P + 4)) * 4;
+  const int64_t strips = (int64_t)batch * R * R / c.P, cells = (int64_t)M * (c.K + 1);
+  const int slices = (int)std::min<int64_t>(std::min<int64_t>(strips, 256), part_cap / cells);
+  if (slices < 1 || strips > (1 << 30)) return false;
+#define MLP_DW(BB, NN)                                                                        \
+  if (mb == BB && nt <= NN) {                                                                 \
+    k_conv_dw<BB, NN><<<slices, 256, lds, s>>>(c, in, dout, (int)strips, part);               \
+    MCHECK(hipGetLastError());                                                                \
+    k_conv_dw_reduce<<<nblk(cells, 256), 256, 0, s>>>(part, slices, M, c.K, dw, db);          \
+    MCHECK(hipGetLastError());                                                                \
+    return true;                                                                              \
+  }
+  MLP_DW(1, 3) MLP_DW(1, 5) MLP_DW(1, 10) MLP_DW(2, 5) MLP_DW(2, 10) MLP_DW(4, 5) MLP_DW(4, 10)
+#undef MLP_DW
+  return false;
+}
+
 Opnd op_row(const void* p, int ld) { return Opnd{p, OP_ROW, ld, 0, 0, 0}; }
-Opnd op_trans(const void* p, int ld) { return Opnd{p, OP_TRANS, ld, 0, 0, 0}; }
 Dst dst_row(void* p, int ld, const float* bias, bool relu, bool bf16) {
-  return Dst{p, 0, ld, 0, 0, bias, 0, relu ? 1 : 0, bf16 ? 1 : 0};
+  return Dst{p, 0, ld, 0, 0, bias, 0, relu ? 1 : 0, bf16 ? 1 : 0, nullptr};
 }
 Dst dst_chan(void* p, int C, int R, const float* bias, bool relu, bool bf16) {
-  return Dst{p, 1, 0, C, R, bias, 1, relu ? 1 : 0, bf16 ? 1 : 0};
+  return Dst{p, 1, 0, C, R, bias, 1, relu ? 1 : 0, bf16 ? 1 : 0, nullptr};
 }
 
 struct Layer {
@@ -405,6 +762,7 @@ struct pecs_mlp {
   float* kpart = nullptr;  // split-k partial sums of the weight gradients
   int64_t kpart_cap = 0;
   float *target = nullptr, *part = nullptr;
+  float* hpart = nullptr;  // pinned host copy of the loss's partial sums
   hipStream_t s = nullptr;
   ~pecs_mlp() {
     if (s) (void)hipStreamSynchronize(s);
@@ -415,6 +773,7 @@ struct pecs_mlp {
     for (float* a : act) f(a);
     for (float* a : dact) f(a);
     for (uint16_t* a : actb) f(a);
+    if (hpart) (void)hipHostFree(hpart);
     if (s) (void)hipStreamDestroy(s);
   }
   int L() const { return (int)layers.size(); }
@@ -450,9 +809,9 @@ struct pecs_mlp {
     const bool relu = l < L();
     const float* bias = p + y.boff;
     if (!y.conv) {
-      mm<T>(op_row(in, y.nin), op_row(w + y.woff, y.nout), dst_row(out, y.nout, bias, relu, bf16out), rows, y.nout,
-            y.nin, s);
-    } else {
+      dense<T>(in, y.nin, 1, w + y.woff, y.nout, 1, dst_row(out, y.nout, bias, relu, bf16out), rows, y.nout, y.nin, s);
+    } else if (!conv<T, 0>(in, y.cin, y.R, y.up, w + y.woff, y.cout, rows,
+                           dst_chan(out, y.cout, y.R, bias, relu, bf16out), s)) {
       const Opnd B{in, OP_IM2COL, 0, y.cin, y.R, y.up};
       mm<T>(op_row(w + y.woff, y.cin * 9), B, dst_chan(out, y.cout, y.R, bias, relu, bf16out), y.cout,
             rows * y.R * y.R, y.cin * 9, s);
@@ -461,55 +820,59 @@ struct pecs_mlp {
   void forward(int rows) {
     for (int l = 1; l <= L(); ++l) layer_fwd<float>(l, rows, act[l - 1], act[l], p, false);
   }
-  // loss gradient in dact[L]; returns the loss (synchronises)
-  float loss_grad(int rows) {
+  // loss gradient in dact[L], its partial sums to hpart (on the stream)
+  void loss_grad(int rows) {
     const int64_t n = (int64_t)rows * nout;
     k_mse<<<256, 256, 0, s>>>(act[L()], target, dact[L()], part, n);
     MCHECK(hipGetLastError());
-    std::vector<float> h(256);
-    MCHECK(hipMemcpyAsync(h.data(), part, 256 * sizeof(float), hipMemcpyDeviceToHost, s));
-    MCHECK(hipStreamSynchronize(s));
+    MCHECK(hipMemcpyAsync(hpart, part, 256 * sizeof(float), hipMemcpyDeviceToHost, s));
+  }
+  float loss(int rows) const {  // once the stream has drained
     double acc = 0.0;
-    for (float x : h) acc += x;
-    return (float)(acc / (double)n);
+    for (int i = 0; i < 256; ++i) acc += hpart[i];
+    return (float)(acc / (double)((int64_t)rows * nout));
   }
   void backward(int rows) {
     for (int l = L(); l >= 1; --l) {
       const Layer& y = layers[l - 1];
+      // (every layer but the last ends in a ReLU: the input gradients are
+      // masked by the layer's output below)
+      const float* below = act[l - 1];
       if (!y.conv) {
         // dW = act[l-1]^T dact[l]; db = colsum(dact[l]); dact[l-1] = dact[l] W^T
-        mm<float>(op_trans(act[l - 1], y.nin), op_row(dact[l], y.nout), dst_row(g + y.woff, y.nout, nullptr, false, false),
-                  y.nin, y.nout, rows, s, kpart, kpart_cap);
+        dense<float>(act[l - 1], 1, y.nin, dact[l], y.nout, 1, dst_row(g + y.woff, y.nout, nullptr, false, false), y.nin,
+                     y.nout, rows, s);
         k_colsum<<<nblk(y.nout, 256), 256, 0, s>>>(dact[l], g + y.boff, rows, y.nout);
         MCHECK(hipGetLastError());
-        if (l > 1)
-          mm<float>(op_row(dact[l], y.nout), op_trans(p + y.woff, y.nout),
-                    dst_row(dact[l - 1], y.nin, nullptr, false, false), rows, y.nin, y.nout, s);
+        if (l > 1) {
+          Dst d = dst_row(dact[l - 1], y.nin, nullptr, false, false);
+          d.mask = below;
+          dense<float>(dact[l], y.nout, 1, p + y.woff, 1, y.nout, d, rows, y.nin, y.nout, s, kpart, kpart_cap);
+        }
       } else {
         const int R2 = y.R * y.R;
         // dW[co][ci t] = sum over (b, px) of dOut[b][co][px] im2col(in)[ci t][b px]
-        mm<float>(Opnd{dact[l], OP_CHAN, 0, y.cout, y.R, 0}, Opnd{act[l - 1], OP_IM2COL_T, 0, y.cin, y.R, y.up},
-                  dst_row(g + y.woff, y.cin * 9, nullptr, false, false), y.cout, y.cin * 9, rows * R2, s, kpart,
-                  kpart_cap);
-        k_chansum<<<y.cout, 256, 0, s>>>(dact[l], g + y.boff, rows, y.cout, R2);
-        MCHECK(hipGetLastError());
+        if (!conv_dw(act[l - 1], y.cin, y.R, y.up, dact[l], y.cout, rows, g + y.woff, g + y.boff, kpart, kpart_cap, s)) {
+          mm<float>(Opnd{dact[l], OP_CHAN, 0, y.cout, y.R, 0}, Opnd{act[l - 1], OP_IM2COL_T, 0, y.cin, y.R, y.up},
+                    dst_row(g + y.woff, y.cin * 9, nullptr, false, false), y.cout, y.cin * 9, rows * R2, s, kpart,
+                    kpart_cap);
+          k_chansum<<<y.cout, 256, 0, s>>>(dact[l], g + y.boff, rows, y.cout, R2);
+          MCHECK(hipGetLastError());
+        }
         if (l > 1) {
           // d(upsampled input)[ci][b px] = sum over (co, t) of W[co][ci][t] dOut[b][co][px - offset(t)]
-          float* dst = y.up ? dup : dact[l - 1];
-          mm<float>(Opnd{p + y.woff, OP_WT, 0, y.cin, 0, 0}, Opnd{dact[l], OP_DCOL, 0, y.cout, y.R, 0},
-                    dst_chan(dst, y.cin, y.R, nullptr, false, false), y.cin, rows * R2, y.cout * 9, s);
+          Dst d = dst_chan(y.up ? dup : dact[l - 1], y.cin, y.R, nullptr, false, false);
+          if (!y.up) d.mask = below;
+          if (!conv<float, 1>(dact[l], y.cout, y.R, 0, p + y.woff, y.cin, rows, d, s))
+            mm<float>(Opnd{p + y.woff, OP_WT, 0, y.cin, 0, 0}, Opnd{dact[l], OP_DCOL, 0, y.cout, y.R, 0}, d, y.cin,
+                      rows * R2, y.cout * 9, s);
           if (y.up) {
             const int Ri = y.R / 2;
             const int64_t n = (int64_t)rows * y.cin * Ri * Ri;
-            k_down2_sum<<<nblk(n, 256), 256, 0, s>>>(dup, dact[l - 1], (int64_t)rows * y.cin, Ri);
+            k_down2_relu<<<nblk(n, 256), 256, 0, s>>>(dup, below, dact[l - 1], (int64_t)rows * y.cin, Ri);
             MCHECK(hipGetLastError());
           }
         }
-      }
-      if (l > 1) {  // every layer but the last ends in a ReLU
-        const int64_t na = (int64_t)rows * size(l - 1);
-        k_relu_back<<<nblk(na, 256), 256, 0, s>>>(dact[l - 1], act[l - 1], na);
-        MCHECK(hipGetLastError());
       }
     }
   }
@@ -534,7 +897,7 @@ void mlp_init(pecs_mlp* net, unsigned seed) {
   }
   net->np = off;
   int64_t wmax = 0;
-  for (const Layer& y : net->layers) wmax = std::max(wmax, y.boff - y.woff);
+  for (const Layer& y : net->layers) wmax = std::max(wmax, y.boff - y.woff + (y.conv ? y.cout : y.nout));
   net->kpart_cap = std::min<int64_t>((int64_t)MAX_SPLIT * wmax, (int64_t)1 << 24);  // larger products do not split
   MCHECK(hipMalloc(&net->kpart, net->kpart_cap * sizeof(float)));
   std::vector<float> h(off, 0.f);
@@ -553,6 +916,7 @@ void mlp_init(pecs_mlp* net, unsigned seed) {
   MCHECK(hipMalloc(&net->v, off * sizeof(float)));
   MCHECK(hipMalloc(&net->pb, off * sizeof(uint16_t)));
   MCHECK(hipMalloc(&net->part, 256 * sizeof(float)));
+  MCHECK(hipHostMalloc((void**)&net->hpart, 256 * sizeof(float), hipHostMallocDefault));
   MCHECK(hipMemcpy(net->p, h.data(), off * sizeof(float), hipMemcpyHostToDevice));
   MCHECK(hipMemset(net->m, 0, off * sizeof(float)));
   MCHECK(hipMemset(net->v, 0, off * sizeof(float)));
@@ -672,11 +1036,11 @@ int pecs_mlp_gradients(pecs_mlp* net, const float* x, const float* y, int batch,
     MCHECK(hipMemcpyAsync(net->act[0], x, (size_t)batch * net->nin * sizeof(float), hipMemcpyHostToDevice, net->s));
     MCHECK(hipMemcpyAsync(net->target, y, (size_t)batch * net->nout * sizeof(float), hipMemcpyHostToDevice, net->s));
     net->forward(batch);
-    const float l = net->loss_grad(batch);
+    net->loss_grad(batch);
     net->backward(batch);
     if (grads) MCHECK(hipMemcpyAsync(grads, net->g, net->np * sizeof(float), hipMemcpyDeviceToHost, net->s));
     MCHECK(hipStreamSynchronize(net->s));
-    if (loss) *loss = l;
+    if (loss) *loss = net->loss(batch);
   } catch (const std::exception& e) {
     return mlp_fail(e);
   }
