@@ -120,7 +120,7 @@ struct pecs_ctx {
   double* rH = nullptr;  // B multiplier right-hand sides, h-major
   double* tH = nullptr;
   double* old[5] = {};
-  double* acc = nullptr;  // 2 per instance
+  double* acc = nullptr;  // 2 per instance, pinned host memory
   double* rpart = nullptr;  // residual partial sums: 5 vectors x RES_PARTS pairs per instance
   double* io[4] = {};     // staging for host-pointer calls (one instance)
   std::vector<double> last_res;
@@ -163,6 +163,7 @@ struct pecs_ctx {
     if (join_ev) (void)hipEventDestroy(join_ev);
     for (hipEvent_t e : events) (void)hipEventDestroy(e);
     for (void* p : allocs) (void)hipFree(p);
+    if (acc) (void)hipHostFree(acc);
     factor_handle_destroy(blas);
   }
 };
@@ -990,33 +991,37 @@ void step_once(pecs_ctx* c) {
 // copy, the step and the residual are ordered by the graph's edges.)
 void save_old(pecs_ctx* c, hipStream_t s) {
   const int64_t nsv[5] = {c->Ns, c->Ns, c->Ne, c->Ne, c->NP};
-  for (int j = 0; j < 4; ++j) HIPCHECK((hipError_t)launch_copy(c->u[j], c->old[j], c->B * nsv[j], s));
-  HIPCHECK((hipError_t)launch_copy(c->pv, c->old[4], c->B * nsv[4], s));
+  VecPairs v{};
+  v.nvec = 5;
+  for (int j = 0; j < 5; ++j) {
+    v.a[j] = j < 4 ? c->u[j] : c->pv;
+    v.b[j] = c->old[j];
+    v.n[j] = c->B * nsv[j];
+  }
+  HIPCHECK((hipError_t)launch_copy(v, s));
 }
 
 // ||x^{n+1} - x^n||^2 and ||x^n||^2 over the five state vectors, per
-// instance, into c->acc (2 per instance).
+// instance, into c->acc (2 per instance; pinned host memory, so that the last
+// kernel of the step hands them over and no copy follows it).
 void launch_residual(pecs_ctx* c, hipStream_t s) {
   const int64_t nsv[5] = {c->Ns, c->Ns, c->Ne, c->Ne, c->NP};
-  const int B = c->B;
-  for (int b = 0; b < B; ++b) {
-    for (int j = 0; j < 5; ++j) {
-      const double* cur = j < 4 ? c->u[j] : c->pv;
-      HIPCHECK((hipError_t)launch_diff_norms(cur + b * nsv[j], c->old[j] + b * nsv[j], nsv[j],
-                                             c->rpart + (size_t)(5 * b + j) * 2 * RES_PARTS, s));
-    }
+  VecPairs v{};
+  v.nvec = 5;
+  for (int j = 0; j < 5; ++j) {
+    v.a[j] = j < 4 ? c->u[j] : c->pv;
+    v.b[j] = c->old[j];
+    v.n[j] = v.stride[j] = nsv[j];
   }
-  HIPCHECK((hipError_t)launch_sum_partials(c->rpart, 5, c->acc, B, s));
+  HIPCHECK((hipError_t)launch_norms(v, c->rpart, c->acc, c->B, s));
 }
 
-// c->acc to the host (after the stream has drained), then the residuals.
+// The residuals from c->acc, after the stream has drained.
 void finish_residual(pecs_ctx* c) {
-  std::vector<double> h(2 * c->B);
-  HIPCHECK(hipMemcpy(h.data(), c->acc, 2 * c->B * sizeof(double), hipMemcpyDeviceToHost));
+  const double* h = c->acc;
   for (int b = 0; b < c->B; ++b)
     c->last_res[b] = (h[2 * b + 1] > 0) ? std::sqrt(h[2 * b] / h[2 * b + 1]) / c->P.dt : 0.0;
 }
-
 
 // Capture into a graph (once per context), on c->cap with the context's own
 // stream swapped for it; the side-stream fork/join of the region solves
@@ -1368,7 +1373,7 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     c->yP = dalloc<double>(c.get(), B * c->ysz);
     c->rH = dalloc<double>(c.get(), B * (size_t)c->FH.n);
     c->tH = dalloc<double>(c.get(), std::max(B, scratch_rhs(B)) * (size_t)c->FH.n);
-    c->acc = dalloc<double>(c.get(), 2 * B);
+    HIPCHECK(hipHostMalloc((void**)&c->acc, 2 * B * sizeof(double), hipHostMallocDefault));
     c->rpart = dalloc<double>(c.get(), (size_t)10 * RES_PARTS * B);
     c->last_res.assign(B, -1.0);
     HIPCHECK(hipDeviceSynchronize());
@@ -1847,13 +1852,15 @@ int pecs_last_density_change(pecs_ctx* ctx, double* out) {
     const int B = ctx->B;
     if (!ctx->dacc) ctx->dacc = dalloc<double>(ctx, 2 * (size_t)B);
     const int64_t nsv[4] = {ctx->Ns, ctx->Ns, ctx->Ne, ctx->Ne};
-    for (int b = 0; b < B; ++b)
-      for (int j = 0; j < 4; ++j) {
-        const int64_t n = nsv[j], off = b * n + 2 * n / 3;  // the density block of [Jx | Jy | u]
-        HIPCHECK((hipError_t)launch_diff_norms(ctx->u[j] + off, ctx->old[j] + off, n / 3,
-                                               ctx->rpart + (size_t)(4 * b + j) * 2 * RES_PARTS, ctx->stream));
-      }
-    HIPCHECK((hipError_t)launch_sum_partials(ctx->rpart, 4, ctx->dacc, B, ctx->stream));
+    VecPairs v{};
+    v.nvec = 4;
+    for (int j = 0; j < 4; ++j) {  // the density block of [Jx | Jy | u]
+      v.a[j] = ctx->u[j] + 2 * nsv[j] / 3;
+      v.b[j] = ctx->old[j] + 2 * nsv[j] / 3;
+      v.n[j] = nsv[j] / 3;
+      v.stride[j] = nsv[j];
+    }
+    HIPCHECK((hipError_t)launch_norms(v, ctx->rpart, ctx->dacc, B, ctx->stream));
     std::vector<double> h(2 * (size_t)B);
     d2h(ctx, h.data(), ctx->dacc, 2 * (int64_t)B);
     for (int b = 0; b < B; ++b) out[b] = h[2 * b + 1] > 0 ? std::sqrt(h[2 * b] / h[2 * b + 1]) : 0.0;

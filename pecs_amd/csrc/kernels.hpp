@@ -272,14 +272,22 @@ int launch_poisson_recover(int k, const DevPoisson& P, const double* lam, const 
 int launch_poisson_rhs_assemble(int k, const DevPoisson& P, const DevTabs& T, const DevPhys* phs, const double* un,
                                 const double* up, const double* ur, const double* uo, int ncs, int nce, double* b,
                                 hipStream_t s);
-// Steady residual: per vector, RES_PARTS partial pairs (|a-b|^2, |b|^2) into
-// part[0 .. 2 RES_PARTS); then per instance the sum of nvec vectors' partials
-// (stored consecutively, instance after instance) into acc[2 i], acc[2 i + 1].
+// Up to 5 vector pairs; instance i of pair j begins stride[j] entries after
+// instance i - 1.
+struct VecPairs {
+  int nvec;
+  const double* a[5];
+  double* b[5];
+  int64_t n[5], stride[5];
+};
+// b = a of every pair (one instance), as a kernel (stays on the stream's
+// compute queue)
+int launch_copy(const VecPairs& v, hipStream_t s);
+// Steady residual: acc[2 i], acc[2 i + 1] = the sums of |a - b|^2 and |b|^2
+// over instance i's vectors; part: scratch, 2 RES_PARTS doubles per vector and
+// instance.  acc may be pinned host memory.
 constexpr int RES_PARTS = 1024;
-int launch_diff_norms(const double* a, const double* b, int64_t n, double* part, hipStream_t s);
-int launch_sum_partials(const double* part, int nvec, double* acc, int ninst, hipStream_t s);
-// dst[0:n] = src[0:n] as a kernel (stays on the stream's compute queue)
-int launch_copy(const double* src, double* dst, int64_t n, hipStream_t s);
+int launch_norms(const VecPairs& v, double* part, double* acc, int ninst, hipStream_t s);
 // Density of a carrier vector (region refinement r) at the G x G logical
 // cell centres of its region, and the density block from such a grid
 // (nodal values of the grid's bilinear interpolant).
