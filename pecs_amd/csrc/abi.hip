@@ -1276,6 +1276,14 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
     P.type = upload(c.get(), op.type);
     P.table = upload(c.get(), op.table);
     P.stride = op.type_stride;
+    {
+      const size_t nl = op.nloc;
+      std::vector<double> t((size_t)op.ntype * nl * nl);
+      for (int ty = 0; ty < op.ntype; ++ty)
+        for (size_t i = 0; i < nl; ++i)
+          for (size_t j = 0; j < nl; ++j) t[(ty * nl + j) * nl + i] = op.table[ty * (size_t)op.type_stride + i * nl + j];
+      P.tab_t = upload(c.get(), t);
+    }
     {  // wave-uniform cell list for the recovery (as for the Schur kernels)
       const char* su = std::getenv("PECS_SCHUR_UNIFORM");
       std::vector<int> own = wave_groups(m.ncellP, 1, [&](int K, int* key) { key[0] = op.type[K]; });

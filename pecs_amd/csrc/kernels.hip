@@ -1524,43 +1524,6 @@ __device__ __forceinline__ void poisson_mdir(const DevPoisson& P, const DevTabs&
   }
 }
 
-// UNI: cells from P.ucell (waves share the cell type: scalar table reads)
-template <int K, bool UNI>
-__global__ __launch_bounds__(64) void k_poisson_cell(DevPoisson P, DevTabs T, const DevPhys* __restrict__ phs,
-                                                     const double* __restrict__ un, const double* __restrict__ up,
-                                                     const double* __restrict__ ur, const double* __restrict__ uo,
-                                                     int ncs, int nce, double* __restrict__ y, int64_t ss, int64_t se,
-                                                     int64_t sy) {
-  const DevPhys ph = phs[blockIdx.y];
-  {
-    const int64_t i = blockIdx.y;
-    un += i * ss;
-    up += i * ss;
-    ur += i * se;
-    uo += i * se;
-    y += i * sy;
-  }
-  using S = Sz<K>;
-  constexpr int NRT = S::NRT, NL = S::NL, NPHI = S::NPHI;
-  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int Kc = UNI ? (t0 < P.nucell ? P.ucell[t0] : -1) : (t0 < P.ncell ? t0 : -1);
-  if (Kc < 0) return;
-  double f[NL];
-  const int ty = UNI ? __builtin_amdgcn_readfirstlane(P.type[Kc]) : P.type[Kc];
-  const double* tb = P.table + (size_t)ty * P.stride;
-#pragma unroll
-  for (int i = 0; i < NRT; ++i) f[i] = poisson_bias<K>(tb, ph, i);
-  if (P.mdir) poisson_mdir<K>(P, T, Kc, f);
-  poisson_fphi<K>(P, T, ph, Kc, un, up, ur, uo, ncs, nce, f + NRT);
-  for (int i = 0; i < NL; ++i) {
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < NL; ++j) s += tb[i * NL + j] * f[j];
-    y[(size_t)Kc * NL + i] = s;
-  }
-  (void)NPHI;
-}
-
 // face DoF ownership for the continuous D layout: left/bottom faces belong to
 // the cell; right/top faces only on the right/top boundary.
 template <int K>
@@ -1585,26 +1548,140 @@ __device__ __forceinline__ bool owns_face(const DevPoisson& P, int Kc, int f) {
   return (P.own[Kc] >> f) & 1;
 }
 
-template <int K>
-__global__ __launch_bounds__(64) void k_poisson_cell_from_b(DevPoisson P, const double* __restrict__ b,
-                                                            double* __restrict__ y) {
+// y = A^{-1} f of cells whose f is in LDS, or (assemble) f into the global
+// right-hand side
+template <int K, int IG, int NC>
+__device__ __forceinline__ void poisson_store(const DevPoisson& P, const double (&sf)[IG][NC][Sz<K>::NL], int c0, int i0,
+                                              int ninst, double* __restrict__ y, int64_t sy, int assemble) {
   constexpr int NL = Sz<K>::NL, NRT = Sz<K>::NRT;
-  const int Kc = blockIdx.x * blockDim.x + threadIdx.x;
-  if (Kc >= P.ncell) return;
-  const int* id = P.idx + (size_t)Kc * NL;
-  double f[NL];
-  for (int i = 0; i < NL; ++i) {
+  for (int e = threadIdx.x; e < NC * NL; e += 256) {
+    const int i = e % NL, lc = e / NL, Kc = c0 + lc;
+    if (Kc >= P.ncell) break;
+    if (assemble) {
+      int m;
+      const int fc = i < NRT ? face_of_local<K>(i, m) : -1;
+      if (fc < 0 || owns_face<K>(P, Kc, fc)) y[P.idx[(size_t)Kc * NL + i]] = sf[0][lc][i];
+      continue;
+    }
+    const double* __restrict__ tb = P.tab_t + (size_t)P.type[Kc] * NL * NL + i;
+    double s[IG];
+#pragma unroll
+    for (int g = 0; g < IG; ++g) s[g] = 0.0;
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const double a = tb[j * NL];
+#pragma unroll
+      for (int g = 0; g < IG; ++g) s[g] += a * sf[g][lc][j];
+    }
+#pragma unroll
+    for (int g = 0; g < IG; ++g)
+      if (i0 + g < ninst) y[(i0 + g) * sy + (size_t)Kc * NL + i] = s[g];
+  }
+}
+
+// Cell right-hand side f (D rows: bias data; Phi rows: -<phi, rho>) and, unless
+// `assemble`, its condensation y = A^{-1} f (into y); assemble: f itself into
+// the global right-hand side y.  A wave takes 16 cells of one instance: the
+// charge at the quadrature points and its moments are FP64 MFMA products, as in
+// k_rhs_carrier; then a thread takes a (cell, row) and applies A^{-1} from LDS,
+// its table row (A^{-1} transposed: coalesced over the rows) for all IG
+// instances.  IG 4: 16 cells of 4 instances per workgroup, else 64 cells.
+// One thread per cell took 26 us at refinement 8, k = 2 and 20 us at
+// refinement 4, k = 3.
+template <int K, int IG>
+__global__ __launch_bounds__(256) void k_poisson_cell(DevPoisson P, DevTabs T, const DevPhys* __restrict__ phs,
+                                                      const double* __restrict__ un, const double* __restrict__ up,
+                                                      const double* __restrict__ ur, const double* __restrict__ uo,
+                                                      int ncs, int nce, double* __restrict__ y, int64_t ss, int64_t se,
+                                                      int64_t sy, int ninst, int assemble) {
+  using S = Sz<K>;
+  constexpr int NB = S::NB, NQ = S::NQ, NRT = S::NRT, NL = S::NL, NPHI = S::NPHI;
+  constexpr int SA = (NB + 3) / 4, QB = (NQ + 15) / 16, NC = 64 / IG;
+  __shared__ double sf[IG][NC][NL];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int col = lane & 15, kq = lane >> 4;
+  const int c0 = blockIdx.x * NC, i0 = blockIdx.y * IG;
+  {
+    const int ig = IG > 1 ? wave : 0, lc = (IG > 1 ? 0 : 16 * wave) + col;
+    const int i = min(i0 + ig, ninst - 1);  // (instances and cells past the last repeat it and store nothing)
+    const int Kc = min(c0 + lc, P.ncell - 1);
+    const bool semi = Kc < ncs;
+    const int c = semi ? Kc : Kc - ncs, nc = semi ? ncs : nce;
+    const double* __restrict__ u1 = semi ? un + i * ss : ur + i * se;
+    const double* __restrict__ u2 = semi ? up + i * ss : uo + i * se;
+    const double rho0 = semi ? phs[i].ne - phs[i].pe : 0.0;  // N_D - N_A (SolarCell.cpp:542-548)
+    const size_t ub = 2 * (size_t)nc * NB + (size_t)c * NB;
+    double v[8], d[SA];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = P.V[8 * (size_t)Kc + t];
+#pragma unroll
+    for (int t = 0; t < SA; ++t) {
+      const int a = 4 * t + kq;
+      d[t] = a < NB ? u2[ub + a] - u1[ub + a] : 0.0;
+    }
+    v4d f = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      v4d rho = {0.0, 0.0, 0.0, 0.0};
+      const int qr = 16 * qb + col;
+#pragma unroll
+      for (int t = 0; t < SA; ++t) {
+        const int a = 4 * t + kq;
+        rho = __builtin_amdgcn_mfma_f64_16x16x4f64((qr < NQ && a < NB) ? T.phi[a * NQ + qr] : 0.0, d[t], rho, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (16 * qb + 4 * r >= NQ) continue;
+        const int q = 16 * qb + 4 * r + kq;
+        const bool in = q < NQ;
+        const int qc = in ? q : NQ - 1;
+        const GeoD g = bilin(v, T.qx[qc], T.qy[qc]);
+        double w = rho0 + rho[r];
+        if (P.msrc) w += P.msrc[(size_t)Kc * NQ + qc];
+        w = in ? -w * T.qw[qc] * g.det : 0.0;
+        f = __builtin_amdgcn_mfma_f64_16x16x4f64((in && col < NPHI) ? T.phiP[col * NQ + q] : 0.0, w, f, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < (NPHI + 3) / 4; ++r)
+      if (4 * r + kq < NPHI) sf[ig][lc][NRT + 4 * r + kq] = f[r];
+  }
+  for (int e = threadIdx.x; e < IG * NC * NRT; e += 256) {  // D rows
+    const int i = e % NRT, lc = e / NRT % NC, ig = e / (NRT * NC);
+    const int Kc = min(c0 + lc, P.ncell - 1);
+    sf[ig][lc][i] = poisson_bias<K>(P.table + (size_t)P.type[Kc] * P.stride, phs[min(i0 + ig, ninst - 1)], i);
+  }
+  __syncthreads();
+  if (P.mdir) {
+    for (int lc = threadIdx.x; lc < NC; lc += 256) {
+      double f[NRT];
+#pragma unroll
+      for (int i = 0; i < NRT; ++i) f[i] = 0.0;
+      if (c0 + lc < P.ncell) poisson_mdir<K>(P, T, c0 + lc, f);
+      for (int ig = 0; ig < IG; ++ig)
+        for (int i = 0; i < NRT; ++i) sf[ig][lc][i] += f[i];
+    }
+    __syncthreads();
+  }
+  poisson_store<K, IG, NC>(P, sf, c0, i0, ninst, y, sy, assemble);
+}
+
+// condensation of a given right-hand side b (in the global layout)
+template <int K>
+__global__ __launch_bounds__(256) void k_poisson_cell_from_b(DevPoisson P, const double* __restrict__ b,
+                                                             double* __restrict__ y) {
+  constexpr int NL = Sz<K>::NL, NRT = Sz<K>::NRT, NC = 16;
+  __shared__ double sf[1][NC][NL];
+  const int c0 = blockIdx.x * NC;
+  for (int e = threadIdx.x; e < NC * NL; e += 256) {
+    const int i = e % NL, lc = e / NL, Kc = c0 + lc;
+    if (Kc >= P.ncell) break;
     int m;
     const int fc = (i < NRT) ? face_of_local<K>(i, m) : -1;
-    f[i] = (fc < 0 || owns_face<K>(P, Kc, fc)) ? b[id[i]] : 0.0;
+    sf[0][lc][i] = (fc < 0 || owns_face<K>(P, Kc, fc)) ? b[P.idx[(size_t)Kc * NL + i]] : 0.0;
   }
-  const double* tb = P.table + (size_t)P.type[Kc] * P.stride;
-  for (int i = 0; i < NL; ++i) {
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < NL; ++j) s += tb[i * NL + j] * f[j];
-    y[(size_t)Kc * NL + i] = s;
-  }
+  __syncthreads();
+  poisson_store<K, 1, NC>(P, sf, c0, 0, 1, y, 0, 0);
 }
 
 __global__ __launch_bounds__(256) void k_poisson_face(DevPoisson P, const double* __restrict__ y,
@@ -1621,47 +1698,54 @@ __global__ __launch_bounds__(256) void k_poisson_face(DevPoisson P, const double
   r[P.mult_perm[m]] = s;
 }
 
-// UNI: cells from P.ucell, whose waves share the cell type, so the table
-// offsets are wave-uniform (scalar-cache reads).  Faces without multipliers
-// contribute exact zeros (s - 0 = s), so the sum equals the one over the
-// faces that have them.
-template <int K, bool UNI>
-__global__ __launch_bounds__(64) void k_poisson_recover(DevPoisson P, const double* __restrict__ lam,
-                                                        const double* __restrict__ y, double* __restrict__ out,
-                                                        int64_t sl, int64_t sy, int64_t so) {
-  constexpr int NL = Sz<K>::NL, NRT = Sz<K>::NRT;
-  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int Kc = UNI ? (t0 < P.nucell ? P.ucell[t0] : -1) : (t0 < P.ncell ? t0 : -1);
-  if (Kc < 0) return;
-  lam += blockIdx.y * sl;
-  y += blockIdx.y * sy;
-  out += blockIdx.y * so;
-  double e[4 * K];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
+// x_K = y - A^{-1} E^T lambda, a (cell, row) per thread, 32 cells per
+// workgroup, the cell's weighted multipliers in LDS, the table entries for all
+// IG instances of the workgroup.
+template <int K, int IG>
+__global__ __launch_bounds__(256) void k_poisson_recover(DevPoisson P, const double* __restrict__ lam,
+                                                         const double* __restrict__ y, double* __restrict__ out,
+                                                         int64_t sl, int64_t sy, int64_t so, int ninst) {
+  constexpr int NL = Sz<K>::NL, NRT = Sz<K>::NRT, NC = 32, NE = 4 * K;
+  __shared__ double se[IG][NC][NE];
+  const int c0 = blockIdx.x * NC, i0 = blockIdx.y * IG;
+  for (int e = threadIdx.x; e < NC * NE; e += 256) {
+    const int fm = e % NE, lc = e / NE, Kc = c0 + lc, f = fm / K, m = fm - f * K;
+    if (Kc >= P.ncell) break;
     const int base = P.mult_face[4 * (size_t)Kc + f];
-    const double sf = (f == 1 || f == 3) ? 1.0 : -1.0;
+    const double w = (f == 1 || f == 3) ? P.gw[m] : -P.gw[m];
+    const int p = base < 0 ? 0 : P.mult_perm[base + m];
 #pragma unroll
-    for (int m = 0; m < K; ++m) e[f * K + m] = base < 0 ? 0.0 : sf * P.gw[m] * lam[P.mult_perm[base + m]];
+    for (int g = 0; g < IG; ++g) se[g][lc][fm] = base < 0 ? 0.0 : w * lam[min(i0 + g, ninst - 1) * sl + p];
   }
-  const int ty = UNI ? __builtin_amdgcn_readfirstlane(P.type[Kc]) : P.type[Kc];
-  const double* tb = P.table + (size_t)ty * P.stride;
-  const int* id = P.idx + (size_t)Kc * NL;
-  for (int i = 0; i < NL; ++i) {
-    double s = y[(size_t)Kc * NL + i];
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int m = 0; m < K; ++m) s -= tb[i * NL + rt_face<K>(f, m)] * e[f * K + m];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NC * NL; e += 256) {
+    const int i = e % NL, lc = e / NL, Kc = c0 + lc;
+    if (Kc >= P.ncell) break;
+    bool zero = false;
     if (i < NRT) {
       int m;
       const int fc = face_of_local<K>(i, m);
       if (fc >= 0) {
         if (!owns_face<K>(P, Kc, fc)) continue;
-        if (P.pbid[4 * (size_t)Kc + fc] == 2) s = 0.0;  // Neumann D.n = 0 (Poisson.cpp:41-47)
+        zero = P.pbid[4 * (size_t)Kc + fc] == 2;  // Neumann D.n = 0 (Poisson.cpp:41-47)
       }
     }
-    out[id[i]] = s;
+    const double* __restrict__ tb = P.tab_t + (size_t)P.type[Kc] * NL * NL + i;
+    double s[IG];
+#pragma unroll
+    for (int g = 0; g < IG; ++g) s[g] = y[min(i0 + g, ninst - 1) * sy + (size_t)Kc * NL + i];
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        const double a = tb[rt_face<K>(f, m) * NL];
+#pragma unroll
+        for (int g = 0; g < IG; ++g) s[g] -= a * se[g][lc][f * K + m];
+      }
+    const int id = P.idx[(size_t)Kc * NL + i];
+#pragma unroll
+    for (int g = 0; g < IG; ++g)
+      if (i0 + g < ninst) out[(i0 + g) * so + id] = zero ? 0.0 : s[g];
   }
 }
 
@@ -1748,35 +1832,6 @@ __global__ __launch_bounds__(64) void k_poisson_recover_f32(DevPoisson P, const 
     }
     out[id[i]] = s;
   }
-}
-
-template <int K>
-__global__ __launch_bounds__(64) void k_poisson_rhs_assemble(DevPoisson P, DevTabs T, const DevPhys* __restrict__ phs,
-                                                             const double* __restrict__ un,
-                                                             const double* __restrict__ up,
-                                                             const double* __restrict__ ur,
-                                                             const double* __restrict__ uo, int ncs, int nce,
-                                                             double* __restrict__ b) {
-  constexpr int NL = Sz<K>::NL, NRT = Sz<K>::NRT, NPHI = Sz<K>::NPHI;
-  const int Kc = blockIdx.x * blockDim.x + threadIdx.x;
-  if (Kc >= P.ncell) return;
-  const DevPhys ph = phs[0];
-  double fphi[NPHI];
-  poisson_fphi<K>(P, T, ph, Kc, un, up, ur, uo, ncs, nce, fphi);
-  const int* id = P.idx + (size_t)Kc * NL;
-  const double* tb = P.table + (size_t)P.type[Kc] * P.stride;
-  double fd[NRT];
-#pragma unroll
-  for (int i = 0; i < NRT; ++i) fd[i] = poisson_bias<K>(tb, ph, i);
-  if (P.mdir) poisson_mdir<K>(P, T, Kc, fd);
-  for (int i = 0; i < NRT; ++i) {
-    int m;
-    const int fc = face_of_local<K>(i, m);
-    if (fc >= 0 && !owns_face<K>(P, Kc, fc)) continue;
-    b[id[i]] = fd[i];
-  }
-#pragma unroll
-  for (int l = 0; l < NPHI; ++l) b[id[NRT + l]] = fphi[l];
 }
 
 // dst = src of up to 5 vectors, one launch (blockIdx.y: the vector)
@@ -2337,19 +2392,19 @@ int launch_poisson_cell(int k, const DevPoisson& P, const DevTabs& T, const DevP
                            P, T, phs, un, up, ur, uo, ncs, nce, y, ss, se, sy)));
     return (int)hipGetLastError();
   }
-  if (P.ucell) {
-    PECS_DISPATCH_K(k, (k_poisson_cell<KK, true><<<dim3(nblk(P.nucell, 64), nb), 64, 0, s>>>(
-                           P, T, phs, un, up, ur, uo, ncs, nce, y, ss, se, sy)));
+  if (nb >= 4) {
+    PECS_DISPATCH_K(k, (k_poisson_cell<KK, 4><<<dim3(nblk(P.ncell, 16), nblk(nb, 4)), 256, 0, s>>>(
+                           P, T, phs, un, up, ur, uo, ncs, nce, y, ss, se, sy, nb, 0)));
   } else {
-    PECS_DISPATCH_K(k, (k_poisson_cell<KK, false><<<dim3(nblk(P.ncell, 64), nb), 64, 0, s>>>(
-                           P, T, phs, un, up, ur, uo, ncs, nce, y, ss, se, sy)));
+    PECS_DISPATCH_K(k, (k_poisson_cell<KK, 1><<<dim3(nblk(P.ncell, 64), nb), 256, 0, s>>>(
+                           P, T, phs, un, up, ur, uo, ncs, nce, y, ss, se, sy, nb, 0)));
   }
   return (int)hipGetLastError();
 }
 
 int launch_poisson_cell_from_b(const DevPoisson& P, const double* b, double* y, hipStream_t s) {
   const int k = (P.nphi == 1) ? 1 : (P.nphi == 4 ? 2 : 3);
-  PECS_DISPATCH_K(k, (k_poisson_cell_from_b<KK><<<nblk(P.ncell, 64), 64, 0, s>>>(P, b, y)));
+  PECS_DISPATCH_K(k, (k_poisson_cell_from_b<KK><<<nblk(P.ncell, 16), 256, 0, s>>>(P, b, y)));
   return (int)hipGetLastError();
 }
 
@@ -2366,12 +2421,12 @@ static int launch_poisson_recover_main(int k, const DevPoisson& P, const double*
                                                                                               so)));
     return (int)hipGetLastError();
   }
-  if (P.ucell) {
-    PECS_DISPATCH_K(k, (k_poisson_recover<KK, true><<<dim3(nblk(P.nucell, 64), nb), 64, 0, s>>>(P, lam, y, out, sl,
-                                                                                                 sy, so)));
+  if (nb >= 4) {
+    PECS_DISPATCH_K(k, (k_poisson_recover<KK, 4><<<dim3(nblk(P.ncell, 32), nblk(nb, 4)), 256, 0, s>>>(
+                           P, lam, y, out, sl, sy, so, nb)));
   } else {
-    PECS_DISPATCH_K(k, (k_poisson_recover<KK, false><<<dim3(nblk(P.ncell, 64), nb), 64, 0, s>>>(P, lam, y, out, sl,
-                                                                                                  sy, so)));
+    PECS_DISPATCH_K(k, (k_poisson_recover<KK, 1><<<dim3(nblk(P.ncell, 32), nb), 256, 0, s>>>(P, lam, y, out, sl, sy, so,
+                                                                                             nb)));
   }
   return (int)hipGetLastError();
 }
@@ -2475,8 +2530,8 @@ int launch_poisson_recover(int k, const DevPoisson& P, const double* lam, const 
 int launch_poisson_rhs_assemble(int k, const DevPoisson& P, const DevTabs& T, const DevPhys* phs, const double* un,
                                 const double* up, const double* ur, const double* uo, int ncs, int nce, double* b,
                                 hipStream_t s) {
-  PECS_DISPATCH_K(k, (k_poisson_rhs_assemble<KK><<<nblk(P.ncell, 64), 64, 0, s>>>(P, T, phs, un, up, ur, uo, ncs,
-                                                                                   nce, b)));
+  PECS_DISPATCH_K(k, (k_poisson_cell<KK, 1><<<dim3(nblk(P.ncell, 64), 1), 256, 0, s>>>(P, T, phs, un, up, ur, uo, ncs,
+                                                                                       nce, b, 0, 0, 0, 1, 1)));
   return (int)hipGetLastError();
 }
 

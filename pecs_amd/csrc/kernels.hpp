@@ -60,6 +60,7 @@ struct DevPoisson {
   const int* idx;        // nloc global DoFs per cell
   const int* type;
   const double* table;   // per type: Ainv | U0 | U1 | U2 (unit Dirichlet data of phi_bi, phi_app, phi_sch)
+  const double* tab_t;   // per type: Ainv transposed
   int stride;
   const int* pbid;       // 4 per cell
   const int* pI;
