@@ -766,9 +766,10 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
       bym[hb.M].push_back({hb.X, (int)h});
     }
     auto csr = [&](const std::vector<std::vector<std::pair<int, int>>>& L, const int*& cell, const int*& ptr,
-                   const int*& other, const int*& bi) {
-      std::vector<int> vc, vp{0}, vo, vb;
+                   const int*& other, const int*& bi, const int*& all) {
+      std::vector<int> vc, vp{0}, vo, vb, va{0};
       for (int x = 0; x < R.ncell; ++x) {
+        va.push_back(va.back() + (int)L[x].size());
         if (L[x].empty()) continue;
         vc.push_back(x);
         for (const auto& pr : L[x]) {
@@ -781,10 +782,11 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
       ptr = upload(c, vp);
       other = upload(c, vo);
       bi = upload(c, vb);
+      all = upload(c, va);
       return (int)vc.size();
     };
-    d.nhx = csr(byx, d.hx_cell, d.hx_ptr, d.hx_src, d.hx_blk);
-    d.nhm = csr(bym, d.hm_cell, d.hm_ptr, d.hm_dst, d.hm_blk);
+    d.nhx = csr(byx, d.hx_cell, d.hx_ptr, d.hx_src, d.hx_blk, d.hx_all);
+    d.nhm = csr(bym, d.hm_cell, d.hm_ptr, d.hm_dst, d.hm_blk, d.hm_all);
     d.hblk = upload(c, blk);
   }
   // Wave-uniform cell lists for the Schur kernels, kept when the padding to
@@ -1336,6 +1338,14 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
           ptr.push_back((int)q + 1);
         }
       }
+      std::vector<int> all(m.ncellP + 1, 0), mh(op.nmult, -1);
+      for (size_t q = 0; q < hs.size(); ++q) {
+        all[hs[q].coarse + 1]++;
+        for (int a = 0; a < c->k; ++a) mh[hs[q].mbase + a] = (int)q;
+      }
+      for (int K = 0; K < m.ncellP; ++K) all[K + 1] += all[K];
+      P.hc_all = upload(c.get(), all);
+      P.mhang = upload(c.get(), mh);
       P.nhang = (int)hs.size();
       P.nhc = (int)cells.size();
       P.h_cell = upload(c.get(), hc);

@@ -381,6 +381,11 @@ __device__ __forceinline__ int wave_type(const DevRegion& R, int M) {
 // A lane keeps its rows of the tables in registers and runs over `per`
 // instances of a batch; a cell's W, u and s pass between its lanes in LDS.
 // A lane's node lies on at most two faces: one of x = 0, 1 and one of y = 0, 1.
+// HANG: the couplings across hanging faces, whole blocks, by the lanes of the
+// few cells that have one (kernels of their own, a cell per thread, took 25 +
+// 25 us and 23 + 22 us per step on the boundary-layer mesh at
+// refinement 5; the step 354 -> 256 us).  The loop costs up to 70
+// registers, so a system without hanging faces has its own variant.
 // One thread per cell with whole blocks (its chain of 700 to 4000 dependent
 // products and, on conic meshes, 9.7 KB of table per cell set the time) ->
 // this, per step: refinement 4, k = 3, distinct mobilities 344 -> 236 us;
@@ -448,7 +453,7 @@ __global__ __launch_bounds__(256) void k_carrier_w(SchurPair P, int nrhs, int ni
 }
 
 // g = f_v + B^T W: the cell's own block and its face neighbours' traces of W
-template <int K>
+template <int K, bool HANG>
 __global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ninst, int per) {
   using S = SchurLane<K>;
   constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
@@ -480,6 +485,8 @@ __global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ni
     }
     pm = R.perm[at];
   }
+  const bool hg = HANG && on && R.hx_all;
+  const int h0 = hg ? R.hx_all[c] : 0, h1 = hg ? R.hx_all[c + 1] : 0;
   int buf = 0;
   const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
   for (int i = blockIdx.y * per; i < i1; ++i)
@@ -500,6 +507,12 @@ __global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ni
             acc += bf[e][m] * wm[n] + bf[e][N1 + m] * wm[nb + n];
           }
         }
+        for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
+          const double* wm = w + (size_t)R.hx_src[e] * NB;
+          const double* B = R.hblk + (size_t)R.hx_blk[e] * 2 * NB * NB + a;
+#pragma unroll
+          for (int q = 0; q < NB; ++q) acc += B[q * NB] * wm[q] + B[(NB + q) * NB] * wm[nb + q];
+        }
       }
       __syncthreads();
       if (on) {
@@ -511,7 +524,7 @@ __global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ni
 }
 
 // q = W - mu A^{-1} B u; writes [Jx | Jy | u]
-template <int K>
+template <int K, bool HANG>
 __global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, int ninst, int per) {
   using S = SchurLane<K>;
   constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
@@ -550,6 +563,8 @@ __global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, in
     }
     pm = R.perm[at];
   }
+  const bool hg = HANG && on && R.hm_all;
+  const int h0 = hg ? R.hm_all[c] : 0, h1 = hg ? R.hm_all[c + 1] : 0;
   const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
   for (int i = blockIdx.y * per; i < i1; ++i)
     for (int h = 0; h < nrhs; ++h) {
@@ -570,6 +585,16 @@ __global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, in
             const double v = x[pn[e][j]];
             s0 += bf[e][0][j] * v;
             s1 += bf[e][1][j] * v;
+          }
+        }
+        for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
+          const int* px = R.perm + (size_t)R.hm_dst[e] * NB;
+          const double* B = R.hblk + (size_t)R.hm_blk[e] * 2 * NB * NB + a * NB;
+#pragma unroll
+          for (int q = 0; q < NB; ++q) {
+            const double v = x[px[q]];
+            s0 += B[q] * v;
+            s1 += B[NB * NB + q] * v;
           }
         }
       }
@@ -1695,6 +1720,16 @@ __global__ __launch_bounds__(256) void k_poisson_face(DevPoisson P, const double
     const int c = P.mcell[2 * m + e];
     if (c >= 0) s += P.mcoef[2 * m + e] * y[(size_t)c * P.nloc + P.mloc[2 * m + e]];
   }
+  const int h = P.mhang ? P.mhang[m] : -1;
+  if (h >= 0) {  // the coarse side of a hanging face
+    const int k = P.nphi == 1 ? 1 : P.nphi == 4 ? 2 : 3, f = P.h_face[h];
+    const double* E = P.hE + (P.h_sub[h] * k + m - P.h_mbase[h]) * k;
+    const double* yc = y + (size_t)P.h_cell[h] * P.nloc;
+    double t = 0.0;
+    for (int j = 0; j < k; ++j)
+      t += E[j] * yc[k == 1 ? rt_face<1>(f, j) : k == 2 ? rt_face<2>(f, j) : rt_face<3>(f, j)];
+    s += (f == 1 || f == 3) ? t : -t;
+  }
   r[P.mult_perm[m]] = s;
 }
 
@@ -1716,6 +1751,20 @@ __global__ __launch_bounds__(256) void k_poisson_recover(DevPoisson P, const dou
     const int p = base < 0 ? 0 : P.mult_perm[base + m];
 #pragma unroll
     for (int g = 0; g < IG; ++g) se[g][lc][fm] = base < 0 ? 0.0 : w * lam[min(i0 + g, ninst - 1) * sl + p];
+    if (P.hc_all) {  // the coarse side of hanging faces: the fine faces' multipliers against this DoF
+      for (int q = P.hc_all[Kc]; q < P.hc_all[Kc + 1]; ++q) {
+        if (P.h_face[q] != f) continue;
+        for (int mm = 0; mm < K; ++mm) {
+          const double c = P.hE[(P.h_sub[q] * K + mm) * K + m];
+          const int pp = P.mult_perm[P.h_mbase[q] + mm];
+#pragma unroll
+          for (int g = 0; g < IG; ++g) {
+            const double l = lam[min(i0 + g, ninst - 1) * sl + pp];
+            se[g][lc][fm] += c * ((f == 1 || f == 3) ? l : -l);
+          }
+        }
+      }
+    }
   }
   __syncthreads();
   for (int e = threadIdx.x; e < NC * NL; e += 256) {
@@ -1984,12 +2033,11 @@ inline int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 // ------------------------------------------------------------------------
 // Hanging faces of boundary-layer refinement
 // ------------------------------------------------------------------------
-// The Schur kernels leave out the couplings across hanging faces (those faces
-// are absent from the neighbour lists); these kernels add them afterwards, in
-// FP64, one thread per cell that has such a coupling.  Both are linear in the
-// terms they add, so the sum equals the one over all couplings.
-// W: the current part of b holds W (the FP64 path), else f_p.
-template <int K, int NRHS, bool W>
+// The mixed-precision kernels leave out the couplings across hanging faces
+// (those faces are absent from the neighbour lists); these kernels add them
+// afterwards, in FP64, one thread per cell that has such a coupling.  Both are
+// linear in the terms they add, so the sum equals the one over all couplings.
+template <int K, int NRHS>
 __global__ __launch_bounds__(64) void k_schur_rhs_hang(DevRegion R, const double* __restrict__ b1,
                                                        const double* __restrict__ b2, double mu1, double mu2,
                                                        double* __restrict__ g1, double* __restrict__ g2, int64_t sb,
@@ -2012,21 +2060,8 @@ __global__ __launch_bounds__(64) void k_schur_rhs_hang(DevRegion R, const double
     const double* B = R.hblk + (size_t)R.hx_blk[e] * 2 * NB * NB;
     const int ty = R.type[M];
     double w1[2 * NB], w2[2 * NB];
-    if (W) {
-      const size_t nc = R.ncell;
-#pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        w1[a] = b1[(size_t)M * NB + a];
-        w1[NB + a] = b1[nc * NB + (size_t)M * NB + a];
-        if (NRHS > 1) {
-          w2[a] = b2[(size_t)M * NB + a];
-          w2[NB + a] = b2[nc * NB + (size_t)M * NB + a];
-        }
-      }
-    } else {
-      schur_w<K>(R, b1, mu1, M, ty, w1);
-      if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
-    }
+    schur_w<K>(R, b1, mu1, M, ty, w1);
+    if (NRHS > 1) schur_w<K>(R, b2, mu2, M, ty, w2);
     for (int i = 0; i < 2 * NB; ++i) {
 #pragma unroll
       for (int a = 0; a < NB; ++a) {
@@ -2097,26 +2132,8 @@ __global__ __launch_bounds__(64) void k_schur_recover_hang(DevRegion R, const do
     }
 }
 
-// H right-hand side: the coarse side's contribution to the fine faces'
-// multipliers, one thread per (hanging pair, multiplier DoF)
-template <int K>
-__global__ __launch_bounds__(64) void k_poisson_face_hang(DevPoisson P, const double* __restrict__ y,
-                                                          double* __restrict__ r, int64_t sy, int64_t sr) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= P.nhang * K) return;
-  y += blockIdx.y * sy;
-  r += blockIdx.y * sr;
-  const int h = t / K, m = t % K;
-  const int Kc = P.h_cell[h], f = P.h_face[h], sub = P.h_sub[h];
-  const double sf = (f == 1 || f == 3) ? 1.0 : -1.0;
-  double s = 0.0;
-#pragma unroll
-  for (int j = 0; j < K; ++j) s += P.hE[(sub * K + m) * K + j] * y[(size_t)Kc * P.nloc + rt_face<K>(f, j)];
-  r[P.mult_perm[P.h_mbase[h] + m]] += sf * s;
-}
-
-// Recovery: x_K -= A_K^{-1} E_K^T lambda over the coarse cell's hanging faces
-// (with the same write rules as k_poisson_recover)
+// Recovery in mixed precision: x_K -= A_K^{-1} E_K^T lambda over the coarse
+// cell's hanging faces (with the same write rules as k_poisson_recover)
 template <int K>
 __global__ __launch_bounds__(64) void k_poisson_recover_hang(DevPoisson P, const double* __restrict__ lam,
                                                              double* __restrict__ out, int64_t sl, int64_t so) {
@@ -2184,20 +2201,26 @@ static int schur_per(int nblk, int nb) {
 
 int schur_ctab_size(int k) { return 3 * (k + 1) * (k + 1) * (k + 1) * (k + 1) + 8 * (k + 1) * (k + 1); }
 
-#define PECS_SCHUR_LAUNCH(KERNEL)                                                        \
-  P.nblk0 = nblk1(P.side[0].ncell, 256 / ((k + 1) * (k + 1)));                           \
-  const int n = P.nblk0 + nblk1(P.side[1].ncell, 256 / ((k + 1) * (k + 1)));             \
-  if (n == 0) return 0;                                                                  \
-  const int per = schur_per(n, nb);                                                      \
-  PECS_DISPATCH_K(k, (KERNEL<KK><<<dim3(n, nblk1(nb, per)), 256, 0, s>>>(P, nrhs, nb, per))); \
-  return (int)hipGetLastError()
+#define PECS_SCHUR_LAUNCH(KERNEL, ...)                                                       \
+  do {                                                                                       \
+    P.nblk0 = nblk1(P.side[0].ncell, 256 / ((k + 1) * (k + 1)));                             \
+    const int n = P.nblk0 + nblk1(P.side[1].ncell, 256 / ((k + 1) * (k + 1)));               \
+    if (n == 0) return 0;                                                                    \
+    const int per = schur_per(n, nb);                                                        \
+    PECS_DISPATCH_K(k, (KERNEL<KK, ##__VA_ARGS__><<<dim3(n, nblk1(nb, per)), 256, 0, s>>>(P, nrhs, nb, per))); \
+    return (int)hipGetLastError();                                                           \
+  } while (0)
 
 int launch_carrier_w(int k, SchurPair P, int nrhs, hipStream_t s, int nb) { PECS_SCHUR_LAUNCH(k_carrier_w); }
 
-static int launch_schur_rhs_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) { PECS_SCHUR_LAUNCH(k_schur_rhs); }
+static int launch_schur_rhs_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
+  if (P.side[0].hx_all || P.side[1].hx_all) PECS_SCHUR_LAUNCH(k_schur_rhs, true);
+  PECS_SCHUR_LAUNCH(k_schur_rhs, false);
+}
 
 static int launch_schur_recover_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
-  PECS_SCHUR_LAUNCH(k_schur_recover);
+  if (P.side[0].hm_all || P.side[1].hm_all) PECS_SCHUR_LAUNCH(k_schur_recover, true);
+  PECS_SCHUR_LAUNCH(k_schur_recover, false);
 }
 #undef PECS_SCHUR_LAUNCH
 
@@ -2408,7 +2431,7 @@ int launch_poisson_cell_from_b(const DevPoisson& P, const double* b, double* y, 
   return (int)hipGetLastError();
 }
 
-static int launch_poisson_face_main(const DevPoisson& P, const double* y, double* r, hipStream_t s, int nb, int64_t sy,
+int launch_poisson_face(const DevPoisson& P, const double* y, double* r, hipStream_t s, int nb, int64_t sy,
                         int64_t sr) {
   k_poisson_face<<<dim3(nblk(P.nmult, 256), nb), 256, 0, s>>>(P, y, r, sy, sr);
   return (int)hipGetLastError();
@@ -2433,8 +2456,9 @@ static int launch_poisson_recover_main(int k, const DevPoisson& P, const double*
 
 SchurSide schur_side_of(const DevRegion& R, const double* b1, const double* b2, double* w1, double* w2, double mu1,
                         double mu2, double* g1, double* g2, double* o1, double* o2, int64_t sb, int64_t sg, int64_t so) {
-  return SchurSide{R.ncell, R.nbr, R.type, R.perm, R.ctab, {b1, b2}, {w1, w2}, {g1, g2}, {o1, o2}, {mu1, mu2}, sb, sg,
-                   so};
+  return SchurSide{R.ncell,   R.nbr,    R.type,   R.perm,     R.ctab, {b1, b2}, {w1, w2},
+                   {g1, g2},  {o1, o2}, {mu1, mu2}, sb,       sg,     so,       R.hx_all,
+                   R.hx_src,  R.hx_blk, R.hm_all, R.hm_dst,   R.hm_blk, R.hblk};
 }
 
 int launch_schur_rhs(int k, const DevRegion* const* R, const SchurPair& P, int nrhs, hipStream_t s, int nb) {
@@ -2457,21 +2481,15 @@ int launch_schur_rhs(int k, const DevRegion* const* R, const SchurPair& P, int n
                                                                     S.g[0], S.sb, S.sg)));
       }
     }
-    if (R[r]->nhx == 0) continue;
+    if (!f32 || R[r]->nhx == 0) continue;
     const dim3 g(nblk(R[r]->nhx, 64), nb);
-#define PECS_HANG(NN, WW, B1, B2)                                                                              \
-  PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, NN, WW><<<g, 64, 0, s>>>(*R[r], B1, B2, S.mu[0], S.mu[NN - 1], S.g[0], \
-                                                                    S.g[NN - 1], S.sb, S.sg)))
-    if (f32 && nrhs == 2) {
-      PECS_HANG(2, false, S.b[0], S.b[1]);
-    } else if (f32) {
-      PECS_HANG(1, false, S.b[0], S.b[0]);
-    } else if (nrhs == 2) {
-      PECS_HANG(2, true, S.w[0], S.w[1]);
+    if (nrhs == 2) {
+      PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, 2><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[1], S.mu[0], S.mu[1], S.g[0],
+                                                                   S.g[1], S.sb, S.sg)));
     } else {
-      PECS_HANG(1, true, S.w[0], S.w[0]);
+      PECS_DISPATCH_K(k, (k_schur_rhs_hang<KK, 1><<<g, 64, 0, s>>>(*R[r], S.b[0], S.b[0], S.mu[0], S.mu[0], S.g[0],
+                                                                   S.g[0], S.sb, S.sg)));
     }
-#undef PECS_HANG
   }
   return (int)hipGetLastError();
 }
@@ -2497,7 +2515,7 @@ int launch_schur_recover(int k, const DevRegion* const* R, const SchurPair& P, i
                                                                         S.mu[0], S.o[0], S.o[0], S.sb, S.sg, S.so)));
       }
     }
-    if (R[r]->nhm == 0) continue;
+    if (!f32 || R[r]->nhm == 0) continue;
     const dim3 g(nblk(R[r]->nhm, 64), nb);
     if (nrhs == 2) {
       PECS_DISPATCH_K(k, (k_schur_recover_hang<KK, 2><<<g, 64, 0, s>>>(*R[r], S.g[0], S.g[1], S.mu[0], S.mu[1], S.o[0],
@@ -2510,19 +2528,10 @@ int launch_schur_recover(int k, const DevRegion* const* R, const SchurPair& P, i
   return (int)hipGetLastError();
 }
 
-int launch_poisson_face(const DevPoisson& P, const double* y, double* r, hipStream_t s, int nb, int64_t sy,
-                        int64_t sr) {
-  const int rc = launch_poisson_face_main(P, y, r, s, nb, sy, sr);
-  if (rc || P.nhang == 0) return rc;
-  const int k = (P.nphi == 1) ? 1 : (P.nphi == 4 ? 2 : 3);
-  PECS_DISPATCH_K(k, (k_poisson_face_hang<KK><<<dim3(nblk(P.nhang * k, 64), nb), 64, 0, s>>>(P, y, r, sy, sr)));
-  return (int)hipGetLastError();
-}
-
 int launch_poisson_recover(int k, const DevPoisson& P, const double* lam, const double* y, double* out,
                            hipStream_t s, int nb, int64_t sl, int64_t sy, int64_t so) {
   const int rc = launch_poisson_recover_main(k, P, lam, y, out, s, nb, sl, sy, so);
-  if (rc || P.nhc == 0) return rc;
+  if (rc || P.nhc == 0 || !P.table_f) return rc;
   PECS_DISPATCH_K(k, (k_poisson_recover_hang<KK><<<dim3(nblk(P.nhc, 64), nb), 64, 0, s>>>(P, lam, out, sl, so)));
   return (int)hipGetLastError();
 }

@@ -44,14 +44,15 @@ struct DevRegion {
   const double* mflux;
   // hanging faces of boundary-layer refinement (nhx = nhm = 0: none).  Their
   // couplings B_{M,X} (2nb x nb blocks in hblk: cell M's current rows, cell
-  // X's density columns) are not in nbr / table; they are applied after the
-  // kernels above by target cell X (right-hand side: g_X += B^T W_M; entries
+  // X's density columns) are not in nbr / table; the Schur kernels add them
+  // (mixed precision: kernels of their own after them) by target cell X (right-hand side: g_X += B^T W_M; entries
   // hx_ptr[t] .. hx_ptr[t+1] of target hx_cell[t] name M in hx_src and the
   // block in hx_blk) and by row cell M (recovery: q_M -= mu Minv_M B u_X).
   int nhx, nhm;
   const int *hx_cell, *hx_ptr, *hx_src, *hx_blk;
   const int *hm_cell, *hm_ptr, *hm_dst, *hm_blk;
   const double* hblk;
+  const int *hx_all, *hm_all;  // the entries of every cell (ncell + 1; null: no hanging faces)
 };
 
 struct DevPoisson {
@@ -93,6 +94,8 @@ struct DevPoisson {
   const int *h_cell, *h_face, *h_sub, *h_mbase;
   const int *hc_cell, *hc_ptr;
   const double* hE;
+  const int *hc_all;  // the pairs of every cell (ncell + 1; null: no hanging faces)
+  const int *mhang;   // per multiplier: the hanging pair of its (fine) face, or -1 (null: none)
 };
 
 struct DevPhys {
@@ -211,6 +214,9 @@ struct SchurSide {
   double* o[2];
   double mu[2];
   int64_t sb, sg, so;
+  // hanging faces (as in DevRegion; null: none)
+  const int *hx_all, *hx_src, *hx_blk, *hm_all, *hm_dst, *hm_blk;
+  const double* hblk;
 };
 // Both regions (side[1].ncell 0: one); nblk0 is set by the launchers.
 struct SchurPair {
