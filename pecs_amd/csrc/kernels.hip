@@ -453,11 +453,11 @@ __global__ __launch_bounds__(256) void k_carrier_w(SchurPair P, int nrhs, int ni
 }
 
 // g = f_v + B^T W: the cell's own block and its face neighbours' traces of W
-template <int K, bool HANG>
-__global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ninst, int per) {
+template <int K, int NRHS, bool HANG>
+__global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int ninst, int per) {
   using S = SchurLane<K>;
   constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
-  __shared__ double sw[2][2][CPB * NB];  // two buffers: one barrier per right-hand side
+  __shared__ double sw[2][NRHS][2][CPB * NB];  // two buffers: one barrier per instance
   int c0;
   const SchurSide& R = schur_side<K>(P, c0);
   const int t = threadIdx.x, lc = t / NB, a = t % NB, c = c0 + lc;
@@ -489,46 +489,58 @@ __global__ __launch_bounds__(256) void k_schur_rhs(SchurPair P, int nrhs, int ni
   const int h0 = hg ? R.hx_all[c] : 0, h1 = hg ? R.hx_all[c + 1] : 0;
   int buf = 0;
   const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
-  for (int i = blockIdx.y * per; i < i1; ++i)
-    for (int h = 0; h < nrhs; ++h, buf ^= 1) {
-      const double* w = R.w[h] + i * R.sb;
-      double acc = 0.0;
-      if (on) {
-        sw[buf][0][t] = w[at];
-        sw[buf][1][t] = w[nb + at];
-        acc = R.b[h][i * R.sb + 2 * nb + at];
+  for (int i = blockIdx.y * per; i < i1; ++i, buf ^= 1) {
+    double acc[NRHS];
+    if (on) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          if (M[e] < 0) continue;
-          const double* wm = w + (size_t)M[e] * NB;
+      for (int h = 0; h < NRHS; ++h) {
+        const double* w = R.w[h] + i * R.sb;
+        sw[buf][h][0][t] = w[at];
+        sw[buf][h][1][t] = w[nb + at];
+        acc[h] = R.b[h][i * R.sb + 2 * nb + at];
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        if (M[e] < 0) continue;
+#pragma unroll
+        for (int h = 0; h < NRHS; ++h) {
+          const double* wm = R.w[h] + i * R.sb + (size_t)M[e] * NB;
 #pragma unroll
           for (int m = 0; m < N1; ++m) {
             const int n = S::node(fc[e] ^ 1, m);
-            acc += bf[e][m] * wm[n] + bf[e][N1 + m] * wm[nb + n];
+            acc[h] += bf[e][m] * wm[n] + bf[e][N1 + m] * wm[nb + n];
           }
         }
-        for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
-          const double* wm = w + (size_t)R.hx_src[e] * NB;
-          const double* B = R.hblk + (size_t)R.hx_blk[e] * 2 * NB * NB + a;
+      }
+      for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
+        const double* B = R.hblk + (size_t)R.hx_blk[e] * 2 * NB * NB + a;
 #pragma unroll
-          for (int q = 0; q < NB; ++q) acc += B[q * NB] * wm[q] + B[(NB + q) * NB] * wm[nb + q];
+        for (int h = 0; h < NRHS; ++h) {
+          const double* wm = R.w[h] + i * R.sb + (size_t)R.hx_src[e] * NB;
+#pragma unroll
+          for (int q = 0; q < NB; ++q) acc[h] += B[q * NB] * wm[q] + B[(NB + q) * NB] * wm[nb + q];
         }
       }
-      __syncthreads();
-      if (on) {
+    }
+    __syncthreads();
+    if (on) {
 #pragma unroll
-        for (int q = 0; q < NB; ++q) acc += bs[q] * sw[buf][0][lc * NB + q] + bs[NB + q] * sw[buf][1][lc * NB + q];
-        R.g[h][i * R.sg + pm] = acc;
+      for (int h = 0; h < NRHS; ++h) {
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+          acc[h] += bs[q] * sw[buf][h][0][lc * NB + q] + bs[NB + q] * sw[buf][h][1][lc * NB + q];
+        R.g[h][i * R.sg + pm] = acc[h];
       }
     }
+  }
 }
 
 // q = W - mu A^{-1} B u; writes [Jx | Jy | u]
-template <int K, bool HANG>
-__global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, int ninst, int per) {
+template <int K, int NRHS, bool HANG>
+__global__ __launch_bounds__(256, K == 2 && !HANG ? 4 : 1) void k_schur_recover(SchurPair P, int ninst, int per) {
   using S = SchurLane<K>;
   constexpr int NB = S::NB, N1 = S::N1, CPB = S::CPB;
-  __shared__ double su[CPB * NB], ss[2][CPB * NB];
+  __shared__ double su[NRHS][CPB * NB], ss[NRHS][2][CPB * NB];
   int c0;
   const SchurSide& R = schur_side<K>(P, c0);
   const int t = threadIdx.x, lc = t / NB, a = t % NB, c = c0 + lc;
@@ -566,61 +578,72 @@ __global__ __launch_bounds__(256) void k_schur_recover(SchurPair P, int nrhs, in
   const bool hg = HANG && on && R.hm_all;
   const int h0 = hg ? R.hm_all[c] : 0, h1 = hg ? R.hm_all[c + 1] : 0;
   const int i1 = min(ninst, ((int)blockIdx.y + 1) * per);
-  for (int i = blockIdx.y * per; i < i1; ++i)
-    for (int h = 0; h < nrhs; ++h) {
-      const double* x = R.g[h] + i * R.sg;
-      double* o = R.o[h] + i * R.so;
-      double s0 = 0.0, s1 = 0.0, w0 = 0.0, w1 = 0.0;
-      if (on) {
-        const double u = x[pm];
-        su[t] = u;
-        o[2 * nb + at] = u;
-        w0 = R.w[h][i * R.sb + at];
-        w1 = R.w[h][i * R.sb + nb + at];
+  for (int i = blockIdx.y * per; i < i1; ++i) {
+    double s0[NRHS], s1[NRHS], w0[NRHS], w1[NRHS];
+    if (on) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          if (M[e] < 0) continue;
+      for (int h = 0; h < NRHS; ++h) {
+        const double u = R.g[h][i * R.sg + pm];
+        su[h][t] = u;
+        R.o[h][i * R.so + 2 * nb + at] = u;
+        w0[h] = R.w[h][i * R.sb + at];
+        w1[h] = R.w[h][i * R.sb + nb + at];
+        s0[h] = s1[h] = 0.0;
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        if (M[e] < 0) continue;
+#pragma unroll
+        for (int h = 0; h < NRHS; ++h)
 #pragma unroll
           for (int j = 0; j < N1; ++j) {
-            const double v = x[pn[e][j]];
-            s0 += bf[e][0][j] * v;
-            s1 += bf[e][1][j] * v;
+            const double v = R.g[h][i * R.sg + pn[e][j]];
+            s0[h] += bf[e][0][j] * v;
+            s1[h] += bf[e][1][j] * v;
           }
-        }
-        for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
-          const int* px = R.perm + (size_t)R.hm_dst[e] * NB;
-          const double* B = R.hblk + (size_t)R.hm_blk[e] * 2 * NB * NB + a * NB;
-#pragma unroll
-          for (int q = 0; q < NB; ++q) {
-            const double v = x[px[q]];
-            s0 += B[q] * v;
-            s1 += B[NB * NB + q] * v;
-          }
-        }
       }
-      __syncthreads();
-      if (on) {
+      for (int e = h0; HANG && e < h1; ++e) {  // hanging faces
+        const int* px = R.perm + (size_t)R.hm_dst[e] * NB;
+        const double* B = R.hblk + (size_t)R.hm_blk[e] * 2 * NB * NB + a * NB;
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+          for (int h = 0; h < NRHS; ++h) {
+            const double v = R.g[h][i * R.sg + px[q]];
+            s0[h] += B[q] * v;
+            s1[h] += B[NB * NB + q] * v;
+          }
+      }
+    }
+    __syncthreads();
+    if (on) {
+#pragma unroll
+      for (int h = 0; h < NRHS; ++h) {
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
-          const double v = su[lc * NB + q];
-          s0 += bs[0][q] * v;
-          s1 += bs[1][q] * v;
+          const double v = su[h][lc * NB + q];
+          s0[h] += bs[0][q] * v;
+          s1[h] += bs[1][q] * v;
         }
-        ss[0][t] = s0;
-        ss[1][t] = s1;
+        ss[h][0][t] = s0[h];
+        ss[h][1][t] = s1[h];
       }
-      __syncthreads();
-      if (on) {
+    }
+    __syncthreads();
+    if (on) {
+#pragma unroll
+      for (int h = 0; h < NRHS; ++h) {
         double q0 = 0.0, q1 = 0.0;
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
-          q0 += mi[q] * ss[0][lc * NB + q];
-          q1 += mi[q] * ss[1][lc * NB + q];
+          q0 += mi[q] * ss[h][0][lc * NB + q];
+          q1 += mi[q] * ss[h][1][lc * NB + q];
         }
-        o[at] = w0 - R.mu[h] * q0;
-        o[nb + at] = w1 - R.mu[h] * q1;
+        R.o[h][i * R.so + at] = w0[h] - R.mu[h] * q0;
+        R.o[h][i * R.so + nb + at] = w1[h] - R.mu[h] * q1;
       }
     }
+  }
 }
 
 // ------------------------------------------------------------------------
@@ -2201,27 +2224,39 @@ static int schur_per(int nblk, int nb) {
 
 int schur_ctab_size(int k) { return 3 * (k + 1) * (k + 1) * (k + 1) * (k + 1) + 8 * (k + 1) * (k + 1); }
 
-#define PECS_SCHUR_LAUNCH(KERNEL, ...)                                                       \
+#define PECS_SCHUR_LAUNCH(KERNEL, ARGS)                                                      \
   do {                                                                                       \
     P.nblk0 = nblk1(P.side[0].ncell, 256 / ((k + 1) * (k + 1)));                             \
     const int n = P.nblk0 + nblk1(P.side[1].ncell, 256 / ((k + 1) * (k + 1)));               \
     if (n == 0) return 0;                                                                    \
     const int per = schur_per(n, nb);                                                        \
-    PECS_DISPATCH_K(k, (KERNEL<KK, ##__VA_ARGS__><<<dim3(n, nblk1(nb, per)), 256, 0, s>>>(P, nrhs, nb, per))); \
+    PECS_DISPATCH_K(k, (KERNEL<<<dim3(n, nblk1(nb, per)), 256, 0, s>>>ARGS));                \
     return (int)hipGetLastError();                                                           \
   } while (0)
+#define PECS_SCHUR_CASE(KERNEL, NRHS, HANG)                                                  \
+  if (nrhs == NRHS && hang == HANG) PECS_SCHUR_LAUNCH((KERNEL<KK, NRHS, HANG>), (P, nb, per))
+#define PECS_SCHUR_CASES(KERNEL)                                                             \
+  PECS_SCHUR_CASE(KERNEL, 1, false);                                                         \
+  PECS_SCHUR_CASE(KERNEL, 2, false);                                                         \
+  PECS_SCHUR_CASE(KERNEL, 1, true);                                                          \
+  PECS_SCHUR_CASE(KERNEL, 2, true);                                                          \
+  return (int)hipErrorInvalidValue
 
-int launch_carrier_w(int k, SchurPair P, int nrhs, hipStream_t s, int nb) { PECS_SCHUR_LAUNCH(k_carrier_w); }
+int launch_carrier_w(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
+  PECS_SCHUR_LAUNCH((k_carrier_w<KK>), (P, nrhs, nb, per));
+}
 
 static int launch_schur_rhs_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
-  if (P.side[0].hx_all || P.side[1].hx_all) PECS_SCHUR_LAUNCH(k_schur_rhs, true);
-  PECS_SCHUR_LAUNCH(k_schur_rhs, false);
+  const bool hang = P.side[0].hx_all || P.side[1].hx_all;
+  PECS_SCHUR_CASES(k_schur_rhs);
 }
 
 static int launch_schur_recover_main(int k, SchurPair P, int nrhs, hipStream_t s, int nb) {
-  if (P.side[0].hm_all || P.side[1].hm_all) PECS_SCHUR_LAUNCH(k_schur_recover, true);
-  PECS_SCHUR_LAUNCH(k_schur_recover, false);
+  const bool hang = P.side[0].hm_all || P.side[1].hm_all;
+  PECS_SCHUR_CASES(k_schur_recover);
 }
+#undef PECS_SCHUR_CASES
+#undef PECS_SCHUR_CASE
 #undef PECS_SCHUR_LAUNCH
 
 template <int NRHS, bool FWD>
