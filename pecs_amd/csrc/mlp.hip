@@ -35,6 +35,7 @@
 #include <random>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pecs_abi.h"
@@ -341,19 +342,32 @@ struct Conv {
   int ch() const { return (P / R + 2) * (R + 2); }  // staged entries per channel
 };
 
-// One wave stages one row at a time (two where a row is at most 32 entries).
+// The rows of the strip and one above and below, all channels, 8 loads per
+// thread in flight (one row per wave at a time, W entries in passes of 64, cost
+// a load latency per row: 32 channels at R = 64 staged for longer than they
+// were multiplied).  R is a power of two (it divides P); the border columns are
+// zero by themselves.
 template <class T>
 __device__ __forceinline__ void conv_stage(const Conv& c, const T* __restrict__ in, int smp, int y0, T* sIn) {
-  const int W = c.R + 2, rows = c.P / c.R + 2, Ri = c.R >> c.up;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int par = W <= 32 ? 2 : 1, sub = W <= 32 ? lane >> 5 : 0, x0 = W <= 32 ? lane & 31 : lane, xs = 64 / par;
-  for (int q = wave * par + sub; q < c.C * rows; q += 4 * par) {
-    const int ci = q / rows, yy = q - ci * rows, y = y0 + yy - 1;
-    const bool yin = y >= 0 && y < c.R;
-    const T* src = in + (((int64_t)smp * c.C + ci) * Ri + (yin ? y >> c.up : 0)) * Ri;
-    for (int xx = x0; xx < W; xx += xs) {
-      const int x = xx - 1;
-      sIn[q * W + xx] = yin && x >= 0 && x < c.R ? src[x >> c.up] : T(0);
+  const int W = c.R + 2, rows = c.P / c.R + 2, Ri = c.R >> c.up, nrow = c.C * rows;
+  const int sh = 31 - __clz(c.R), n = nrow << sh;
+  const uint32_t inv = 0xffffffffu / (uint32_t)rows + 1;  // q / rows = umulhi(q, inv) for q < 2^16 (rows >= 3)
+  const T* src = in + (int64_t)smp * c.C * Ri * Ri;
+  for (int q = threadIdx.x; q < nrow; q += 256) sIn[q * W] = sIn[q * W + W - 1] = T(0);
+  constexpr int U = 8;
+  for (int e0 = threadIdx.x; e0 < n; e0 += 256 * U) {
+    T v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = min(e0 + 256 * u, n - 1), x = e & (c.R - 1), q = e >> sh;
+      const int ci = (int)__umulhi((uint32_t)q, inv), y = y0 + q - ci * rows - 1;
+      const T t = src[(ci * Ri + (min(max(y, 0), c.R - 1) >> c.up)) * Ri + (x >> c.up)];
+      v[u] = y >= 0 && y < c.R ? t : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + 256 * u;
+      if (e < n) sIn[(e >> sh) * W + (e & (c.R - 1)) + 1] = v[u];
     }
   }
 }
@@ -408,7 +422,7 @@ __global__ __launch_bounds__(256) void k_conv(Conv c, const T* __restrict__ in, 
         o[u][e] = k < c.K ? ko.x : -1;
       }
   };
-  auto mma = [&](const T (&x)[DU][E], const int (&o)[DU][E]) {
+  auto mma = [&](const T (&x)[DU][E], const int (&o)[DU][E], auto tail) {  // tail: some k past the end
 #pragma unroll
     for (int u = 0; u < DU; ++u)
 #pragma unroll
@@ -416,8 +430,12 @@ __global__ __launch_bounds__(256) void k_conv(Conv c, const T* __restrict__ in, 
         T b[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-          const T v = sIn[max(o[u][e], 0) + po[j]];
-          b[e] = o[u][e] >= 0 ? v : T(0);
+          if constexpr (decltype(tail)::value) {
+            const T v = sIn[max(o[u][e], 0) + po[j]];
+            b[e] = o[u][e] >= 0 ? v : T(0);
+          } else {
+            b[e] = sIn[o[u][e] + po[j]];
+          }
         }
         if constexpr (BF) {
           v4s xa, yb;
@@ -432,21 +450,36 @@ __global__ __launch_bounds__(256) void k_conv(Conv c, const T* __restrict__ in, 
         }
       }
   };
+  constexpr int KG = DU * KS;
+  auto group = [&](int k0, int h) {
+    if (k0 + KG <= c.K) mma(A[h], O[h], std::false_type{});
+    else mma(A[h], O[h], std::true_type{});
+  };
   load(0, A[0], O[0]);
-  for (int k0 = 0; k0 < c.K; k0 += 2 * DU * KS) {
-    if (k0 + DU * KS < c.K) load(k0 + DU * KS, A[1], O[1]);
-    mma(A[0], O[0]);
-    if (k0 + DU * KS >= c.K) break;
-    if (k0 + 2 * DU * KS < c.K) load(k0 + 2 * DU * KS, A[0], O[0]);
-    mma(A[1], O[1]);
+  for (int k0 = 0; k0 < c.K; k0 += 2 * KG) {
+    if (k0 + KG < c.K) load(k0 + KG, A[1], O[1]);
+    group(k0, 0);
+    if (k0 + KG >= c.K) break;
+    if (k0 + 2 * KG < c.K) load(k0 + 2 * KG, A[0], O[0]);
+    group(k0 + KG, 1);
   }
+  // mm_store of channel m, pixel px0 + px[j] of sample smp
 #pragma unroll
-  for (int j = 0; j < NC; ++j)
+  for (int r = 0; r < 4; ++r) {
+    const int m = m0 + 4 * lq + r;
+    if (m >= c.M) continue;
+    const float bias = D.bias ? D.bias[m] : 0.f;
+    const int64_t o0 = ((int64_t)smp * D.C + m) * R2 + px0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 4 * lq + r;
-      if (m < c.M) mm_store(D, m, (int)(n0 + px[j]), acc[j][r]);
+    for (int j = 0; j < NC; ++j) {
+      float v = acc[j][r];
+      if (D.bias) v += bias;
+      if (D.relu && v < 0.f) v = 0.f;
+      if (D.mask && D.mask[o0 + px[j]] <= 0.f) v = 0.f;
+      if (D.bf16) static_cast<uint16_t*>(D.p)[o0 + px[j]] = f32_to_bf16(v);
+      else static_cast<float*>(D.p)[o0 + px[j]] = v;
     }
+  }
 }
 
 // dW[co][ci t] = sum over pixels of dOut[co][px] in[ci][px + off(t)], and the
@@ -466,7 +499,9 @@ __global__ __launch_bounds__(256) void k_conv_dw(Conv c, const float* __restrict
   float* sA = sIn + c.C * CH;  // output gradient of the strip: [co][pixel]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lq = lane >> 4;
-  const int ncol = c.K + 1, nblk = (ncol + 15) / 16;  // column K: ones
+  const int ncol = c.K + 1;  // column K: ones
+  const int sh = 31 - __clz(c.R);
+  constexpr int G = 4;  // groups of 4 pixels whose LDS reads go out together (P is a multiple of 16)
   int off[NT];  // tap offset of this lane's column; -1: ones, -2: none
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
@@ -488,21 +523,25 @@ __global__ __launch_bounds__(256) void k_conv_dw(Conv c, const float* __restrict
       for (int x = lane; x < c.P; x += 64)
         sA[m * lda + x] = m < c.M ? dout[((int64_t)smp * c.M + m) * R2 + px0 + x] : 0.f;
     __syncthreads();
-    for (int y = 0; y < c.P / c.R; ++y)
-      for (int x = 0; x < c.R; x += 4) {
-        float a[MB];
+    for (int g = 0; g < c.P; g += 4 * G) {
+      float a[G][MB], b[G][NT];
 #pragma unroll
-        for (int i = 0; i < MB; ++i) a[i] = sA[(16 * i + li) * lda + y * c.R + x + lq];
-        const int po = y * W + x + lq;
+      for (int u = 0; u < G; ++u) {
+        const int x = g + 4 * u + lq, po = (x >> sh) * W + (x & (c.R - 1));
+#pragma unroll
+        for (int i = 0; i < MB; ++i) a[u][i] = sA[(16 * i + li) * lda + x];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) b[u][j] = sIn[max(off[j], 0) + po];
+      }
+#pragma unroll
+      for (int u = 0; u < G; ++u)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          if (wave + 4 * j >= nblk) continue;  // wave-uniform
-          const float v = sIn[max(off[j], 0) + po];
-          const float b = off[j] >= 0 ? v : off[j] == -1 ? 1.f : 0.f;
+          const float v = off[j] >= 0 ? b[u][j] : off[j] == -1 ? 1.f : 0.f;
 #pragma unroll
-          for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b, acc[i][j], 0, 0, 0);
+          for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], v, acc[i][j], 0, 0, 0);
         }
-      }
+    }
   }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -515,18 +554,29 @@ __global__ __launch_bounds__(256) void k_conv_dw(Conv c, const float* __restrict
       }
 }
 
+// The sum over the workgroups' parts: 16 threads per entry, each every 16th
+// part, their sums added in order (one thread per entry went through 256 parts
+// in 15 us).
 __global__ __launch_bounds__(256) void k_conv_dw_reduce(const float* __restrict__ part, int slices, int M, int K,
                                                         float* __restrict__ dw, float* __restrict__ db) {
-  const int e = blockIdx.x * 256 + threadIdx.x, ncol = K + 1, n = M * ncol;
-  if (e >= n) return;
+  __shared__ float sv[16][17];
+  const int x = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int ncol = K + 1, n = M * ncol, e = blockIdx.x * 16 + x;
   float v = 0.f;
-  for (int z0 = 0; z0 < slices; z0 += 8) {  // 8 loads in flight, added in order
-    float q[8];
+  if (e < n)
+    for (int z0 = g; z0 < slices; z0 += 16 * 8) {  // 8 loads in flight, added in order
+      float q[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) q[u] = z0 + u < slices ? part[(int64_t)(z0 + u) * n + e] : 0.f;
+      for (int u = 0; u < 8; ++u) q[u] = z0 + 16 * u < slices ? part[(int64_t)(z0 + 16 * u) * n + e] : 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v += q[u];
-  }
+      for (int u = 0; u < 8; ++u) v += q[u];
+    }
+  sv[g][x] = v;
+  __syncthreads();
+  if (g || e >= n) return;
+  v = 0.f;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) v += sv[u][x];
   const int m = e / ncol, c = e - m * ncol;
   if (c < K) dw[m * K + c] = v;
   else db[m] = v;
@@ -706,18 +756,25 @@ inline bool conv_dw(const float* in, int C, int R, int up, const float* dout, in
   Conv c{C, R, up, 0, M, C * 9};
   const int mb = nblk(M, 16), nt = nblk(nblk(c.K + 1, 16), 4);
   if (R % 4 || mb > 4 || nt > 10 || mb == 3) return false;
-  bool fits = false;
-  for (int px = 256; px >= 16 && !fits; px /= 2) fits = conv_strip(c, px, 4, (size_t)16 * mb * (px + 4) * 4);
-  if (!fits) return false;
+  // the largest strip with which 512 workgroups have work, else the smallest
+  // that is there: 256 workgroups, one wave per SIMD, waited on every LDS read
+  int best = 0;
+  for (int px = 256; px >= 16; px /= 2) {
+    if (!conv_strip(c, px, 4, (size_t)16 * mb * (px + 4) * 4)) continue;
+    best = px;
+    if ((int64_t)batch * R * R / px >= 512) break;
+  }
+  if (!best) return false;
+  c.P = best;
   const size_t lds = ((size_t)C * c.ch() + (size_t)16 * mb * (c.P + 4)) * 4;
   const int64_t strips = (int64_t)batch * R * R / c.P, cells = (int64_t)M * (c.K + 1);
-  const int slices = (int)std::min<int64_t>(std::min<int64_t>(strips, 256), part_cap / cells);
+  const int slices = (int)std::min<int64_t>(std::min<int64_t>(strips, 512), part_cap / cells);
   if (slices < 1 || strips > (1 << 30)) return false;
 #define MLP_DW(BB, NN)                                                                        \
   if (mb == BB && nt <= NN) {                                                                 \
     k_conv_dw<BB, NN><<<slices, 256, lds, s>>>(c, in, dout, (int)strips, part);               \
     MCHECK(hipGetLastError());                                                                \
-    k_conv_dw_reduce<<<nblk(cells, 256), 256, 0, s>>>(part, slices, M, c.K, dw, db);          \
+    k_conv_dw_reduce<<<nblk(cells, 16), 256, 0, s>>>(part, slices, M, c.K, dw, db);          \
     MCHECK(hipGetLastError());                                                                \
     return true;                                                                              \
   }
