@@ -411,6 +411,16 @@ __global__ __launch_bounds__(256) void k_conv(Conv c, const T* __restrict__ in, 
   T A[2][DU][E];
   int O[2][DU][E];
   auto load = [&](int k0, T (&x)[DU][E], int (&o)[DU][E]) {
+    if (BF && !FLIP && k0 + DU * KS <= c.K) {  // a lane's 4 weights are consecutive: one load of 8 bytes
+#pragma unroll
+      for (int u = 0; u < DU; ++u) {
+        const int k = k0 + u * KS + lq * E;
+        memcpy(x[u], wm + k, E * sizeof(T));
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[u][e] = sK[k + e].x;
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < DU; ++u)
 #pragma unroll
