@@ -740,8 +740,8 @@ def main():
     workload = (f"PECS half cell, refinement {args.refine} ({1 << args.refine}x{1 << args.refine} quads/region), "
                 f"LDG k={args.degree}, RT{args.degree - 1}xDGQ{args.degree - 1} Poisson, dt={args.dt}")
     U = 2 * g.n_semi + 2 * g.n_elec + g.n_poisson
-    # the production path (pecs_step replaying the captured step graphs, the
-    # two regions' chains on two streams) gives value; the run with
+    # the production path (pecs_step replaying the captured step graphs) gives
+    # value; the run with
     # per-phase events (kernel by kernel, phases one after another) gives the
     # phase times and the roofline's kernel time
     ms_timed = elapsed / args.steps * 1e3

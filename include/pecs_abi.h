@@ -264,7 +264,7 @@ int pecs_use_graph(pecs_ctx* ctx, int enable);
 /* Per-phase timing of pecs_step with hipEvents on the context stream
  * (the TimerOutput sections of SolarCell.cpp:1905-2087): phases 0 rhs semi,
  * 1 rhs elec, 2 Schur transforms of both regions, 3 carrier Cholesky solves of
- * both regions (concurrent on two streams), 4 recoveries of both regions,
+ * both regions (one forest factor, or two on two streams), 4 recoveries of both regions,
  * 5 Poisson condensation, 6 Poisson multiplier Cholesky, 7 Poisson recovery.
  * ms[] accumulates since enable. */
 int pecs_enable_timing(pecs_ctx* ctx, int enable);
@@ -280,7 +280,7 @@ int pecs_factor_bytes(pecs_ctx* ctx, int which, double* bytes);
  * solve has no tunable shape). */
 int pecs_sweep_config(pecs_ctx* ctx, int which, int* out, int n, int* nlevels);
 
-/* Which cell-local kernels take wave-uniform cell lists (cells grouped so
+/* Which cell-local kernels have wave-uniform cell lists for mixed precision (cells grouped so
  * that every 64-cell wave shares the operator types it reads): bit 0/1
  * semiconductor Schur recovery / right-hand side, bit 2/3 the same for the
  * electrolyte, bit 4 the Poisson condensation and recovery.  No counterpart

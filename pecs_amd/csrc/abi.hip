@@ -68,7 +68,7 @@ struct FactorDev {
 struct pecs_ctx {
   std::string err;
   hipStream_t stream = nullptr;
-  hipStream_t side = nullptr;            // second stream for the concurrent region solves
+  hipStream_t side = nullptr;            // second stream, for the second factor where the regions' systems do not fit one forest
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   // one time step captured as a graph (pecs_step replays it); cap is the
   // stream it is captured on (capture needs a stream other than the null stream)
@@ -789,7 +789,7 @@ DevRegion make_region_dev(pecs_ctx* c, int reg, const Region& R, const LdgRegion
     d.nhm = csr(bym, d.hm_cell, d.hm_ptr, d.hm_dst, d.hm_blk, d.hm_all);
     d.hblk = upload(c, blk);
   }
-  // Wave-uniform cell lists for the Schur kernels, kept when the padding to
+  // Wave-uniform cell lists for the mixed-precision Schur kernels, kept when the padding to
   // whole waves adds at most max(ncell, 2048) cells (meshes with few
   // operator types; on conic meshes every cell has its own type and the
   // lists are not used).
@@ -1286,7 +1286,7 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
           for (size_t j = 0; j < nl; ++j) t[(ty * nl + j) * nl + i] = op.table[ty * (size_t)op.type_stride + i * nl + j];
       P.tab_t = upload(c.get(), t);
     }
-    {  // wave-uniform cell list for the recovery (as for the Schur kernels)
+    {  // wave-uniform cell list (mixed precision, as for the Schur kernels)
       const char* su = std::getenv("PECS_SCHUR_UNIFORM");
       std::vector<int> own = wave_groups(m.ncellP, 1, [&](int K, int* key) { key[0] = op.type[K]; });
       if (!(su && su[0] == '0') && own.size() <= std::max<size_t>(2 * (size_t)m.ncellP, (size_t)m.ncellP + 2048)) {

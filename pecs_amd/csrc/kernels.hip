@@ -1,24 +1,26 @@
 // HIP kernels of the PECS per-time-step IMEX path for gfx950 (CDNA4).
 //
 // Per step (SolarCell.cpp:2057-2075):
-//   k_rhs_carrier   assemble_{semiconductor,electrolyte}_rhs: one thread per
-//                   cell, geometry rebuilt from the 4 vertices (MappingQ1),
-//                   old densities, Poisson field (Piola) and lagged traces of
-//                   the other region evaluated at QGauss(k+2) points.
-//   k_schur_rhs     g = f_v + B^T W (cell + 4 face neighbours), with
-//                   W = mu A^{-1} f_p recomputed per cell from the RHS.
+//   k_rhs_carrier   assemble_{semiconductor,electrolyte}_rhs, both regions in
+//                   one launch: geometry rebuilt from the 4 vertices
+//                   (MappingQ1), old densities, Poisson field (Piola) and
+//                   lagged traces of the other region at QGauss(k+2) points,
+//                   contracted on FP64 MFMA; stores W = mu A^{-1} f_p in
+//                   place of the current part f_p.
+//   k_schur_rhs     g = f_v + B^T W (cell, face neighbours, hanging faces), a
+//                   lane per density DoF.
 //   k_fwd_gather / k_sweep  supernodal triangular solves
-//                   with S = L L^T, level by level on the elimination tree:
+//                   with S = L L^T of both regions, level by level on the
+//                   elimination forest:
 //                   row tiles of dense [Linv; L21 Linv] panels, vector chunks
 //                   staged in LDS, W lanes per row (deterministic, no atomics).
 //   k_schur_recover q = W - A^{-1} B u; writes [Jx | Jy | u].
 //   k_poisson_*     hybridised mixed Poisson: cell condensation, face
 //                   assembly, multiplier solve, cell recovery.
 // Batches of instances sharing the factors: k_sweep_mfma (FP64 MFMA) with
-// RHS-interleaved vectors and their gathers.  The Schur and Poisson cell
-// kernels take wave-uniform cell lists where the mesh has few cell types
-// (table entries as scalar operands), and FP32 variants (*_f32) serve the
-// mixed-precision mode.
+// RHS-interleaved vectors and their gathers.  FP32 variants (*_f32) of the
+// Schur and Poisson cell kernels, a thread per cell on wave-uniform cell lists
+// (table entries as scalar operands), serve the mixed-precision mode.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"

@@ -7,7 +7,7 @@ A triangular solve is a sequence of launches (per supernode level: a gather and
 a sweep, forward then backward, then one copy).  Its dispatches are found in
 the trace as the window between the marker kernels that bracket it in every
 step: k_schur_rhs ... k_schur_recover for the carrier solves of both regions
-(which run concurrently on two streams) and k_poisson_face ...
+and k_poisson_face ...
 k_poisson_recover for the Poisson multipliers.
 
 `trace` prints per-kernel statistics and, per window, the sum of kernel
