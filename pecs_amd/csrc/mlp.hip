@@ -17,8 +17,10 @@
 //   k_conv     the convolutions and their input gradients as implicit GEMMs on
 //              input strips staged in LDS
 //   k_conv_dw  their weight and bias gradients on the same strips
-//   k_mm       any of the convolution products, im2col gathered element by
-//              element: maps that do not divide into strips of whole rows
+//   k_mm       64 x 64 tiles staged in LDS: dense products that fill the chip
+//              with them, and any of the convolution products, im2col gathered
+//              element by element, on maps that do not divide into strips of
+//              whole rows
 // Every product adds its k terms in ascending order in groups of 4 (FP32) or
 // 16 (BF16), whichever kernel runs it: the forward pass is the same bit by bit.
 //
@@ -82,6 +84,7 @@ __device__ __forceinline__ float ldv<uint16_t>(const uint16_t* p, int64_t i) {
 // An operand matrix of k_mm, read element by element while staging tiles.
 enum OpKind {
   OP_ROW = 0,     // (r, c) = p[r ld + c]
+  OP_TRANS = 1,   // (r, c) = p[c ld + r]
   OP_IM2COL = 2,  // (ci 9 + t, b R^2 + px): input pixel under tap t of output pixel px (conv forward B)
   OP_IM2COL_T = 3,  // its transpose (weight gradient B)
   OP_CHAN = 4,    // (ch, b R^2 + px) of a C x R x R map per sample (weight gradient A)
@@ -92,7 +95,7 @@ enum OpKind {
 struct Opnd {
   const void* p;
   int kind;
-  int ld;  // OP_ROW
+  int ld;  // OP_ROW / OP_TRANS
   int C;   // channels of the map read (OP_WT: cin)
   int R;   // side of the convolution's output (and upsampled input)
   int up;  // OP_IM2COL*: the input map is R/2 x R/2, upsampled by 2 (nearest)
@@ -104,6 +107,8 @@ __device__ __forceinline__ float opnd(const Opnd& o, int r, int c) {
   switch (o.kind) {
     case OP_ROW:
       return ldv(p, (int64_t)r * o.ld + c);
+    case OP_TRANS:
+      return ldv(p, (int64_t)c * o.ld + r);
     case OP_IM2COL:
     case OP_IM2COL_T: {
       const int k = o.kind == OP_IM2COL ? r : c, n = o.kind == OP_IM2COL ? c : r;
@@ -682,6 +687,9 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ a, ui
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+Opnd op_row(const void* p, int ld) { return Opnd{p, OP_ROW, ld, 0, 0, 0}; }
+Opnd op_trans(const void* p, int ld) { return Opnd{p, OP_TRANS, ld, 0, 0, 0}; }
+
 // k slices for an M x N x K product: enough workgroups to fill the chip
 // when the output has few tiles, slices of at least 1024 deep (a multiple
 // of TK), at most MAX_SPLIT
@@ -711,9 +719,22 @@ void mm(const Opnd& A, const Opnd& B, const Dst& D, int M, int N, int K, hipStre
 
 // Dense product.  k slices (where a scratch array is given) until about 512
 // waves are at work, each slice at least 128 deep.
+// With enough whole 64 x 64 tiles k_mm is faster, whose tiles read an operand
+// entry once per 64 outputs instead of 16: from 512 tiles on (two workgroups
+// per CU), or 256 where b is read across its rows, 64 bytes of each per step
+// here (the input gradients).  256 x 256 weights, k_mm against k_dense, in us:
+// forward 2048 rows 50 / 19, 4096 50 / 34, 8192 54 / 72 (BF16 45 / 65), 32768
+// 123 / 252; input gradients 2048 rows 38 / 31, 4096 40 / 61, 8192 51 / 117.
+// 256 x 4096 weights, forward: 512 rows 54 / 72, 4096 197 / 503.  Where a is
+// read across its rows (the weight gradients) k_dense is faster throughout:
+// 256 x 4096 weights, 4096 rows 694 / 188.
 template <class T>
 void dense(const T* a, int am, int ak, const T* b, int bk, int bn, const Dst& D, int M, int N, int K, hipStream_t s,
            float* part = nullptr, int64_t part_cap = 0) {
+  if (ak == 1 && (int64_t)(M / TM) * (N / TN) >= (bn == 1 ? 512 : 256)) {
+    mm<T>(op_row(a, am), bn == 1 ? op_row(b, bk) : op_trans(b, bn), D, M, N, K, s);
+    return;
+  }
   const int64_t waves = (int64_t)nblk(N, 16) * nblk(M, 16);
   int splits = part ? (int)std::max<int64_t>(1, std::min<int64_t>(512 / waves, K / 128)) : 1;
   if ((int64_t)splits * M * N > part_cap) splits = 1;
@@ -793,7 +814,6 @@ inline bool conv_dw(const float* in, int C, int R, int up, const float* dout, in
   return false;
 }
 
-Opnd op_row(const void* p, int ld) { return Opnd{p, OP_ROW, ld, 0, 0, 0}; }
 Dst dst_row(void* p, int ld, const float* bias, bool relu, bool bf16) {
   return Dst{p, 0, ld, 0, 0, bias, 0, relu ? 1 : 0, bf16 ? 1 : 0, nullptr};
 }

@@ -69,6 +69,40 @@ def test_rejects_bad_sizes():
         pecs_amd.WarmStartNet(0, 8, 2, 4)
 
 
+# Large minibatches: from 512 whole 64 x 64 tiles on (256 for the input
+# gradients) the dense products change kernel.  Both add their products in the
+# same order, so a prediction's rows have the bits of a small batch's, with the
+# same hidden units on, and the gradient is the batch-weighted mean of the
+# small batches' up to the rounding of its sums: about sqrt(K) eps of their
+# largest, 1.3e-5 at K = 10947 rows; bar 2e-5 of each block's largest.
+@pytest.mark.parametrize("dims,rows", [((4, 256, 2, 70), (4096, 4163, 8191, 8192, 8197)), ((5, 200, 2, 64), (10943, 10947))])
+def test_large_batches_match_small_ones(dims, rows):
+    nin, nh, nl, nout = dims
+    net = pecs_amd.WarmStartNet(nin, nh, nl, nout, seed=6)
+    lay, _ = layout(nin, nh, nl, nout)
+    rng = np.random.default_rng(13)
+    x = rng.normal(size=(max(rows), nin)).astype(np.float32)
+    y = rng.normal(size=(max(rows), nout)).astype(np.float32)
+    step = 1000  # (4 x 16 tiles of 64 x 64: the small kernel)
+    parts = {bf: np.concatenate([net.predict(x[i:i + step], bf16=bf) for i in range(0, len(x), step)])
+             for bf in (False, True)}
+    for b in rows:
+        _say(f"[gpu] mlp large batch {dims} rows {b}")
+        for bf in (False, True):
+            assert np.array_equal(net.predict(x[:b], bf16=bf), parts[bf][:b]), (b, bf)
+        loss, g = net.gradients(x[:b], y[:b])
+        rloss, rg = 0.0, 0.0
+        for i in range(0, b, step):
+            n = min(step, b - i)
+            pl, pg = net.gradients(x[i:i + n], y[i:i + n])
+            rloss, rg = rloss + pl * (n / b), rg + pg.astype(np.float64) * (n / b)
+        assert abs(loss - rloss) <= 1e-5 * rloss
+        for lo, hi in [(w[0], w[0] + w[1] * w[2]) for w, _ in lay] + [(v[0], v[0] + v[1]) for _, v in lay]:
+            d = np.abs(g[lo:hi] - rg[lo:hi]).max() / np.abs(rg[lo:hi]).max()
+            assert d <= 2e-5, (b, lo, hi, d)
+    net.close()
+
+
 # encoder + convolutional decoder: (nin, nh, nl, c0, g0, stages, batch); the
 # shapes cross tile edges (64-row / 64-column tiles, 16-deep k steps)
 DECODERS = [
