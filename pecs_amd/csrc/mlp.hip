@@ -718,7 +718,10 @@ void mm(const Opnd& A, const Opnd& B, const Dst& D, int M, int N, int K, hipStre
 }
 
 // Dense product.  k slices (where a scratch array is given) until about 512
-// waves are at work, each slice at least 128 deep.
+// waves are at work, each slice at least 128 deep, and never fewer than k_mm
+// takes: a weight gradient over many rows is not one chain of sums (256 x 256
+// weights in us, 8192 rows 150 -> 33 with the sum of the slices, 32768 593 -> 115; k_mm 190 and
+// 228).
 // With enough whole 64 x 64 tiles k_mm is faster, whose tiles read an operand
 // entry once per 64 outputs instead of 16: from 512 tiles on (two workgroups
 // per CU), or 256 where b is read across its rows, 64 bytes of each per step
@@ -736,8 +739,8 @@ void dense(const T* a, int am, int ak, const T* b, int bk, int bn, const Dst& D,
     return;
   }
   const int64_t waves = (int64_t)nblk(N, 16) * nblk(M, 16);
-  int splits = part ? (int)std::max<int64_t>(1, std::min<int64_t>(512 / waves, K / 128)) : 1;
-  if ((int64_t)splits * M * N > part_cap) splits = 1;
+  int splits = part ? (int)std::max<int64_t>(mm_splits(M, N, K), std::min<int64_t>(512 / waves, K / 128)) : 1;
+  splits = (int)std::max<int64_t>(1, std::min<int64_t>(splits, part_cap / ((int64_t)M * N)));
   const int kchunk = splits > 1 ? ((K + splits - 1) / splits + 15) / 16 * 16 : K;
   if (splits > 1) splits = (K + kchunk - 1) / kchunk;
   k_dense<T><<<dim3(nblk(N, 64), nblk(M, 16), splits), 256, 0, s>>>(a, am, ak, b, bk, bn, D, M, N, K, kchunk,
@@ -928,7 +931,7 @@ struct pecs_mlp {
       if (!y.conv) {
         // dW = act[l-1]^T dact[l]; db = colsum(dact[l]); dact[l-1] = dact[l] W^T
         dense<float>(act[l - 1], 1, y.nin, dact[l], y.nout, 1, dst_row(g + y.woff, y.nout, nullptr, false, false), y.nin,
-                     y.nout, rows, s);
+                     y.nout, rows, s, kpart, kpart_cap);
         k_colsum<<<nblk(y.nout, 256), 256, 0, s>>>(dact[l], g + y.boff, rows, y.nout);
         MCHECK(hipGetLastError());
         if (l > 1) {

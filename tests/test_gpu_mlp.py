@@ -103,6 +103,31 @@ def test_large_batches_match_small_ones(dims, rows):
     net.close()
 
 
+# The weight gradients of a large minibatch are summed in slices: one chain of
+# n terms of one sign is off by about 0.41 u sqrt(n / 3) (u = 2^-24 half a unit
+# in the last place, partial sums growing evenly), 2.6e-6 for 32768 terms added
+# one by one and up to 4 times that at the worst of 4096 entries; slices of
+# 1024 rows and their sum give 4.6e-7.  Bar: 6 times that, 2.8e-6, of every
+# entry (targets far below the outputs, so that no term changes sign).
+def test_weight_gradients_of_many_rows():
+    nin, nh, nl, nout, b = 4, 64, 2, 64, 32768
+    _say(f"[gpu] mlp weight gradients over {b} rows")
+    net = pecs_amd.WarmStartNet(nin, nh, nl, nout, seed=8)
+    rng = np.random.default_rng(14)
+    x = rng.uniform(0.5, 1.5, size=(b, nin)).astype(np.float32)
+    y = rng.uniform(-101, -99, size=(b, nout)).astype(np.float32)
+    lay, _ = layout(nin, nh, nl, nout)
+    _, rg = loss_and_grad(net.params().astype(np.float64), lay, x, y)
+    _, g = net.gradients(x, y)
+    (lo, fi, fo), _ = lay[-1]
+    g, rg = g[lo:lo + fi * fo].reshape(fi, fo), rg[lo:lo + fi * fo].reshape(fi, fo)
+    on = np.abs(rg).max(axis=1) > 1e-2 * np.abs(rg).max()  # (units that hardly ever turn on sum little)
+    assert on.sum() >= nh // 4
+    err = np.abs(g[on] / rg[on] - 1.0).max()
+    assert err <= 2.8e-6, err
+    net.close()
+
+
 # encoder + convolutional decoder: (nin, nh, nl, c0, g0, stages, batch); the
 # shapes cross tile edges (64-row / 64-column tiles, 16-deep k steps)
 DECODERS = [
