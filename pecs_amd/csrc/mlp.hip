@@ -720,8 +720,8 @@ void mm(const Opnd& A, const Opnd& B, const Dst& D, int M, int N, int K, hipStre
 // Dense product.  k slices (where a scratch array is given) until about 512
 // waves are at work, each slice at least 128 deep, and never fewer than k_mm
 // takes: a weight gradient over many rows is not one chain of sums (256 x 256
-// weights in us, 8192 rows 150 -> 33 with the sum of the slices, 32768 593 -> 115; k_mm 190 and
-// 228).
+// weights in us, with the sum of the slices: 8192 rows 150 -> 33, 32768 593 ->
+// 115; k_mm 190 and 228).
 // With enough whole 64 x 64 tiles k_mm is faster, whose tiles read an operand
 // entry once per 64 outputs instead of 16: from 512 tiles on (two workgroups
 // per CU), or 256 where b is read across its rows, 64 bytes of each per step
@@ -788,8 +788,9 @@ bool conv(const T* in, int C, int R, int up, const T* w, int M, int batch, const
 inline bool conv_dw(const float* in, int C, int R, int up, const float* dout, int M, int batch, float* dw, float* db,
                     float* part, int64_t part_cap, hipStream_t s) {
   Conv c{C, R, up, 0, M, C * 9};
-  const int mb = nblk(M, 16), nt = nblk(nblk(c.K + 1, 16), 4);
-  if (R % 4 || mb > 4 || nt > 10 || mb == 3) return false;
+  // (three row blocks take the variant of four, whose last one is zero)
+  const int mb = M > 32 && M <= 48 ? 4 : nblk(M, 16), nt = nblk(nblk(c.K + 1, 16), 4);
+  if (R % 4 || mb > 4 || nt > 10) return false;
   // the largest strip with which 512 workgroups have work, else the smallest
   // that is there: 256 workgroups, one wave per SIMD, waited on every LDS read
   int best = 0;
