@@ -853,7 +853,7 @@ struct pecs_mlp {
   float* kpart = nullptr;  // split-k partial sums of the weight gradients
   int64_t kpart_cap = 0;
   float *target = nullptr, *part = nullptr;
-  float* hpart = nullptr;  // pinned host copy of the loss's partial sums
+  float* hpart = nullptr;  // pinned host copy of the loss's partial sums, from the first gradient call on
   hipStream_t s = nullptr;
   ~pecs_mlp() {
     if (s) (void)hipStreamSynchronize(s);
@@ -914,6 +914,7 @@ struct pecs_mlp {
   // loss gradient in dact[L], its partial sums to hpart (on the stream)
   void loss_grad(int rows) {
     const int64_t n = (int64_t)rows * nout;
+    if (!hpart) MCHECK(hipHostMalloc((void**)&hpart, 256 * sizeof(float), hipHostMallocDefault));
     k_mse<<<256, 256, 0, s>>>(act[L()], target, dact[L()], part, n);
     MCHECK(hipGetLastError());
     MCHECK(hipMemcpyAsync(hpart, part, 256 * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -1007,7 +1008,6 @@ void mlp_init(pecs_mlp* net, unsigned seed) {
   MCHECK(hipMalloc(&net->v, off * sizeof(float)));
   MCHECK(hipMalloc(&net->pb, off * sizeof(uint16_t)));
   MCHECK(hipMalloc(&net->part, 256 * sizeof(float)));
-  MCHECK(hipHostMalloc((void**)&net->hpart, 256 * sizeof(float), hipHostMallocDefault));
   MCHECK(hipMemcpy(net->p, h.data(), off * sizeof(float), hipMemcpyHostToDevice));
   MCHECK(hipMemset(net->m, 0, off * sizeof(float)));
   MCHECK(hipMemset(net->v, 0, off * sizeof(float)));
