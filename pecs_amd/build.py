@@ -18,6 +18,7 @@ SELFTEST = os.path.join(BUILD, "pecs_selftest")
 HOST = os.path.join(HERE, "host")
 RUNNER = os.path.join(BUILD, "pecs_run")
 HOST_TEST = os.path.join(BUILD, "pecs_host_test")
+FACTOR_TEST = os.path.join(BUILD, "pecs_devfactor_test")
 
 HOST_SRC = ["mesh.cpp", "ops.cpp", "cholesky.cpp", "vtu.cpp", "dealii_layout.cpp"]
 HIP_SRC = ["kernels.hip", "devfactor.hip", "mlp.hip", "abi.hip"]
@@ -57,6 +58,7 @@ def build(verbose=False):
     link = ["-L" + HERE, "-lpecs_amd", "-Wl,-rpath,$ORIGIN/.."]
     _run(["g++", "-O2", "-std=c++17", os.path.join(HOST, "main.cpp"), "-o", RUNNER] + link, verbose)
     _run(["g++", "-O2", "-std=c++17", os.path.join(HOST, "host_test.cpp"), "-o", HOST_TEST] + link, verbose)
+    _run([hipcc] + HIPFLAGS + [os.path.join(CSRC, "devfactor_test.cpp"), "-o", FACTOR_TEST] + link, verbose)
     return LIB
 
 

@@ -785,13 +785,8 @@ void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::ve
         if (v == 0.0 || q < p) continue;
         const int s = plan.node_of[p];
         const SNode& N = F.nodes[s];
-        int r = q - N.p0;
-        if (r >= N.ns) {
-          const auto it = std::lower_bound(F.rows.begin() + N.rows_off, F.rows.begin() + N.rows_off + N.ms, q);
-          if (it == F.rows.begin() + N.rows_off + N.ms || *it != q)
-            throw std::runtime_error("execute_plan_host: an entry outside its front");
-          r = N.ns + (int)(it - F.rows.begin() - N.rows_off);
-        }
+        const int r = front_row(q, N.p0, N.ns, N.ms, F.rows.data() + N.rows_off);
+        if (r < 0) throw std::runtime_error("execute_plan_host: an entry outside its front");
         fr.at(plan.front_off[s] + (int64_t)r * (N.ns + N.ms) + (p - N.p0)) += v;
       }
   for (int l = 0; l < F.nlevels; ++l) {

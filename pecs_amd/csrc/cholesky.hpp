@@ -79,6 +79,22 @@ inline SupernodalFactor cholesky_factor(const BlockSPD& S, int leaf_cells) {
   return cholesky_factor(Systems{&S}, leaf_cells);
 }
 
+// Row of permuted index q in the front of a node with own rows [p0, p0 + ns)
+// and ms ascending struct rows, q >= p0; -1: q is not in the front.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline int front_row(int q, int p0, int ns, int ms, const int* rows) {
+  if (q - p0 < ns) return q - p0;
+  int lo = 0, hi = ms;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (rows[mid] < q) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo < ms && rows[lo] == q ? ns + lo : -1;
+}
+
 // Index plan of the multifrontal factorisation for execution on the device:
 // each node's dense nf x nf row-major front (nf = ns + ms; fronts of one level
 // contiguous), the S blocks (every entry (p, q), p <= q in permuted order, goes

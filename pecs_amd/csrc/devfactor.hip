@@ -81,13 +81,14 @@ struct Pool {
 // S blocks into the fronts: one wave per block.  Entry (p, q) in permuted
 // order, p <= q, goes to column p of the front of the node that owns p, at q's
 // row: own, or found in the node's ascending struct rows.  The entries write
-// disjoint positions of zeroed fronts.
+// disjoint positions of zeroed fronts.  lost counts the entries whose row is
+// not in the front.
 __global__ __launch_bounds__(64) void k_front_scatter(const double* __restrict__ sv, const SbItem* __restrict__ items,
                                                       const int* __restrict__ perm, const int* __restrict__ node_of,
                                                       const int* __restrict__ p0_, const int* __restrict__ ns_,
                                                       const int* __restrict__ ms_, const int64_t* __restrict__ rows_off,
                                                       const int* __restrict__ rows_, const int64_t* __restrict__ front_off,
-                                                      double* __restrict__ fr) {
+                                                      double* __restrict__ fr, int* __restrict__ lost) {
   const SbItem I = items[blockIdx.x];
   const int n = I.nx * I.ny;
   for (int e = threadIdx.x; e < n; e += 64) {
@@ -96,17 +97,10 @@ __global__ __launch_bounds__(64) void k_front_scatter(const double* __restrict__
     const int p = perm[I.x + a], q = perm[I.y + b];
     if (v == 0.0 || q < p) continue;
     const int s = node_of[p], ns = ns_[s], ms = ms_[s];
-    int r = q - p0_[s];
-    if (r >= ns) {
-      const int* rows = rows_ + rows_off[s];
-      int lo = 0, hi = ms;
-      while (lo < hi) {
-        const int mid = (lo + hi) / 2;
-        if (rows[mid] < q) lo = mid + 1;
-        else hi = mid;
-      }
-      if (lo == ms || rows[lo] != q) continue;  // (the row structure holds every coupling)
-      r = ns + lo;
+    const int r = front_row(q, p0_[s], ns, ms, rows_ + rows_off[s]);
+    if (r < 0) {
+      atomicAdd(lost, 1);
+      continue;
     }
     fr[front_off[s] + (int64_t)r * (ns + ms) + (p - p0_[s])] = v;
   }
@@ -305,8 +299,8 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
     }
   }
   double** d_ptrs = pool.up(ptrs, st);
-  rocblas_int* d_info = pool.alloc<rocblas_int>(ninfo);
-  DFCHECK(hipMemsetAsync(d_info, 0, std::max<size_t>(ninfo, 1) * sizeof(rocblas_int), st));
+  rocblas_int* d_info = pool.alloc<rocblas_int>(ninfo + 1);  // (the last one: entries outside their fronts)
+  DFCHECK(hipMemsetAsync(d_info, 0, (ninfo + 1) * sizeof(rocblas_int), st));
   // PECS_SETUP_TRACE=1: per-level times of the assembly kernels and the dense calls on stderr
   const char* tr = std::getenv("PECS_SETUP_TRACE");
   const bool trace = tr && std::string(tr) == "1";
@@ -324,7 +318,7 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
     if (trace) DFCHECK(hipEventRecord(ev[0], st));
     if (!sb.empty())
       k_front_scatter<<<(unsigned)sb.size(), 64, 0, st>>>(sv, d_sb, d_perm, d_node_of, d_p0, d_ns, d_ms, d_rows_off,
-                                                          d_rows, d_front_off, fr);
+                                                          d_rows, d_front_off, fr, d_info + ninfo);
     for (int l = 0; l < F.nlevels; ++l) {
       for (int pass = 0; pass < plan.npass; ++pass) {
         const int e0 = plan.ea_level[(size_t)plan.npass * l + pass], e1 = plan.ea_level[(size_t)plan.npass * l + pass + 1];
@@ -410,9 +404,12 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
                                                        bwd);
     DFCHECK(hipGetLastError());
     if (trace) DFCHECK(hipEventRecord(ev[2 * F.nlevels + 1], st));
-    std::vector<rocblas_int> info(ninfo);
-    if (ninfo) DFCHECK(hipMemcpyAsync(info.data(), d_info, ninfo * sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
+    std::vector<rocblas_int> info(ninfo + 1);
+    DFCHECK(hipMemcpyAsync(info.data(), d_info, (ninfo + 1) * sizeof(rocblas_int), hipMemcpyDeviceToHost, st));
     DFCHECK(hipStreamSynchronize(st));
+    if (info[ninfo])
+      throw std::runtime_error("device factorisation: " + std::to_string(info[ninfo]) +
+                               " entries of the matrix lie outside their fronts");
     for (const Group& g : groups)
       for (int i = 0; i < 2 * g.count; ++i)
         if (info[g.info0 + i] != 0)

@@ -340,18 +340,8 @@ static void device_factor_emulate(const FrontPlan& plan, const SupernodalFactor&
         const int p = F.perm[plan.sb_x[it] + a], q = F.perm[plan.sb_y[it] + b];
         if (v == 0.0 || q < p) continue;
         const int s = plan.node_of[p], ns = P.ns[s], ms = P.ms[s];
-        int r = q - P.p0[s];
-        if (r >= ns) {
-          const int* rows = P.rows.data() + P.rows_off[s];
-          int lo = 0, hi = ms;
-          while (lo < hi) {
-            const int mid = (lo + hi) / 2;
-            if (rows[mid] < q) lo = mid + 1;
-            else hi = mid;
-          }
-          DEV_CHECK(lo < ms && rows[lo] == q, "struct row");
-          r = ns + lo;
-        }
+        const int r = front_row(q, P.p0[s], ns, ms, P.rows.data() + P.rows_off[s]);
+        DEV_CHECK(r >= 0, "struct row");
         FR(plan.front_off[s] + (int64_t)r * (ns + ms) + (p - P.p0[s])) = v;
       }
   }

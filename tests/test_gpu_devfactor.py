@@ -6,6 +6,9 @@ the scalar sweeps (single instance) and the MFMA sweeps over blocked copies
 (batched instances), and the trajectories against the oracle are covered by
 the other GPU tests, which run on the device factors by default.
 """
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -71,3 +74,10 @@ def test_device_factor_batched_mfma_matches_host_factor(monkeypatch):
     for i in range(3):
         for c in "nproP":
             assert _rel(dev[i][c], host[i][c]) < 1e-11, (i, c, _rel(dev[i][c], host[i][c]))
+
+
+def test_entries_outside_their_fronts_are_refused():
+    _say("[gpu] device factorisation with a struct row missing")
+    exe = os.path.join(os.path.dirname(pecs_amd.__file__), "_build", "pecs_devfactor_test")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
