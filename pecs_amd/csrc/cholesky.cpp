@@ -68,7 +68,7 @@ struct DofGraph {
           const int xi = X % S.NXc, xj = X / S.NXc;
           for (int a = 0; a < nx; ++a) {
             int64_t cnt = 0;
-            const int64_t at = ptr[dof0[k][X] + a];
+            const int64_t at = pass ? ptr[dof0[k][X] + a] : 0;  // (the counting pass writes ptr)
             for (int o = 0; o < no; ++o) {
               const int yi = xi + S.offi[o], yj = xj + S.offj[o];
               if (yi < 0 || yi >= S.NXc || yj < 0 || yj >= S.NYc) continue;
