@@ -413,26 +413,28 @@ void structure(const DofGraph& G, const std::vector<NDNode>& nodes, std::vector<
   std::vector<std::vector<int>> by(nl);
   for (int s = 0; s < nn; ++s) by[lv[s]].push_back(s);
   st.assign(nn, {});
-#pragma omp parallel
-  {
-    std::vector<int> mark(G.n, -1);
-    for (int l = 0; l < nl; ++l) {
-#pragma omp for schedule(dynamic, 4)
-      for (size_t i = 0; i < by[l].size(); ++i) {
-        const int s = by[l][i];
-        std::vector<int>& r = st[s];
-        auto consider = [&](int q) {
-          if (q >= p1[s] && mark[q] != s) {
-            mark[q] = s;
-            r.push_back(q);
-          }
-        };
-        for (int d : nodes[s].dofs)
-          for (int64_t q = G.ptr[d]; q < G.ptr[d + 1]; ++q) consider(pos[G.adj[q]]);
-        for (int c : nodes[s].children)
-          for (int q : st[c]) consider(q);
-        std::sort(r.begin(), r.end());
-      }
+  for (int l = 0; l < nl; ++l) {
+#pragma omp parallel for schedule(dynamic, 4)
+    for (size_t i = 0; i < by[l].size(); ++i) {
+      const int s = by[l][i];
+      std::vector<int>& r = st[s];
+      // (sorted, not marked in an array over all DoFs, of which every thread
+      // would hold one; neighbours have most rows in common, so that a small
+      // table of recent ones keeps most repeats out)
+      int recent[1024];
+      std::fill(recent, recent + 1024, -1);
+      auto consider = [&](int q) {
+        if (q < p1[s] || recent[q & 1023] == q) return;
+        recent[q & 1023] = q;
+        r.push_back(q);
+      };
+      for (int d : nodes[s].dofs)
+        for (int64_t q = G.ptr[d]; q < G.ptr[d + 1]; ++q) consider(pos[G.adj[q]]);
+      for (int c : nodes[s].children)
+        for (int q : st[c]) consider(q);
+      std::sort(r.begin(), r.end());
+      r.erase(std::unique(r.begin(), r.end()), r.end());
+      r.shrink_to_fit();
     }
   }
 }
@@ -603,10 +605,9 @@ SupernodalFactor cholesky_factor(const Systems& Ss, int leaf_cells, const SolveC
   // nodes of one level are independent (their children are in lower levels).
   std::vector<std::vector<double>> upd(nn);
   const int nthreads = omp_get_max_threads();
-  std::vector<std::vector<int>> loc_t(nthreads, std::vector<int>(F.n, -1));
   std::vector<double> flops_t(nthreads, 0.0), ta_t(nthreads, 0.0), tf_t(nthreads, 0.0), ti_t(nthreads, 0.0);
+  std::vector<int64_t> lost_t(nthreads, 0);  // entries outside their fronts
   auto process = [&](int s, int tid) {
-    std::vector<int>& loc = loc_t[tid];  // permuted index -> struct row of this front
     const SNode& N = F.nodes[s];
     const int ns = N.ns, ms = N.ms, nf = ns + ms;
     const bool big = nf > 1024;
@@ -614,7 +615,6 @@ SupernodalFactor cholesky_factor(const Systems& Ss, int leaf_cells, const SolveC
     std::vector<double> Fr((size_t)nf * nf);
 #pragma omp parallel for schedule(static) if (big)
     for (int r = 0; r < nf; ++r) std::fill(&Fr[(size_t)r * nf], &Fr[(size_t)r * nf] + r + 1, 0.0);
-    for (int r = 0; r < ms; ++r) loc[F.rows[N.rows_off + r]] = ns + r;
     // original entries (p, q), p own and p <= q, into column p
     for (int c = 0; c < ns; ++c) {
       const int d = dof_at[N.p0 + c], X = G.cell[d];
@@ -632,12 +632,15 @@ SupernodalFactor cholesky_factor(const Systems& Ss, int leaf_cells, const SolveC
           const double v = B[(size_t)a * ny + b];
           const int q = F.perm[dof0[Y] + b];
           if (v == 0.0 || q < N.p0 + c) continue;
-          const int r = q < N.p0 + ns ? q - N.p0 : loc[q];
+          const int r = front_row(q, N.p0, ns, ms, F.rows.data() + N.rows_off);
+          if (r < 0) {
+            ++lost_t[tid];
+            continue;
+          }
           Fr[(size_t)r * nf + c] += v;
         }
       }
     }
-    for (int r = 0; r < ms; ++r) loc[F.rows[N.rows_off + r]] = -1;
     // extend-add children
     for (int c : F.children[s]) {
       const int mc = F.nodes[c].ms;
@@ -681,6 +684,7 @@ SupernodalFactor cholesky_factor(const Systems& Ss, int leaf_cells, const SolveC
     }
   }
   for (int t = 0; t < nthreads; ++t) {
+    if (lost_t[t]) throw std::runtime_error("cholesky_factor: an entry outside its front");
     F.flops += flops_t[t];
     F.t_assemble += ta_t[t];
     F.t_factor += tf_t[t];

@@ -2,10 +2,14 @@
 // builds the meshes, local operators, the SPD Schur / multiplier matrices,
 // factors them and checks ||S x - b|| / ||b|| of the stored factor through a
 // plain host triangular solve written only for this test.
+#include <omp.h>
+
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 #include <random>
 
 #include "cholesky.hpp"
@@ -13,6 +17,16 @@
 #include "ops.hpp"
 
 using namespace pecs;
+
+// Bytes asked of new so far.
+static std::atomic<int64_t> g_bytes{0};
+void* operator new(size_t n) {
+  g_bytes += (int64_t)n;
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 static void block_matvec(const Systems& Ss, const SupernodalFactor& F, const double* x, double* y) {
   for (int k = 0; k < (int)Ss.size(); ++k) {
@@ -678,6 +692,24 @@ int main(int argc, char** argv) {
         std::printf("twin systems ordered differently\n");
         return 2;
       }
+  }
+  {  // the symbolic phase's memory does not grow with the number of threads:
+     // with 64, less than 8 arrays over the DoFs more than with one
+    const int threads = omp_get_max_threads();
+    int64_t bytes[2];
+    int n = 0;
+    for (int i = 0; i < 2; ++i) {
+      omp_set_num_threads(i ? 64 : 1);
+      bytes[i] = -g_bytes;
+      FrontPlan plan;
+      n = cholesky_symbolic({&Ss, &Se}, leaf, plan, costs[1]).n;
+      bytes[i] += g_bytes;
+    }
+    omp_set_num_threads(threads);
+    if (bytes[1] - bytes[0] > 8 * 4 * (int64_t)n) {
+      std::printf("symbolic phase allocated %.1f MB with 64 threads, %.1f MB with one\n", bytes[1] * 1e-6, bytes[0] * 1e-6);
+      return 2;
+    }
   }
   std::printf("%s\n", worst < 1e-12 ? "SELFTEST OK" : "SELFTEST FAIL");
   return worst < 1e-12 ? 0 : 1;
