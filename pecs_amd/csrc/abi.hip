@@ -1346,7 +1346,6 @@ int create_impl(const pecs_mesh* mesh, const pecs_params* params, int B, pecs_ct
       for (int K = 0; K < m.ncellP; ++K) all[K + 1] += all[K];
       P.hc_all = upload(c.get(), all);
       P.mhang = upload(c.get(), mh);
-      P.nhang = (int)hs.size();
       P.nhc = (int)cells.size();
       P.h_cell = upload(c.get(), hc);
       P.h_face = upload(c.get(), hf);

@@ -358,16 +358,10 @@ __device__ __forceinline__ void schur_w(const DevRegion& R, const double* __rest
 // wave's cells share the operator types the kernel reads (groups padded to
 // whole waves with -1), so that the table offsets are wave-uniform and the
 // table entries are fetched once per wave through the scalar cache.
-template <bool UNI>
-__device__ __forceinline__ int schur_cell(const int* __restrict__ list, int n, int t) {
-  if (UNI) return t < n ? list[t] : -1;
-  return t < n ? t : -1;
-}
+__device__ __forceinline__ int schur_cell(const int* __restrict__ list, int n, int t) { return t < n ? list[t] : -1; }
 
-template <bool UNI>
 __device__ __forceinline__ int wave_type(const DevRegion& R, int M) {
-  const int t = R.type[M];
-  return UNI ? __builtin_amdgcn_readfirstlane(t) : t;
+  return __builtin_amdgcn_readfirstlane(R.type[M]);
 }
 
 // The FP64 Schur kernels: one lane per (cell, density DoF a), NB = (K + 1)^2
@@ -669,7 +663,7 @@ __device__ __forceinline__ void schur_rhs_one_f32(const DevRegion& R, const doub
   for (int f = -1; f < 4; ++f) {
     const int M = f < 0 ? X : R.nbr[4 * (size_t)X + f];
     if (M < 0) continue;
-    const int ty = wave_type<true>(R, M);
+    const int ty = wave_type(R, M);
     const float* Minv = R.table_f + (size_t)ty * R.stride;
     const float* B = Minv + NB * NB + (f < 0 ? 0 : 2 * NB * NB + (f ^ 1) * 2 * NB * NB);
     float fx[NB], fy[NB], w[2 * NB];
@@ -704,7 +698,7 @@ __global__ __launch_bounds__(64) void k_schur_rhs_f32(DevRegion R, const double*
                                                       const double* __restrict__ b2, double mu1, double mu2,
                                                       double* __restrict__ g1, double* __restrict__ g2, int64_t sb,
                                                       int64_t sg) {
-  const int X = schur_cell<true>(R.ucell_nbh, R.nu_nbh, blockIdx.x * blockDim.x + threadIdx.x);
+  const int X = schur_cell(R.ucell_nbh, R.nu_nbh, blockIdx.x * blockDim.x + threadIdx.x);
   if (X < 0) return;
   const int64_t i = blockIdx.y;
   schur_rhs_one_f32<K>(R, b1 + i * sb, mu1, g1 + i * sg, X);
@@ -772,10 +766,10 @@ __global__ __launch_bounds__(64) void k_schur_recover_f32(DevRegion R, const dou
                                                           const double* __restrict__ x2, double mu1, double mu2,
                                                           double* __restrict__ o1, double* __restrict__ o2,
                                                           int64_t sb, int64_t sx, int64_t so) {
-  const int M = schur_cell<true>(R.ucell_own, R.nu_own, blockIdx.x * blockDim.x + threadIdx.x);
+  const int M = schur_cell(R.ucell_own, R.nu_own, blockIdx.x * blockDim.x + threadIdx.x);
   if (M < 0) return;
   const int64_t i = blockIdx.y;
-  const float* tb = R.table_f + (size_t)wave_type<true>(R, M) * R.stride;
+  const float* tb = R.table_f + (size_t)wave_type(R, M) * R.stride;
   schur_recover_one_f32<K>(R, tb, b1 + i * sb, x1 + i * sx, mu1, o1 + i * so, M);
   if (NRHS > 1) schur_recover_one_f32<K>(R, tb, b2 + i * sb, x2 + i * sx, mu2, o2 + i * so, M);
 }

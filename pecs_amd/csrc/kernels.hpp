@@ -85,12 +85,12 @@ struct DevPoisson {
   // per cell: bit f set if the cell writes face f's D DoFs
   const unsigned char* own;
   // hanging faces: the coarse side's D.n couples to the fine faces'
-  // multipliers.  Per hanging pair h (nhang): coarse cell, coarse face,
+  // multipliers.  Per hanging pair h: coarse cell, coarse face,
   // subface and first multiplier of the fine face; the coupling of
   // multiplier (s, m) to the coarse face's local DoF j is
   // sign(face) * hE[(s k + m) k + j].  hc_cell / hc_ptr group the pairs by
   // coarse cell (nhc cells).
-  int nhang, nhc;
+  int nhc;
   const int *h_cell, *h_face, *h_sub, *h_mbase;
   const int *hc_cell, *hc_ptr;
   const double* hE;

@@ -274,7 +274,6 @@ static BlockSPD schur_matrix_lattice(const Region& R, const LdgRegionOps& ops, d
   BlockSPD S;
   S.NXc = R.NXg;
   S.NYc = R.NYg;
-  S.sep_width = 0;
   const size_t NG = (size_t)S.NXc * S.NYc;
   S.ndof.assign(NG, 0);
   auto gid = [&](int c) { return (size_t)R.ci[c] + (size_t)S.NXc * R.cj[c]; };
@@ -349,7 +348,6 @@ BlockSPD schur_matrix(const Region& R, const LdgRegionOps& ops, double mu) {
   S.NXc = N;
   S.NYc = N;
   S.ndof.assign(N * N, nb);
-  S.sep_width = 2;
   for (int dj = -2; dj <= 2; ++dj)
     for (int di = -2; di <= 2; ++di)
       if (std::abs(di) + std::abs(dj) <= 2) {
@@ -709,7 +707,6 @@ static BlockSPD multiplier_matrix_local(const SolarCellMesh& m, const PoissonOps
   S.NXc = m.NX;
   S.NYc = m.NY;
   S.ndof = O.ndof_owner;
-  S.sep_width = 0;
   const size_t NG = (size_t)m.NX * m.NY;
   std::vector<int> owner_of(O.nmult);
   for (size_t G = 0; G < NG; ++G)
@@ -774,7 +771,6 @@ BlockSPD multiplier_matrix(const SolarCellMesh& m, const PoissonOps& O, const Re
   S.NXc = m.NX;
   S.NYc = m.NY;
   S.ndof = O.ndof_owner;
-  S.sep_width = 1;
   const int oi[7] = {0, 1, -1, 0, 0, 1, -1}, oj[7] = {0, 0, 0, 1, -1, -1, 1};
   for (int o = 0; o < 7; ++o) {
     S.offi.push_back(oi[o]);

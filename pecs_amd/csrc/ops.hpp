@@ -81,15 +81,11 @@ struct LdgRegionOps {
 LdgRegionOps build_ldg_ops(const Region& R, const RefTables& T, const Params& P);
 
 // Block-sparse SPD matrix on a structured cell grid (input to the Cholesky).
-// sep_width = 0: every nested-dissection separator is made as wide as the
-// couplings across it require (meshes embedded in a lattice with empty
-// positions, whose coupling offsets differ from place to place).
 struct BlockSPD {
   int NXc = 0, NYc = 0;
   std::vector<int> ndof;          // per grid cell gid = i + NXc*j
   std::vector<int> offi, offj;    // coupling offsets
   std::vector<std::vector<double>> blk;  // [gid*noff + o]: ndof[gid] x ndof[nbr]
-  int sep_width = 1;
   int noff() const { return (int)offi.size(); }
 };
 
