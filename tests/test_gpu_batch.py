@@ -192,3 +192,39 @@ def test_single_solves_on_lds_shaped_factors(shape, seed):
             assert _rel(x, o.solve(key, b)) < 1e-11, (key, _rel(x, o.solve(key, b)))
     finally:
         g.close()
+
+
+# (batch, mobilities): with one region's pair equal and the other's distinct
+# the regions have a factor each, the second solved on the second stream, and
+# the batch of 2 shapes one of them for 2 right-hand sides and the other, with
+# 4, for MFMA; with both distinct, 3 instances take MFMA shapes on a forest of
+# four systems, of which a carrier's solve runs one.
+@pytest.mark.parametrize("B,mobility", [(1, dict(mu_p=0.7)), (1, dict(mu_o=0.5)), (2, dict(mu_n=1.3, mu_p=0.7)),
+                                        (2, dict(mu_r=2.0, mu_o=0.5)), (3, dict(mu_p=0.7)),
+                                        (3, dict(mu_n=1.3, mu_p=0.7, mu_r=2.0, mu_o=0.5))])
+def test_mobilities_distinct_per_region(B, mobility, seed):
+    import pecs_amd
+    _say(f"[gpu] batch of {B}, mobilities {mobility}")
+    prms = [dict(p, **mobility) for p in _batch(B, seed + 13, r=3)]
+    g = pecs_amd.SolarCellGPU(prms if B > 1 else prms[0])
+    g.initial_state()
+    g.step(STEPS)
+    oracles = [OracleSolarCell(p) for p in prms]
+    for i, o in enumerate(oracles):
+        a, b = g.get_state(i), o.run(STEPS)
+        for c in "nproP":
+            assert _rel(a[c], b[c]) < 1e-10, (i, c, _rel(a[c], b[c]))
+    rng = np.random.default_rng(seed)
+    for which, key in ((pecs_amd.ELECTRONS, "n"), (pecs_amd.HOLES, "p"), (pecs_amd.REDUCTANTS, "r"),
+                       (pecs_amd.OXIDANTS, "o"), (pecs_amd.POISSON, "P")):
+        n = {"n": g.n_semi, "p": g.n_semi, "r": g.n_elec, "o": g.n_elec, "P": g.n_poisson}[key]
+        b = rng.standard_normal(n)
+        x = oracles[0].solve(key, b)
+        assert _rel(g.solve(which, b), x) < 1e-11, (key, _rel(g.solve(which, b), x))
+    # the solves leave the steps' scratch usable
+    g.step(1)
+    for i, o in enumerate(oracles):
+        a, b = g.get_state(i), o.run(STEPS + 1)
+        for c in "nproP":
+            assert _rel(a[c], b[c]) < 1e-10, (i, c, _rel(a[c], b[c]))
+    g.close()

@@ -3,7 +3,8 @@
 The no-allocation variant runs the same kernels in the same order on a static
 device scratch array instead of the context's buffers, so its solutions must
 equal pecs_solve_dev's bit for bit, for every system, on two contexts in a
-row (the second one smaller: the array keeps the first call's contents).  It
+row (the second one smaller: the array keeps the first call's contents), with
+systems shared by a region's carriers or not.  It
 must leave the device's free memory unchanged, and reject batched contexts
 and systems whose scratch exceeds the limit with an error.
 """
@@ -73,15 +74,21 @@ class _Hip:
         self.bufs = []
 
 
-def test_noalloc_matches_solve_dev(seed):
+# one system per region, one per carrier, one region of each kind (two factors)
+MOBILITIES = {"equal": {}, "distinct": dict(mu_n=1.3, mu_p=0.7, mu_r=2.0, mu_o=0.5), "holes": dict(mu_p=0.7),
+              "oxidants": dict(mu_o=0.5)}
+
+
+@pytest.mark.parametrize("mobility", list(MOBILITIES))
+def test_noalloc_matches_solve_dev(mobility, seed):
     import pecs_amd
     L = _lib()
     hip = _Hip()
     rng = np.random.default_rng(seed)
     for r, k in ((5, 2), (3, 1)):  # the second context is smaller
         p = pecs_amd.workload_params(r, k, 5e-4)
-        p.update(phi_bi=0.4, phi_app=0.1)
-        _say(f"[gpu] no-alloc solve vs pecs_solve_dev: refinement {r}, k={k}")
+        p.update(phi_bi=0.4, phi_app=0.1, **MOBILITIES[mobility])
+        _say(f"[gpu] no-alloc solve vs pecs_solve_dev: refinement {r}, k={k}, mobilities {mobility}")
         g = pecs_amd.SolarCellGPU(p)
         for which, n in ((pecs_amd.ELECTRONS, g.n_semi), (pecs_amd.HOLES, g.n_semi),
                          (pecs_amd.REDUCTANTS, g.n_elec), (pecs_amd.OXIDANTS, g.n_elec),
@@ -102,6 +109,10 @@ def test_noalloc_matches_solve_dev(seed):
             assert np.array_equal(xn, xr), (r, which, float(np.abs(xn - xr).max()))
             # and the host-pointer solve (pecs_solve) agrees with both
             assert np.array_equal(g.solve(which, bh), xr)
+            # in place: the right-hand side's vector takes the solution
+            assert L.pecs_solve_dev(g.ctx, which, b, b) == 0
+            hip.sync()
+            assert np.array_equal(hip.get(b, n), xr), which
         g.close()
     hip.release()
 
