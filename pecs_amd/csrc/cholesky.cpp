@@ -700,9 +700,7 @@ SupernodalFactor cholesky_symbolic(const Systems& Ss, int leaf_cells, FrontPlan&
   const int nn = (int)F.nodes.size();
   plan = FrontPlan{};
   plan.nlevels = F.nlevels;
-  // S blocks, concatenated
-  std::vector<const std::vector<double>*> blocks;
-  int64_t sv = 0;
+  // S blocks
   for (size_t k = 0; k < Ss.size(); ++k) {
     const BlockSPD& S = *Ss[k];
     const int NG = S.NXc * S.NYc, no = S.noff();
@@ -712,19 +710,15 @@ SupernodalFactor cholesky_symbolic(const Systems& Ss, int leaf_cells, FrontPlan&
         if (B.empty()) continue;
         const int Y = X + S.offi[o] + S.NXc * S.offj[o];
         if (S.ndof[X] == 0 || S.ndof[Y] == 0) continue;
-        blocks.push_back(&B);
-        plan.sb_src.push_back(sv);
+        plan.sb_val.push_back(B.data());
+        plan.sb_src.push_back(plan.nvals);
         plan.sb_x.push_back(G.dof0[k][X]);
         plan.sb_y.push_back(G.dof0[k][Y]);
         plan.sb_nx.push_back(S.ndof[X]);
         plan.sb_ny.push_back(S.ndof[Y]);
-        sv += (int64_t)B.size();
+        plan.nvals += (int64_t)B.size();
       }
   }
-  plan.svals.resize(sv);
-#pragma omp parallel for schedule(static)
-  for (size_t i = 0; i < blocks.size(); ++i)
-    std::copy(blocks[i]->begin(), blocks[i]->end(), &plan.svals[plan.sb_src[i]]);
   plan.node_of.resize(F.n);
   for (int s = 0; s < nn; ++s)
     std::fill_n(plan.node_of.begin() + F.nodes[s].p0, F.nodes[s].ns, s);
@@ -774,6 +768,12 @@ SupernodalFactor cholesky_symbolic(const Systems& Ss, int leaf_cells, FrontPlan&
   return F;
 }
 
+void copy_blocks(const FrontPlan& plan, size_t i0, size_t i1, double* dst) {
+#pragma omp parallel for schedule(static)
+  for (size_t i = i0; i < i1; ++i)
+    std::copy_n(plan.sb_val[i], plan.sb_nx[i] * plan.sb_ny[i], dst + (plan.sb_src[i] - plan.sb_src[i0]));
+}
+
 void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::vector<double>& Linv,
                        std::vector<double>& L21) {
   const int nn = (int)F.nodes.size();
@@ -784,7 +784,7 @@ void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::ve
   for (size_t i = 0; i < plan.sb_src.size(); ++i)
     for (int a = 0; a < plan.sb_nx[i]; ++a)
       for (int b = 0; b < plan.sb_ny[i]; ++b) {
-        const double v = plan.svals.at(plan.sb_src[i] + (int64_t)a * plan.sb_ny[i] + b);
+        const double v = plan.sb_val[i][a * plan.sb_ny[i] + b];
         const int p = F.perm[plan.sb_x[i] + a], q = F.perm[plan.sb_y[i] + b];
         if (v == 0.0 || q < p) continue;
         const int s = plan.node_of[p];

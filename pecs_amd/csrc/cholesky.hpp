@@ -105,10 +105,13 @@ struct FrontPlan {
   int nlevels = 0, npass = 0;
   std::vector<int64_t> front_off, level_front;  // per node; per level [begin, end)
   int64_t front_total = 0;
-  std::vector<double> svals;                    // S blocks concatenated
-  // per nonempty block: values offset, first DoF and count of its rows / columns
+  // per nonempty S block: its values (in the systems, which the plan does not
+  // outlive), their offset with all blocks' values one after the other, first
+  // DoF and count of its rows / columns
+  std::vector<const double*> sb_val;
   std::vector<int64_t> sb_src;
   std::vector<int> sb_x, sb_y, sb_nx, sb_ny;
+  int64_t nvals = 0;                            // of all blocks
   std::vector<int> node_of;                     // per permuted index: its node
   std::vector<int> ea_child, ea_row, ea_parent, ea_level;  // extend-add rows; ea_level per (level, pass)
   std::vector<int> ea_map;                      // per child: its panel rows' positions in the parent front
@@ -118,6 +121,8 @@ struct FrontPlan {
 // values: Linv / L21 stay empty) and the device plan of its numeric phase.
 SupernodalFactor cholesky_symbolic(const Systems& S, int leaf_cells, FrontPlan& plan, const SolveCost& cost = {},
                                    const std::vector<int>& twin = {});
+// The values of blocks [i0, i1) of a plan, one after the other.
+void copy_blocks(const FrontPlan& plan, size_t i0, size_t i1, double* dst);
 // Host execution of a plan (for checking the plan's indexing against
 // cholesky_factor): fills Linv and L21 as cholesky_factor does.
 void execute_plan_host(const FrontPlan& plan, const SupernodalFactor& F, std::vector<double>& Linv,

@@ -243,7 +243,7 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
   {  // the fronts are the large allocation: fail with a clear message, not inside the dense calls
     size_t free_b = 0, total_b = 0;
     DFCHECK(hipMemGetInfo(&free_b, &total_b));
-    const double need = 8.0 * (double)plan.front_total + 8.0 * (double)plan.svals.size() + (256.0 * (1 << 20));
+    const double need = 8.0 * (double)plan.front_total + 8.0 * (double)plan.nvals + (256.0 * (1 << 20));
     if (need > (double)free_b)
       throw std::runtime_error("device factorisation: the fronts need " + std::to_string(need * 1e-9) +
                                " GB, the device has " + std::to_string(free_b * 1e-9) + " GB free");
@@ -258,7 +258,17 @@ DeviceFactorStats factor_on_device(const FrontPlan& plan, const SupernodalFactor
   std::vector<PkItem> pk;
   for (int s = 0; s < nn; ++s)
     for (int j0 = 0; j0 < P.ns[s]; j0 += 16) pk.push_back(PkItem{s, j0});
-  double* sv = pool.up(plan.svals, st);
+  double* sv = pool.alloc<double>(plan.nvals);
+  {  // the blocks' values through a buffer of 64 MB: the host holds no second copy of the systems
+    std::vector<double> stage(std::min<int64_t>(plan.nvals, (int64_t)8 << 20));
+    for (size_t i = 0, j; i < sb.size(); i = j) {
+      auto end = [&](size_t b) { return sb[b].src + (int64_t)sb[b].nx * sb[b].ny - sb[i].src; };
+      for (j = i + 1; j < sb.size() && end(j) <= (int64_t)stage.size();) ++j;
+      copy_blocks(plan, i, j, stage.data());
+      DFCHECK(hipMemcpyAsync(sv + sb[i].src, stage.data(), end(j - 1) * sizeof(double), hipMemcpyHostToDevice, st));
+      DFCHECK(hipStreamSynchronize(st));
+    }
+  }
   SbItem* d_sb = pool.up(sb, st);
   int* d_perm = pool.up(F.perm, st);
   int* d_node_of = pool.up(plan.node_of, st);

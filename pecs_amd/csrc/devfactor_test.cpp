@@ -44,7 +44,7 @@ int main() {
     for (int e = 0; e < plan.sb_nx[i] * plan.sb_ny[i] && damaged.empty(); ++e) {
       const int p = F.perm[plan.sb_x[i] + e / plan.sb_ny[i]], q = F.perm[plan.sb_y[i] + e % plan.sb_ny[i]];
       const SNode& N = F.nodes[plan.node_of[p]];
-      if (plan.svals[plan.sb_src[i] + e] == 0.0 || q < p) continue;
+      if (plan.sb_val[i][e] == 0.0 || q < p) continue;
       const int r = front_row(q, N.p0, N.ns, N.ms, &F.rows[N.rows_off]) - N.ns;
       if (r < 0 || r + 1 >= N.ms) continue;
       Q.rows[N.rows_off + r] = Q.rows[N.rows_off + r + 1];

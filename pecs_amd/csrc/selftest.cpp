@@ -342,14 +342,16 @@ static void device_factor_emulate(const FrontPlan& plan, const SupernodalFactor&
     DEV_CHECK(i >= 0 && i < P.nvals, "bwd");
     return bwd[i];
   };
+  std::vector<double> sv(plan.nvals);
+  copy_blocks(plan, 0, plan.sb_src.size(), sv.data());
   // k_front_scatter: 64 lanes per block
   for (size_t it = 0; it < plan.sb_src.size(); ++it) {
     const int nx = plan.sb_nx[it], ny = plan.sb_ny[it];
     for (int t = 0; t < 64; ++t)
       for (int e = t; e < nx * ny; e += 64) {
         const int a = e / ny, b = e - a * ny;
-        DEV_CHECK(plan.sb_src[it] + e < (int64_t)plan.svals.size(), "svals");
-        const double v = plan.svals[plan.sb_src[it] + e];
+        DEV_CHECK(plan.sb_src[it] + e < plan.nvals, "block values");
+        const double v = sv[plan.sb_src[it] + e];
         DEV_CHECK(plan.sb_x[it] + a < F.n && plan.sb_y[it] + b < F.n, "perm");
         const int p = F.perm[plan.sb_x[it] + a], q = F.perm[plan.sb_y[it] + b];
         if (v == 0.0 || q < p) continue;
