@@ -298,7 +298,9 @@ int pecs_uniform_lists(pecs_ctx* ctx, int* flags);
  * relative L2 differences from the FP64 path of about 5e-8 in the densities
  * after 20 steps at refinement 4, 2e-4 (carrier vectors) after 200 steps at
  * refinement 6 and 8e-4 after 200 steps at refinement 8; the potential stays
- * near 3e-7.  No counterpart in the reference (FP64 throughout); it replaces
+ * near 3e-7.  It is slower than FP64, whose cell kernels spread a cell over
+ * lanes where these take a thread per cell (refinement 8, k = 2: one instance
+ * 1.67 against 1.63 ms per step, a batch of 16 5.75 against 5.27).  No counterpart in the reference (FP64 throughout); it replaces
  * nothing. */
 int pecs_set_mixed_precision(pecs_ctx* ctx, int enable);
 
@@ -370,8 +372,8 @@ int pecs_solve_dev(pecs_ctx* ctx, int which, const double* rhs, double* x);
  * static device array of 64 MiB per GPU, held until the process ends, instead
  * of the context's buffers.  Single-instance contexts only.  A system whose
  * scratch exceeds 64 MiB is rejected with an error (refinement 8, k = 2
- * needs 32.7 MB for a carrier and 42.2 MB for the Poisson system).  The
- * array is found on the device that is current at the call; contexts created
+ * needs 27.6 MB for a carrier, 29.9 MB with distinct mobilities, and 37.5 MB
+ * for the Poisson system).  The array is found on the device that is current at the call; contexts created
  * on that device set it up.  Every call on a GPU shares that GPU's array:
  * calls that overlap on one GPU (two streams, two host threads) race. */
 int pecs_solve_dev_noalloc(pecs_ctx* ctx, int which, const double* rhs, double* x);

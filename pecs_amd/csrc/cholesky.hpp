@@ -17,8 +17,8 @@
 // of the cut, 2 (k + 1) per cell of its length where whole cells to the reach
 // of the couplings would be 2 (k + 1)^2; for the multipliers the cut's own
 // faces, k where an owner cell holds 2 k.  The dense blocks of the large
-// separators shrink with the square: refinement 8, k = 2 stores 135 M entries
-// per Schur factor with leaves of 16 cells instead of 645 M.
+// separators shrink with the square: refinement 8, k = 2 stores 112 M entries
+// per Schur factor (leaves of 4 cells, levels merged) instead of 645 M.
 //
 // Adjacent tree levels are then merged where a launch costs more than the
 // entries the merge adds (merge_levels): each node of the merged range absorbs
