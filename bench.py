@@ -21,7 +21,7 @@ state vectors falls to 1e-8 (the reference has no criterion of its own),
 on the measured workload and, beside the CPU restatement, on the small
 workload (refinement 4, k = 1, dt = 1e-3).
 
-batched: an I-V sweep of 16 applied biases on the measured mesh stepped
+batched: an I-V sweep of 64 applied biases on the measured mesh stepped
 together (one read of each factor per sweep for all of them, FP64 MFMA):
 aggregate step throughput and time to steady state per bias point.
 
